@@ -46,16 +46,16 @@ struct Level {
   float* uf = nullptr;               // FP32 copies for mixed smoothing
   float* bf = nullptr;
   int8_t* bc = nullptr;              // (n1+3)(n2+3)
-  // multi-block levels: rotating states (index 0 is u or uf) and the
-  // residual partial sums of the sweep kernels (kRing slots x blocks)
+  // multi-block levels: FP64 rotating states (index 0 is u) and the residual
+  // partial sums of the sweep kernels (kRing slots x blocks); mixed the
+  // states after the down visit (index 0, uf) and the up visit (index 1)
   bool mb = false;
   bool small_tiles = false;          // multi-block sweeps on 32-wide tiles
   void* rot[kRot] = {};
   int nbx = 0, nby = 0;
   double* partials = nullptr;
   // FP64: sweeps of the first launch of the level's down and up visits, one
-  // more than each visit took in the previous V-cycle; mixed: the visits'
-  // fixed sweep counts
+  // more than each visit took in the previous V-cycle
   int first_dn = kSweepsPerLaunch, first_up = kSweepsPerLaunch;
 };
 
@@ -174,7 +174,6 @@ struct lepic_ctx {
   int32_t mg_epoch = 0;              // epoch of the last multi-block level visit
   lepic::LevelCtrl* d_ctrl = nullptr;   // [kMaxLevels+1]
   double* d_partials = nullptr;      // FP64 residual partial sums of the finest level
-  void* d_erot = nullptr;            // mixed: device array of the level-1 FP32 correction buffers
   int64_t partials_cap = 0;
   double* d_scalar = nullptr;        // small scratch (res0 etc.)
   double* h_pinned = nullptr;        // pinned host scratch (kPinnedDoubles)

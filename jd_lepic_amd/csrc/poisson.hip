@@ -5,7 +5,7 @@
 // A kernel launch costs about 3 us on MI355X whatever it does, and a grid-wide
 // software barrier costs more, so the solver is organised to launch few
 // kernels and to need no grid synchronisation:
-//  * Fine ("multi-block") levels run k_sweeps: each block owns a 64-wide tile,
+//  * FP64 fine ("multi-block") levels run k_sweeps: each block owns a 64-wide tile,
 //    stages the tile plus a halo of 2S+1 nodes in LDS and performs S red-black
 //    sweeps on it, recomputing the halo redundantly instead of exchanging it.
 //    After every sweep it writes the tile to that sweep's state buffer (S+1
@@ -15,16 +15,19 @@
 //    from the same partial sums in the same order, so all blocks agree and no
 //    atomics or host round trips are needed.  A visit with the reference's
 //    limit of 10 sweeps takes two launches.
-//  * Coarse levels (at most mg_tail_nodes nodes) run in k_tail, one workgroup
-//    of 1024 threads that performs the whole lower part of the V-cycle (down
-//    sweeps, restrictions, the coarsest solve, prolongations and up sweeps),
-//    with the levels that fit in its LDS (up to 158 KB) held there.
-//  * Grid transfers between multi-block levels: FP64 runs them as kernels
-//    between the visits (k_restrict, LDS-tiled; k_prolong).  In mixed mode a
-//    down visit's last sweep launch computes the restriction of its tile from
-//    the region still in LDS (one node of extra halo), and an up visit's
-//    first launch adds the prolonged coarse correction to its region as it
-//    loads it.
+//  * Coarse levels (at most mg_tail_nodes nodes) run in one workgroup that
+//    performs the whole lower part of the V-cycle (down sweeps, restrictions,
+//    the coarsest solve, prolongations and up sweeps), with the levels that
+//    fit in its LDS (up to 158 KB) held there: k_tail (FP64; the mixed form
+//    where a level is too wide for strips) and k_tail32 (mixed).
+//  * Grid transfers between FP64 multi-block levels are kernels between the
+//    visits (k_restrict, LDS-tiled; k_prolong).
+//  * Mixed mode runs each visit of a multi-block level in one launch of
+//    k_tile32 (mg_strip.h): the sweeps of a fixed count on register strips,
+//    with the prolongation on load, the restriction after the last sweep, and
+//    on the finest level the correction added to phi.  The sweep counts and
+//    so every buffer are known at launch, nothing is read back but the
+//    V-cycle's FP64 residual.
 // FP64 mode computes the reference's expressions in their order (no
 // contraction), so a sweep is bit-identical to sors.f90; only the order of
 // the L1 residual sum differs.  Mixed mode runs the same V-cycle in FP32 on
@@ -39,8 +42,10 @@
 #include <vector>
 
 #include "lepic_internal.h"
+#include "mg_strip.h"
 
 using namespace lepic;
+using namespace lepic_mg;
 
 namespace {
 
@@ -78,12 +83,13 @@ constexpr int kFixDn = kNr, kFixUp = 2;
 constexpr int kWaveNodes = 320;               // tail levels with at most this many interior nodes run in one wave
 constexpr int kRowBlocks = 1024;              // row-loop blocks of the grid-transfer kernels (one row each up to 1024 rows)
 
-template <typename T> struct TileY;
-template <> struct TileY<float> { static constexpr int v = 32; };
-template <> struct TileY<double> { static constexpr int v = 16; };
-template <typename T> struct SmallTileY;
-template <> struct SmallTileY<float> { static constexpr int v = 16; };
-template <> struct SmallTileY<double> { static constexpr int v = 8; };
+constexpr int kTileY = 16, kSmallTileY = 8;
+// mixed form: a visit's sweeps run in one launch of k_tile32 unless its tiles,
+// small behind a deep halo (84 x 20 nodes for 10 sweeps and the restriction),
+// then need more than two blocks per CU; two launches of 5 sweeps cost one
+// more load and launch (about 5 us) but sweep 1.8 instead of 4.9 times the
+// tiles' nodes
+constexpr int kTileMaxBlocks = 512;
 
 // ---- SOR update of one node (sors.f90:108-110 / 238-240) ----
 // FP64 divides like the reference; the FP32 smoother of the mixed form
@@ -110,13 +116,6 @@ __device__ __forceinline__ T getres(PU u, PB b, int ir, int jr, int n1, T aw, T 
   T uij = u[c], un = u[c + W], us = u[c - W], ue = u[c + 1], uw = u[c - 1];
   T urhs = b[(int64_t)(jr - 1) * (n1 + 1) + (ir - 1)];
   return urhs - (aw * uw + aw * ue + an * un + an * us + ac * uij);
-}
-
-// getres of the node at index x of an LDS region with rows of RW (same
-// expression and order)
-template <typename T>
-__device__ __forceinline__ T lds_getres(const T* su, const T* sb, int x, int RW, T aw, T an, T ac) {
-  return sb[x] - (aw * su[x - 1] + aw * su[x + 1] + an * su[x + RW] + an * su[x - RW] + ac * su[x]);
 }
 
 // mg.f90:386-414: the weighted sum of the centre residual g9 and the eight
@@ -174,24 +173,6 @@ __device__ __forceinline__ void prolong_node(PU u, PC bc, int n1, PE e2h, int m1
   if (bc[c - 1] <= 0) u[c - 1] = u[c - 1] + (r1 + r4) / (T)2.0;
 }
 
-// The correction prolong_node adds to fine node (I, J) (1..n1+1, 1..n2+1):
-// the coarse node (I/2 + 1, J/2 + 1) and its west / south neighbours, with
-// prolong_node's expressions.
-template <typename T>
-__device__ __forceinline__ T prolong_at(const T* e2h, int m1, int I, int J) {
-  const int64_t Wc = m1 + 3;
-  const int ci = I / 2 + 1, cj = J / 2 + 1;
-  const T r1 = e2h[(int64_t)cj * Wc + ci];
-  if (I & 1) {
-    if (J & 1) return r1;
-    return (r1 + e2h[(int64_t)(cj - 1) * Wc + ci]) / (T)2.0;
-  }
-  const T r4 = e2h[(int64_t)cj * Wc + ci - 1];
-  if (J & 1) return (r1 + r4) / (T)2.0;
-  const T r2 = e2h[(int64_t)(cj - 1) * Wc + ci], r3 = e2h[(int64_t)(cj - 1) * Wc + ci - 1];
-  return (r1 + r2 + r3 + r4) / (T)4.0;
-}
-
 // ---------------------------------------------------------------------------
 // visit control of multi-block levels
 // ---------------------------------------------------------------------------
@@ -203,7 +184,6 @@ struct VisitRef {
   double eps;
   int nexec;               // sweeps launched in the visit
   int klast0;              // sweeps before the visit's last launch
-  int fixed;               // the visit runs exactly nexec sweeps (mixed form)
   int* visit;
   double* vres;
 };
@@ -263,14 +243,6 @@ __device__ Resolved resolve_visit(const VisitRef& V, bool writer, bool canon) {
   LevelCtrl* c = V.ctrl;
   const int c0 = c->cur[(V.epoch - 1) & 1];
   Resolved out{0, -1, 0.0};
-  if (V.fixed) {
-    // exactly nexec sweeps ran and the state after them is the result (the
-    // host logs the count)
-    out.ks = V.nexec;
-    out.buf = (c0 + V.nexec) % kRot;
-    if (writer && threadIdx.x == 0) c->cur[V.epoch & 1] = canon ? 0 : out.buf;
-    return out;
-  }
   if (c->done_epoch == V.epoch) {
     out.ks = c->ksor;
     out.res = c->res;
@@ -300,31 +272,15 @@ struct SweepArgs {
   double* partials;
   int nbx, nby;
   int epoch, dig, nr;
-  int fixed;               // run the launch's sweeps without the exit test (mixed form)
-  int nores;               // no residuals (a visit whose sweep count nothing reads back): only the last state is written
   double eps;
-  // mixed form, first launch of an up visit: the coarse level's correction
-  // is added to the region as it is loaded (the prolongation of
-  // mg.f90:585-611, no kernel of its own); pcrot / pvc as in k_prolong
-  int pro, pro_mb, pm1;
-  T* pcrot[kRot];
-  VisitRef pvc;
-  // mixed form, last launch of a down visit: the restriction onto the level
-  // below (k_restrict's work, from the final state in LDS; the launch's halo
-  // is one sweep wider than its sweeps need) and the fine visit's record
-  int rst;
-  T* r2h;
-  const int8_t* bc2h;
-  T* rcrot[kRot];
-  LevelCtrl* rcctrl;       // null when the coarse level runs in k_tail
 };
 
 // Sweeps k0+1 .. k0+kexec (kexec <= KS) of a visit on one TX x TY tile with
 // NT threads (see the file comment).  A launch that continues a visit first
 // takes the reference's exit test for the sweeps of the visit's previous
 // launch, kchk .. k0.
-template <typename T, int kTX, int TY, int kSweepThreads, int KS, bool RST = false>
-__global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs<T> A, int k0, int kexec, int kchk) {
+template <typename T, int kTX, int TY, int kSweepThreads, int KS>
+__global__ __launch_bounds__(kSweepThreads) void k_sweeps(SweepArgs<T> A, int k0, int kexec, int kchk) {
   constexpr int kHalo = Halo<KS>::v;
   // a block's tile is kTX x TY nodes, or one node wider (taller) in the last
   // column (row) of tiles when the level's node count leaves one node over
@@ -336,23 +292,15 @@ __global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs
   __shared__ T su[RN];
   __shared__ T sb[RN];
   __shared__ int8_t sbc[RN];
-  __shared__ int s_go, s_c0, s_pb, s_rb;
+  __shared__ int s_go, s_c0;
   __shared__ double ws[kSweepThreads / 64];
   const int nb = A.nbx * A.nby;
   const int bid = blockIdx.y * A.nbx + blockIdx.x;
-  const bool pro = A.pro && k0 == 0;
   if (threadIdx.x < 64) {
     LevelCtrl* c = A.ctrl;
     int go = 1;
-    int pb = 0;
-    if (pro && A.pro_mb) {  // the coarse level's up visit, as k_prolong resolves it
-      Resolved r = resolve_visit(A.pvc, bid == 0, false);
-      pb = r.buf < 0 ? 0 : r.buf;
-    }
     const int c0 = c->cur[(A.epoch - 1) & 1];
-    if (A.fixed) {
-      go = 1;
-    } else if (__hip_atomic_load(&c->done_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == A.epoch) {
+    if (__hip_atomic_load(&c->done_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == A.epoch) {
       go = 0;
     } else if (k0 > 0) {
       double r = 0.0;
@@ -369,8 +317,6 @@ __global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs
     if (threadIdx.x == 0) {
       s_go = go;
       s_c0 = c0;
-      s_pb = pb;
-      s_rb = (A.rst && A.rcctrl) ? A.rcctrl->cur[(A.epoch - 1) & 1] : 0;   // k_restrict's coarse buffer
     }
   }
   __syncthreads();
@@ -383,12 +329,11 @@ __global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs
   const int gi0 = 1 + (int)blockIdx.x * kTX - kHalo;  // global i of region column 0
   const int gj0 = 1 + (int)blockIdx.y * TY - kHalo;
   const T* uin = A.rot[(s_c0 + k0) % kRot];
-  const T* e2h = pro ? A.pcrot[s_pb] : nullptr;
   {
     // every load of the region is issued before any LDS store: one memory
     // latency for the whole region instead of one per loop trip
     constexpr int kIt = (RN + kSweepThreads - 1) / kSweepThreads;
-    T lu[kIt], lb[kIt], lp[kIt];
+    T lu[kIt], lb[kIt];
     int8_t lc[kIt];
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
@@ -399,12 +344,10 @@ __global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs
       lu[it] = in ? uin[(int64_t)j * W + i] : (T)0;
       lc[it] = in ? A.bc[(int64_t)j * W + i] : (int8_t)1;
       lb[it] = in ? A.b[(int64_t)(j - 1) * (n1 + 1) + (i - 1)] : (T)0;
-      lp[it] = e2h ? prolong_at<T>(e2h, A.pm1, in ? i : 1, in ? j : 1) : (T)0;
     }
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
       const int q = threadIdx.x + it * kSweepThreads;
-      if (e2h && lc[it] <= 0) lu[it] = lu[it] + lp[it];   // prolong_node: bcnd <= 0 nodes
       if (q < RN) { su[q] = lu[it]; sbc[q] = lc[it]; sb[q] = lb[it]; }
     }
   }
@@ -438,15 +381,6 @@ __global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs
       __syncthreads();
     }
     T* uout = A.rot[(s_c0 + k0 + s) % kRot];
-    if (A.nores) {
-      if (s == kexec)
-        for (int q = threadIdx.x; q < kTP * kTYP; q += kSweepThreads) {
-          const int tr = q / kTP, tc = q - tr * kTP;
-          if (tc < tw && tr < th)
-            uout[(int64_t)(gj0 + kHalo + tr) * W + gi0 + kHalo + tc] = su[(kHalo + tr) * RW + kHalo + tc];
-        }
-      continue;
-    }
     double rr = 0.0;
     for (int q0 = threadIdx.x; q0 < kTP * kTYP; q0 += NB * kSweepThreads) {
       int x[NB], gi[NB], gj[NB];
@@ -477,55 +411,6 @@ __global__ __launch_bounds__(kSweepThreads, RST ? 8 : 1) void k_sweeps(SweepArgs
     if (threadIdx.x < 64) {  // fixed-order sum of the 16 wave sums
       const double t = wave_sum(threadIdx.x < kSweepThreads / 64 ? ws[threadIdx.x] : 0.0);
       if (threadIdx.x == 0) A.partials[(size_t)((k0 + s) % kRing) * nb + bid] = t;
-    }
-  }
-  if (RST && A.rst) {  // the last colour pass ended with a barrier
-    // the fine visit's record (resolve_visit of a fixed-length visit)
-    if (bid == 0 && threadIdx.x == 0) A.ctrl->cur[A.epoch & 1] = (s_c0 + k0 + kexec) % kRot;
-    // the coarse nodes whose fine centre (2ci-1, 2cj-1) lies in this tile,
-    // plus the coarse border next to the domain's edge for the zeroing
-    const int m1 = n1 / 2;
-    const int ti0 = 1 + (int)blockIdx.x * kTX, tj0 = 1 + (int)blockIdx.y * TY;
-    const int ci0 = (ti0 + 1) / 2, ci1 = (ti0 + tw) / 2, cj0 = (tj0 + 1) / 2, cj1 = (tj0 + th) / 2;
-    const int zi0 = ci0 - (blockIdx.x == 0), zi1 = ci1 + ((int)blockIdx.x == A.nbx - 1);
-    const int zj0 = cj0 - (blockIdx.y == 0), zj1 = cj1 + ((int)blockIdx.y == A.nby - 1);
-    const int zw = zi1 - zi0 + 1, zn = zw * (zj1 - zj0 + 1);
-    T* e2h = A.rcrot[0];  // selected without a dynamic index into the argument
-#pragma unroll
-    for (int r = 1; r < kRot; ++r) e2h = s_rb == r ? A.rcrot[r] : e2h;
-    const int64_t Wc = m1 + 3;
-    for (int q = threadIdx.x; q < zn; q += kSweepThreads) {
-      const int ci = zi0 + q % zw, cj = zj0 + q / zw;
-      e2h[(int64_t)cj * Wc + ci] = (T)0;
-      if (ci < ci0 || ci > ci1 || cj < cj0 || cj > cj1) continue;
-      T out = (T)0;
-      if (A.bc2h[(int64_t)cj * Wc + ci] <= 0) {
-        const int ir = 2 * ci - 1, jr = 2 * cj - 1;
-        // region index of fine node (ir + dx, jr + dy), unclamped (bc flags)
-        // and clamped into the interior (getres, as restrict_node evaluates it)
-        const int xr = (jr - gj0) * RW + (ir - gi0);
-        const int dxe = ir + 1 <= n1 + 1 ? 1 : 0, dxw = ir - 1 >= 1 ? -1 : 0;
-        const int dyn = jr + 1 <= n2 + 1 ? RW : 0, dys = jr - 1 >= 1 ? -RW : 0;
-        const bool xe = ir != n1 + 1, xw = ir != 1, yn = jr != n2 + 1, ys = jr != 1;
-        const bool f1 = xe && yn && sbc[xr + 1 + RW] <= 0;
-        const bool f2 = xe && sbc[xr + 1] <= 0;
-        const bool f3 = sbc[xr + 1 - RW] <= 0 && xe && ys;
-        const bool f4 = sbc[xr - RW] <= 0 && ys;
-        const bool f5 = sbc[xr - 1 - RW] <= 0 && xw && ys;
-        const bool f6 = sbc[xr - 1] <= 0 && xw;
-        const bool f7 = sbc[xr - 1 + RW] <= 0 && xw && yn;
-        const bool f8 = sbc[xr + RW] <= 0 && yn;
-        out = full_weight<T>(lds_getres<T>(su, sb, xr, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dxe + dyn, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dxe, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dxe + dys, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dys, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dxw + dys, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dxw, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dxw + dyn, RW, aw, an, ac),
-                             lds_getres<T>(su, sb, xr + dyn, RW, aw, an, ac), f1, f2, f3, f4, f5, f6, f7, f8);
-      }
-      A.r2h[(int64_t)(cj - 1) * (m1 + 1) + (ci - 1)] = out;
     }
   }
 }
@@ -697,54 +582,23 @@ __global__ __launch_bounds__(256) void k_finish64(Finish64Args A) {
       A.rot[0][(int64_t)j * W + i] = A.rot[s_buf][(int64_t)j * W + i];
 }
 
-// Mixed mode, end of a V-cycle: phi += e (bcnd <= 0 nodes) with the FP32
-// correction of the up visit, which is then zeroed for the next V-cycle.
-struct AddCorrArgs {
-  double* phi;
-  float* rot[kRot];
-  const int8_t* bc;
-  int n1, n2;
-  int mb;
-  VisitRef v;
-};
-
-__global__ __launch_bounds__(256) void k_add_corr(AddCorrArgs A) {
-  __shared__ int s_buf;
-  if (threadIdx.x < 64) {
-    int buf = 0;
-    if (A.mb) {
-      const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-      Resolved r = resolve_visit(A.v, writer, false);
-      buf = r.buf < 0 ? 0 : r.buf;
-    }
-    if (threadIdx.x == 0) s_buf = buf;
-  }
-  __syncthreads();
-  float* e = A.rot[s_buf];
-  const int64_t W = A.n1 + 3;
-  for (int j = blockIdx.y + 1; j <= A.n2 + 1; j += gridDim.y)
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x + 1; i <= A.n1 + 1; i += gridDim.x * blockDim.x) {
-      const int64_t q = (int64_t)j * W + i;
-      if (A.bc[q] <= 0) A.phi[q] = A.phi[q] + (double)e[q];
-      e[q] = 0.0f;
-    }
+// Mixed mode with the finest level in k_tail: phi += e (bcnd <= 0 nodes) at
+// the end of a V-cycle (otherwise the last up visit adds its own state).
+__global__ __launch_bounds__(256) void k_add_corr(double* __restrict__ phi, const float* __restrict__ e,
+                                                  const int8_t* __restrict__ bc, int64_t n) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n && bc[q] <= 0) phi[q] = phi[q] + (double)e[q];
 }
 
 // FP64 L1 residual of phi on the finest level (the reference's definition,
 // sors.f90:348-349 order); in mixed mode it also becomes the FP32 right-hand
 // side of the next correction equation.  One partial sum per block; blocks
-// walk rows j = blockIdx.x + 1 + m*gridDim.x.  erot also clears the level-1
-// FP32 correction buffer the next visit starts from.
+// walk rows j = blockIdx.x + 1 + m*gridDim.x.
 __global__ __launch_bounds__(256) void k_resid64(const double* __restrict__ u, const double* __restrict__ b,
                                                  const int8_t* __restrict__ bc, int n1, int n2, double aw,
                                                  double an, double ac, float* __restrict__ bf,
-                                                 float* const* __restrict__ erot, const LevelCtrl* ctrl,
-                                                 int epoch_next, double* __restrict__ partials) {
+                                                 double* __restrict__ partials) {
   __shared__ double ws[4];
-  __shared__ int s_zb;
-  if (threadIdx.x == 0) s_zb = erot ? (ctrl ? ctrl->cur[(epoch_next - 1) & 1] : 0) : -1;
-  __syncthreads();
-  float* ez = s_zb >= 0 ? erot[s_zb] : nullptr;
   const int64_t W = n1 + 3;
   double r = 0.0;
   for (int j = blockIdx.x + 1; j <= n2 + 1; j += gridDim.x) {
@@ -755,7 +609,6 @@ __global__ __launch_bounds__(256) void k_resid64(const double* __restrict__ u, c
       if (bc[c] == -1)
         rij = b[q] - (aw * u[c - 1] + an * u[c + W] + an * u[c - W] + aw * u[c + 1] + ac * u[c]);
       if (bf) bf[q] = (float)rij;
-      if (ez) ez[c] = 0.0f;
       r += fabs(rij);
     }
   }
@@ -1276,6 +1129,101 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs<T> A) {
   if (L.lds) copy_l2g(L.gu, smem + L.ou, (L.n1 + 3) * (L.n2 + 3) * (int)sizeof(T));
 }
 
+// The same work for the mixed form, on register strips (mg_strip.h; 28 us a
+// launch at 65^2 nodes and below against 60 us for k_tail, of 65e3 cycles:
+// load 4e3, down visits 13e3 (65^2), 9e3 (33^2), 6.2-6.9e3 each below, up
+// visits 2.5-5.2e3; a pass costs about 225 cycles in one wave, most of them
+// the LDS exchange): every
+// level above the coarsest runs its fixed sweeps from registers, its arrays in
+// LDS between the visits.  Levels whose strips fit one wave run in wave 0
+// without block barriers.  The coarsest level keeps the exit test of
+// sors.f90:371-377 on the arrays in LDS.
+struct Tail32Level {
+  StripLevel s;
+  int two;                     // strips of 2 rows (else 4); always in wave 0
+  uint32_t ou, ob, obc;        // LDS offsets of the correction, right-hand side and bc arrays
+};
+
+struct Tail32Args {
+  int Ls, ng, k;
+  int Lw;                      // levels Ls .. Lw-1 by the whole block, Lw .. ng-1 by wave 0
+  int cw;                      // the coarsest level by wave 0
+  int fix_dn, fix_up;
+  double eps;
+  const int8_t* bc_img;
+  int bc_bytes;
+  uint32_t u_begin, u_end, oed;
+  const float* gb;             // level Ls: right-hand side, and where its correction goes
+  float* gu;
+  double* phi;                 // not null when Ls is the finest level
+  float omega, caw, can, cac;  // coarsest level
+  int* visit;
+  double* vres;
+  Tail32Level lv[kMaxLevels + 1];
+};
+
+template <bool ISO>
+__global__ __launch_bounds__(kTailThreads) void k_tail32(Tail32Args A) {
+  extern __shared__ __align__(16) char smem[];
+  __shared__ double ws[32];
+  const int Ls = A.Ls, ng = A.ng, tid = threadIdx.x;
+  auto U = [&](int l) { return (float*)(smem + A.lv[l].ou); };
+  auto B = [&](int l) { return (float*)(smem + A.lv[l].ob); };
+  auto M = [&](int l) { return (const int8_t*)(smem + A.lv[l].obc); };
+  float* ed = (float*)(smem + A.oed);
+  {
+    const StripLevel& L = A.lv[Ls].s;
+    copy3_g2l(smem, A.bc_img, A.bc_bytes, smem + A.lv[Ls].ob, A.gb, (L.n1 + 1) * (L.n2 + 1) * 4, smem, A.bc_img, 0);
+  }
+  for (uint32_t q = A.u_begin + 16u * tid; q < A.u_end; q += 16u * blockDim.x)
+    *(float4*)(smem + q) = make_float4(0.f, 0.f, 0.f, 0.f);
+  __syncthreads();
+  int ks = 0;
+  double res = 0.0;
+  TLevel<float> C;
+  C.n1 = A.lv[ng].s.n1; C.n2 = A.lv[ng].s.n2;
+  C.aw = A.caw; C.an = A.can; C.ac = A.cac;
+  C.gu = nullptr; C.gb = nullptr; C.gbc = nullptr;
+  C.lds = 1;
+  C.ou = C.ob = C.obc = 0;
+  const int nr = A.k == 1 ? 1000000 : kNr;
+  for (int l = Ls; l < A.Lw; ++l) {
+    const Tail32Level& L = A.lv[l];
+    if (L.two) strip_down<2, ISO, false>(L.s, L.s.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
+    else strip_down<4, ISO, false>(L.s, L.s.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
+    if (tid == 0) A.visit[l] = A.fix_dn;
+  }
+  if (A.cw) {
+    if (tid < 64) {
+      for (int l = A.Lw; l < ng; ++l) {
+        const Tail32Level& L = A.lv[l];
+        strip_down<2, ISO, true>(L.s, L.s.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
+        if (tid == 0) A.visit[l] = A.fix_dn;
+      }
+      smooth_level<float, true>(C, U(ng), B(ng), M(ng), A.omega, A.eps, 0, nr, ws, &ks, &res);
+      if (tid == 0) { A.visit[ng] = ks; A.vres[ng] = res; }
+      for (int l = ng - 1; l >= A.Lw; --l) {
+        const Tail32Level& L = A.lv[l];
+        strip_up<2, ISO, true>(L.s, L.s.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), l == Ls ? A.gu : nullptr,
+                               l == Ls ? A.phi : nullptr);
+        if (tid == 0) A.visit[2 * ng - l] = A.fix_up;
+      }
+    }
+  } else {                     // Lw == ng
+    smooth_level<float>(C, U(ng), B(ng), M(ng), A.omega, A.eps, 0, nr, ws, &ks, &res);
+    if (tid == 0) { A.visit[ng] = ks; A.vres[ng] = res; }
+  }
+  __syncthreads();
+  for (int l = A.Lw - 1; l >= Ls; --l) {
+    const Tail32Level& L = A.lv[l];
+    float* gu = l == Ls ? A.gu : nullptr;
+    double* phi = l == Ls ? A.phi : nullptr;
+    if (L.two) strip_up<2, ISO, false>(L.s, L.s.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), gu, phi);
+    else strip_up<4, ISO, false>(L.s, L.s.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), gu, phi);
+    if (tid == 0) A.visit[2 * ng - l] = A.fix_up;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1293,7 +1241,7 @@ double* d_vres_of(lepic_ctx* ctx) { return ctx->d_scalar + 32; }
 int* d_status_of(lepic_ctx* ctx) { return (int*)(ctx->d_scalar + 64) + kVisitLog; }
 
 VisitRef visit_ref(lepic_ctx* ctx, int l, int epoch, int dig, int nr, int ig, double eps, int nexec,
-                   int klast0 = -1, int fixed = 0) {
+                   int klast0 = -1) {
   Level& L = ctx->lv[l];
   VisitRef v;
   v.ctrl = ctx->d_ctrl + l;
@@ -1302,7 +1250,6 @@ VisitRef visit_ref(lepic_ctx* ctx, int l, int epoch, int dig, int nr, int ig, do
   v.epoch = epoch; v.dig = dig; v.nr = nr; v.ig = ig; v.eps = eps;
   v.nexec = nexec;
   v.klast0 = klast0 >= 0 ? klast0 : ((nexec - 1) / kS) * kS;
-  v.fixed = fixed;
   v.visit = d_visit_of(ctx);
   v.vres = d_vres_of(ctx);
   return v;
@@ -1319,107 +1266,135 @@ int last_launch_start(int k0, int k_end, int first) {
   return last;
 }
 
-// How a multi-block level's visit runs.  FP64: the reference's exit test
+// How a multi-block level's FP64 visit runs: the reference's exit test
 // (sors.f90:371-377) decides, the first launch `first` sweeps and
-// continuations up to kNr.  Mixed: the visit runs its fixed count
-// (kFineDn / kFineUp on the finest level, kFixDn / kFixUp below) and no
-// continuation launch tests anything.
+// continuations up to kNr.
 struct VisitPlan {
-  int k_end, first, klast0, fixed;
+  int k_end, first, klast0;
 };
 
-VisitPlan visit_plan(const Level& L, bool up, bool f32) {
+VisitPlan visit_plan(const Level& L, bool up) {
   const int f = up ? L.first_up : L.first_dn;
-  if (!f32) return VisitPlan{kNr, f, last_launch_start(0, kNr, f), 0};
-  const int first = std::min(f, kS);
-  return VisitPlan{f, first, last_launch_start(0, f, first), 1};
+  return VisitPlan{kNr, f, last_launch_start(0, kNr, f)};
 }
 
-// the launch size KS (halo 2 KS + 1) is kexec, or kexec + 1 for a launch
-// that restricts (its full weighting reads the state two nodes past the tile)
-template <typename T, int kTX, int TY, int NT>
-void launch_sweeps(lepic_ctx* ctx, const Level& L, const SweepArgs<T>& A, int k, int kexec, int kchk) {
+// the launch size KS (halo 2 KS + 1) is kexec
+template <int kTX, int TY, int NT>
+void launch_sweeps(lepic_ctx* ctx, const Level& L, const SweepArgs<double>& A, int k, int kexec, int kchk) {
   const dim3 g(L.nbx, L.nby);
-  if (A.rst) {
-    // mixed form only: FP64 restricts in its own kernel
-    if constexpr (sizeof(T) == 4) {
-      const int ks = kexec + 1;
-      if (ks <= 3) hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, 3, true>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-      else if (ks <= 4) hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, 4, true>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-      else if (ks <= kS) hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, kS, true>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-      else hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, kS + 1, true>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-    }
-    return;
-  }
-  if (kexec <= 2) hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, 2>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-  else if (kexec <= 3) hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, 3>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-  else if (kexec <= 4) hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, 4>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-  else hipLaunchKernelGGL((k_sweeps<T, kTX, TY, NT, kS>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
+  if (kexec <= 2) hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, 2>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
+  else if (kexec <= 3) hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, 3>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
+  else if (kexec <= 4) hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, 4>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
+  else hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, kS>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
 }
 
-// launches of one visit of a multi-block level: sweeps k0+1 .. k_end, the
+// launches of one FP64 visit of a multi-block level: sweeps k0+1 .. k_end, the
 // first launch `first` sweeps (one more than the same visit took in the
 // previous V-cycle: most visits then finish in one launch of a small
 // halo), the others kS; each continuation first tests the previous launch's
 // sweeps and returns at once when the visit has stopped there
-template <typename T>
-int launch_visit(lepic_ctx* ctx, int l, bool f32, int epoch, int dig, int nr, double eps, int k0, int k_end,
-                 int first = kS, int fixed = 0, bool pro = false, bool rst = false) {
+int launch_visit(lepic_ctx* ctx, int l, int epoch, int dig, int nr, double eps, int k0, int k_end, int first = kS) {
   Level& L = ctx->lv[l];
-  SweepArgs<T> A;
-  A.rst = 0;
-  if (rst) {  // the down visit's last launch restricts onto level l + 1
-    Level& C = ctx->lv[l + 1];
-    A.r2h = b_of<T>(C, f32);
-    A.bc2h = C.bc;
-    for (int r = 0; r < kRot; ++r) A.rcrot[r] = C.mb ? rot_of<T>(C, r) : u_of<T>(C, f32);
-    A.rcctrl = C.mb ? ctx->d_ctrl + (l + 1) : nullptr;
-  } else {
-    A.r2h = nullptr;
-    A.bc2h = nullptr;
-    for (int r = 0; r < kRot; ++r) A.rcrot[r] = nullptr;
-    A.rcctrl = nullptr;
-  }
-  A.pro = pro ? 1 : 0;
-  A.pro_mb = 0;
-  A.pm1 = L.n1 / 2;
-  A.pvc = VisitRef{};
-  if (pro) {  // the up visit's first launch takes the prolongation from level l + 1
-    Level& C = ctx->lv[l + 1];
-    for (int r = 0; r < kRot; ++r) A.pcrot[r] = C.mb ? rot_of<T>(C, r) : u_of<T>(C, f32);
-    A.pro_mb = C.mb ? 1 : 0;
-    if (C.mb) {
-      const VisitPlan pc = visit_plan(C, true, f32);
-      A.pvc = visit_ref(ctx, l + 1, epoch, ctx->ng - (l + 1), kNr, 2 * ctx->ng - (l + 1), eps, pc.k_end, pc.klast0,
-                        pc.fixed);
-    }
-  } else {
-    for (int r = 0; r < kRot; ++r) A.pcrot[r] = nullptr;
-  }
-  for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<T>(L, r);
-  A.b = b_of<T>(L, f32);
+  SweepArgs<double> A;
+  for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<double>(L, r);
+  A.b = L.b;
   A.bc = L.bc;
   A.n1 = L.n1; A.n2 = L.n2;
-  A.aw = (T)L.aw; A.an = (T)L.an; A.ac = (T)L.ac;
-  A.omega = (f32 && l == 1) ? (T)kFineOmega : (T)1.4;   // iterative_solver.f90:27
+  A.aw = L.aw; A.an = L.an; A.ac = L.ac;
+  A.omega = 1.4;                                  // iterative_solver.f90:27
   A.ctrl = ctx->d_ctrl + l;
   A.partials = L.partials;
   A.nbx = L.nbx; A.nby = L.nby;
   A.epoch = epoch; A.dig = dig; A.nr = nr; A.eps = eps;
-  A.fixed = fixed;
-  // the mixed form's visits run fixed counts: their residuals feed nothing
-  A.nores = (f32 && fixed) ? 1 : 0;
   int kchk = 0;
   for (int k = k0, size = std::min(std::max(first, 1), kS); k < k_end; size = kS) {
     const int kexec = std::min(size, k_end - k);
-    A.rst = (rst && k + kexec == k_end) ? 1 : 0;
-    if (L.small_tiles) launch_sweeps<T, kSmallTX, SmallTileY<T>::v, kSmallThreads>(ctx, L, A, k, kexec, kchk);
-    else launch_sweeps<T, kTX, TileY<T>::v, kSweepThreads>(ctx, L, A, k, kexec, kchk);
+    if (L.small_tiles) launch_sweeps<kSmallTX, kSmallTileY, kSmallThreads>(ctx, L, A, k, kexec, kchk);
+    else launch_sweeps<kTX, kTileY, kSweepThreads>(ctx, L, A, k, kexec, kchk);
     kchk = k + 1;
     k += kexec;
   }
   LEPIC_HIP(hipGetLastError());
   return 0;
+}
+
+// ---- mixed form: visits of fixed sweep counts in k_tile32 ----
+StripCoef strip_coef(const Level& L, float omega) {
+  StripCoef k;
+  k.aw = (float)L.aw; k.an = (float)L.an; k.ac = (float)L.ac;
+  k.om = omega; k.om1 = 1.0f - omega; k.rac = 1.0f / k.ac;
+  return k;
+}
+
+bool strip_iso(const Level& L) { return (float)L.aw == (float)L.an; }
+
+// One launch of nsw sweeps.  Bound by VALU issue (eleven instructions of about
+// 4.7 cycles per node and pass) behind the launch's load latency of about
+// 3 us.  Regions of 128 x 64 nodes as 16 waves x 4 rows, four waves per SIMD to
+// cover the LDS exchange (8 waves x 8 rows: 9.9, 11.9, 11.7, 11.3 us for the
+// four down visits of 1025^2 .. 129^2 against 9.2, 12.3, 10.6, 10.0); for
+// halos of at most 4 nodes 128 x 32, whose passes take half as long.  The
+// sweeps on a region in LDS that this replaces took 23.5 us for the 1025^2
+// down visit (4 sweeps) and 29.6, 20.4, 21.2 us for the 10 sweeps of the
+// others in two launches each.
+int launch_tile32(lepic_ctx* ctx, const Level& L, TileArgs A) {
+  A.halo = 2 * A.nsw + (A.r2h ? 2 : 0);
+  const int rows = A.halo <= 4 ? 32 : 64;
+  const int tx = 128 - 2 * A.halo, ty = rows - 2 * A.halo;
+  const dim3 g((unsigned)((L.n1 - 1 + tx - 1) / tx), (unsigned)((L.n2 - 1 + ty - 1) / ty));
+  if (strip_iso(L)) {
+    if (rows == 32) hipLaunchKernelGGL((k_tile32<4, 8, true>), g, dim3(512), 0, ctx->stream, A);
+    else hipLaunchKernelGGL((k_tile32<4, 16, true>), g, dim3(1024), 0, ctx->stream, A);
+  } else {
+    if (rows == 32) hipLaunchKernelGGL((k_tile32<4, 8, false>), g, dim3(512), 0, ctx->stream, A);
+    else hipLaunchKernelGGL((k_tile32<4, 16, false>), g, dim3(1024), 0, ctx->stream, A);
+  }
+  LEPIC_HIP(hipGetLastError());
+  return 0;
+}
+
+TileArgs tile_args(lepic_ctx* ctx, int l) {
+  Level& L = ctx->lv[l];
+  TileArgs A{};
+  A.b = L.bf; A.bc = L.bc; A.n1 = L.n1; A.n2 = L.n2;
+  A.k = strip_coef(L, l == 1 ? kFineOmega : 1.4f);
+  return A;
+}
+
+// down visit of level l: from zero into rot[0], the restricted residual to
+// level l + 1's right-hand side
+int tile_down(lepic_ctx* ctx, int l) {
+  Level& L = ctx->lv[l];
+  const int nsw = l == 1 ? kFineDn : kFixDn;
+  TileArgs A = tile_args(ctx, l);
+  A.u_out = rot_of<float>(L, 0);
+  const int h = 2 * nsw + 2;
+  const int64_t nb = (int64_t)((L.n1 - 1 + 127 - 2 * h) / (128 - 2 * h)) * ((L.n2 - 1 + 63 - 2 * h) / (64 - 2 * h));
+  A.nsw = nsw;
+  if (nsw > kS && nb > kTileMaxBlocks) {
+    A.nsw = kS;
+    A.u_out = rot_of<float>(L, 1);
+    if (int rc = launch_tile32(ctx, L, A)) return rc;
+    A.u_in = rot_of<float>(L, 1);
+    A.u_out = rot_of<float>(L, 0);
+    A.nsw = nsw - kS;
+  }
+  A.r2h = ctx->lv[l + 1].bf;
+  return launch_tile32(ctx, L, A);
+}
+
+// up visit: rot[0] and the prolonged correction of level l + 1 into rot[1], on
+// the finest level added to phi
+int tile_up(lepic_ctx* ctx, int l) {
+  Level& L = ctx->lv[l];
+  Level& C = ctx->lv[l + 1];
+  TileArgs A = tile_args(ctx, l);
+  A.u_in = rot_of<float>(L, 0);
+  if (l == 1) A.phi = ctx->phi;
+  else A.u_out = rot_of<float>(L, 1);
+  A.e2h = C.mb ? rot_of<float>(C, 1) : C.uf;
+  A.nsw = l == 1 ? kFineUp : kFixUp;
+  return launch_tile32(ctx, L, A);
 }
 
 template <typename T>
@@ -1428,8 +1403,8 @@ int launch_restrict(lepic_ctx* ctx, int l, bool f32, int epoch, double eps) {
   Level& F = ctx->lv[l];
   Level& C = ctx->lv[l + 1];
   RestrictArgs<T> A;
-  const VisitPlan pf = visit_plan(F, false, std::is_same<T, float>::value);
-  A.vf = visit_ref(ctx, l, epoch, l - ng, kNr, l, eps, pf.k_end, pf.klast0, pf.fixed);
+  const VisitPlan pf = visit_plan(F, false);
+  A.vf = visit_ref(ctx, l, epoch, l - ng, kNr, l, eps, pf.k_end, pf.klast0);
   for (int r = 0; r < kRot; ++r) A.frot[r] = rot_of<T>(F, r);
   A.fb = b_of<T>(F, f32);
   A.fbc = F.bc;
@@ -1461,12 +1436,135 @@ int launch_prolong(lepic_ctx* ctx, int l, bool f32, int epoch_up, double eps) {
   A.coarse_mb = C.mb ? 1 : 0;
   if (C.mb)
   {
-    const VisitPlan pc = visit_plan(C, true, std::is_same<T, float>::value);
-    A.vc = visit_ref(ctx, l + 1, epoch_up, ng - (l + 1), kNr, 2 * ng - (l + 1), eps, pc.k_end, pc.klast0, pc.fixed);
+    const VisitPlan pc = visit_plan(C, true);
+    A.vc = visit_ref(ctx, l + 1, epoch_up, ng - (l + 1), kNr, 2 * ng - (l + 1), eps, pc.k_end, pc.klast0);
   }
   else A.vc = VisitRef{};
   dim3 g((C.n1 + 1 + 127) / 128, std::min(C.n2 + 1, kRowBlocks));
   hipLaunchKernelGGL(k_prolong<T>, g, dim3(128), 0, ctx->stream, A);
+  LEPIC_HIP(hipGetLastError());
+  return 0;
+}
+
+// The bc arrays of levels ng .. Lr, coarsest first, each from a 16-byte
+// boundary: rebuilt when the boundary or the layout changes.
+int tail_bc_image(lepic_ctx* ctx, int Lr, bool f32) {
+  const int key = Lr * 2 + (f32 ? 1 : 0);
+  if (ctx->tail_bc_key == key) return 0;
+  auto bytes_of = [&](int l) { return (size_t)(ctx->lv[l].n1 + 3) * (ctx->lv[l].n2 + 3); };
+  size_t total = 0;
+  for (int l = ctx->ng; l >= Lr; --l) total = (total + bytes_of(l) + 15) & ~size_t(15);
+  if (total > ctx->tail_bc_cap) {
+    if (ctx->d_tail_bc) LEPIC_HIP(hipFree(ctx->d_tail_bc));
+    LEPIC_HIP(hipMalloc(&ctx->d_tail_bc, total));
+    ctx->tail_bc_cap = total;
+  }
+  size_t off = 0;
+  for (int l = ctx->ng; l >= Lr; --l) {
+    LEPIC_HIP(hipMemcpyAsync(ctx->d_tail_bc + off, ctx->lv[l].bc, bytes_of(l), hipMemcpyDeviceToDevice, ctx->stream));
+    off = (off + bytes_of(l) + 15) & ~size_t(15);
+  }
+  ctx->tail_bc_key = key;
+  return 0;
+}
+
+// k_tail32's layout, or false where a level above the coarsest does not fit
+// its strips (wider than 128 columns or more than 16 waves) or the LDS.
+bool tail32_plan(lepic_ctx* ctx, Tail32Args& A, size_t& lds, int& threads) {
+  if (ctx->Lc == ctx->ng) return false;   // the coarsest level alone
+  const int ng = ctx->ng, Ls = ctx->Lc;
+  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
+  A.Ls = Ls; A.ng = ng; A.Lw = ng;
+  int waves = 4;
+  size_t ed = 0;
+  for (int l = Ls; l < ng; ++l) {
+    const Level& L = ctx->lv[l];
+    Tail32Level& T = A.lv[l];
+    StripLevel& S = T.s;
+    S.n1 = L.n1; S.n2 = L.n2;
+    S.Lx = (L.n1 + 1) / 2;
+    if (S.Lx > 64) return false;
+    S.SW = 64 / S.Lx;
+    S.inv = 65536 / S.Lx + 1;
+    // strips of two rows where they fit four waves, one per SIMD; strips of
+    // four rows where a level has work for every SIMD anyway (65^2: 13e3
+    // cycles a down visit in 8 waves of 4 rows, 18e3 in 4 waves of 8)
+    T.two = ((L.n2 - 1 + 1) / 2 + S.SW - 1) / S.SW <= 4;
+    const int R = T.two ? 2 : 4;
+    S.nst = (L.n2 - 1 + R - 1) / R;
+    const int w = (S.nst + S.SW - 1) / S.SW;
+    if (w > 16) return false;
+    if (w == 1 && T.two) A.Lw = std::min(A.Lw, l);
+    else if (A.Lw < l) return false;
+    waves = std::max(waves, w);
+    S.k = strip_coef(L, 1.4f);
+    ed = std::max(ed, (size_t)4 * (S.nst + 2) * S.Lx * 4);
+  }
+  const Level& C = ctx->lv[ng];
+  A.lv[ng].s.n1 = C.n1; A.lv[ng].s.n2 = C.n2;
+  A.cw = (C.n1 + 1) * (C.n2 + 1) <= kWaveNodes ? 1 : 0;
+  if (!A.cw && A.Lw < ng) return false;
+  size_t off = 0;
+  for (int l = ng; l >= Ls; --l) {
+    A.lv[l].obc = (uint32_t)off;
+    off = al(off + (size_t)(ctx->lv[l].n1 + 3) * (ctx->lv[l].n2 + 3));
+  }
+  A.bc_bytes = (int)off;
+  A.u_begin = (uint32_t)off;
+  for (int l = ng; l >= Ls; --l) {
+    A.lv[l].ou = (uint32_t)off;
+    off = al(off + (size_t)(ctx->lv[l].n1 + 3) * (ctx->lv[l].n2 + 3) * 4);
+  }
+  A.u_end = (uint32_t)off;
+  for (int l = ng; l >= Ls; --l) {
+    A.lv[l].ob = (uint32_t)off;
+    off = al(off + (size_t)(ctx->lv[l].n1 + 1) * (ctx->lv[l].n2 + 1) * 4);
+  }
+  A.oed = (uint32_t)off;
+  lds = off + ed;
+  threads = 64 * waves;
+  return lds <= kTailLds;
+}
+
+template <typename T>
+int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps);
+
+int launch_tail32(lepic_ctx* ctx, int k, double eps) {
+  Tail32Args A{};
+  size_t lds = 0;
+  int threads = 0;
+  const Level& L = ctx->lv[ctx->Lc];
+  if (!tail32_plan(ctx, A, lds, threads)) {
+    // the generic kernel starts from the state in global memory: zero
+    const int64_t n = (int64_t)(L.n1 + 3) * (L.n2 + 3);
+    if (int rc = zero_async(ctx, L.uf, n * 4)) return rc;
+    if (int rc = launch_tail<float>(ctx, true, k, eps)) return rc;
+    if (ctx->Lc == 1) {
+      hipLaunchKernelGGL(k_add_corr, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, ctx->phi,
+                         (const float*)L.uf, (const int8_t*)ctx->bc, n);
+      LEPIC_HIP(hipGetLastError());
+    }
+    return 0;
+  }
+  if (int rc = tail_bc_image(ctx, ctx->Lc, true)) return rc;
+  A.k = k; A.eps = eps;
+  A.fix_dn = kFixDn; A.fix_up = kFixUp;
+  A.bc_img = ctx->d_tail_bc;
+  A.gb = L.bf;
+  A.gu = L.uf;
+  A.phi = ctx->Lc == 1 ? ctx->phi : nullptr;
+  const Level& C = ctx->lv[ctx->ng];
+  A.omega = 1.4f; A.caw = (float)C.aw; A.can = (float)C.an; A.cac = (float)C.ac;
+  A.visit = d_visit_of(ctx);
+  A.vres = d_vres_of(ctx);
+  static bool attr_set = false;
+  if (!attr_set) {
+    LEPIC_HIP(hipFuncSetAttribute((const void*)k_tail32<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
+    LEPIC_HIP(hipFuncSetAttribute((const void*)k_tail32<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
+    attr_set = true;
+  }
+  if (strip_iso(L)) hipLaunchKernelGGL(k_tail32<true>, dim3(1), dim3(threads), lds, ctx->stream, A);
+  else hipLaunchKernelGGL(k_tail32<false>, dim3(1), dim3(threads), lds, ctx->stream, A);
   LEPIC_HIP(hipGetLastError());
   return 0;
 }
@@ -1513,21 +1611,7 @@ int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps) {
       C.ob = (uint32_t)off; off = al(off + (size_t)(L.n1 + 1) * (L.n2 + 1) * sizeof(T));
     }
   }
-  // the bc image, rebuilt when the boundary or the layout changes
-  const int key = Lr * 2 + (f32 ? 1 : 0);
-  if (ctx->tail_bc_key != key) {
-    if (bc_bytes > ctx->tail_bc_cap) {
-      if (ctx->d_tail_bc) LEPIC_HIP(hipFree(ctx->d_tail_bc));
-      LEPIC_HIP(hipMalloc(&ctx->d_tail_bc, bc_bytes));
-      ctx->tail_bc_cap = bc_bytes;
-    }
-    for (int l = ctx->ng; l >= Lr; --l) {
-      const Level& L = ctx->lv[l];
-      LEPIC_HIP(hipMemcpyAsync(ctx->d_tail_bc + A.lv[l].obc, L.bc, (size_t)(L.n1 + 3) * (L.n2 + 3),
-                               hipMemcpyDeviceToDevice, ctx->stream));
-    }
-    ctx->tail_bc_key = key;
-  }
+  if (int rc = tail_bc_image(ctx, Lr, f32)) return rc;
   A.bc_img = ctx->d_tail_bc;
   A.bc_bytes = (int)bc_bytes;
   static bool attr_set = false;   // per instantiation; the attribute is per kernel
@@ -1541,53 +1625,46 @@ int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps) {
   return 0;
 }
 
-// One V-cycle (mg.f90:85-225) at precision T: levels 1..Ls-1 multi-block,
-// Ls..ng in k_tail; then the end-of-cycle kernel of the mode.
-template <typename T>
-int vcycle(lepic_ctx* ctx, bool f32, int k, double eps) {
+// One FP64 V-cycle (mg.f90:85-225): levels 1..Ls-1 multi-block, Ls..ng in
+// k_tail; then the end-of-cycle kernel.
+int vcycle64(lepic_ctx* ctx, int k, double eps) {
   const int ng = ctx->ng, Ls = ctx->Lc;
   const int e_dn = ctx->mg_epoch + 1, e_up = ctx->mg_epoch + 2;
   ctx->mg_epoch += 2;
   for (int l = 1; l < Ls; ++l) {  // down leg
-    // FP64: the restriction kernel; mixed: folded into the visit's last launch
-    const VisitPlan pl = visit_plan(ctx->lv[l], false, f32);
-    if (int rc = launch_visit<T>(ctx, l, f32, e_dn, l - ng, kNr, eps, 0, pl.k_end, pl.first, pl.fixed, false, f32))
-      return rc;
-    if constexpr (sizeof(T) == 8)
-      if (int rc = launch_restrict<T>(ctx, l, f32, e_dn, eps)) return rc;
+    const VisitPlan pl = visit_plan(ctx->lv[l], false);
+    if (int rc = launch_visit(ctx, l, e_dn, l - ng, kNr, eps, 0, pl.k_end, pl.first)) return rc;
+    if (int rc = launch_restrict<double>(ctx, l, false, e_dn, eps)) return rc;
   }
-  if (int rc = launch_tail<T>(ctx, f32, k, eps)) return rc;
+  if (int rc = launch_tail<double>(ctx, false, k, eps)) return rc;
   for (int l = Ls - 1; l >= 1; --l) {  // up leg
-    // FP64: the prolongation kernel; mixed: folded into the up visit's first launch
-    if constexpr (sizeof(T) == 8)
-      if (int rc = launch_prolong<T>(ctx, l, f32, e_up, eps)) return rc;
-    const VisitPlan pl = visit_plan(ctx->lv[l], true, f32);
-    if (int rc = launch_visit<T>(ctx, l, f32, e_up, ng - l, kNr, eps, 0, pl.k_end, pl.first, pl.fixed, f32)) return rc;
+    if (int rc = launch_prolong<double>(ctx, l, false, e_up, eps)) return rc;
+    const VisitPlan pl = visit_plan(ctx->lv[l], true);
+    if (int rc = launch_visit(ctx, l, e_up, ng - l, kNr, eps, 0, pl.k_end, pl.first)) return rc;
   }
   Level& L1 = ctx->lv[1];
-  const unsigned gx = (unsigned)((L1.n1 + 1 + 255) / 256);
-  if (!f32) {
-    if (L1.mb) {
-      Finish64Args A;
-      const VisitPlan p1 = visit_plan(L1, true, false);
-      A.v = visit_ref(ctx, 1, e_up, ng - 1, kNr, 2 * ng - 1, eps, p1.k_end, p1.klast0, p1.fixed);
-      for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<double>(L1, r);
-      A.n1 = L1.n1; A.n2 = L1.n2;
-      A.status = d_status_of(ctx);
-      hipLaunchKernelGGL(k_finish64, dim3(gx, std::min(L1.n2 + 1, kRowBlocks)), dim3(256), 0, ctx->stream, A);
-    }
-  } else {
-    AddCorrArgs A;
-    A.phi = ctx->phi;
-    for (int r = 0; r < kRot; ++r) A.rot[r] = L1.mb ? rot_of<float>(L1, r) : L1.uf;
-    A.bc = ctx->bc;
+  if (L1.mb) {
+    Finish64Args A;
+    const VisitPlan p1 = visit_plan(L1, true);
+    A.v = visit_ref(ctx, 1, e_up, ng - 1, kNr, 2 * ng - 1, eps, p1.k_end, p1.klast0);
+    for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<double>(L1, r);
     A.n1 = L1.n1; A.n2 = L1.n2;
-    A.mb = L1.mb ? 1 : 0;
-    const VisitPlan p1 = visit_plan(L1, true, true);
-    A.v = L1.mb ? visit_ref(ctx, 1, e_up, ng - 1, kNr, 2 * ng - 1, eps, p1.k_end, p1.klast0, p1.fixed) : VisitRef{};
-    hipLaunchKernelGGL(k_add_corr, dim3(gx, std::min(L1.n2 + 1, kRowBlocks)), dim3(256), 0, ctx->stream, A);
+    A.status = d_status_of(ctx);
+    hipLaunchKernelGGL(k_finish64, dim3((unsigned)((L1.n1 + 1 + 255) / 256), std::min(L1.n2 + 1, kRowBlocks)),
+                       dim3(256), 0, ctx->stream, A);
   }
   LEPIC_HIP(hipGetLastError());
+  return 0;
+}
+
+// One V-cycle of the mixed form on the FP32 correction equation; adds the
+// correction to phi.
+int vcycle32(lepic_ctx* ctx, int k, double eps) {
+  for (int l = 1; l < ctx->Lc; ++l)
+    if (int rc = tile_down(ctx, l)) return rc;
+  if (int rc = launch_tail32(ctx, k, eps)) return rc;
+  for (int l = ctx->Lc - 1; l >= 1; --l)
+    if (int rc = tile_up(ctx, l)) return rc;
   return 0;
 }
 
@@ -1598,16 +1675,12 @@ double alpha_of(lepic_ctx* ctx) {
 
 int resid_blocks(lepic_ctx* ctx) { return std::min(ctx->g.n2 + 1, kResidBlocks); }
 
-// FP64 residual of phi; fills the FP32 right-hand side (and clears the
-// correction the next visit starts from) when fill_f32
+// FP64 residual of phi; fills the FP32 right-hand side when fill_f32
 int launch_resid64(lepic_ctx* ctx, bool fill_f32, const double* u = nullptr) {
   Level& L = ctx->lv[1];
-  float* const* erot = nullptr;
-  if (fill_f32) erot = (float* const*)ctx->d_erot;
   hipLaunchKernelGGL(k_resid64, dim3(resid_blocks(ctx)), dim3(256), 0, ctx->stream, u ? u : (const double*)ctx->phi,
                      (const double*)ctx->rhs, (const int8_t*)ctx->bc, L.n1, L.n2, L.aw, L.an, L.ac,
-                     fill_f32 ? L.bf : nullptr, erot, L.mb ? (const LevelCtrl*)(ctx->d_ctrl + 1) : nullptr,
-                     ctx->mg_epoch + 1, ctx->d_partials);
+                     fill_f32 ? L.bf : nullptr, ctx->d_partials);
   LEPIC_HIP(hipGetLastError());
   return 0;
 }
@@ -1694,43 +1767,35 @@ int poisson_setup(lepic_ctx* ctx) {
     if ((int64_t)(L.n1 + 1) * (L.n2 + 1) <= tail_nodes) { ctx->Lc = l; break; }
   }
   if (ng == 1 && (int64_t)(ctx->lv[1].n1 + 1) * (ctx->lv[1].n2 + 1) > tail_nodes) ctx->Lc = 2;
-  const size_t esz = mixed ? 4 : 8;
-  const int ty = mixed ? TileY<float>::v : TileY<double>::v;
   for (int l = 1; l < ctx->Lc && l <= ng; ++l) {
     Level& L = ctx->lv[l];
     L.mb = true;
-    // the mixed form's visits run fixed counts; FP64 first launches start at kS
-    L.first_dn = mixed ? (l == 1 ? kFineDn : kFixDn) : kS;
-    L.first_up = mixed ? (l == 1 ? kFineUp : kFixUp) : kS;
     const size_t nn = (size_t)(L.n1 + 3) * (L.n2 + 3);
-    L.rot[0] = mixed ? (void*)L.uf : (void*)L.u;
+    if (mixed) {
+      // the states after the down and the up visit; walls stay zero
+      L.rot[0] = L.uf;
+      LEPIC_HIP(hipMalloc(&L.rot[1], nn * 4));
+      LEPIC_HIP(hipMemsetAsync(L.rot[1], 0, nn * 4, ctx->stream));
+      continue;
+    }
+    L.first_dn = L.first_up = kS;
+    L.rot[0] = L.u;
     for (int r = 1; r < kRot; ++r) {
-      LEPIC_HIP(hipMalloc(&L.rot[r], nn * esz));
-      LEPIC_HIP(hipMemsetAsync(L.rot[r], 0, nn * esz, ctx->stream));
+      LEPIC_HIP(hipMalloc(&L.rot[r], nn * 8));
+      LEPIC_HIP(hipMemsetAsync(L.rot[r], 0, nn * 8, ctx->stream));
     }
     L.nbx = tiles_of(L.n1 + 1, kTX);
-    L.nby = tiles_of(L.n2 + 1, ty);
+    L.nby = tiles_of(L.n2 + 1, kTileY);
     // few wide tiles leave most CUs idle: the level takes small tiles, whose
     // launch latency is lower (each block has less than half the nodes)
     L.small_tiles = L.nbx * L.nby < kSmallTileBelow;
     if (L.small_tiles) {
-      const int sty = mixed ? SmallTileY<float>::v : SmallTileY<double>::v;
       L.nbx = tiles_of(L.n1 + 1, kSmallTX);
-      L.nby = tiles_of(L.n2 + 1, sty);
+      L.nby = tiles_of(L.n2 + 1, kSmallTileY);
     }
     const size_t np = (size_t)kRing * L.nbx * L.nby;
     LEPIC_HIP(hipMalloc(&L.partials, np * 8));
     LEPIC_HIP(hipMemsetAsync(L.partials, 0, np * 8, ctx->stream));
-  }
-  if (mixed && ctx->lv[1].mb) {
-    LEPIC_HIP(hipMalloc(&ctx->d_erot, kRot * sizeof(float*)));
-    LEPIC_HIP(hipMemcpyAsync(ctx->d_erot, ctx->lv[1].rot, kRot * sizeof(float*), hipMemcpyHostToDevice, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-  } else if (mixed) {
-    std::vector<float*> e(kRot, ctx->lv[1].uf);
-    LEPIC_HIP(hipMalloc(&ctx->d_erot, kRot * sizeof(float*)));
-    LEPIC_HIP(hipMemcpyAsync(ctx->d_erot, e.data(), kRot * sizeof(float*), hipMemcpyHostToDevice, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
   }
   LEPIC_HIP(hipMalloc(&ctx->d_ctrl, (kMaxLevels + 1) * sizeof(LevelCtrl)));
   LEPIC_HIP(hipMemsetAsync(ctx->d_ctrl, 0, (kMaxLevels + 1) * sizeof(LevelCtrl), ctx->stream));
@@ -1753,7 +1818,6 @@ void poisson_teardown(lepic_ctx* ctx) {
       if (L.rot[r]) (void)hipFree(L.rot[r]);
     if (L.partials) (void)hipFree(L.partials);
   }
-  if (ctx->d_erot) (void)hipFree(ctx->d_erot);
   if (ctx->d_tail_bc) (void)hipFree(ctx->d_tail_bc);
   ctx->d_tail_bc = nullptr;
   ctx->tail_bc_cap = 0;
@@ -1821,7 +1885,7 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
       int k0 = 0, ks = 0;
       while (k0 < nr) {
         const int k_end = std::min(nr, k0 + 16 * kS);
-        if (int rc = launch_visit<double>(ctx, 1, false, e, 0, nr, alpha * eps, k0, k_end)) return rc;
+        if (int rc = launch_visit(ctx, 1, e, 0, nr, alpha * eps, k0, k_end)) return rc;
         k0 = k_end;
         Level& L1 = ctx->lv[1];
         Finish64Args A;
@@ -1840,12 +1904,12 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
       if (!ks) return ctx->fail(LEPIC_ERR_STATE, "SOR visit did not finish");
       if (int rc = read_back(ctx, visit, vres, nullptr)) return rc;
     } else if (!mixed) {
-      if (int rc = vcycle<double>(ctx, false, k, alpha * eps)) return rc;
+      if (int rc = vcycle64(ctx, k, alpha * eps)) return rc;
       if (int rc = read_back(ctx, visit, vres, nullptr)) return rc;
     } else {
       // FP32 correction V-cycle on the FP64 residual, then phi += e; the new
       // FP64 residual is both the convergence test and the next right-hand side
-      if (int rc = vcycle<float>(ctx, true, k, alpha * eps)) return rc;
+      if (int rc = vcycle32(ctx, k, alpha * eps)) return rc;
       if (int rc = launch_resid64(ctx, true)) return rc;
       double rs = 0.0;
       if (int rc = read_back(ctx, visit, vres, &rs)) return rc;
@@ -1862,8 +1926,8 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
           L.first_dn = std::min(std::max(visit[l] + 1, 2), kS);
           L.first_up = std::min(std::max(visit[2 * ng - l] + 1, 2), kS);
         } else {   // the mixed form's fixed counts
-          visit[l] = L.first_dn;
-          visit[2 * ng - l] = L.first_up;
+          visit[l] = l == 1 ? kFineDn : kFixDn;
+          visit[2 * ng - l] = l == 1 ? kFineUp : kFixUp;
         }
       }
     for (int ig = 1; ig <= nvis; ++ig) {
