@@ -5,13 +5,13 @@
 // part_moments: one block per 1024-slot particle segment (the particle
 // layout of the mover), thread t owning four consecutive slots; each
 // particle adds k1*kq*w*(|v|^2, vx, vy, vz) to the four nodes around its
-// half-step-back position on the grid coarsened by size_na.  Consecutive
-// particles of one thread that share a coarse cell are summed in registers
-// first (the species is cell-sorted every few steps); the sums go to the
-// FP64 moment grid with atomics, so only the summation order differs from
-// the reference's serial loop.  calc_avg and the phi/E averages are
-// elementwise over nodes.  Diagnostics: called every navg steps, so these
-// kernels are HBM/atomic bound without further tuning.
+// half-step-back position on the grid coarsened by size_na.  Runs of
+// particles in one coarse cell are summed in registers over a thread's
+// slots, then over adjacent lanes (segmented DPP sums), go to an LDS window
+// of coarse nodes around the segment's first particle and from there to the
+// FP64 moment grid, one atomic per node and quantity of a segment; only the
+// summation order differs from the reference's serial loop.  calc_avg and
+// the phi/E averages are elementwise over nodes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,75 +32,157 @@ struct MomArgs {
   const float *fx, *fy, *fvx, *fvy, *fvz;
   const int8_t* bc;              // fine bcnd: kq = 2 where bc != -1
   int n1, size_na, na1, na2;
-  double h1, h2, ha1, ha2, xmax, ymax, half_dt, k1;
+  double h1, h2, ra1, ra2, xmax, ymax, half_dt, k1;   // ra = 1/(size_na h)
   double* pm;                    // (na2+1)(na1+1) x 4: |v|^2, vx, vy, vz
 };
 
-__device__ __forceinline__ double kq_at(const MomArgs& a, int ix, int iy) {
-  return a.bc[(int64_t)iy * (a.n1 + 3) + ix] != -1 ? 2.0 : 1.0;
-}
+// LDS window of coarse nodes, kMomX0 columns left and kMomY0 rows below the
+// segment's first particle: a sorted segment spans up to 1024 / (particles
+// per cell) columns of one row and drifts a few cells between sorts; runs in
+// cells outside go to the moment grid directly.  16 KB of LDS: ten blocks per
+// CU.
+constexpr int kMomCols = 64, kMomRows = 8, kMomX0 = 8, kMomY0 = 3;
+constexpr int kMomWin = kMomCols * kMomRows;
 
-template <bool MIXED>
-__global__ __launch_bounds__(kBlock) void k_part_moments(MomArgs a) {
-  const int cnt = a.seg[blockIdx.x];
-  const int64_t i0 = (int64_t)blockIdx.x * kChunk + (int64_t)kItems * threadIdx.x;
-  const int nv = min(max(cnt - kItems * (int)threadIdx.x, 0), kItems);
-  // running sum of consecutive particles in one coarse cell
-  int cur = -1, cix = 0, ciy = 0;
-  double acc[4][4] = {};         // [corner][|v|^2, vx, vy, vz]
-  auto flush = [&]() {
-    if (cur < 0) return;
-    const int cx[4] = {cix, cix + 1, cix + 1, cix}, cy[4] = {ciy, ciy, ciy + 1, ciy + 1};
-    for (int c = 0; c < 4; ++c) {
-      if (cx[c] > a.na1 + 1 || cy[c] > a.na2 + 1) continue;
-      double* m = a.pm + 4 * ((int64_t)(cy[c] - 1) * (a.na1 + 1) + (cx[c] - 1));
+// a run's sums (corner, quantity) into the window or the moment grid, scaled
+// by k1 and each corner's kq: at the fine node next to the coarse node's, as
+// utils.f90:103-135 indexes it.  A factor 2 is exact, so it is applied to the
+// sum instead of every particle.
+__device__ __forceinline__ void mom_flush(const MomArgs& a, double (*win)[4], int wx0, int wy0, int ix, int iy,
+                                          const double acc[16]) {
+  const int ixf = a.size_na * ix - (a.size_na - 1), iyf = a.size_na * iy - (a.size_na - 1);
+  const bool in = ix >= wx0 && ix + 1 < wx0 + kMomCols && iy >= wy0 && iy + 1 < wy0 + kMomRows;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int dx = (c == 1 || c == 2) ? 1 : 0, dy = c >= 2 ? 1 : 0;
+    const double k = (a.bc[(int64_t)(iyf + dy) * (a.n1 + 3) + ixf + dx] != -1 ? 2.0 : 1.0) * a.k1;
+    if (in) {
+      double* w = win[(iy + dy - wy0) * kMomCols + ix + dx - wx0];
+#pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (acc[c][q] != 0.0) atomic_add_f64(m + q, acc[c][q]);
-    }
-  };
-  for (int k = 0; k < nv; ++k) {
-    const int64_t i = i0 + k;
-    double xp, yp, vx, vy, vz;
-    if (MIXED) {
-      const int c = a.cell[i];
-      vx = a.fvx[i]; vy = a.fvy[i]; vz = a.fvz[i];
-      xp = ((double)((c & 0xFFFF) - 1) + (double)a.fx[i]) * a.h1;
-      yp = ((double)((c >> 16) - 1) + (double)a.fy[i]) * a.h2;
-    } else {
-      vx = a.vx[i]; vy = a.vy[i]; vz = a.vz[i];
-      xp = a.x[i];
-      yp = a.y[i];
-    }
-    xp = xp - vx * a.half_dt;
-    yp = yp - vy * a.half_dt;
-    if (xp > a.xmax || xp < 0.0 || yp > a.ymax || yp < 0.0) continue;
-    const double Eki = vx * vx + vy * vy + vz * vz;
-    const int ix = (int)(xp / a.ha1) + 1;
-    const double px = (ix * a.ha1 - xp) / a.ha1;
-    const int iy = (int)(yp / a.ha2) + 1;
-    const double py = (iy * a.ha2 - yp) / a.ha2;
-    const int key = iy * (a.na1 + 3) + ix;
-    if (key != cur) {
-      flush();
-      cur = key; cix = ix; ciy = iy;
-      for (int c = 0; c < 4; ++c)
-        for (int q = 0; q < 4; ++q) acc[c][q] = 0.0;
-    }
-    const double ki[4] = {a.k1 * px * py, a.k1 * (1.0 - px) * py, a.k1 * (1.0 - px) * (1.0 - py),
-                          a.k1 * px * (1.0 - py)};
-    const int ixf = a.size_na * ix - (a.size_na - 1), iyf = a.size_na * iy - (a.size_na - 1);
-    // kq at the fine node next to the coarse node's, as utils.f90:103-135 indexes it
-    const double kq[4] = {kq_at(a, ixf, iyf), kq_at(a, ixf + 1, iyf), kq_at(a, ixf + 1, iyf + 1),
-                          kq_at(a, ixf, iyf + 1)};
-    for (int c = 0; c < 4; ++c) {
-      const double kt = kq[c] * ki[c];
-      acc[c][0] += kt * Eki;
-      acc[c][1] += kt * vx;
-      acc[c][2] += kt * vy;
-      acc[c][3] += kt * vz;
+        __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double*)(w + q), k * acc[4 * c + q]);
+    } else if (ix + dx <= a.na1 + 1 && iy + dy <= a.na2 + 1) {
+      double* m = a.pm + 4 * ((int64_t)(iy + dy - 1) * (a.na1 + 1) + (ix + dx - 1));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) atomic_add_f64(m + q, k * acc[4 * c + q]);
     }
   }
-  flush();
+}
+
+// one stage of the segmented sum: the values CTRL lanes back join the lanes
+// whose run reaches them (one change of the active lanes for all sixteen)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void mom_stage(double acc[16], bool take) {
+  double o[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) o[c] = dpp_move<CTRL, ROWS>(acc[c]);
+  if (take) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] += o[c];
+  }
+}
+
+// Bound by FP64 issue: about 75 operations a particle and 290 a wave of 256
+// particles for the lane sums, against 24 B (mixed) or 40 B (FP64) read.
+// 26.2e6 particles at 100 per cell, mixed, size_na 2: 0.206 ms, 3.05 TB/s of
+// the 24 B a particle; 7.11 ms with 16 atomics on the moment grid per thread.
+template <bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_part_moments(MomArgs a) {
+  __shared__ double win[kMomWin][4];
+  __shared__ int s_w[2];
+  const int t = threadIdx.x, lane = t & 63;
+  const int cnt = a.seg[blockIdx.x];
+  if (cnt <= 0) return;          // block-uniform
+  const int64_t i0 = (int64_t)blockIdx.x * kChunk + (int64_t)kItems * t;
+  const int nv = min(max(cnt - kItems * t, 0), kItems);
+  double X[kItems], Y[kItems], V[kItems][3];
+  // the arrays are padded to whole segments: vector loads past the count stay inside
+  if (MIXED) {
+    const int4 c4 = *(const int4*)(a.cell + i0);
+    const float4 fx4 = *(const float4*)(a.fx + i0), fy4 = *(const float4*)(a.fy + i0);
+    const float4 u4 = *(const float4*)(a.fvx + i0), v4 = *(const float4*)(a.fvy + i0), w4 = *(const float4*)(a.fvz + i0);
+    const int c[4] = {c4.x, c4.y, c4.z, c4.w};
+    const float fx[4] = {fx4.x, fx4.y, fx4.z, fx4.w}, fy[4] = {fy4.x, fy4.y, fy4.z, fy4.w};
+    const float u[4] = {u4.x, u4.y, u4.z, u4.w}, v[4] = {v4.x, v4.y, v4.z, v4.w}, w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+      X[k] = ((double)((c[k] & 0xFFFF) - 1) + (double)fx[k]) * a.h1;
+      Y[k] = ((double)((c[k] >> 16) - 1) + (double)fy[k]) * a.h2;
+      V[k][0] = u[k]; V[k][1] = v[k]; V[k][2] = w[k];
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < kItems; k += 2) {
+      const double2 x2 = *(const double2*)(a.x + i0 + k), y2 = *(const double2*)(a.y + i0 + k);
+      const double2 u2 = *(const double2*)(a.vx + i0 + k), v2 = *(const double2*)(a.vy + i0 + k);
+      const double2 w2 = *(const double2*)(a.vz + i0 + k);
+      X[k] = x2.x; X[k + 1] = x2.y; Y[k] = y2.x; Y[k + 1] = y2.y;
+      V[k][0] = u2.x; V[k + 1][0] = u2.y; V[k][1] = v2.x; V[k + 1][1] = v2.y; V[k][2] = w2.x; V[k + 1][2] = w2.y;
+    }
+  }
+  for (int e = t; e < 4 * kMomWin; e += kBlock) (&win[0][0])[e] = 0.0;
+  if (t == 0) {
+    s_w[0] = max((int)(X[0] * a.ra1) + 1 - kMomX0, 1);
+    s_w[1] = max((int)(Y[0] * a.ra2) + 1 - kMomY0, 1);
+  }
+  __syncthreads();
+  const int wx0 = s_w[0], wy0 = s_w[1];
+  // running sum of consecutive particles in one coarse cell
+  int cur = -1;
+  double acc[16];                // [corner][|v|^2, vx, vy, vz]
+#pragma unroll
+  for (int c = 0; c < 16; ++c) acc[c] = 0.0;
+  const int S = a.na1 + 3;
+#pragma unroll
+  for (int k = 0; k < kItems; ++k) {
+    const double vx = V[k][0], vy = V[k][1], vz = V[k][2];
+    const double xp = X[k] - vx * a.half_dt, yp = Y[k] - vy * a.half_dt;
+    if (k >= nv || !(xp <= a.xmax && xp >= 0.0 && yp <= a.ymax && yp >= 0.0)) continue;
+    const double sx = xp * a.ra1, sy = yp * a.ra2;
+    const int ix = (int)sx + 1, iy = (int)sy + 1;
+    const double px = (double)ix - sx, py = (double)iy - sy;
+    const int key = iy * S + ix;
+    if (key != cur) {
+      if (cur >= 0) mom_flush(a, win, wx0, wy0, cur % S, cur / S, acc);
+      cur = key;
+#pragma unroll
+      for (int c = 0; c < 16; ++c) acc[c] = 0.0;
+    }
+    const double e = vx * vx + vy * vy + vz * vz;
+    const double ki[4] = {px * py, (1.0 - px) * py, (1.0 - px) * (1.0 - py), px * (1.0 - py)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      acc[4 * c] = fma(ki[c], e, acc[4 * c]);
+      acc[4 * c + 1] = fma(ki[c], vx, acc[4 * c + 1]);
+      acc[4 * c + 2] = fma(ki[c], vy, acc[4 * c + 2]);
+      acc[4 * c + 3] = fma(ki[c], vz, acc[4 * c + 3]);
+    }
+  }
+  // the run that ends the thread, over runs of equal cell in adjacent lanes
+  const uint64_t act = __ballot(cur >= 0);
+  if (act != 0) {                // wave-uniform
+    const int kk = cur >= 0 ? cur : -2 - lane;
+    const int kp = __shfl_up(kk, 1, 64);
+    const uint64_t heads = __ballot(lane == 0 || kp != kk);
+    if (__popcll(heads & act) != __popcll(act)) {
+      const int s = 63 - __builtin_clzll(heads & ((2ull << lane) - 1ull));
+      mom_stage<0x111, 0xf>(acc, lane - 1 >= s && (lane & 15) >= 1);
+      mom_stage<0x112, 0xf>(acc, lane - 2 >= s && (lane & 15) >= 2);
+      mom_stage<0x114, 0xf>(acc, lane - 4 >= s && (lane & 15) >= 4);
+      mom_stage<0x118, 0xf>(acc, lane - 8 >= s && (lane & 15) >= 8);
+      mom_stage<0x142, 0xa>(acc, (lane & 16) && (lane & ~15) - 1 >= s);
+      mom_stage<0x143, 0xc>(acc, lane >= 32 && s <= 31);
+    }
+    const bool tail = lane == 63 || ((heads >> (lane + 1)) & 1ull);
+    if (tail && cur >= 0) mom_flush(a, win, wx0, wy0, cur % S, cur / S, acc);
+  }
+  __syncthreads();
+  for (int e = t; e < 4 * kMomWin; e += kBlock) {
+    const double v = (&win[0][0])[e];
+    const int nd = e >> 2, ix = wx0 + nd % kMomCols, iy = wy0 + nd / kMomCols;
+    if (v != 0.0 && ix <= a.na1 + 1 && iy <= a.na2 + 1)
+      atomic_add_f64(a.pm + 4 * ((int64_t)(iy - 1) * (a.na1 + 1) + (ix - 1)) + (e & 3), v);
+  }
 }
 
 struct AvgArgs {
@@ -253,10 +335,11 @@ int lepic_moments_accumulate(lepic_ctx* ctx, int32_t size_na) {
     a.bc = ctx->bc;
     a.n1 = ctx->g.n1; a.size_na = size_na; a.na1 = na1; a.na2 = na2;
     a.h1 = ctx->g.h1; a.h2 = ctx->g.h2;
-    a.ha1 = size_na * ctx->g.h1; a.ha2 = size_na * ctx->g.h2;
+    const double ha1 = size_na * ctx->g.h1, ha2 = size_na * ctx->g.h2;
+    a.ra1 = 1.0 / ha1; a.ra2 = 1.0 / ha2;
     a.xmax = ctx->g.n1 * ctx->g.h1; a.ymax = ctx->g.n2 * ctx->g.h2;
     a.half_dt = ctx->g.dt / 2.0;
-    a.k1 = s.Nm / (a.ha1 * a.ha2 * ctx->g.zmax);
+    a.k1 = s.Nm / (ha1 * ha2 * ctx->g.zmax);
     a.pm = M.pm;
     const int64_t nb = nseg_of(s);
     if (nb > 0) {
