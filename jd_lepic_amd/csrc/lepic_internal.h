@@ -24,7 +24,7 @@ constexpr int kMaxTypes = 32;
 constexpr int kBlock = 256;          // threads per block of the particle kernels
 constexpr int kItems = 4;            // particles per thread in the mover
 constexpr int kChunk = kBlock * kItems;  // slots per particle segment
-constexpr int kSweepsPerLaunch = 5;  // red-black sweeps per launch on multi-block MG levels
+constexpr int kSweepsPerLaunch = 8;  // most red-black sweeps of a launch on multi-block MG levels
 constexpr int kRot = kSweepsPerLaunch + 1;  // rotating state buffers of a multi-block level
 constexpr int kRing = 16;            // residual partial-sum slots (sweep index mod kRing)
 constexpr int kPinnedDoubles = 1024; // pinned host scratch (doubles)
@@ -47,16 +47,16 @@ struct Level {
   float* bf = nullptr;
   int8_t* bc = nullptr;              // (n1+3)(n2+3)
   // multi-block levels: FP64 rotating states (index 0 is u) and the residual
-  // partial sums of the sweep kernels (kRing slots x blocks); mixed the
-  // states after the down visit (index 0, uf) and the up visit (index 1)
+  // partial sums of the sweep kernel (kRing slots of part_stride blocks);
+  // mixed the states after the down visit (index 0, uf) and the up visit
+  // (index 1)
   bool mb = false;
-  bool small_tiles = false;          // multi-block sweeps on 32-wide tiles
   void* rot[kRot] = {};
-  int nbx = 0, nby = 0;
   double* partials = nullptr;
+  int part_stride = 0;
   // FP64: sweeps of the first launch of the level's down and up visits, one
   // more than each visit took in the previous V-cycle
-  int first_dn = kSweepsPerLaunch, first_up = kSweepsPerLaunch;
+  int first_dn = 0, first_up = 0;
 };
 
 // Device-side state of a multi-block MG level across its visits.  A visit

@@ -1,5 +1,6 @@
-// mg_strip.h -- red-black SOR of the mixed form's FP32 correction equation on
-// register strips (sors.f90:93-260 in the fixed schedule of poisson.hip).
+// mg_strip.h -- red-black SOR (sors.f90:93-260) on register strips: FP32, the
+// mixed form's correction equation in the fixed schedule of poisson.hip, and
+// FP64, the reference's sweeps and residuals.
 //
 // A lane holds two neighbouring columns (i even, i + 1) of R rows (first row
 // even), so every row of a colour pass updates the same one of the two nodes
@@ -30,14 +31,30 @@ __device__ __forceinline__ float from_east(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));   // wave_shl:1
 }
 
-struct StripCoef {
-  float aw, an, ac, om, om1, rac;   // om1 = 1 - omega, rac = 1 / ac
+__device__ __forceinline__ double from_west(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xf, 0xf, true);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xf, 0xf, true), lo);
+}
+__device__ __forceinline__ double from_east(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xf, 0xf, true);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xf, 0xf, true), lo);
+}
+
+// om1 = 1 - omega, rac = 1 / ac rounded, racl (FP64) what the rounding left
+template <typename T> struct StripCoef;
+template <> struct StripCoef<float> {
+  float aw, an, ac, om, om1, rac;
+};
+template <> struct StripCoef<double> {
+  double aw, an, ac, om, om1, rac, racl;
 };
 
 // The coefficients as values the compiler keeps in scalar registers: it would
 // load them from the kernel's arguments again for every node of a pass.
-__device__ __forceinline__ StripCoef strip_hold(StripCoef k) {
+template <typename T>
+__device__ __forceinline__ StripCoef<T> strip_hold(StripCoef<T> k) {
   asm volatile("" : "+s"(k.aw), "+s"(k.an), "+s"(k.ac), "+s"(k.om), "+s"(k.om1), "+s"(k.rac));
+  if constexpr (sizeof(T) == 8) asm volatile("" : "+s"(k.racl));
   return k;
 }
 
@@ -46,29 +63,40 @@ __device__ __forceinline__ StripCoef strip_hold(StripCoef k) {
 __device__ __forceinline__ float strip_select(uint32_t m, float v, float u) {
   return __uint_as_float((m & __float_as_uint(v)) | (~m & __float_as_uint(u)));
 }
+__device__ __forceinline__ double strip_select(uint32_t m, double v, double u) {
+  const uint32_t hi = (m & (uint32_t)__double2hiint(v)) | (~m & (uint32_t)__double2hiint(u));
+  const uint32_t lo = (m & (uint32_t)__double2loint(v)) | (~m & (uint32_t)__double2loint(u));
+  return __hiloint2double((int)hi, (int)lo);
+}
+__device__ __forceinline__ float strip_clear(uint32_t m, float v) { return __uint_as_float(m & __float_as_uint(v)); }
+__device__ __forceinline__ double strip_clear(uint32_t m, double v) {
+  return __hiloint2double((int)(m & (uint32_t)__double2hiint(v)), (int)(m & (uint32_t)__double2loint(v)));
+}
 __device__ __forceinline__ uint32_t strip_mask(bool b) { return b ? 0xFFFFFFFFu : 0u; }
 
 // u: state, p = aw u, q = an u (ISO: aw = an and only p is used), b:
 // right-hand side, m: all bits set where bcnd <= 0 (walls keep u, which is
 // zero there).
-template <int R, bool ISO>
+template <typename T, int R, bool ISO>
 struct Strip {
-  float u[R][2], p[R][2], q[R][2], b[R][2];
+  T u[R][2], p[R][2], q[R][2], b[R][2];
   uint32_t m[R][2];
-  __device__ __forceinline__ float north(int r, int P) const { return ISO ? p[r][P] : q[r][P]; }   // an u
-  __device__ __forceinline__ void products(const StripCoef& k, int r, int P) {
+  __device__ __forceinline__ T north(int r, int P) const { return ISO ? p[r][P] : q[r][P]; }   // an u
+  __device__ __forceinline__ void products(const StripCoef<T>& k, int r, int P) {
     p[r][P] = k.aw * u[r][P];
     if (!ISO) q[r][P] = k.an * u[r][P];
   }
 };
 
-struct __attribute__((packed, aligned(4))) F2 { float x, y; };
-struct __attribute__((packed, aligned(8))) D2 { double x, y; };
+// a pair of neighbouring nodes, aligned like one
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) P2 { T x, y; };
+using F2 = P2<float>;
+using D2 = P2<double>;
 struct __attribute__((packed, aligned(1))) B2 { int8_t x, y; };
 
 // sor_update of node (r, P) given an u of its northern and southern neighbours
 template <int R, bool ISO, int P>
-__device__ __forceinline__ void strip_update(Strip<R, ISO>& s, const StripCoef& k, int r, float qn, float qs) {
+__device__ __forceinline__ void strip_update(Strip<float, R, ISO>& s, const StripCoef<float>& k, int r, float qn, float qs) {
   const float pw = P ? s.p[r][0] : from_west(s.p[r][1]), pe = P ? from_east(s.p[r][0]) : s.p[r][1];
   const float x = s.b[r][P] - pw - qn - qs - pe;
   const float v = k.om1 * s.u[r][P] + k.om * x * k.rac;
@@ -77,19 +105,20 @@ __device__ __forceinline__ void strip_update(Strip<R, ISO>& s, const StripCoef& 
 }
 
 // getres of node (r, P), zero on walls (the restriction counts bcnd <= 0 nodes only)
-template <int R, bool ISO, int P>
-__device__ __forceinline__ float strip_resid(const Strip<R, ISO>& s, const StripCoef& k, int r, float qn, float qs) {
-  const float pw = P ? s.p[r][0] : from_west(s.p[r][1]), pe = P ? from_east(s.p[r][0]) : s.p[r][1];
-  const float v = s.b[r][P] - (pw + pe + qn + qs + k.ac * s.u[r][P]);
-  return __uint_as_float(s.m[r][P] & __float_as_uint(v));
+template <typename T, int R, bool ISO, int P>
+__device__ __forceinline__ T strip_resid(const Strip<T, R, ISO>& s, const StripCoef<T>& k, int r, T qn, T qs) {
+  const T pw = P ? s.p[r][0] : from_west(s.p[r][1]), pe = P ? from_east(s.p[r][0]) : s.p[r][1];
+  const T v = s.b[r][P] - (pw + pe + qn + qs + k.ac * s.u[r][P]);
+  return strip_clear(s.m[r][P], v);
 }
 
 // Edge rows in LDS (an u), for each colour (0 red, 1 black) the first and the
 // last row of every strip: ed[(2 colour + last) * E + (strip + 1) * Lx + lane].
 // o is the lane's own entry; the guard strips before the first and after the
 // last are zero.
+template <typename T>
 struct Edges {
-  float* ed;
+  T* ed;
   int E, Lx, o;
   bool write;                  // the lane belongs to a strip
 };
@@ -97,7 +126,7 @@ struct Edges {
 // One colour pass: red (i + j odd) is the second node of even rows and the
 // first of odd ones.
 template <int R, bool ISO, bool RED>
-__device__ __forceinline__ void strip_pass(Strip<R, ISO>& s, const StripCoef& k, const Edges& e) {
+__device__ __forceinline__ void strip_pass(Strip<float, R, ISO>& s, const StripCoef<float>& k, const Edges<float>& e) {
   constexpr int E0 = RED ? 1 : 0, O0 = 1 - E0;            // position in even and odd rows
   constexpr int other = RED ? 1 : 0, own = 1 - other;     // colours of the neighbours and of the pass
   const float above = e.ed[(2 * other) * e.E + e.o + e.Lx], below = e.ed[(2 * other + 1) * e.E + e.o - e.Lx];
@@ -131,7 +160,7 @@ __device__ __forceinline__ void strip_sync() {
 // pass writes only its own colour's edges and reads the other's, so one
 // synchronisation per pass suffices.
 template <int R, bool ISO, bool WAVE>
-__device__ __forceinline__ void strip_sweeps(Strip<R, ISO>& s, const StripCoef& k, int nsw, const Edges& e) {
+__device__ __forceinline__ void strip_sweeps(Strip<float, R, ISO>& s, const StripCoef<float>& k, int nsw, const Edges<float>& e) {
   for (int it = 0; it < nsw; ++it) {
     strip_pass<R, ISO, true>(s, k, e);
     strip_sync<WAVE>();
@@ -141,8 +170,8 @@ __device__ __forceinline__ void strip_sweeps(Strip<R, ISO>& s, const StripCoef& 
 }
 
 // the black edges of a starting state that is not zero
-template <int R, bool ISO>
-__device__ __forceinline__ void strip_publish_black(const Strip<R, ISO>& s, const Edges& e) {
+template <typename T, int R, bool ISO>
+__device__ __forceinline__ void strip_publish_black(const Strip<T, R, ISO>& s, const Edges<T>& e) {
   if (e.write) {
     e.ed[2 * e.E + e.o] = s.north(0, 0);
     e.ed[3 * e.E + e.o] = s.north(R - 1, 1);
@@ -152,19 +181,19 @@ __device__ __forceinline__ void strip_publish_black(const Strip<R, ISO>& s, cons
 // Full weighting (mg.f90:386-414) of the residuals at the coarse nodes of the
 // strip, the second node of every odd row.  out[t]: coarse node of row 2t + 1.
 // All edges are in LDS; contains two synchronisations.
-template <int R, bool ISO, bool WAVE>
-__device__ __forceinline__ void strip_restrict(const Strip<R, ISO>& s, const StripCoef& k, const Edges& e,
-                                               float out[R / 2]) {
-  float g[R + 1][2];
+template <typename T, int R, bool ISO, bool WAVE>
+__device__ __forceinline__ void strip_restrict(const Strip<T, R, ISO>& s, const StripCoef<T>& k, const Edges<T>& e,
+                                               T out[R / 2]) {
+  T g[R + 1][2];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    float n0, n1, s0, s1;      // an u of the two nodes' northern and southern neighbours
+    T n0, n1, s0, s1;          // an u of the two nodes' northern and southern neighbours
     if (r + 1 < R) { n0 = s.north(r + 1 < R ? r + 1 : r, 0); n1 = s.north(r + 1 < R ? r + 1 : r, 1); }
     else { n0 = e.ed[2 * e.E + e.o + e.Lx]; n1 = e.ed[e.o + e.Lx]; }          // even row: black, red
     if (r > 0) { s0 = s.north(r > 0 ? r - 1 : r, 0); s1 = s.north(r > 0 ? r - 1 : r, 1); }
     else { s0 = e.ed[e.E + e.o - e.Lx]; s1 = e.ed[3 * e.E + e.o - e.Lx]; }     // odd row: red, black
-    g[r][0] = strip_resid<R, ISO, 0>(s, k, r, n0, s0);
-    g[r][1] = strip_resid<R, ISO, 1>(s, k, r, n1, s1);
+    g[r][0] = strip_resid<T, R, ISO, 0>(s, k, r, n0, s0);
+    g[r][1] = strip_resid<T, R, ISO, 1>(s, k, r, n1, s1);
   }
   strip_sync<WAVE>();          // every edge has been read
   if (e.write) {
@@ -174,32 +203,124 @@ __device__ __forceinline__ void strip_restrict(const Strip<R, ISO>& s, const Str
   strip_sync<WAVE>();
   g[R][0] = e.ed[e.o + e.Lx];
   g[R][1] = e.ed[2 * e.E + e.o + e.Lx];
-  float ge[R + 1];             // the first node of the next lane
+  T ge[R + 1];                 // the first node of the next lane
 #pragma unroll
   for (int r = 0; r <= R; ++r) ge[r] = from_east(g[r][0]);
 #pragma unroll
   for (int t = 0; t < R / 2; ++t) {
     const int c = 2 * t + 1;
-    const float v = (4.0f * g[c][1] + 2.0f * (ge[c] + g[c - 1][1] + g[c][0] + g[c + 1][1]) + ge[c + 1] + ge[c - 1] +
-                     g[c - 1][0] + g[c + 1][0]) / 16.0f;
-    out[t] = __uint_as_float(s.m[c][1] & __float_as_uint(v));
+    const T v = ((T)4 * g[c][1] + (T)2 * (ge[c] + g[c - 1][1] + g[c][0] + g[c + 1][1]) + ge[c + 1] + ge[c - 1] +
+                 g[c - 1][0] + g[c + 1][0]) / (T)16;
+    out[t] = strip_clear(s.m[c][1], v);
   }
 }
 
 // The bilinear correction (mg.f90:585-611) of the strip's nodes added to u on
 // bcnd <= 0 nodes.  c[t]: coarse values (ci - 1, ci) of coarse row j0/2 + t,
 // ci = i0/2 + 1, for the strip's first row j0 and first column i0.
-template <int R, bool ISO>
-__device__ __forceinline__ void strip_prolong(Strip<R, ISO>& s, const F2 c[R / 2 + 1]) {
+template <typename T, int R, bool ISO>
+__device__ __forceinline__ void strip_prolong(Strip<T, R, ISO>& s, const P2<T> c[R / 2 + 1]) {
 #pragma unroll
   for (int t = 0; t < R / 2; ++t) {
-    const F2 a = c[t], b = c[t + 1];
-    const float v[2][2] = {{(b.y + a.y + a.x + b.x) / 4.0f, (b.y + a.y) / 2.0f}, {(b.y + b.x) / 2.0f, b.y}};
+    const P2<T> a = c[t], b = c[t + 1];
+    const T v[2][2] = {{(b.y + a.y + a.x + b.x) / (T)4, (b.y + a.y) / (T)2}, {(b.y + b.x) / (T)2, b.y}};
 #pragma unroll
     for (int d = 0; d < 2; ++d)
 #pragma unroll
       for (int P = 0; P < 2; ++P)
         s.u[2 * t + d][P] = strip_select(s.m[2 * t + d][P], s.u[2 * t + d][P] + v[d][P], s.u[2 * t + d][P]);
+  }
+}
+
+// ---- FP64: the reference's sweeps with the residual of every sweep ----
+
+// x / ac, correctly rounded as the reference's division: the quotient from the
+// reciprocal in two parts is within one unit in the last place, so the
+// remainder is exact and one correction rounds it right (Markstein's theorem,
+// IBM J. Res. Dev. 34, 1990); four operations where the general division
+// takes a dozen.
+__device__ __forceinline__ double strip_div(double x, const StripCoef<double>& k) {
+  const double q = __builtin_fma(x, k.rac, x * k.racl);
+  return __builtin_fma(__builtin_fma(-k.ac, q, x), k.rac, q);
+}
+
+// sors.f90:108-110 of node (r, P).  The residual (sors.f90:348-349 order) is
+// taken where its neighbours are at hand: a black node's of this sweep right
+// after its update, a red node's of the sweep before right before it.
+// Returns |residual|, zero on walls.
+template <int R, bool ISO, int P, bool RED, bool RES, bool UPD>
+__device__ __forceinline__ double strip_node64(Strip<double, R, ISO>& s, const StripCoef<double>& k, int r, double qn,
+                                               double qs) {
+  const double pw = P ? s.p[r][0] : from_west(s.p[r][1]), pe = P ? from_east(s.p[r][0]) : s.p[r][1];
+  const double u = s.u[r][P], b = s.b[r][P];
+  double res = 0.0;
+  if (RES && RED) res = b - (pw + qn + qs + pe + k.ac * u);
+  if (UPD) {
+    const double v = k.om1 * u + strip_div(k.om * (b - pw - qn - qs - pe), k);
+    s.u[r][P] = strip_select(s.m[r][P], v, u);
+    s.products(k, r, P);
+  }
+  if (RES && !RED) res = b - (pw + qn + qs + pe + k.ac * s.u[r][P]);
+  return RES ? fabs(strip_clear(s.m[r][P], res)) : 0.0;
+}
+
+// One colour pass; UPD false: the residual of the red nodes alone.
+template <int R, bool ISO, bool RED, bool RES, bool UPD>
+__device__ __forceinline__ double strip_pass64(Strip<double, R, ISO>& s, const StripCoef<double>& k,
+                                               const Edges<double>& e) {
+  constexpr int E0 = RED ? 1 : 0, O0 = 1 - E0;            // position in even and odd rows
+  constexpr int other = RED ? 1 : 0, own = 1 - other;     // colours of the neighbours and of the pass
+  const double above = e.ed[(2 * other) * e.E + e.o + e.Lx], below = e.ed[(2 * other + 1) * e.E + e.o - e.Lx];
+  double rr = 0.0;
+#pragma unroll
+  for (int r = 1; r + 1 < R; ++r) {
+    if (r & 1) rr += strip_node64<R, ISO, O0, RED, RES, UPD>(s, k, r, s.north(r + 1, O0), s.north(r - 1, O0));
+    else rr += strip_node64<R, ISO, E0, RED, RES, UPD>(s, k, r, s.north(r + 1, E0), s.north(r - 1, E0));
+  }
+  rr += strip_node64<R, ISO, E0, RED, RES, UPD>(s, k, 0, s.north(1, E0), below);
+  rr += strip_node64<R, ISO, O0, RED, RES, UPD>(s, k, R - 1, above, s.north(R - 2, O0));
+  if (UPD && e.write) {
+    e.ed[(2 * own) * e.E + e.o] = s.north(0, E0);
+    e.ed[(2 * own + 1) * e.E + e.o] = s.north(R - 1, O0);
+  }
+  return rr;
+}
+
+// A region's u, b and bc on the lane's strip: columns i0, i0 + 1, rows j0 .. +
+// R - 1; all loads are issued before the first is used, from clamped
+// positions.  uin null: zero.  The outer walls come from uw, the level's
+// array 0: the other state buffers hold the nodes between them.
+template <int R, bool ISO>
+__device__ __forceinline__ void strip_region_load(Strip<double, R, ISO>& s, const double* uin, const double* uw,
+                                                  const double* b, const int8_t* bc, int n1, int n2, int i0, int j0) {
+  const int W = n1 + 3;
+  const bool oki = i0 >= 0 && i0 <= n1 + 1, okb = i0 >= 2 && i0 <= n1;
+  D2 lu[R], lb[R];
+  B2 lc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int j = j0 + r;
+    const bool ok = oki && j >= 1 && j <= n2 + 1;
+    const int64_t q = ok ? (int64_t)j * W + i0 : (int64_t)2 * W + 2;
+    const int64_t qb = okb && j >= 2 && j <= n2 ? (int64_t)(j - 1) * (n1 + 1) + (i0 - 1) : (int64_t)(n1 + 2);
+    lu[r] = D2{0.0, 0.0};
+    if (uin) {
+      const double* base = i0 == 0 || i0 == n1 + 1 || j == 1 || j == n2 + 1 ? uw : uin;
+      lu[r] = *(const D2*)(base + q);
+    }
+    lb[r] = *(const D2*)(b + qb);
+    lc[r] = *(const B2*)(bc + q);
+    if (!ok) lc[r] = B2{1, 1};
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool ok = oki && j0 + r >= 1 && j0 + r <= n2 + 1;
+    s.m[r][0] = strip_mask(lc[r].x <= 0);
+    s.m[r][1] = strip_mask(lc[r].y <= 0);
+    s.u[r][0] = ok ? lu[r].x : 0.0;
+    s.u[r][1] = ok ? lu[r].y : 0.0;
+    s.b[r][0] = lb[r].x;
+    s.b[r][1] = lb[r].y;
   }
 }
 
@@ -212,7 +333,7 @@ struct TileArgs {
   const float* b;
   const int8_t* bc;
   int n1, n2;
-  StripCoef k;
+  StripCoef<float> k;
   int nsw, halo;               // sweeps; halo nodes around a tile (even)
   const float* e2h;            // up visit: the coarse correction to prolong
   float* r2h;                  // last launch of a down visit: the coarse right-hand side
@@ -234,7 +355,7 @@ __global__ __launch_bounds__(64 * NW) void k_tile32(TileArgs A) {
   const int i0 = 2 + (int)blockIdx.x * TX - A.halo + 2 * lane;
   const int j0 = 2 + (int)blockIdx.y * TY - A.halo + w * R;
   const bool oki = i0 >= 2 && i0 <= n1;
-  const StripCoef k = strip_hold(A.k);
+  const StripCoef<float> k = strip_hold(A.k);
   // what leaves the block: the tile's nodes
   const bool colo = oki && 2 * lane >= A.halo && 2 * lane < 128 - A.halo;
   const int lr0 = w * R;
@@ -248,7 +369,7 @@ __global__ __launch_bounds__(64 * NW) void k_tile32(TileArgs A) {
     for (int r = 0; r < R; ++r)
       ph[r] = *(const D2*)(A.phi + (own[r] ? (int64_t)(j0 + r) * W + i0 : (int64_t)2 * W + 2));
   }
-  Strip<R, ISO> s;
+  Strip<float, R, ISO> s;
   {
     F2 lu[R], lb[R];
     B2 lc[R];
@@ -282,17 +403,17 @@ __global__ __launch_bounds__(64 * NW) void k_tile32(TileArgs A) {
       const int cj = min(max((j0 >> 1) + t, 1), m2 + 1);
       c[t] = *(const F2*)(A.e2h + (int64_t)cj * Wc + ci - 1);
     }
-    strip_prolong<R, ISO>(s, c);
+    strip_prolong<float, R, ISO>(s, c);
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     s.products(k, r, 0);
     s.products(k, r, 1);
   }
-  Edges e{ed, E, 64, (w + 1) * 64 + lane, true};
+  Edges<float> e{ed, E, 64, (w + 1) * 64 + lane, true};
   __syncthreads();
   if (A.u_in) {
-    strip_publish_black<R, ISO>(s, e);
+    strip_publish_black<float, R, ISO>(s, e);
     __syncthreads();
   }
   strip_sweeps<R, ISO, false>(s, k, A.nsw, e);
@@ -309,7 +430,7 @@ __global__ __launch_bounds__(64 * NW) void k_tile32(TileArgs A) {
   }
   if (A.r2h) {                 // block-uniform
     float out[R / 2];
-    strip_restrict<R, ISO, false>(s, k, e, out);
+    strip_restrict<float, R, ISO, false>(s, k, e, out);
     const int m1 = n1 / 2;
 #pragma unroll
     for (int t = 0; t < R / 2; ++t) {
@@ -327,7 +448,7 @@ struct StripLevel {
   int n1, n2;
   int Lx, SW, nst;             // lanes per strip row ((n1 + 1) / 2), strips per wave, strips
   int inv;                     // 65536 / Lx + 1: lane / Lx = lane inv >> 16 for lane < 64, Lx <= 64
-  StripCoef k;
+  StripCoef<float> k;
 };
 
 // the lane's strip of a level: wave w holds strips w SW .. w SW + SW - 1,
@@ -351,7 +472,7 @@ __device__ __forceinline__ StripPos strip_pos(const StripLevel& L, int w) {
 
 // All loads are issued before the first is used, from clamped positions.
 template <int R, bool ISO>
-__device__ __forceinline__ void strip_load(Strip<R, ISO>& s, const StripLevel& L, const StripPos& p, const float* u,
+__device__ __forceinline__ void strip_load(Strip<float, R, ISO>& s, const StripLevel& L, const StripPos& p, const float* u,
                                            const float* b, const int8_t* bc) {
   const int W = L.n1 + 3;
   int8_t c[R][2];
@@ -384,23 +505,23 @@ __device__ __forceinline__ void strip_load(Strip<R, ISO>& s, const StripLevel& L
 // The lane's edges: zero guards below the first and above the last strip, and
 // the starting state's black edges (north: their an u).
 template <int R, bool ISO>
-__device__ __forceinline__ void strip_edges(const Strip<R, ISO>& s, const StripLevel& L, const StripPos& p,
-                                            const Edges& e) {
+__device__ __forceinline__ void strip_edges(const Strip<float, R, ISO>& s, const StripLevel& L, const StripPos& p,
+                                            const Edges<float>& e) {
   if (!p.act) return;
   if (p.strip == 0) e.ed[e.E + p.lx] = e.ed[3 * e.E + p.lx] = 0.0f;
   if (p.strip == L.nst - 1) e.ed[e.o + e.Lx] = e.ed[2 * e.E + e.o + e.Lx] = 0.0f;
-  strip_publish_black<R, ISO>(s, e);
+  strip_publish_black<float, R, ISO>(s, e);
 }
 
 // Down visit: nsw sweeps from zero, the state to u, the restricted residual
 // to the coarse right-hand side b2.
 template <int R, bool ISO, bool WAVE>
-__device__ __forceinline__ void strip_down(const StripLevel& L, const StripCoef& kl, int nsw, float* ed, float* u,
+__device__ __forceinline__ void strip_down(const StripLevel& L, const StripCoef<float>& kl, int nsw, float* ed, float* u,
                                            const float* b, const int8_t* bc, float* b2) {
-  const StripCoef k = strip_hold(kl);
+  const StripCoef<float> k = strip_hold(kl);
   const StripPos p = strip_pos(L, WAVE ? 0 : (int)(threadIdx.x >> 6));
-  Edges e{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
-  Strip<R, ISO> s;
+  Edges<float> e{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
+  Strip<float, R, ISO> s;
   strip_load<R, ISO>(s, L, p, nullptr, b, bc);
 #pragma unroll
   for (int r = 0; r < R; ++r) s.p[r][0] = s.p[r][1] = s.q[r][0] = s.q[r][1] = 0.0f;
@@ -417,7 +538,7 @@ __device__ __forceinline__ void strip_down(const StripLevel& L, const StripCoef&
       }
   }
   float out[R / 2];
-  strip_restrict<R, ISO, WAVE>(s, k, e, out);
+  strip_restrict<float, R, ISO, WAVE>(s, k, e, out);
   if (p.act && p.i0 + 1 <= L.n1) {
 #pragma unroll
     for (int t = 0; t < R / 2; ++t)
@@ -429,12 +550,12 @@ __device__ __forceinline__ void strip_down(const StripLevel& L, const StripCoef&
 // Up visit: the coarse correction u2 prolonged onto u, nsw sweeps, the state
 // to u, to the global array gu, or added to phi.
 template <int R, bool ISO, bool WAVE>
-__device__ __forceinline__ void strip_up(const StripLevel& L, const StripCoef& kl, int nsw, float* ed, float* u,
+__device__ __forceinline__ void strip_up(const StripLevel& L, const StripCoef<float>& kl, int nsw, float* ed, float* u,
                                          const float* b, const int8_t* bc, const float* u2, float* gu, double* phi) {
-  const StripCoef k = strip_hold(kl);
+  const StripCoef<float> k = strip_hold(kl);
   const StripPos p = strip_pos(L, WAVE ? 0 : (int)(threadIdx.x >> 6));
-  Edges e{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
-  Strip<R, ISO> s;
+  Edges<float> e{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
+  Strip<float, R, ISO> s;
   strip_load<R, ISO>(s, L, p, u, b, bc);
   const int W = L.n1 + 3, m1 = L.n1 / 2, m2 = L.n2 / 2, j0 = 2 + p.strip * R;
   F2 c[R / 2 + 1];
@@ -444,7 +565,7 @@ __device__ __forceinline__ void strip_up(const StripLevel& L, const StripCoef& k
     const int q = cj * (m1 + 3) + min(p.i0 / 2, m1);
     c[t] = F2{u2[q], u2[q + 1]};
   }
-  strip_prolong<R, ISO>(s, c);
+  strip_prolong<float, R, ISO>(s, c);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     s.products(k, r, 0);

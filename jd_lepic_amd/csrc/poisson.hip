@@ -5,23 +5,25 @@
 // A kernel launch costs about 3 us on MI355X whatever it does, and a grid-wide
 // software barrier costs more, so the solver is organised to launch few
 // kernels and to need no grid synchronisation:
-//  * FP64 fine ("multi-block") levels run k_sweeps: each block owns a 64-wide tile,
-//    stages the tile plus a halo of 2S+1 nodes in LDS and performs S red-black
-//    sweeps on it, recomputing the halo redundantly instead of exchanging it.
-//    After every sweep it writes the tile to that sweep's state buffer (S+1
-//    rotating buffers per level) and its share of the L1 residual.  The exit
-//    test of sors.f90:371-377 for those sweeps is taken at the start of the
-//    next launch (or by the kernel that consumes the level), by every block
-//    from the same partial sums in the same order, so all blocks agree and no
-//    atomics or host round trips are needed.  A visit with the reference's
-//    limit of 10 sweeps takes two launches.
+//  * FP64 fine ("multi-block") levels run k_visit64: each block holds a tile
+//    and a halo of 2S+1 nodes on register strips (mg_strip.h) and performs S
+//    red-black sweeps on it, recomputing the halo redundantly instead of
+//    exchanging it.  After every sweep it writes the tile to that sweep's
+//    state buffer (kRot rotating buffers per level) and its share of the L1
+//    residual.  The exit test of sors.f90:371-377 for those sweeps is taken
+//    at the start of the next launch (or by the kernel that consumes the
+//    level), by every block from the same partial sums in the same order, so
+//    all blocks agree and no atomics or host round trips are needed.  A visit
+//    takes two launches, of which the second mostly finds it finished.  An up
+//    visit prolongs the coarse correction while it loads; the restriction
+//    needs the visit's outcome and is a kernel of its own (k_restrict64).
+//    Between the V-cycles the finest state stays in its buffer; the solve's
+//    end moves it to phi.
 //  * Coarse levels (at most mg_tail_nodes nodes) run in one workgroup that
 //    performs the whole lower part of the V-cycle (down sweeps, restrictions,
 //    the coarsest solve, prolongations and up sweeps), with the levels that
 //    fit in its LDS (up to 158 KB) held there: k_tail (FP64; the mixed form
 //    where a level is too wide for strips) and k_tail32 (mixed).
-//  * Grid transfers between FP64 multi-block levels are kernels between the
-//    visits (k_restrict, LDS-tiled; k_prolong).
 //  * Mixed mode runs each visit of a multi-block level in one launch of
 //    k_tile32 (mg_strip.h): the sweeps of a fixed count on register strips,
 //    with the prolongation on load, the restriction after the last sweep, and
@@ -53,13 +55,6 @@ constexpr int kVisitLog = 2 * kMaxLevels;     // ig = 1 .. 2ng-1
 constexpr size_t kTailLds = 160 * 1024 - 2048;  // dynamic LDS of k_tail (static arrays take < 2 KB)
 constexpr int kTailThreads = 1024;
 constexpr int kS = kSweepsPerLaunch;          // most sweeps of one launch (kRot - 1 state buffers ahead)
-// halo of a launch of at most KS sweeps: validity shrinks by one node per colour pass
-template <int KS> struct Halo { static constexpr int v = 2 * KS + 1; };
-constexpr int kTX = 64;                       // wide tiles: 64 x TileY nodes, 1024 threads
-constexpr int kSmallTX = 32;                  // small tiles: 32 x SmallTileY nodes, 512 threads
-constexpr int kSmallThreads = 512;
-constexpr int kSmallTileBelow = 64;           // a level with fewer wide tiles than this takes small ones
-constexpr int kSweepThreads = 1024;
 constexpr int kDefaultTailNodes = 5000;
 constexpr int kResidBlocks = 512;             // blocks of the FP64 finest-level residual (their partial sums fit the pinned read-back)
 // byte offset of the residual partials behind the scalars, visit log and status
@@ -81,15 +76,13 @@ constexpr int kFineDn = 4, kFineUp = 3;
 constexpr float kFineOmega = 1.15f;
 constexpr int kFixDn = kNr, kFixUp = 2;
 constexpr int kWaveNodes = 320;               // tail levels with at most this many interior nodes run in one wave
-constexpr int kRowBlocks = 1024;              // row-loop blocks of the grid-transfer kernels (one row each up to 1024 rows)
 
-constexpr int kTileY = 16, kSmallTileY = 8;
 // mixed form: a visit's sweeps run in one launch of k_tile32 unless its tiles,
 // small behind a deep halo (84 x 20 nodes for 10 sweeps and the restriction),
 // then need more than two blocks per CU; two launches of 5 sweeps cost one
 // more load and launch (about 5 us) but sweep 1.8 instead of 4.9 times the
 // tiles' nodes
-constexpr int kTileMaxBlocks = 512;
+constexpr int kTileMaxBlocks = 512, kTileSplit = 5;
 
 // ---- SOR update of one node (sors.f90:108-110 / 238-240) ----
 // FP64 divides like the reference; the FP32 smoother of the mixed form
@@ -174,53 +167,42 @@ __device__ __forceinline__ void prolong_node(PU u, PC bc, int n1, PE e2h, int m1
 }
 
 // ---------------------------------------------------------------------------
-// visit control of multi-block levels
+// visit control of multi-block levels (FP64)
 // ---------------------------------------------------------------------------
-struct VisitRef {
-  LevelCtrl* ctrl;
+// What the exit test of a launch reads: the partial sums of the launch's
+// sweeps by nb1 blocks, of the sweep before them by nb0.
+struct StopTest {
   const double* partials;
-  int nb;                  // blocks of the level's sweep kernel
-  int epoch, dig, nr, ig;
+  int stride, nb0, nb1;
+  int dig, nr;
   double eps;
-  int nexec;               // sweeps launched in the visit
-  int klast0;              // sweeps before the visit's last launch
-  int* visit;
-  double* vres;
 };
 
-// L1 residuals after sweeps kf-1 .. kt of the current visit (kt-kf+2 <= kS+1
-// values): the blocks' partial sums in a fixed order (lane strides, then a
-// shuffle tree).  All loads are issued before any sum, so the evaluation
-// costs one memory round trip.  Wave 0, all lanes; r[0] is sweep kf-1 (zero
-// when kf = 1).
-__device__ void ring_res(const double* partials, int nb, int kf, int kt, double* r) {
-  const int lane = threadIdx.x & 63;
-  double s[kS + 1];
-#pragma unroll
-  for (int m = 0; m <= kS; ++m) {
+// sors.f90:371-377 for sweeps kf .. kt (of one launch): the first sweep after
+// which the reference stops (0 if none), from the blocks' partial sums of the
+// L1 residual in a fixed order (lane strides, then a tree); the sweep before
+// the visit's first counts as zero.  Called by every thread of a block, which
+// all get the same answer; a wave sums one sweep at a time.  s_res: kS + 1
+// doubles.
+__device__ int first_stop(const StopTest& T, int kf, int kt, double* s_res, double* r_out) {
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  for (int m = threadIdx.x >> 6; m <= kt - kf + 1; m += nw) {
     const int k = kf - 1 + m;
-    s[m] = 0.0;
-    if (k >= 1 && k <= kt) {
-      const double* p = partials + (size_t)(k % kRing) * nb;
-      for (int q = lane; q < nb; q += 64) s[m] += p[q];
+    double s = 0.0;
+    if (k >= 1) {
+      const double* p = T.partials + (size_t)(k % kRing) * T.stride;
+      const int nb = m == 0 ? T.nb0 : T.nb1;
+      for (int q = lane; q < nb; q += 64) s += p[q];
+      s = wave_sum(s);
     }
+    if (lane == 0) s_res[m] = s;
   }
-#pragma unroll
-  for (int m = 0; m <= kS; ++m) r[m] = wave_sum(s[m]);
-}
-
-// sors.f90:371-377 for sweeps kf..kt (at most kS of them): the first sweep
-// after which the reference stops (0 if none); res_s is the previous
-// sweep's residual, zero before the first sweep of a visit.
-__device__ int first_stop(const double* partials, int nb, int kf, int kt, int dig, double eps, int nr,
-                          double* r_out) {
-  double r[kS + 1];
-  ring_res(partials, nb, kf, kt, r);
-  double prev = r[0];
+  __syncthreads();
+  double prev = s_res[0];
   for (int k = kf; k <= kt; ++k) {
-    const double rk = r[k - kf + 1];
-    bool stop = (dig == 0) ? (rk <= eps) : (prev > 0.0 && rk / prev <= 0.6);
-    if (k >= nr) stop = true;
+    const double rk = s_res[k - kf + 1];
+    bool stop = (T.dig == 0) ? (rk <= T.eps) : (prev > 0.0 && rk / prev <= 0.6);
+    if (k >= T.nr) stop = true;
     if (stop) {
       *r_out = rk;
       return k;
@@ -230,356 +212,254 @@ __device__ int first_stop(const double* partials, int nb, int kf, int kt, int di
   return 0;
 }
 
+struct VisitRef {
+  LevelCtrl* ctrl;
+  StopTest t;              // of the visit's last launch
+  int epoch, ig;
+  int nexec;               // sweeps launched in the visit
+  int klast0;              // sweeps before the visit's last launch
+  int* visit;
+  double* vres;
+};
+
 struct Resolved {
   int ks;                  // sweeps of the visit (0: not finished)
   int buf;                 // rotating buffer holding the state after them
-  double res;
 };
 
 // Outcome of a visit after all its launches; every block of the consuming
-// kernel evaluates it (wave 0) and block 0 records it.  `canon` records
-// buffer 0 as the level's state (the caller copies the result there).
-__device__ Resolved resolve_visit(const VisitRef& V, bool writer, bool canon) {
+// kernel evaluates it (all threads) and one records it.
+__device__ Resolved resolve_visit(const VisitRef& V, bool writer, double* s_res) {
   LevelCtrl* c = V.ctrl;
   const int c0 = c->cur[(V.epoch - 1) & 1];
-  Resolved out{0, -1, 0.0};
+  Resolved out{0, 0};
+  double res = 0.0;
   if (c->done_epoch == V.epoch) {
     out.ks = c->ksor;
-    out.res = c->res;
+    res = c->res;
   } else {
-    out.ks = first_stop(V.partials, V.nb, V.klast0 + 1, V.nexec, V.dig, V.eps, V.nr, &out.res);
+    out.ks = first_stop(V.t, V.klast0 + 1, V.nexec, s_res, &res);
   }
   if (out.ks) out.buf = (c0 + out.ks) % kRot;
   if (writer && out.ks && threadIdx.x == 0) {
-    c->cur[V.epoch & 1] = canon ? 0 : out.buf;
+    c->cur[V.epoch & 1] = out.buf;
     V.visit[V.ig] = out.ks;
-    V.vres[V.ig] = out.res;
+    V.vres[V.ig] = res;
   }
   return out;
 }
 
 // ---------------------------------------------------------------------------
-// multi-block levels
+// multi-block levels (FP64)
 // ---------------------------------------------------------------------------
-template <typename T>
-struct SweepArgs {
-  T* rot[kRot];
-  const T* b;
+constexpr int kVR = 4;                        // rows of a strip
+constexpr int kVisitMaxWaves = 16;
+
+struct VisitArgs {
+  double* rot[kRot];
+  const double* b;
   const int8_t* bc;
   int n1, n2;
-  T aw, an, ac, omega;
+  StripCoef<double> k;
   LevelCtrl* ctrl;
   double* partials;
-  int nbx, nby;
-  int epoch, dig, nr;
-  double eps;
+  StopTest t;              // of the visit's previous launch
+  int epoch;
+  int k0, kexec, kchk;     // sweeps k0+1 .. k0+kexec; the previous launch's kchk .. k0 (kchk 0: no test)
+  int halo_x, halo_y;      // region around a tile; halo_y a multiple of kVR
+  int zero;                // the visit starts from zero
+  const double* crot[kRot];   // up visit's first launch: the coarse correction (null: none), from the buffer
+  int coarse_mb;              // that the coarse level's visit ends in, or from buffer 0
+  VisitRef vc;
 };
 
-// Sweeps k0+1 .. k0+kexec (kexec <= KS) of a visit on one TX x TY tile with
-// NT threads (see the file comment).  A launch that continues a visit first
-// takes the reference's exit test for the sweeps of the visit's previous
-// launch, kchk .. k0.
-template <typename T, int kTX, int TY, int kSweepThreads, int KS>
-__global__ __launch_bounds__(kSweepThreads) void k_sweeps(SweepArgs<T> A, int k0, int kexec, int kchk) {
-  constexpr int kHalo = Halo<KS>::v;
-  // a block's tile is kTX x TY nodes, or one node wider (taller) in the last
-  // column (row) of tiles when the level's node count leaves one node over
-  // (2^k + 1 nodes per side); the region has room for that and stays even
-  constexpr int kTP = kTX + 1, kTYP = TY + 1;
-  constexpr int RW = kTX + 2 + 2 * kHalo, RH = kTYP + 2 * kHalo, RN = RW * RH;
-  constexpr int HW = (RW - 2) / 2;  // nodes of one colour per inner region row
-  static_assert((RW & 1) == 0, "region width must be even");
-  __shared__ T su[RN];
-  __shared__ T sb[RN];
-  __shared__ int8_t sbc[RN];
-  __shared__ int s_go, s_c0;
-  __shared__ double ws[kSweepThreads / 64];
-  const int nb = A.nbx * A.nby;
-  const int bid = blockIdx.y * A.nbx + blockIdx.x;
-  if (threadIdx.x < 64) {
-    LevelCtrl* c = A.ctrl;
-    int go = 1;
-    const int c0 = c->cur[(A.epoch - 1) & 1];
-    if (__hip_atomic_load(&c->done_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == A.epoch) {
-      go = 0;
-    } else if (k0 > 0) {
-      double r = 0.0;
-      const int ks = first_stop(A.partials, nb, kchk, k0, A.dig, A.eps, A.nr, &r);
-      if (ks) {
-        go = 0;
-        if (bid == 0 && threadIdx.x == 0) {
-          c->ksor = ks;
-          c->res = r;
-          __hip_atomic_store(&c->done_epoch, A.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    }
-    if (threadIdx.x == 0) {
-      s_go = go;
-      s_c0 = c0;
-    }
-  }
-  __syncthreads();
-  if (!s_go) return;
-
+// Sweeps of a visit on one tile (see the file comment).  Bound by VALU issue:
+// an update costs 19 FP64 operations where aw = an (four of them the
+// division), its residual 8 more, against six LDS reads, the index arithmetic
+// and a division of a dozen operations per node and pass on a region in LDS,
+// the residual in a third pass.  1025 x 513 nodes, 5 sweeps: 34-39 us so
+// before, 16 now; 257 x 129: 14, now 9; a launch that finds the visit finished
+// takes 4.5 us either way.  The region of 128
+// columns x kVR rows per wave is the tile and a halo of 2 kexec + 1 nodes at
+// least (validity shrinks by one node per colour pass, and the residual reads
+// one more).  Tiles start at (2, 2).  A wave takes part only in the sweeps
+// whose outcome still reaches the tile, and only waves of tile rows (halo_y is
+// a multiple of a strip's rows) evaluate residuals and write states.
+template <bool ISO>
+__global__ __launch_bounds__(64 * kVisitMaxWaves) void k_visit64(VisitArgs A) {
+  __shared__ double ed[4 * (kVisitMaxWaves + 2) * 64];
+  __shared__ double ws[kS][kVisitMaxWaves];
+  __shared__ double s_res[2][kS + 1];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int E = (nw + 2) * 64;
   const int n1 = A.n1, n2 = A.n2;
-  const int64_t W = n1 + 3;
-  const int tw = (int)blockIdx.x == A.nbx - 1 ? n1 + 1 - (int)blockIdx.x * kTX : kTX;
-  const int th = (int)blockIdx.y == A.nby - 1 ? n2 + 1 - (int)blockIdx.y * TY : TY;
-  const int gi0 = 1 + (int)blockIdx.x * kTX - kHalo;  // global i of region column 0
-  const int gj0 = 1 + (int)blockIdx.y * TY - kHalo;
-  const T* uin = A.rot[(s_c0 + k0) % kRot];
-  {
-    // every load of the region is issued before any LDS store: one memory
-    // latency for the whole region instead of one per loop trip
-    constexpr int kIt = (RN + kSweepThreads - 1) / kSweepThreads;
-    T lu[kIt], lb[kIt];
-    int8_t lc[kIt];
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-      const int q = threadIdx.x + it * kSweepThreads;
-      const int r = q / RW, cc = q - r * RW;
-      const int i = gi0 + cc, j = gj0 + r;
-      const bool in = q < RN && i >= 1 && i <= n1 + 1 && j >= 1 && j <= n2 + 1;
-      lu[it] = in ? uin[(int64_t)j * W + i] : (T)0;
-      lc[it] = in ? A.bc[(int64_t)j * W + i] : (int8_t)1;
-      lb[it] = in ? A.b[(int64_t)(j - 1) * (n1 + 1) + (i - 1)] : (T)0;
-    }
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-      const int q = threadIdx.x + it * kSweepThreads;
-      if (q < RN) { su[q] = lu[it]; sbc[q] = lc[it]; sb[q] = lb[it]; }
+  const int TX = 128 - 2 * A.halo_x, TY = nw * kVR - 2 * A.halo_y;
+  const int i0 = 2 + (int)blockIdx.x * TX - A.halo_x + 2 * lane;
+  const int j0 = 2 + (int)blockIdx.y * TY - A.halo_y + w * kVR;
+  const int nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
+  LevelCtrl* c = A.ctrl;
+  const int c0 = c->cur[(A.epoch - 1) & 1];
+  Strip<double, kVR, ISO> s;
+  strip_region_load<kVR, ISO>(s, A.zero ? nullptr : A.rot[(c0 + A.k0) % kRot], A.rot[0], A.b, A.bc, n1, n2, i0, j0);
+  if (A.kchk > 0) {
+    // Another block may record the stop while this one looks, so every wave
+    // takes part in the test; a stop recorded by an earlier launch counts
+    // whatever the test says of sweeps that were not run.
+    const int done = __hip_atomic_load(&c->done_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    double r = 0.0;
+    const int ks = first_stop(A.t, A.kchk, A.k0, s_res[0], &r);
+    if (done == A.epoch) return;
+    if (ks) {
+      if (bid == 0 && threadIdx.x == 0) {
+        c->ksor = ks;
+        c->res = r;
+        __hip_atomic_store(&c->done_epoch, A.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      return;
     }
   }
+  if (A.crot[0]) {
+    int cb = 0;
+    if (A.coarse_mb) cb = resolve_visit(A.vc, bid == 0, s_res[1]).buf;
+    const double* e2h = A.crot[cb];
+    const int m1 = n1 / 2, m2 = n2 / 2, Wc = m1 + 3;
+    const int ci = min(max(i0 / 2 + 1, 2), m1 + 1);
+    D2 e[kVR / 2 + 1];
+#pragma unroll
+    for (int t = 0; t <= kVR / 2; ++t) {
+      const int cj = min(max((j0 >> 1) + t, 1), m2 + 1);
+      e[t] = *(const D2*)(e2h + (int64_t)cj * Wc + ci - 1);
+    }
+    strip_prolong<double, kVR, ISO>(s, e);
+  }
+  const StripCoef<double> k = strip_hold(A.k);
+#pragma unroll
+  for (int r = 0; r < kVR; ++r) {
+    s.products(k, r, 0);
+    s.products(k, r, 1);
+  }
+  Edges<double> e{ed, E, 64, (w + 1) * 64 + lane, true};
+  if (w == 0) ed[E + lane] = ed[3 * E + lane] = 0.0;
+  if (w == nw - 1) ed[e.o + 64] = ed[2 * E + e.o + 64] = 0.0;
+  strip_publish_black<double, kVR, ISO>(s, e);
   __syncthreads();
-  const T aw = A.aw, an = A.an, ac = A.ac, om = A.omega;
-  constexpr int NB = 4;  // slots per thread whose loads are issued together
-  constexpr int kPass = (RH - 2) * HW;
-  for (int s = 1; s <= kexec; ++s) {
-    for (int color = 1; color >= 0; --color) {  // red (i+j odd), then black
-      // nodes of one colour never read each other, so a thread gathers all
-      // its slots before it writes any
-      for (int q0 = threadIdx.x; q0 < kPass; q0 += NB * kSweepThreads) {
-        int x[NB];
-        int8_t m[NB];
-        T c[NB], w[NB], e[NB], n[NB], so[NB], bb[NB];
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-          const int q = q0 + k * kSweepThreads;
-          const int qq = q < kPass ? q : 0;
-          const int r = 1 + qq / HW;
-          x[k] = r * RW + 1 + 2 * (qq % HW) + ((color ^ ((gi0 + gj0 + r + 1) & 1)) & 1);
-          m[k] = sbc[x[k]];
-          if (q >= kPass) m[k] = 1;
-          c[k] = su[x[k]]; w[k] = su[x[k] - 1]; e[k] = su[x[k] + 1];
-          n[k] = su[x[k] + RW]; so[k] = su[x[k] - RW]; bb[k] = sb[x[k]];
-        }
-#pragma unroll
-        for (int k = 0; k < NB; ++k)
-          if (m[k] <= 0) su[x[k]] = sor_update(c[k], bb[k], w[k], n[k], so[k], e[k], aw, an, ac, om);
-      }
-      __syncthreads();
+  const int P = 2 * A.kexec, dist = min(kVR * w + kVR - 1, kVR * (nw - w) - 1);
+  const int last = (dist + 2 + P - A.halo_y) / 2;            // the wave's last sweep
+  const bool own = kVR * w >= A.halo_y && kVR * (w + 1) <= kVR * nw - A.halo_y;
+  const bool colo = 2 * lane >= A.halo_x && 2 * lane < 128 - A.halo_x && i0 <= n1;
+  const int W = n1 + 3;
+  auto log = [&](int it, double rr) {                        // the wave's share of sweep it's residual
+    const double t = wave_sum(colo ? rr : 0.0);
+    if (lane == 0) ws[it - 1][w] = t;
+  };
+  double rb = 0.0;
+  for (int it = 1; it <= A.kexec; ++it) {
+    if (it <= last) {
+      if (own && it > 1) log(it - 1, rb + strip_pass64<kVR, ISO, true, true, true>(s, k, e));
+      else strip_pass64<kVR, ISO, true, false, true>(s, k, e);
     }
-    T* uout = A.rot[(s_c0 + k0 + s) % kRot];
-    double rr = 0.0;
-    for (int q0 = threadIdx.x; q0 < kTP * kTYP; q0 += NB * kSweepThreads) {
-      int x[NB], gi[NB], gj[NB];
-      int8_t m[NB];
-      T c[NB], w[NB], e[NB], n[NB], so[NB], bb[NB];
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        const int q = q0 + k * kSweepThreads;
-        const int qq = q < kTP * kTYP ? q : 0;
-        const int tr = qq / kTP, tc = qq - tr * kTP;
-        x[k] = (kHalo + tr) * RW + kHalo + tc;
-        gi[k] = (q < kTP * kTYP && tc < tw && tr < th) ? gi0 + kHalo + tc : n1 + 2;   // n1 + 2: not this tile's
-        gj[k] = gj0 + kHalo + tr;
-        m[k] = sbc[x[k]];
-        c[k] = su[x[k]]; w[k] = su[x[k] - 1]; e[k] = su[x[k] + 1];
-        n[k] = su[x[k] + RW]; so[k] = su[x[k] - RW]; bb[k] = sb[x[k]];
-      }
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        if (gi[k] > n1 + 1 || gj[k] > n2 + 1) continue;
-        if (m[k] == -1) rr += fabs(sor_resid(c[k], bb[k], w[k], n[k], so[k], e[k], aw, an, ac));
-        uout[(int64_t)gj[k] * W + gi[k]] = c[k];
-      }
-    }
-    rr = wave_sum(rr);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = rr;
     __syncthreads();
-    if (threadIdx.x < 64) {  // fixed-order sum of the 16 wave sums
-      const double t = wave_sum(threadIdx.x < kSweepThreads / 64 ? ws[threadIdx.x] : 0.0);
-      if (threadIdx.x == 0) A.partials[(size_t)((k0 + s) % kRing) * nb + bid] = t;
+    if (it <= last) {
+      if (own) {
+        rb = strip_pass64<kVR, ISO, false, true, true>(s, k, e);
+        double* uout = A.rot[(c0 + A.k0 + it) % kRot];
+        if (colo) {
+#pragma unroll
+          for (int r = 0; r < kVR; ++r)
+            if (j0 + r <= n2) *(D2*)(uout + (int64_t)(j0 + r) * W + i0) = D2{s.u[r][0], s.u[r][1]};
+        }
+      } else {
+        strip_pass64<kVR, ISO, false, false, true>(s, k, e);
+      }
     }
+    __syncthreads();
+  }
+  if (own) log(A.kexec, rb + strip_pass64<kVR, ISO, true, true, false>(s, k, e));
+  __syncthreads();
+  const int w0 = A.halo_y / kVR, nown = nw - 2 * w0;
+  for (int it = 1 + w; it <= A.kexec; it += nw) {
+    const double t = wave_sum(lane < nown ? ws[it - 1][w0 + lane] : 0.0);
+    if (lane == 0) A.partials[(size_t)((A.k0 + it) % kRing) * A.t.stride + bid] = t;
   }
 }
 
 // restriction, mg.f90:335-444, from a multi-block level: resolves the fine
-// level's down visit, writes the coarse right-hand side and zeroes the
-// coarse correction in the buffer the coarse level's visit starts from.
-template <typename T>
+// level's down visit and writes the coarse right-hand side; `zero`, when not
+// null, is the coarse correction, cleared for the single-workgroup kernel (a
+// multi-block level's down visit knows that it starts from zero).
 struct RestrictArgs {
   VisitRef vf;
-  T* frot[kRot];
-  const T* fb;
+  const double* frot[kRot];
+  const double* fb;
   const int8_t* fbc;
   int n1, n2;
-  T aw, an, ac;
-  T* r2h;
-  const int8_t* bc2h;
-  T* crot[kRot];
-  LevelCtrl* cctrl;        // null when the coarse level runs in k_tail
-  int cepoch;
+  StripCoef<double> k;
+  double* r2h;
+  double* zero;
 };
 
-// A block restricts a tile of kRcx x kRcy coarse nodes: the fine residuals
-// its nodes weight (2 kRcx + 1 by 2 kRcy + 1 positions) are evaluated once
-// each into LDS, with their bc flags, and every coarse node then combines
-// nine of them; the residual at a position is getres at the position clamped
-// into the interior, as restrict_node evaluates it.  Each block also zeroes
-// a slice of the coarse correction.
-constexpr int kRcx = 32, kRcy = 8;
-constexpr int kRrx = 2 * kRcx + 1, kRry = 2 * kRcy + 1;
-constexpr int kRestrictThreads = kRcx * kRcy;
-
-template <typename T>
-__global__ __launch_bounds__(kRestrictThreads) void k_restrict(RestrictArgs<T> A) {
-  constexpr int kRN = kRrx * kRry;
-  constexpr int kIt = (kRN + kRestrictThreads - 1) / kRestrictThreads;
-  __shared__ int s_fb, s_cb;
-  __shared__ T sr[kRN];
-  __shared__ int8_t sf[kRN];
-  const int t = threadIdx.x;
-  if (t < 64) {
-    const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-    Resolved r = resolve_visit(A.vf, writer, false);
-    if (t == 0) {
-      s_fb = r.buf < 0 ? 0 : r.buf;
-      s_cb = A.cctrl ? A.cctrl->cur[(A.cepoch - 1) & 1] : 0;
-    }
-  }
-  __syncthreads();
-  const T* u = A.frot[s_fb];
-  T* e2h = A.crot[s_cb];
+// A block's region is 128 x 32 nodes with 2 around the tile; bound by latency
+// (the visit's outcome, then the loads): 1025 x 513 nodes 20 us with every
+// residual's neighbours read from memory, 7.8 so.
+constexpr int kRestrictWaves = 8;
+template <bool ISO>
+__global__ __launch_bounds__(64 * kRestrictWaves) void k_restrict64(RestrictArgs A) {
+  constexpr int NW = kRestrictWaves, E = (NW + 2) * 64;
+  __shared__ double ed[4 * E];
+  __shared__ double s_res[kS + 1];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int n1 = A.n1, n2 = A.n2, m1 = n1 / 2, m2 = n2 / 2;
-  const int64_t W = n1 + 3;
-  {
+  const int nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
+  const int i0 = (int)blockIdx.x * 124 + 2 * lane, j0 = (int)blockIdx.y * (NW * kVR - 4) + w * kVR;
+  if (A.zero) {
     const int64_t nc = (int64_t)(m1 + 3) * (m2 + 3);
-    const int64_t nbk = (int64_t)gridDim.x * gridDim.y, bk = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    const int64_t per = (nc + nbk - 1) / nbk, q1 = min(nc, (bk + 1) * per);
-    for (int64_t q = bk * per + t; q < q1; q += kRestrictThreads) e2h[q] = (T)0;
+    for (int64_t q = (int64_t)bid * blockDim.x + threadIdx.x; q < nc; q += (int64_t)nb * blockDim.x) A.zero[q] = 0.0;
   }
-  const int ci0 = 1 + (int)blockIdx.x * kRcx, cj0 = 1 + (int)blockIdx.y * kRcy;
-  const int fa0 = 2 * ci0 - 2, fc0 = 2 * cj0 - 2;   // fine position of region (0, 0)
-  {
-    T g[kIt];
-    int8_t fl[kIt];
+  const int buf = resolve_visit(A.vf, bid == 0, s_res).buf;
+  Strip<double, kVR, ISO> s;
+  strip_region_load<kVR, ISO>(s, A.frot[buf], A.frot[0], A.fb, A.fbc, n1, n2, i0, j0);
+  const StripCoef<double> k = strip_hold(A.k);
 #pragma unroll
-    for (int k = 0; k < kIt; ++k) {
-      const int q = t + k * kRestrictThreads;
-      const int qq = q < kRN ? q : 0;
-      const int y = qq / kRrx, x = qq - y * kRrx;
-      const int a = fa0 + x, c = fc0 + y;
-      const int ac = a < 1 ? 1 : (a > n1 + 1 ? n1 + 1 : a);
-      const int cc = c < 1 ? 1 : (c > n2 + 1 ? n2 + 1 : c);
-      g[k] = getres(u, A.fb, ac, cc, n1, A.aw, A.an, A.ac);
-      fl[k] = (a <= n1 + 2 && c <= n2 + 2) ? A.fbc[(int64_t)c * W + a] : (int8_t)1;
-    }
-#pragma unroll
-    for (int k = 0; k < kIt; ++k) {
-      const int q = t + k * kRestrictThreads;
-      if (q < kRN) { sr[q] = g[k]; sf[q] = fl[k]; }
-    }
+  for (int r = 0; r < kVR; ++r) {
+    s.products(k, r, 0);
+    s.products(k, r, 1);
   }
+  Edges<double> e{ed, E, 64, (w + 1) * 64 + lane, true};
+  if (w == 0) ed[E + lane] = ed[3 * E + lane] = 0.0;
+  if (w == NW - 1) ed[e.o + 64] = ed[2 * E + e.o + 64] = 0.0;
+  strip_publish_black<double, kVR, ISO>(s, e);
+  ed[e.o] = s.north(0, 1);                         // red edges
+  ed[E + e.o] = s.north(kVR - 1, 0);
   __syncthreads();
-  const int ti = t % kRcx, tj = t / kRcx;
-  const int i = ci0 + ti, j = cj0 + tj;
-  if (i > m1 + 1 || j > m2 + 1) return;
-  T out = (T)0;
-  if (A.bc2h[(int64_t)j * (m1 + 3) + i] <= 0) {
-    const int ir = 2 * i - 1, jr = 2 * j - 1;
-    const int x0 = 2 * ti + 1, y0 = 2 * tj + 1;      // region position of (ir, jr)
-    auto R = [&](int dx, int dy) { return sr[(y0 + dy) * kRrx + x0 + dx]; };
-    auto B = [&](int dx, int dy) { return sf[(y0 + dy) * kRrx + x0 + dx]; };
-    const bool xe = ir != n1 + 1, xw = ir != 1, yn = jr != n2 + 1, ys = jr != 1;
-    const bool f1 = xe && yn && B(1, 1) <= 0;
-    const bool f2 = xe && B(1, 0) <= 0;
-    const bool f3 = B(1, -1) <= 0 && xe && ys;
-    const bool f4 = B(0, -1) <= 0 && ys;
-    const bool f5 = B(-1, -1) <= 0 && xw && ys;
-    const bool f6 = B(-1, 0) <= 0 && xw;
-    const bool f7 = B(-1, 1) <= 0 && xw && yn;
-    const bool f8 = B(0, 1) <= 0 && yn;
-    out = full_weight<T>(R(0, 0), R(1, 1), R(1, 0), R(1, -1), R(0, -1), R(-1, -1), R(-1, 0), R(-1, 1), R(0, 1),
-                         f1, f2, f3, f4, f5, f6, f7, f8);
+  double out[kVR / 2];
+  strip_restrict<double, kVR, ISO, false>(s, k, e, out);
+  if (lane == 0 || lane == 63 || i0 + 1 > n1) return;
+#pragma unroll
+  for (int t = 0; t < kVR / 2; ++t) {
+    const int r = 2 * t + 1, lr = w * kVR + r, j = j0 + r;
+    if (lr < 2 || lr >= NW * kVR - 2 || j > n2) continue;
+    A.r2h[(int64_t)((j + 1) / 2 - 1) * (m1 + 1) + i0 / 2] = out[t];
   }
-  A.r2h[(int64_t)(j - 1) * (m1 + 1) + (i - 1)] = out;
 }
 
-// prolongation into a multi-block level from the level below (resolving the
-// coarse level's up visit when it is multi-block itself)
-template <typename T>
-struct ProlongArgs {
-  T* frot[kRot];
-  LevelCtrl* fctrl;
-  int fepoch;              // epoch of the fine level's coming up visit
-  const int8_t* bc;
-  int n1, n2;
-  T* crot[kRot];
-  int coarse_mb;
-  VisitRef vc;
-};
-
-template <typename T>
-__global__ __launch_bounds__(128) void k_prolong(ProlongArgs<T> A) {
-  __shared__ int s_fb, s_cb;
-  if (threadIdx.x < 64) {
-    int cb = 0;
-    if (A.coarse_mb) {
-      const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-      Resolved r = resolve_visit(A.vc, writer, false);
-      cb = r.buf < 0 ? 0 : r.buf;
-    }
-    if (threadIdx.x == 0) {
-      s_cb = cb;
-      s_fb = A.fctrl->cur[(A.fepoch - 1) & 1];
-    }
-  }
-  __syncthreads();
-  const int m1 = A.n1 / 2, m2 = A.n2 / 2;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  if (i > m1 + 1) return;
-  for (int j = blockIdx.y + 1; j <= m2 + 1; j += gridDim.y)
-    prolong_node<T>(A.frot[s_fb], A.bc, A.n1, (const T*)A.crot[s_cb], m1, i, j);
-}
-
-// FP64 mode, end of a V-cycle on a multi-block finest level: resolve the up
-// visit and copy its result into phi (buffer 0) when it lies elsewhere.
+// end of a V-cycle on a multi-block finest level: records the up visit
 struct Finish64Args {
   VisitRef v;
-  double* rot[kRot];
-  int n1, n2;
   int* status;             // sweeps of the visit, 0 if not finished
 };
 
-__global__ __launch_bounds__(256) void k_finish64(Finish64Args A) {
-  __shared__ int s_buf, s_ks;
-  if (threadIdx.x < 64) {
-    const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-    Resolved r = resolve_visit(A.v, writer, true);
-    if (threadIdx.x == 0) {
-      s_buf = r.buf;
-      s_ks = r.ks;
-      if (writer) *A.status = r.ks;
-    }
-  }
-  __syncthreads();
-  if (s_ks == 0 || s_buf == 0) return;
-  const int64_t W = A.n1 + 3;
-  for (int j = blockIdx.y + 1; j <= A.n2 + 1; j += gridDim.y)
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x + 1; i <= A.n1 + 1; i += gridDim.x * blockDim.x)
-      A.rot[0][(int64_t)j * W + i] = A.rot[s_buf][(int64_t)j * W + i];
+__global__ __launch_bounds__(64 * (kS + 1)) void k_finish64(Finish64Args A) {
+  __shared__ double s_res[kS + 1];
+  const Resolved r = resolve_visit(A.v, true, s_res);
+  if (threadIdx.x == 0) *A.status = r.ks;
+}
+
+// end of a solve: the finest level's state from buffer `u_in` to phi (buffer 0)
+__global__ __launch_bounds__(256) void k_settle64(double* __restrict__ phi, const double* __restrict__ u_in,
+                                                  const int8_t* __restrict__ bc, int64_t n, LevelCtrl* c) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q == 0) c->cur[0] = c->cur[1] = 0;
+  if (q < n && bc[q] == -1) phi[q] = u_in[q];
 }
 
 // Mixed mode with the finest level in k_tail: phi += e (bcnd <= 0 nodes) at
@@ -1240,87 +1120,122 @@ int* d_visit_of(lepic_ctx* ctx) { return (int*)(ctx->d_scalar + 64); }
 double* d_vres_of(lepic_ctx* ctx) { return ctx->d_scalar + 32; }
 int* d_status_of(lepic_ctx* ctx) { return (int*)(ctx->d_scalar + 64) + kVisitLog; }
 
-VisitRef visit_ref(lepic_ctx* ctx, int l, int epoch, int dig, int nr, int ig, double eps, int nexec,
-                   int klast0 = -1) {
+// A launch of kexec sweeps: the halo, the waves of a block and the grid.
+struct VisitShape {
+  int hx, hy, nw;
+  dim3 g;
+  int nb() const { return (int)(g.x * g.y); }
+};
+
+// The fewest waves of 8, 12, 16 whose launch has at most one block per CU
+// (a block of 8 waves passes its rows in half the time of one of 16, but halos
+// cost it more of them: 8-row tiles in 32 rows against 40 in 64 for 5 sweeps);
+// larger grids take 16.
+constexpr int kVisitBlocks = 256;
+
+VisitShape visit_shape(const Level& L, int kexec) {
+  VisitShape S;
+  S.hx = 2 * kexec + 2;
+  S.hy = (2 * kexec + 1 + kVR - 1) / kVR * kVR;
+  const int tx = 128 - 2 * S.hx;
+  for (S.nw = 8;; S.nw += 4) {
+    const int ty = S.nw * kVR - 2 * S.hy;
+    if (ty < 8) continue;
+    S.g = dim3((unsigned)((L.n1 - 1 + tx - 1) / tx), (unsigned)((L.n2 - 1 + ty - 1) / ty));
+    if (S.nw == kVisitMaxWaves || S.nb() <= kVisitBlocks) return S;
+  }
+}
+
+// How a multi-block level's FP64 visit runs: the reference's exit test
+// (sors.f90:371-377) decides; one launch of `first` sweeps (one more than the
+// same visit took in the previous V-cycle: most visits then finish in one
+// launch of a small halo) and one of the others up to kNr, which first tests
+// the first one's sweeps and returns at once when the visit has stopped there.
+constexpr int kFirstMax = 5;
+static_assert(kNr - 2 <= kS && kFirstMax <= kS && kNr - kFirstMax <= kS, "a visit takes two launches");
+
+VisitRef visit_ref(lepic_ctx* ctx, int l, int epoch, int dig, int nr, int ig, double eps, int nexec, int klast0,
+                   int before) {
   Level& L = ctx->lv[l];
   VisitRef v;
   v.ctrl = ctx->d_ctrl + l;
-  v.nb = L.nbx * L.nby;
-  v.partials = L.partials;
-  v.epoch = epoch; v.dig = dig; v.nr = nr; v.ig = ig; v.eps = eps;
+  v.t = StopTest{L.partials, L.part_stride, before ? visit_shape(L, before).nb() : 0,
+                 visit_shape(L, nexec - klast0).nb(), dig, nr, eps};
+  v.epoch = epoch; v.ig = ig;
   v.nexec = nexec;
-  v.klast0 = klast0 >= 0 ? klast0 : ((nexec - 1) / kS) * kS;
+  v.klast0 = klast0;
   v.visit = d_visit_of(ctx);
   v.vres = d_vres_of(ctx);
   return v;
 }
 
-// Start of the last launch of a visit whose launches cover sweeps
-// k0+1 .. k_end, the first of them `first` sweeps and the others kS.
-int last_launch_start(int k0, int k_end, int first) {
-  int k = k0, last = k0;
-  for (int size = std::min(first, kS); k < k_end; size = kS) {
-    last = k;
-    k += std::min(size, k_end - k);
-  }
-  return last;
+// the down or up visit of a V-cycle
+VisitRef cycle_visit_ref(lepic_ctx* ctx, int l, int epoch, bool up, double eps) {
+  const int f = up ? ctx->lv[l].first_up : ctx->lv[l].first_dn, ng = ctx->ng;
+  return visit_ref(ctx, l, epoch, up ? ng - l : l - ng, kNr, up ? 2 * ng - l : l, eps, kNr, f, f);
 }
 
-// How a multi-block level's FP64 visit runs: the reference's exit test
-// (sors.f90:371-377) decides, the first launch `first` sweeps and
-// continuations up to kNr.
-struct VisitPlan {
-  int k_end, first, klast0;
-};
-
-VisitPlan visit_plan(const Level& L, bool up) {
-  const int f = up ? L.first_up : L.first_dn;
-  return VisitPlan{kNr, f, last_launch_start(0, kNr, f)};
+StripCoef<double> strip_coef64(const Level& L) {
+  StripCoef<double> k;
+  k.aw = L.aw; k.an = L.an; k.ac = L.ac;
+  k.om = 1.4;                                     // iterative_solver.f90:27
+  k.om1 = 1.0 - k.om;
+  k.rac = 1.0 / k.ac;
+  k.racl = std::fma(-k.rac, k.ac, 1.0) / k.ac;
+  return k;
 }
 
-// the launch size KS (halo 2 KS + 1) is kexec
-template <int kTX, int TY, int NT>
-void launch_sweeps(lepic_ctx* ctx, const Level& L, const SweepArgs<double>& A, int k, int kexec, int kchk) {
-  const dim3 g(L.nbx, L.nby);
-  if (kexec <= 2) hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, 2>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-  else if (kexec <= 3) hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, 3>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-  else if (kexec <= 4) hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, 4>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-  else hipLaunchKernelGGL((k_sweeps<double, kTX, TY, NT, kS>), g, dim3(NT), 0, ctx->stream, A, k, kexec, kchk);
-}
-
-// launches of one FP64 visit of a multi-block level: sweeps k0+1 .. k_end, the
-// first launch `first` sweeps (one more than the same visit took in the
-// previous V-cycle: most visits then finish in one launch of a small
-// halo), the others kS; each continuation first tests the previous launch's
-// sweeps and returns at once when the visit has stopped there
-int launch_visit(lepic_ctx* ctx, int l, int epoch, int dig, int nr, double eps, int k0, int k_end, int first = kS) {
+VisitArgs visit_args(lepic_ctx* ctx, int l, int epoch, int dig, int nr, double eps) {
   Level& L = ctx->lv[l];
-  SweepArgs<double> A;
+  VisitArgs A{};
   for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<double>(L, r);
   A.b = L.b;
   A.bc = L.bc;
   A.n1 = L.n1; A.n2 = L.n2;
-  A.aw = L.aw; A.an = L.an; A.ac = L.ac;
-  A.omega = 1.4;                                  // iterative_solver.f90:27
+  A.k = strip_coef64(L);
   A.ctrl = ctx->d_ctrl + l;
   A.partials = L.partials;
-  A.nbx = L.nbx; A.nby = L.nby;
-  A.epoch = epoch; A.dig = dig; A.nr = nr; A.eps = eps;
-  int kchk = 0;
-  for (int k = k0, size = std::min(std::max(first, 1), kS); k < k_end; size = kS) {
-    const int kexec = std::min(size, k_end - k);
-    if (L.small_tiles) launch_sweeps<kSmallTX, kSmallTileY, kSmallThreads>(ctx, L, A, k, kexec, kchk);
-    else launch_sweeps<kTX, kTileY, kSweepThreads>(ctx, L, A, k, kexec, kchk);
-    kchk = k + 1;
-    k += kexec;
-  }
+  A.t = StopTest{L.partials, L.part_stride, 0, 0, dig, nr, eps};
+  A.epoch = epoch;
+  return A;
+}
+
+// one launch: sweeps k0+1 .. k0+kexec; the one before it ran sweeps kchk .. k0
+int launch_sweeps(lepic_ctx* ctx, int l, VisitArgs& A, int k0, int kexec, int kchk) {
+  const Level& L = ctx->lv[l];
+  const VisitShape S = visit_shape(L, kexec);
+  A.k0 = k0; A.kexec = kexec; A.kchk = kchk;
+  A.halo_x = S.hx; A.halo_y = S.hy;
+  if (L.aw == L.an) hipLaunchKernelGGL(k_visit64<true>, S.g, dim3(64 * S.nw), 0, ctx->stream, A);
+  else hipLaunchKernelGGL(k_visit64<false>, S.g, dim3(64 * S.nw), 0, ctx->stream, A);
   LEPIC_HIP(hipGetLastError());
+  A.t.nb0 = A.t.nb1;                              // for the launch after it
+  A.t.nb1 = S.nb();
+  A.zero = 0;
+  A.crot[0] = nullptr;
   return 0;
 }
 
+// the down or up visit of a V-cycle; the up visit starts with the prolonged
+// correction of the level below
+int launch_visit(lepic_ctx* ctx, int l, int epoch, bool up, double eps) {
+  Level& L = ctx->lv[l];
+  const int ng = ctx->ng, first = up ? L.first_up : L.first_dn;
+  VisitArgs A = visit_args(ctx, l, epoch, up ? ng - l : l - ng, kNr, eps);
+  A.zero = !up && l > 1;
+  if (up) {
+    Level& C = ctx->lv[l + 1];
+    for (int r = 0; r < kRot; ++r) A.crot[r] = C.mb ? rot_of<double>(C, r) : C.u;
+    A.coarse_mb = C.mb;
+    if (C.mb) A.vc = cycle_visit_ref(ctx, l + 1, epoch, true, eps);
+  }
+  if (int rc = launch_sweeps(ctx, l, A, 0, first, 0)) return rc;
+  return launch_sweeps(ctx, l, A, first, kNr - first, 1);
+}
+
 // ---- mixed form: visits of fixed sweep counts in k_tile32 ----
-StripCoef strip_coef(const Level& L, float omega) {
-  StripCoef k;
+StripCoef<float> strip_coef(const Level& L, float omega) {
+  StripCoef<float> k;
   k.aw = (float)L.aw; k.an = (float)L.an; k.ac = (float)L.ac;
   k.om = omega; k.om1 = 1.0f - omega; k.rac = 1.0f / k.ac;
   return k;
@@ -1371,13 +1286,13 @@ int tile_down(lepic_ctx* ctx, int l) {
   const int h = 2 * nsw + 2;
   const int64_t nb = (int64_t)((L.n1 - 1 + 127 - 2 * h) / (128 - 2 * h)) * ((L.n2 - 1 + 63 - 2 * h) / (64 - 2 * h));
   A.nsw = nsw;
-  if (nsw > kS && nb > kTileMaxBlocks) {
-    A.nsw = kS;
+  if (nsw > kTileSplit && nb > kTileMaxBlocks) {
+    A.nsw = kTileSplit;
     A.u_out = rot_of<float>(L, 1);
     if (int rc = launch_tile32(ctx, L, A)) return rc;
     A.u_in = rot_of<float>(L, 1);
     A.u_out = rot_of<float>(L, 0);
-    A.nsw = nsw - kS;
+    A.nsw = nsw - kTileSplit;
   }
   A.r2h = ctx->lv[l + 1].bf;
   return launch_tile32(ctx, L, A);
@@ -1397,51 +1312,22 @@ int tile_up(lepic_ctx* ctx, int l) {
   return launch_tile32(ctx, L, A);
 }
 
-template <typename T>
-int launch_restrict(lepic_ctx* ctx, int l, bool f32, int epoch, double eps) {
-  const int ng = ctx->ng;
+int launch_restrict(lepic_ctx* ctx, int l, int epoch, double eps) {
   Level& F = ctx->lv[l];
   Level& C = ctx->lv[l + 1];
-  RestrictArgs<T> A;
-  const VisitPlan pf = visit_plan(F, false);
-  A.vf = visit_ref(ctx, l, epoch, l - ng, kNr, l, eps, pf.k_end, pf.klast0);
-  for (int r = 0; r < kRot; ++r) A.frot[r] = rot_of<T>(F, r);
-  A.fb = b_of<T>(F, f32);
+  RestrictArgs A;
+  A.vf = cycle_visit_ref(ctx, l, epoch, false, eps);
+  for (int r = 0; r < kRot; ++r) A.frot[r] = rot_of<double>(F, r);
+  A.fb = F.b;
   A.fbc = F.bc;
   A.n1 = F.n1; A.n2 = F.n2;
-  A.aw = (T)F.aw; A.an = (T)F.an; A.ac = (T)F.ac;
-  A.r2h = b_of<T>(C, f32);
-  A.bc2h = C.bc;
-  for (int r = 0; r < kRot; ++r) A.crot[r] = C.mb ? rot_of<T>(C, r) : u_of<T>(C, f32);
-  A.cctrl = C.mb ? ctx->d_ctrl + (l + 1) : nullptr;
-  A.cepoch = epoch;
-  const dim3 g((unsigned)((C.n1 + 1 + kRcx - 1) / kRcx), (unsigned)((C.n2 + 1 + kRcy - 1) / kRcy));
-  hipLaunchKernelGGL(k_restrict<T>, g, dim3(kRestrictThreads), 0, ctx->stream, A);
-  LEPIC_HIP(hipGetLastError());
-  return 0;
-}
-
-template <typename T>
-int launch_prolong(lepic_ctx* ctx, int l, bool f32, int epoch_up, double eps) {
-  const int ng = ctx->ng;
-  Level& F = ctx->lv[l];
-  Level& C = ctx->lv[l + 1];
-  ProlongArgs<T> A;
-  for (int r = 0; r < kRot; ++r) A.frot[r] = rot_of<T>(F, r);
-  A.fctrl = ctx->d_ctrl + l;
-  A.fepoch = epoch_up;
-  A.bc = F.bc;
-  A.n1 = F.n1; A.n2 = F.n2;
-  for (int r = 0; r < kRot; ++r) A.crot[r] = C.mb ? rot_of<T>(C, r) : u_of<T>(C, f32);
-  A.coarse_mb = C.mb ? 1 : 0;
-  if (C.mb)
-  {
-    const VisitPlan pc = visit_plan(C, true);
-    A.vc = visit_ref(ctx, l + 1, epoch_up, ng - (l + 1), kNr, 2 * ng - (l + 1), eps, pc.k_end, pc.klast0);
-  }
-  else A.vc = VisitRef{};
-  dim3 g((C.n1 + 1 + 127) / 128, std::min(C.n2 + 1, kRowBlocks));
-  hipLaunchKernelGGL(k_prolong<T>, g, dim3(128), 0, ctx->stream, A);
+  A.k = strip_coef64(F);
+  A.r2h = C.b;
+  A.zero = C.mb ? nullptr : C.u;
+  constexpr int tx = 124, ty = kRestrictWaves * kVR - 4;
+  const dim3 g((unsigned)((F.n1 - 1 + tx - 1) / tx), (unsigned)((F.n2 - 1 + ty - 1) / ty));
+  if (F.aw == F.an) hipLaunchKernelGGL(k_restrict64<true>, g, dim3(64 * kRestrictWaves), 0, ctx->stream, A);
+  else hipLaunchKernelGGL(k_restrict64<false>, g, dim3(64 * kRestrictWaves), 0, ctx->stream, A);
   LEPIC_HIP(hipGetLastError());
   return 0;
 }
@@ -1627,34 +1513,25 @@ int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps) {
 
 // One FP64 V-cycle (mg.f90:85-225): levels 1..Ls-1 multi-block, Ls..ng in
 // k_tail; then the end-of-cycle kernel.
+int launch_finish64(lepic_ctx* ctx, const VisitRef& v) {
+  const Finish64Args A{v, d_status_of(ctx)};
+  hipLaunchKernelGGL(k_finish64, dim3(1), dim3(64 * (kS + 1)), 0, ctx->stream, A);
+  LEPIC_HIP(hipGetLastError());
+  return 0;
+}
+
 int vcycle64(lepic_ctx* ctx, int k, double eps) {
-  const int ng = ctx->ng, Ls = ctx->Lc;
+  const int Ls = ctx->Lc;
   const int e_dn = ctx->mg_epoch + 1, e_up = ctx->mg_epoch + 2;
   ctx->mg_epoch += 2;
   for (int l = 1; l < Ls; ++l) {  // down leg
-    const VisitPlan pl = visit_plan(ctx->lv[l], false);
-    if (int rc = launch_visit(ctx, l, e_dn, l - ng, kNr, eps, 0, pl.k_end, pl.first)) return rc;
-    if (int rc = launch_restrict<double>(ctx, l, false, e_dn, eps)) return rc;
+    if (int rc = launch_visit(ctx, l, e_dn, false, eps)) return rc;
+    if (int rc = launch_restrict(ctx, l, e_dn, eps)) return rc;
   }
   if (int rc = launch_tail<double>(ctx, false, k, eps)) return rc;
-  for (int l = Ls - 1; l >= 1; --l) {  // up leg
-    if (int rc = launch_prolong<double>(ctx, l, false, e_up, eps)) return rc;
-    const VisitPlan pl = visit_plan(ctx->lv[l], true);
-    if (int rc = launch_visit(ctx, l, e_up, ng - l, kNr, eps, 0, pl.k_end, pl.first)) return rc;
-  }
-  Level& L1 = ctx->lv[1];
-  if (L1.mb) {
-    Finish64Args A;
-    const VisitPlan p1 = visit_plan(L1, true);
-    A.v = visit_ref(ctx, 1, e_up, ng - 1, kNr, 2 * ng - 1, eps, p1.k_end, p1.klast0);
-    for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<double>(L1, r);
-    A.n1 = L1.n1; A.n2 = L1.n2;
-    A.status = d_status_of(ctx);
-    hipLaunchKernelGGL(k_finish64, dim3((unsigned)((L1.n1 + 1 + 255) / 256), std::min(L1.n2 + 1, kRowBlocks)),
-                       dim3(256), 0, ctx->stream, A);
-  }
-  LEPIC_HIP(hipGetLastError());
-  return 0;
+  for (int l = Ls - 1; l >= 1; --l)  // up leg
+    if (int rc = launch_visit(ctx, l, e_up, true, eps)) return rc;
+  return ctx->lv[1].mb ? launch_finish64(ctx, cycle_visit_ref(ctx, 1, e_up, true, eps)) : 0;
 }
 
 // One V-cycle of the mixed form on the FP32 correction equation; adds the
@@ -1716,14 +1593,6 @@ int read_back(lepic_ctx* ctx, int* visit, double* vres, double* resid_sum) {
 
 namespace lepic {
 
-// tiles of t nodes along a side of `nodes` nodes; a single node left over
-// joins the last tile (k_sweeps' tiles can be one node wider)
-static int tiles_of(int nodes, int t) {
-  int n = (nodes + t - 1) / t;
-  if (n > 1 && nodes - (n - 1) * t == 1) --n;
-  return n;
-}
-
 int poisson_setup(lepic_ctx* ctx) {
   const int ng = ctx->ng;
   const double eps0 = ctx->g.eps0;
@@ -1778,22 +1647,15 @@ int poisson_setup(lepic_ctx* ctx) {
       LEPIC_HIP(hipMemsetAsync(L.rot[1], 0, nn * 4, ctx->stream));
       continue;
     }
-    L.first_dn = L.first_up = kS;
+    L.first_dn = L.first_up = kFirstMax;
     L.rot[0] = L.u;
     for (int r = 1; r < kRot; ++r) {
       LEPIC_HIP(hipMalloc(&L.rot[r], nn * 8));
       LEPIC_HIP(hipMemsetAsync(L.rot[r], 0, nn * 8, ctx->stream));
     }
-    L.nbx = tiles_of(L.n1 + 1, kTX);
-    L.nby = tiles_of(L.n2 + 1, kTileY);
-    // few wide tiles leave most CUs idle: the level takes small tiles, whose
-    // launch latency is lower (each block has less than half the nodes)
-    L.small_tiles = L.nbx * L.nby < kSmallTileBelow;
-    if (L.small_tiles) {
-      L.nbx = tiles_of(L.n1 + 1, kSmallTX);
-      L.nby = tiles_of(L.n2 + 1, kSmallTileY);
-    }
-    const size_t np = (size_t)kRing * L.nbx * L.nby;
+    L.part_stride = 0;
+    for (int k = 1; k <= kS; ++k) L.part_stride = std::max(L.part_stride, visit_shape(L, k).nb());
+    const size_t np = (size_t)kRing * L.part_stride;
     LEPIC_HIP(hipMalloc(&L.partials, np * 8));
     LEPIC_HIP(hipMemsetAsync(L.partials, 0, np * 8, ctx->stream));
   }
@@ -1875,6 +1737,16 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
   info->res0 = r0 / alpha;
   int k = 1;
   info->status = 0;
+  // FP64 with a multi-block finest level: the buffer that holds its state
+  // (the visits' sweeps add up), and the state's way back to phi
+  int state = 0;
+  auto settle = [&]() -> int {
+    if (state == 0) return 0;
+    hipLaunchKernelGGL(k_settle64, g1, dim3(256), 0, ctx->stream, ctx->phi, (const double*)ctx->lv[1].rot[state],
+                       (const int8_t*)ctx->bc, n, ctx->d_ctrl + 1);
+    LEPIC_HIP(hipGetLastError());
+    return 0;
+  };
   for (;;) {
     if (ng == 1 && ctx->lv[1].mb) {
       // red-black SOR alone on a multi-block grid (mg.f90:197-198 with
@@ -1883,19 +1755,15 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
       const int nr = (k == 1) ? 1000000 : kNr;
       const int e = ++ctx->mg_epoch;
       int k0 = 0, ks = 0;
+      VisitArgs A = visit_args(ctx, 1, e, 0, nr, alpha * eps);
       while (k0 < nr) {
-        const int k_end = std::min(nr, k0 + 16 * kS);
-        if (int rc = launch_visit(ctx, 1, e, 0, nr, alpha * eps, k0, k_end)) return rc;
-        k0 = k_end;
-        Level& L1 = ctx->lv[1];
-        Finish64Args A;
-        A.v = visit_ref(ctx, 1, e, 0, nr, 1, alpha * eps, k0);
-        for (int r = 0; r < kRot; ++r) A.rot[r] = rot_of<double>(L1, r);
-        A.n1 = L1.n1; A.n2 = L1.n2;
-        A.status = d_status_of(ctx);
-        hipLaunchKernelGGL(k_finish64, dim3((unsigned)((L1.n1 + 1 + 255) / 256), std::min(L1.n2 + 1, kRowBlocks)),
-                           dim3(256), 0, ctx->stream, A);
-        LEPIC_HIP(hipGetLastError());
+        const int k_end = std::min(nr, k0 + 16 * kFirstMax);
+        for (int kchk = 0; k0 < k_end; k0 += kFirstMax) {   // nr is a multiple of kFirstMax
+          if (int rc = launch_sweeps(ctx, 1, A, k0, kFirstMax, kchk)) return rc;
+          kchk = k0 + 1;
+        }
+        if (int rc = launch_finish64(ctx, visit_ref(ctx, 1, e, 0, nr, 1, alpha * eps, k0, k0 - kFirstMax,
+                                                    kFirstMax))) return rc;
         LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_status_of(ctx), 4, hipMemcpyDeviceToHost, ctx->stream));
         LEPIC_HIP(hipStreamSynchronize(ctx->stream));
         std::memcpy(&ks, ctx->h_pinned, 4);
@@ -1916,6 +1784,7 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
       vres[2 * ng - 1] = rs;
     }
     const int nvis = 2 * ng - 1;
+    if (ctx->lv[1].mb && !mixed) state = (state + visit[1] + (ng > 1 ? visit[nvis] : 0)) % kRot;
     if (ng > 1)
       for (int l = 1; l < ctx->Lc; ++l) {
         Level& L = ctx->lv[l];
@@ -1923,8 +1792,8 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
         if (!mixed) {
           // one sweep more than last time: a spare sweep costs less than a
           // continuation launch when the count grows by one
-          L.first_dn = std::min(std::max(visit[l] + 1, 2), kS);
-          L.first_up = std::min(std::max(visit[2 * ng - l] + 1, 2), kS);
+          L.first_dn = std::min(std::max(visit[l] + 1, 2), kFirstMax);
+          L.first_up = std::min(std::max(visit[2 * ng - l] + 1, 2), kFirstMax);
         } else {   // the mixed form's fixed counts
           visit[l] = l == 1 ? kFineDn : kFixDn;
           visit[2 * ng - l] = l == 1 ? kFineUp : kFixUp;
@@ -1941,11 +1810,13 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
     else if (std::fabs(res / res_s) > 10.0) {
       info->vcycles = k;
       info->res = res;
+      if (int rc = settle()) return rc;
       return ctx->fail(LEPIC_ERR_DIVERGED, "PDE solver is diverging (iterative_solver.f90:42-49)");
     }
     if (res <= eps || k == ncycl) break;
     ++k;
   }
+  if (int rc = settle()) return rc;
   info->vcycles = k;
   info->status = (res <= eps) ? 0 : 1;
   info->res = res;
