@@ -406,7 +406,6 @@ int lepic_destroy(lepic_ctx* ctx) {
   for (int p = 0; p < kMaxSpecies; ++p)
     for (int k = 0; k < 2; ++k)
       if (ctx->ev_mover[p][k]) (void)hipEventDestroy(ctx->ev_mover[p][k]);
-  if (ctx->ev_sync) (void)hipEventDestroy(ctx->ev_sync);
   for (int p = 0; p < ctx->nsp; ++p) {
     Species& s = ctx->sp[p];
     for (int b = 0; b < 2; ++b) (void)hipFree(s.mem[b]);
@@ -434,6 +433,7 @@ int lepic_destroy(lepic_ctx* ctx) {
     if (ctx->lv[l].bf) (void)hipFree(ctx->lv[l].bf);
   }
   if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
+  if (ctx->h_report) (void)hipHostFree(ctx->h_report);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return 0;

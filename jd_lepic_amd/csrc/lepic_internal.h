@@ -71,6 +71,18 @@ struct LevelCtrl {
   int32_t cur[2];
   double res;
 };
+
+// What the host learns of a V-cycle: the residual and the sweeps of each
+// visit, the finest level's FP64 residual, whether an ng = 1 visit is finished
+// (its sweeps, or 0).  seq, on a line of its own, is written last.
+struct SolveReport {
+  double vres[2 * kMaxLevels];
+  double resid;
+  int32_t visit[2 * kMaxLevels];
+  int32_t status;
+  alignas(128) uint64_t seq;
+};
+
 // Particles of a species live in segments of kChunk slots: segment s holds
 // seg[cur][s] particles in its first slots, and the species' order is the
 // segments' contents in segment order.  The mover compacts each segment in
@@ -174,9 +186,11 @@ struct lepic_ctx {
   int32_t mg_epoch = 0;              // epoch of the last multi-block level visit
   lepic::LevelCtrl* d_ctrl = nullptr;   // [kMaxLevels+1]
   double* d_partials = nullptr;      // FP64 residual partial sums of the finest level
-  int64_t partials_cap = 0;
   double* d_scalar = nullptr;        // small scratch (res0 etc.)
   double* h_pinned = nullptr;        // pinned host scratch (kPinnedDoubles)
+  lepic::SolveReport* h_report = nullptr;   // coherent host memory that a V-cycle's last kernel writes
+  lepic::SolveReport* d_report = nullptr;   // its device address
+  uint64_t report_seq = 0;
   double* d_resid64 = nullptr;       // FP64 residual grid for mixed refinement
   float* d_corr = nullptr;
 
@@ -189,7 +203,6 @@ struct lepic_ctx {
   unsigned long long ticket_base = 0;       // tickets taken by earlier launches
   bool timing = false;                      // lepic_kernel_timing
   hipEvent_t ev_mover[lepic::kMaxSpecies][2] = {};
-  hipEvent_t ev_sync = nullptr;      // polled by the solver's per-V-cycle read-back
   bool ev_recorded[lepic::kMaxSpecies] = {};
   int32_t* d_error = nullptr;        // device-side error flags
 

@@ -56,10 +56,9 @@ constexpr size_t kTailLds = 160 * 1024 - 2048;  // dynamic LDS of k_tail (static
 constexpr int kTailThreads = 1024;
 constexpr int kS = kSweepsPerLaunch;          // most sweeps of one launch (kRot - 1 state buffers ahead)
 constexpr int kDefaultTailNodes = 5000;
-constexpr int kResidBlocks = 512;             // blocks of the FP64 finest-level residual (their partial sums fit the pinned read-back)
-// byte offset of the residual partials behind the scalars, visit log and status
-constexpr size_t kPartialsOff = (64 * 8 + (kVisitLog + 1) * sizeof(int) + 7) / 8 * 8;
-static_assert(kPartialsOff - 32 * 8 + kResidBlocks * 8 <= kPinnedDoubles * 8, "read-back fits the pinned buffer");
+constexpr int kResidBlocks = 512;             // blocks of the FP64 finest-level residual
+// byte offset of the residual partials behind the scalars and the visit log
+constexpr size_t kPartialsOff = (64 * 8 + kVisitLog * sizeof(int) + 7) / 8 * 8;
 constexpr int kNr = 10;                       // sweep limit of sors.f90:63-64
 // Mixed form: the FP32 correction V-cycle is a preconditioner inside FP64
 // refinement to the unchanged tolerance, so its schedule is chosen, not
@@ -225,6 +224,7 @@ struct VisitRef {
 struct Resolved {
   int ks;                  // sweeps of the visit (0: not finished)
   int buf;                 // rotating buffer holding the state after them
+  double res;
 };
 
 // Outcome of a visit after all its launches; every block of the consuming
@@ -232,19 +232,18 @@ struct Resolved {
 __device__ Resolved resolve_visit(const VisitRef& V, bool writer, double* s_res) {
   LevelCtrl* c = V.ctrl;
   const int c0 = c->cur[(V.epoch - 1) & 1];
-  Resolved out{0, 0};
-  double res = 0.0;
+  Resolved out{0, 0, 0.0};
   if (c->done_epoch == V.epoch) {
     out.ks = c->ksor;
-    res = c->res;
+    out.res = c->res;
   } else {
-    out.ks = first_stop(V.t, V.klast0 + 1, V.nexec, s_res, &res);
+    out.ks = first_stop(V.t, V.klast0 + 1, V.nexec, s_res, &out.res);
   }
   if (out.ks) out.buf = (c0 + out.ks) % kRot;
   if (writer && out.ks && threadIdx.x == 0) {
     c->cur[V.epoch & 1] = out.buf;
     V.visit[V.ig] = out.ks;
-    V.vres[V.ig] = res;
+    V.vres[V.ig] = out.res;
   }
   return out;
 }
@@ -442,16 +441,49 @@ __global__ __launch_bounds__(64 * kRestrictWaves) void k_restrict64(RestrictArgs
   }
 }
 
-// end of a V-cycle on a multi-block finest level: records the up visit
-struct Finish64Args {
-  VisitRef v;
-  int* status;             // sweeps of the visit, 0 if not finished
+// The host waits for one kernel per V-cycle, which writes what the host needs
+// straight into its memory and then the sequence number the host polls.
+// Against a copy, an event and the runtime's completion handling this takes
+// about 9 us off a V-cycle (128^2, four of them: 290 to 254 us a solve).
+struct ReportArgs {
+  SolveReport* out;
+  uint64_t seq;
+  const int* visit;
+  const double* vres;
 };
 
-__global__ __launch_bounds__(64 * (kS + 1)) void k_finish64(Finish64Args A) {
+// wave 0; lane `ig` reports ks and res instead of what the log holds (-1: none)
+__device__ void write_report(const ReportArgs& A, int ig, int ks, double res, double resid) {
+  const int lane = threadIdx.x;
+  if (lane < kVisitLog) {
+    A.out->visit[lane] = lane == ig ? ks : A.visit[lane];
+    A.out->vres[lane] = lane == ig ? res : A.vres[lane];
+  }
+  if (lane == 0) {
+    A.out->status = ks;
+    A.out->resid = resid;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");   // system scope
+  if (lane == 0) __hip_atomic_store(&A.out->seq, A.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// end of a V-cycle on a multi-block finest level (FP64): records the up visit
+__global__ __launch_bounds__(64 * (kS + 1)) void k_finish64(VisitRef V, ReportArgs A) {
   __shared__ double s_res[kS + 1];
-  const Resolved r = resolve_visit(A.v, true, s_res);
-  if (threadIdx.x == 0) *A.status = r.ks;
+  const Resolved r = resolve_visit(V, true, s_res);
+  if (threadIdx.x < 64) write_report(A, r.ks ? V.ig : -1, r.ks, r.res, 0.0);
+}
+
+// end of the others: the finest residual's partial sums in a fixed order
+constexpr int kReportThreads = 256;
+__global__ __launch_bounds__(kReportThreads) void k_report(const double* __restrict__ partials, int nb, ReportArgs A) {
+  __shared__ double ws[kReportThreads / 64];
+  double r = 0.0;
+  for (int q = threadIdx.x; q < nb; q += kReportThreads) r += partials[q];
+  r = wave_sum(r);
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = r;
+  __syncthreads();
+  if (threadIdx.x < 64) write_report(A, -1, 0, 0.0, ((ws[0] + ws[1]) + ws[2]) + ws[3]);
 }
 
 // end of a solve: the finest level's state from buffer `u_in` to phi (buffer 0)
@@ -1118,7 +1150,6 @@ T* b_of(Level& L, bool f32) { return f32 ? (T*)L.bf : (T*)L.b; }
 
 int* d_visit_of(lepic_ctx* ctx) { return (int*)(ctx->d_scalar + 64); }
 double* d_vres_of(lepic_ctx* ctx) { return ctx->d_scalar + 32; }
-int* d_status_of(lepic_ctx* ctx) { return (int*)(ctx->d_scalar + 64) + kVisitLog; }
 
 // A launch of kexec sweeps: the halo, the waves of a block and the grid.
 struct VisitShape {
@@ -1513,9 +1544,19 @@ int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps) {
 
 // One FP64 V-cycle (mg.f90:85-225): levels 1..Ls-1 multi-block, Ls..ng in
 // k_tail; then the end-of-cycle kernel.
+ReportArgs report_args(lepic_ctx* ctx) {
+  return ReportArgs{ctx->d_report, ++ctx->report_seq, d_visit_of(ctx), d_vres_of(ctx)};
+}
+
 int launch_finish64(lepic_ctx* ctx, const VisitRef& v) {
-  const Finish64Args A{v, d_status_of(ctx)};
-  hipLaunchKernelGGL(k_finish64, dim3(1), dim3(64 * (kS + 1)), 0, ctx->stream, A);
+  hipLaunchKernelGGL(k_finish64, dim3(1), dim3(64 * (kS + 1)), 0, ctx->stream, v, report_args(ctx));
+  LEPIC_HIP(hipGetLastError());
+  return 0;
+}
+
+int launch_report(lepic_ctx* ctx, int nb) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(kReportThreads), 0, ctx->stream, (const double*)ctx->d_partials, nb,
+                     report_args(ctx));
   LEPIC_HIP(hipGetLastError());
   return 0;
 }
@@ -1531,7 +1572,7 @@ int vcycle64(lepic_ctx* ctx, int k, double eps) {
   if (int rc = launch_tail<double>(ctx, false, k, eps)) return rc;
   for (int l = Ls - 1; l >= 1; --l)  // up leg
     if (int rc = launch_visit(ctx, l, e_up, true, eps)) return rc;
-  return ctx->lv[1].mb ? launch_finish64(ctx, cycle_visit_ref(ctx, 1, e_up, true, eps)) : 0;
+  return ctx->lv[1].mb ? launch_finish64(ctx, cycle_visit_ref(ctx, 1, e_up, true, eps)) : launch_report(ctx, 0);
 }
 
 // One V-cycle of the mixed form on the FP32 correction equation; adds the
@@ -1552,40 +1593,30 @@ double alpha_of(lepic_ctx* ctx) {
 
 int resid_blocks(lepic_ctx* ctx) { return std::min(ctx->g.n2 + 1, kResidBlocks); }
 
-// FP64 residual of phi; fills the FP32 right-hand side when fill_f32
+// FP64 residual of phi, reported; fills the FP32 right-hand side when fill_f32
 int launch_resid64(lepic_ctx* ctx, bool fill_f32, const double* u = nullptr) {
   Level& L = ctx->lv[1];
   hipLaunchKernelGGL(k_resid64, dim3(resid_blocks(ctx)), dim3(256), 0, ctx->stream, u ? u : (const double*)ctx->phi,
                      (const double*)ctx->rhs, (const int8_t*)ctx->bc, L.n1, L.n2, L.aw, L.an, L.ac,
                      fill_f32 ? L.bf : nullptr, ctx->d_partials);
   LEPIC_HIP(hipGetLastError());
-  return 0;
+  return launch_report(ctx, resid_blocks(ctx));
 }
 
-double sum_resid_partials(const double* p, int nb) {
-  double s = 0.0;
-  for (int q = 0; q < nb; ++q) s += p[q];
-  return s;
-}
-
-// read back the visit log, the per-visit residuals and (mixed) the FP64
-// residual partial sums of the finest level
-// The V-cycle's visit residuals and log (and the FP64 residual's partials)
-// in one copy; the host then waits for the stream by polling an event, which
-// returns as soon as the copy lands instead of after a blocking wake-up.
-int read_back(lepic_ctx* ctx, int* visit, double* vres, double* resid_sum) {
-  double* h = ctx->h_pinned;
-  const int nb = resid_blocks(ctx);
-  const size_t bytes = resid_sum ? kPartialsOff - 32 * 8 + (size_t)nb * 8 : 32 * 8 + (kVisitLog + 1) * sizeof(int);
-  LEPIC_HIP(hipMemcpyAsync(h, ctx->d_scalar + 32, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  LEPIC_HIP(hipEventRecord(ctx->ev_sync, ctx->stream));
-  hipError_t q;
-  while ((q = hipEventQuery(ctx->ev_sync)) == hipErrorNotReady) {
+// Waits for the report launched last.  The stream is asked now and then, so
+// that an error on it ends the wait.
+int read_report(lepic_ctx* ctx, int* visit, double* vres) {
+  const SolveReport* h = ctx->h_report;
+  auto arrived = [&]() { return __atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) == ctx->report_seq; };
+  for (uint32_t spin = 1; !arrived(); ++spin) {
+    if (spin % 65536 != 0) continue;
+    const hipError_t q = hipStreamQuery(ctx->stream);
+    if (q == hipErrorNotReady) continue;
+    LEPIC_HIP(q);
+    if (!arrived()) return ctx->fail(LEPIC_ERR_STATE, "a V-cycle ended without its report");
   }
-  LEPIC_HIP(q);
-  std::memcpy(vres, h, kVisitLog * 8);
-  std::memcpy(visit, (char*)h + 32 * 8, kVisitLog * sizeof(int));
-  if (resid_sum) *resid_sum = sum_resid_partials((const double*)((const char*)h + kPartialsOff - 32 * 8), nb);
+  std::memcpy(vres, h->vres, sizeof(h->vres));
+  std::memcpy(visit, h->visit, sizeof(h->visit));
   return 0;
 }
 
@@ -1662,14 +1693,16 @@ int poisson_setup(lepic_ctx* ctx) {
   LEPIC_HIP(hipMalloc(&ctx->d_ctrl, (kMaxLevels + 1) * sizeof(LevelCtrl)));
   LEPIC_HIP(hipMemsetAsync(ctx->d_ctrl, 0, (kMaxLevels + 1) * sizeof(LevelCtrl), ctx->stream));
   ctx->mg_epoch = 0;
-  // one allocation: 64 doubles of scalars (the visit residuals from 32),
-  // the visit log and status, then the FP64 residual's block partials, so a
-  // V-cycle's results come back in one copy
+  // one allocation: 64 doubles of scalars (the visit residuals from 32), the
+  // visit log, then the FP64 residual's block partials
   LEPIC_HIP(hipMalloc(&ctx->d_scalar, kPartialsOff + kResidBlocks * 8));
   LEPIC_HIP(hipMemsetAsync(ctx->d_scalar, 0, kPartialsOff + kResidBlocks * 8, ctx->stream));
   ctx->d_partials = (double*)((char*)ctx->d_scalar + kPartialsOff);
-  ctx->partials_cap = kResidBlocks;
-  if (!ctx->ev_sync) LEPIC_HIP(hipEventCreateWithFlags(&ctx->ev_sync, hipEventDisableTiming));
+  if (!ctx->h_report) {
+    LEPIC_HIP(hipHostMalloc((void**)&ctx->h_report, sizeof(SolveReport), hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset((void*)ctx->h_report, 0, sizeof(SolveReport));
+    LEPIC_HIP(hipHostGetDevicePointer((void**)&ctx->d_report, ctx->h_report, 0));
+  }
   return 0;
 }
 
@@ -1709,9 +1742,11 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
     if (g == 0) {
       double r_prev = 0.0, r_net = 0.0;
       if (int rc = launch_resid64(ctx, false)) return rc;
-      if (int rc = read_back(ctx, visit, vres, &r_prev)) return rc;
+      if (int rc = read_report(ctx, visit, vres)) return rc;
+      r_prev = ctx->h_report->resid;
       if (int rc = launch_resid64(ctx, false, ctx->phi_given)) return rc;
-      if (int rc = read_back(ctx, visit, vres, &r_net)) return rc;
+      if (int rc = read_report(ctx, visit, vres)) return rc;
+      r_net = ctx->h_report->resid;
       net_probe_result(ctx, r_net > 0.0 ? r_prev / r_net : HUGE_VAL);
       if (r_net < r_prev) {
         hipLaunchKernelGGL(k_copy_interior, g1, dim3(256), 0, ctx->stream, ctx->phi,
@@ -1731,10 +1766,9 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
   LEPIC_HIP(hipGetLastError());
   // residual of the starting guess; in mixed mode it also fills the FP32
   // right-hand side of the first correction equation
-  double r0 = 0.0;
   if (int rc = launch_resid64(ctx, mixed)) return rc;
-  if (int rc = read_back(ctx, visit, vres, &r0)) return rc;
-  info->res0 = r0 / alpha;
+  if (int rc = read_report(ctx, visit, vres)) return rc;
+  info->res0 = ctx->h_report->resid / alpha;
   int k = 1;
   info->status = 0;
   // FP64 with a multi-block finest level: the buffer that holds its state
@@ -1764,24 +1798,21 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
         }
         if (int rc = launch_finish64(ctx, visit_ref(ctx, 1, e, 0, nr, 1, alpha * eps, k0, k0 - kFirstMax,
                                                     kFirstMax))) return rc;
-        LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_status_of(ctx), 4, hipMemcpyDeviceToHost, ctx->stream));
-        LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-        std::memcpy(&ks, ctx->h_pinned, 4);
+        if (int rc = read_report(ctx, visit, vres)) return rc;
+        ks = ctx->h_report->status;
         if (ks) break;
       }
       if (!ks) return ctx->fail(LEPIC_ERR_STATE, "SOR visit did not finish");
-      if (int rc = read_back(ctx, visit, vres, nullptr)) return rc;
     } else if (!mixed) {
       if (int rc = vcycle64(ctx, k, alpha * eps)) return rc;
-      if (int rc = read_back(ctx, visit, vres, nullptr)) return rc;
+      if (int rc = read_report(ctx, visit, vres)) return rc;
     } else {
       // FP32 correction V-cycle on the FP64 residual, then phi += e; the new
       // FP64 residual is both the convergence test and the next right-hand side
       if (int rc = vcycle32(ctx, k, alpha * eps)) return rc;
       if (int rc = launch_resid64(ctx, true)) return rc;
-      double rs = 0.0;
-      if (int rc = read_back(ctx, visit, vres, &rs)) return rc;
-      vres[2 * ng - 1] = rs;
+      if (int rc = read_report(ctx, visit, vres)) return rc;
+      vres[2 * ng - 1] = ctx->h_report->resid;
     }
     const int nvis = 2 * ng - 1;
     if (ctx->lv[1].mb && !mixed) state = (state + visit[1] + (ng > 1 ? visit[nvis] : 0)) % kRot;
