@@ -3,12 +3,12 @@
 //
 // One block handles one segment of kChunk = 1024 slots.  Mixed precision:
 // 256 threads, thread t owning the four consecutive slots 4t .. 4t+3 (16-byte
-// vector loads and stores); FP64: 512 threads, thread t owning slots t and
-// t + 512.  Survivors are compacted in particle order (part_expmover.f90:
+// vector loads and stores); FP64: 256 threads, thread t owning slots t, t +
+// 256, ...  Survivors are compacted in particle order (part_expmover.f90:
 // 495-503) by a block ballot scan into the same segment of the other particle
 // buffer; the segments' contents in segment order are the species'
 // particles, so no prefix across blocks is needed and blocks never wait for
-// each other.  The mixed mover reads E, B and the cell wall flags from a
+// each other.  The movers read E, B and the cell wall flags from a
 // field tile of 10 x 32 nodes staged in LDS around the segment's first cell
 // (global memory for particles outside it).  Deposition accumulates in an
 // LDS window of 16 rows x 64 columns of nodes around the segment's first
@@ -50,7 +50,7 @@ constexpr int kWinY0 = 7;
 // neighbouring rows serialise
 constexpr int kWinStride = kWinCols + 1;
 constexpr int kWin = kWinRows * kWinStride;
-// Field tile of the mixed mover: E, B and the cell wall flags of kTileRows x
+// Field tile of the movers: E, B and the cell wall flags of kTileRows x
 // kTileCols nodes staged in LDS per segment, from kTileX0 columns left and
 // kTileY0 rows below the segment's first cell.  A sorted segment of 1024
 // particles at 100 per cell spans about 10 cells of one row, and particles
@@ -76,13 +76,17 @@ constexpr double kFix64 = 4398046511104.0;   // 2^42
 constexpr float kFixMx = 1048576.0f;         // 2^20
 // threads per mover block; a block owns one segment of kChunk slots
 constexpr int kMoverThreadsMixed = kBlock;
-constexpr int kMoverThreads64 = 2 * kBlock;   // two particles per thread: FP64 state of 4 would cost occupancy
+constexpr int kMoverThreads64 = kBlock;
+
+// a divisor, its reciprocal rounded and what the rounding left (div_exact)
+struct ExactDiv { double h, r, rl; };
 
 struct MoverCommon {
   const int8_t* bc;
   const int8_t* cellwall;       // 1 where all four corners of cell (ix,iy) are walls
   int n1, n2;
   double h1, h2, dt, k1;        // k1 = dt*q/(2m)
+  ExactDiv d1, d2;              // h1, h2
   double Nm, mass, NmQ;         // NmQ = Nm*charge for cnt_dead
   int tagneg;
   int flagB, gridB, Bconst, magnetize;
@@ -106,6 +110,19 @@ struct Soa64W { double *x, *y, *z, *vx, *vy, *vz; };
 struct SoaMx { const int32_t* cell; const float *fx, *fy, *z, *vx, *vy, *vz; };
 struct SoaMxW { int32_t* cell; float *fx, *fy, *z, *vx, *vy, *vz; };
 
+// An element of an LDS tile or, where the tile does not hold it, of global
+// memory: the explicit address space keeps the two loads apart, which the
+// compiler would otherwise merge into one flat access.
+template <typename T> using lds_p = __attribute__((address_space(3))) const T*;
+template <typename T>
+__device__ __forceinline__ T lds_get(const T* p) {
+  typedef int vi __attribute__((ext_vector_type(sizeof(T) / 4)));
+  const vi v = *(lds_p<vi>)p;
+  T r;
+  __builtin_memcpy(&r, &v, sizeof(T));
+  return r;
+}
+
 __device__ __forceinline__ uint64_t lanemask_lt() {
   return (1ull << (threadIdx.x & 63)) - 1ull;
 }
@@ -124,7 +141,8 @@ __device__ __forceinline__ void cic_fix(float fx, float fy, int& q0, int& q1, in
   q3 = fixmx(px * fy);
 }
 __device__ __forceinline__ void acc_add(unsigned long long* p, long long v) {
-  atomicAdd(p, (unsigned long long)v);
+  __hip_atomic_fetch_add((__attribute__((address_space(1))) unsigned long long*)p, (unsigned long long)v,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Deposit the four corner sums of FP64 cell (ix,iy) (corners 00,10,11,01 in
@@ -469,151 +487,214 @@ __device__ __forceinline__ void deposit_global_runs(const MoverCommon& a, const 
 // ---------------------------------------------------------------------------
 // FP64 mover
 // ---------------------------------------------------------------------------
+// x / h for the cell sizes, correctly rounded: the quotient from the
+// reciprocal in two parts is within one unit in the last place, so the
+// remainder is exact and one correction rounds it right (Markstein's theorem,
+// IBM J. Res. Dev. 34, 1990); the fix-up gives infinities, NaN and zeros as
+// the division does.
+__device__ __forceinline__ double div_exact(double x, const ExactDiv& d) {
+  const double q = __builtin_fma(x, d.r, x * d.rl);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.h, q, x), d.r, q), d.h, x);
+}
+
+// Bound by memory (96 B a particle) as far as the latencies overlap: a
+// thread's particles are all loaded at once, then the field tile (as the mixed
+// mover's; global memory for particles outside it), and everything up to the
+// deposition into the window runs from registers and LDS before the one
+// barrier that the compaction needs.  Four particles per thread at four waves
+// per SIMD: 26.2 M particles on 512 x 512 cells 748 us with E, B and the walls
+// gathered from memory particle by particle, 518 so (4.9 TB/s; two particles
+// per thread 570, one 570).
 template <int BT>
-__global__ __launch_bounds__(BT) void k_mover64(MoverCommon a, Soa64 in, Soa64W out,
-                                                    int8_t* flag_dead, const double* __restrict__ E,
-                                                    const double* __restrict__ B) {
-  constexpr int IT = kChunk / BT;   // particles per thread
+__global__ __launch_bounds__(BT, 4) void k_mover64(MoverCommon a, Soa64 in, Soa64W out, int8_t* flag_dead,
+                                                     const double* __restrict__ E, const double* __restrict__ B) {
+  constexpr int IT = kChunk / BT;   // particles per thread: slots t, t + BT, ...
   __shared__ unsigned long long win[kWin];
-  __shared__ int s_wx0, s_wy0;
+  __shared__ double2 sE[kFieldTile];
+  __shared__ double2 sB[2][kFieldTile];   // (Bx, By), (Bz, |B|)
+  __shared__ int8_t sW[kFieldTile];
   const int64_t bid = blockIdx.x;
   const int cnt_in = a.seg_in[bid];
-  const int64_t base = bid * (int64_t)(BT * IT);
+  const int64_t base = bid * (int64_t)kChunk;
   const int t = threadIdx.x;
   const int n1 = a.n1, n2 = a.n2;
-  const double h1 = a.h1, h2 = a.h2, dt = a.dt, k1 = a.k1;
-
-  if (a.deposit) {
-    for (int e = t; e < kWin; e += BT) win[e] = 0ull;
-    if (t == 0) {
-      int ix0 = 1, iy0 = 1;
-      if (cnt_in > 0) { ix0 = (int)(in.x[base] / h1) + 1; iy0 = (int)(in.y[base] / h2) + 1; }
-      s_wx0 = ix0 - kWinX0 < 0 ? 0 : ix0 - kWinX0;
-      s_wy0 = iy0 - kWinY0 < 0 ? 0 : iy0 - kWinY0;
-    }
-  }
+  const double h1 = a.d1.h, h2 = a.d2.h, dt = a.dt, k1 = a.k1;
 
   double X[IT], Y[IT], Z[IT], VX[IT], VY[IT], VZ[IT];
+  int8_t dead[IT];
   bool surv[IT];
 #pragma unroll
   for (int k = 0; k < IT; ++k) {
     const int64_t i = base + (int64_t)k * BT + t;
-    surv[k] = false;
-    if (k * BT + t >= cnt_in) continue;
-    double xp = in.x[i], yp = in.y[i], zp = in.z[i];
-    double vx = in.vx[i], vy = in.vy[i], vz = in.vz[i];
-    if (a.check_dead && flag_dead[i] == 1) {  // part_expmover.f90:84-98
-      flag_dead[i] = 0;
-      tally_dead(a, 0.5 * a.Nm * a.mass * (vx * vx + vy * vy + vz * vz));
-      continue;
+    surv[k] = k * BT + t < cnt_in;
+    dead[k] = 0;
+    if (!surv[k]) continue;
+    X[k] = in.x[i]; Y[k] = in.y[i]; Z[k] = in.z[i];
+    VX[k] = in.vx[i]; VY[k] = in.vy[i]; VZ[k] = in.vz[i];
+    if (a.check_dead) dead[k] = flag_dead[i];
+  }
+  int cx0 = 1, cy0 = 1;
+  if (cnt_in > 0) {
+    cx0 = (int)div_exact(in.x[base], a.d1) + 1;
+    cy0 = (int)div_exact(in.y[base], a.d2) + 1;
+  }
+  const int wx0 = max(cx0 - kWinX0, 0), wy0 = max(cy0 - kWinY0, 0);
+  const int fx0 = max(min(cx0 - kTileX0, n1 + 3 - kTileCols), 0);
+  const int fy0 = max(min(cy0 - kTileY0, n2 + 3 - kTileRows), 0);
+  const bool tileB = a.flagB && !a.Bconst && !a.gridB;
+  // the field tile (nodes beyond the grid of a small domain are never read)
+  for (int e = t; e < kFieldTile; e += BT) {
+    const int gx = fx0 + e % kTileCols, gy = fy0 + e / kTileCols;
+    double2 ev = make_double2(0.0, 0.0), b0 = ev, b1 = ev;
+    int8_t wv = 1;
+    if (gx <= n1 + 2 && gy <= n2 + 2) {
+      const int64_t nd = node_index(gx, gy, n1);
+      ev = *(const double2*)(E + 2 * nd);
+      if (tileB) {
+        b0 = *(const double2*)(B + 4 * nd);
+        b1 = *(const double2*)(B + 4 * nd + 2);
+      }
+      wv = a.cellwall[nd];
     }
-    int ix = (int)(xp / h1) + 1;  // INT(), lines 103-104
-    int iy = (int)(yp / h2) + 1;
-    clamp_cell(ix, iy, n1, n2);   // identity for positions inside the box
-    double px = (ix * h1 - xp) / h1;
-    double py = (iy * h2 - yp) / h2;
-    double k0 = px * py, kk1 = (1.0 - px) * py, kk2 = (1.0 - px) * (1.0 - py), kk3 = px * (1.0 - py);
-    const int64_t n00 = node_index(ix, iy, n1), n01 = node_index(ix, iy + 1, n1);
-    const double2 e00 = *(const double2*)(E + 2 * n00), e10 = *(const double2*)(E + 2 * (n00 + 1));
-    const double2 e11 = *(const double2*)(E + 2 * (n01 + 1)), e01 = *(const double2*)(E + 2 * n01);
-    double Exp = k0 * e00.x + kk1 * e10.x + kk2 * e11.x + kk3 * e01.x;
-    double Eyp = k0 * e00.y + kk1 * e10.y + kk2 * e11.y + kk3 * e01.y;
-    bool boris = false;
-    double Bx = 0, By = 0, Bz = 0;
-    if (a.flagB) {  // lines 131-182
-      if (a.Bconst) {
-        Bx = a.Bc0; By = a.Bc1; Bz = a.Bc2;
-        boris = true;
+    sE[e] = ev;
+    sB[0][e] = b0;
+    sB[1][e] = b1;
+    sW[e] = wv;
+  }
+  if (a.deposit)
+    for (int e = t; e < kWin; e += BT) win[e] = 0ull;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    int key = 0, dx = 0, dy = 0;
+    double w[4] = {0, 0, 0, 0};
+    if (surv[k] && dead[k] == 1) {  // part_expmover.f90:84-98
+      flag_dead[base + (int64_t)k * BT + t] = 0;
+      tally_dead(a, 0.5 * a.Nm * a.mass * (VX[k] * VX[k] + VY[k] * VY[k] + VZ[k] * VZ[k]));
+      surv[k] = false;
+    }
+    if (surv[k]) {
+      double xp = X[k], yp = Y[k], zp = Z[k], vx = VX[k], vy = VY[k], vz = VZ[k];
+      int ix = (int)div_exact(xp, a.d1) + 1;  // INT(), lines 103-104
+      int iy = (int)div_exact(yp, a.d2) + 1;
+      clamp_cell(ix, iy, n1, n2);   // identity for positions inside the box
+      double px = div_exact(ix * h1 - xp, a.d1);
+      double py = div_exact(iy * h2 - yp, a.d2);
+      double k0 = px * py, kk1 = (1.0 - px) * py, kk2 = (1.0 - px) * (1.0 - py), kk3 = px * (1.0 - py);
+      // the cell's four nodes from the tile when it holds them
+      const int tx = ix - fx0, ty = iy - fy0;
+      const bool in_tile = (unsigned)tx < (unsigned)(kTileCols - 1) && (unsigned)ty < (unsigned)(kTileRows - 1);
+      const int q = ty * kTileCols + tx;
+      double2 e00, e10, e11, e01;
+      if (in_tile) {
+        e00 = lds_get(sE + q); e10 = lds_get(sE + q + 1);
+        e11 = lds_get(sE + q + kTileCols + 1); e01 = lds_get(sE + q + kTileCols);
       } else {
-        int bx = ix, by = iy;
-        if (a.gridB) {
-          bx = (int)(xp / a.hB1) + 1; by = (int)(yp / a.hB2) + 1;
-          bx = bx < 0 ? 0 : (bx > a.nB1 + 1 ? a.nB1 + 1 : bx);
-          by = by < 0 ? 0 : (by > a.nB2 + 1 ? a.nB2 + 1 : by);
-        }
-        const int64_t bs = a.nB1 + 3;
-        const double* B00 = B + 4 * ((int64_t)by * bs + bx);
-        if (B00[3] > 1.0e-5) {
-          if (a.gridB) {
-            px = (bx * a.hB1 - xp) / a.hB1;
-            py = (by * a.hB2 - yp) / a.hB2;
-            k0 = px * py; kk1 = (1.0 - px) * py; kk2 = (1.0 - px) * (1.0 - py); kk3 = px * (1.0 - py);
-          }
-          const double* B10 = B00 + 4;
-          const double* B01 = B + 4 * ((int64_t)(by + 1) * bs + bx);
-          const double* B11 = B01 + 4;
-          Bx = k0 * B00[0] + kk1 * B10[0] + kk2 * B11[0] + kk3 * B01[0];
-          By = k0 * B00[1] + kk1 * B10[1] + kk2 * B11[1] + kk3 * B01[1];
-          Bz = k0 * B00[2] + kk1 * B10[2] + kk2 * B11[2] + kk3 * B01[2];
+        const int64_t n00 = node_index(ix, iy, n1), n01 = node_index(ix, iy + 1, n1);
+        e00 = *(const double2*)(E + 2 * n00); e10 = *(const double2*)(E + 2 * (n00 + 1));
+        e11 = *(const double2*)(E + 2 * (n01 + 1)); e01 = *(const double2*)(E + 2 * n01);
+      }
+      const double Exp = k0 * e00.x + kk1 * e10.x + kk2 * e11.x + kk3 * e01.x;
+      const double Eyp = k0 * e00.y + kk1 * e10.y + kk2 * e11.y + kk3 * e01.y;
+      bool boris = false;
+      double Bx = 0, By = 0, Bz = 0;
+      if (a.flagB) {  // lines 131-182
+        if (a.Bconst) {
+          Bx = a.Bc0; By = a.Bc1; Bz = a.Bc2;
           boris = true;
+        } else if (tileB && in_tile) {
+          if (sB[1][q].y > 1.0e-5) {
+            const double2 c00 = sB[0][q], c10 = sB[0][q + 1], c11 = sB[0][q + kTileCols + 1], c01 = sB[0][q + kTileCols];
+            Bx = k0 * c00.x + kk1 * c10.x + kk2 * c11.x + kk3 * c01.x;
+            By = k0 * c00.y + kk1 * c10.y + kk2 * c11.y + kk3 * c01.y;
+            Bz = k0 * sB[1][q].x + kk1 * sB[1][q + 1].x + kk2 * sB[1][q + kTileCols + 1].x + kk3 * sB[1][q + kTileCols].x;
+            boris = true;
+          }
+        } else {
+          int bx = ix, by = iy;
+          if (a.gridB) {
+            bx = (int)(xp / a.hB1) + 1; by = (int)(yp / a.hB2) + 1;
+            bx = bx < 0 ? 0 : (bx > a.nB1 + 1 ? a.nB1 + 1 : bx);
+            by = by < 0 ? 0 : (by > a.nB2 + 1 ? a.nB2 + 1 : by);
+          }
+          const int64_t bs = a.nB1 + 3;
+          const double* B00 = B + 4 * ((int64_t)by * bs + bx);
+          if (B00[3] > 1.0e-5) {
+            if (a.gridB) {
+              px = (bx * a.hB1 - xp) / a.hB1;
+              py = (by * a.hB2 - yp) / a.hB2;
+              k0 = px * py; kk1 = (1.0 - px) * py; kk2 = (1.0 - px) * (1.0 - py); kk3 = px * (1.0 - py);
+            }
+            const double* B10 = B00 + 4;
+            const double* B01 = B + 4 * ((int64_t)(by + 1) * bs + bx);
+            const double* B11 = B01 + 4;
+            Bx = k0 * B00[0] + kk1 * B10[0] + kk2 * B11[0] + kk3 * B01[0];
+            By = k0 * B00[1] + kk1 * B10[1] + kk2 * B11[1] + kk3 * B01[1];
+            Bz = k0 * B00[2] + kk1 * B10[2] + kk2 * B11[2] + kk3 * B01[2];
+            boris = true;
+          }
         }
       }
+      if (!a.magnetize) boris = false;  // line 185
+      if (boris) {                       // lines 187-206
+        const double Bt = sqrt(Bx * Bx + By * By + Bz * Bz);
+        const double k2 = k1 * (2.0 / (1.0 + (k1 * Bt) * (k1 * Bt)));
+        const double v1x = vx + k1 * Exp, v1y = vy + k1 * Eyp, v1z = vz;
+        const double v3x = v1x + k1 * (v1y * Bz - v1z * By);
+        const double v3y = v1y + k1 * (v1z * Bx - v1x * Bz);
+        const double v3z = v1z + k1 * (v1x * By - v1y * Bx);
+        const double v2x = v1x + k2 * (v3y * Bz - v3z * By);
+        const double v2y = v1y + k2 * (v3z * Bx - v3x * Bz);
+        const double v2z = v1z + k2 * (v3x * By - v3y * Bx);
+        vx = v2x + k1 * Exp;
+        vy = v2y + k1 * Eyp;
+        vz = v2z;
+      } else {  // lines 210-211
+        vx = vx + 2.0 * k1 * Exp;
+        vy = vy + 2.0 * k1 * Eyp;
+      }
+      xp = xp + dt * vx;  // lines 216-219
+      yp = yp + dt * vy;
+      zp = zp + dt * vz;
+      const double qx = div_exact(xp, a.d1), qy = div_exact(yp, a.d2);
+      ix = (int)floor(qx) + 1;  // FLOOR(), lines 244-245
+      iy = (int)floor(qy) + 1;
+      clamp_cell(ix, iy, n1, n2);
+      // lines 254-258, 314-446, from the tile's wall flags when it holds the cell
+      const int lx = ix - fx0, ly = iy - fy0;
+      const bool w_tile = (unsigned)lx < (unsigned)kTileCols && (unsigned)ly < (unsigned)kTileRows;
+      int8_t wall;
+      if (w_tile) wall = *(lds_p<int8_t>)(sW + ly * kTileCols + lx);
+      else wall = a.cellwall[node_index(ix, iy, n1)];
+      if (wall) {
+        tally_lost(a, xp, yp, ix, iy, 0.5 * a.Nm * a.mass * (vx * vx + vy * vy + vz * vz));
+        surv[k] = false;
+      } else {
+        X[k] = xp; Y[k] = yp; Z[k] = zp; VX[k] = vx; VY[k] = vy; VZ[k] = vz;
+        // charge_deposition, part_expmover.f90:555-584, at the new position
+        dx = (int)qx + 1;
+        dy = (int)qy + 1;
+        px = div_exact(dx * h1 - xp, a.d1);
+        py = div_exact(dy * h2 - yp, a.d2);
+        w[0] = px * py;
+        w[1] = (1.0 - px) * py;
+        w[2] = (1.0 - px) * (1.0 - py);
+        w[3] = px * (1.0 - py);
+        key = (int)node_index(dx, dy, n1);
+      }
     }
-    if (!a.magnetize) boris = false;  // line 185
-    if (boris) {                       // lines 187-206
-      double Bt = sqrt(Bx * Bx + By * By + Bz * Bz);
-      double k2 = k1 * (2.0 / (1.0 + (k1 * Bt) * (k1 * Bt)));
-      double v1x = vx + k1 * Exp, v1y = vy + k1 * Eyp, v1z = vz;
-      double v3x = v1x + k1 * (v1y * Bz - v1z * By);
-      double v3y = v1y + k1 * (v1z * Bx - v1x * Bz);
-      double v3z = v1z + k1 * (v1x * By - v1y * Bx);
-      double v2x = v1x + k2 * (v3y * Bz - v3z * By);
-      double v2y = v1y + k2 * (v3z * Bx - v3x * Bz);
-      double v2z = v1z + k2 * (v3x * By - v3y * Bx);
-      vx = v2x + k1 * Exp;
-      vy = v2y + k1 * Eyp;
-      vz = v2z;
-    } else {  // lines 210-211
-      vx = vx + 2.0 * k1 * Exp;
-      vy = vy + 2.0 * k1 * Eyp;
-    }
-    xp = xp + dt * vx;  // lines 216-219
-    yp = yp + dt * vy;
-    zp = zp + dt * vz;
-    ix = (int)floor(xp / h1) + 1;  // FLOOR(), lines 244-245
-    iy = (int)floor(yp / h2) + 1;
-    clamp_cell(ix, iy, n1, n2);
-    if (a.cellwall[node_index(ix, iy, n1)]) {  // lines 254-258, 314-446
-      tally_lost(a, xp, yp, ix, iy, 0.5 * a.Nm * a.mass * (vx * vx + vy * vy + vz * vz));
-      continue;
-    }
-    X[k] = xp; Y[k] = yp; Z[k] = zp; VX[k] = vx; VY[k] = vy; VZ[k] = vz;
-    surv[k] = true;
+    if (a.deposit) deposit_runs64(a, win, wx0, wy0, surv[k], key, dx, dy, w);
   }
-
   uint32_t off[IT];
-  compact_offsets<BT>(a, bid, cnt_in, surv, off);  // contains __syncthreads
-  const int64_t gbase = base;
+  compact_offsets<BT>(a, bid, cnt_in, surv, off);  // its barrier also completes the window
 #pragma unroll
   for (int k = 0; k < IT; ++k) {
     if (!surv[k]) continue;
-    const int64_t o = gbase + off[k];
+    const int64_t o = base + off[k];
     out.x[o] = X[k]; out.y[o] = Y[k]; out.z[o] = Z[k];
     out.vx[o] = VX[k]; out.vy[o] = VY[k]; out.vz[o] = VZ[k];
   }
-  if (!a.deposit) return;
-  const int wx0 = s_wx0, wy0 = s_wy0;
-#pragma unroll
-  for (int k = 0; k < IT; ++k) {
-    // charge_deposition, part_expmover.f90:555-584, at the new position
-    int64_t key = -2 - (int64_t)t;
-    double w[4] = {0, 0, 0, 0};
-    int ix = 0, iy = 0;
-    if (surv[k]) {
-      ix = (int)(X[k] / h1) + 1;
-      iy = (int)(Y[k] / h2) + 1;
-      double px = (ix * h1 - X[k]) / h1;
-      double py = (iy * h2 - Y[k]) / h2;
-      w[0] = px * py;
-      w[1] = (1.0 - px) * py;
-      w[2] = (1.0 - px) * (1.0 - py);
-      w[3] = px * (1.0 - py);
-      key = node_index(ix, iy, n1);
-    }
-    deposit_runs64(a, win, wx0, wy0, surv[k], (int)key, ix, iy, w);
-  }
-  __syncthreads();
-  flush_window(a, win, wx0, wy0);
+  if (a.deposit) flush_window(a, win, wx0, wy0);
 }
 
 // ---------------------------------------------------------------------------
@@ -627,11 +708,11 @@ struct MixedParams {
   float hB1r, hB2r;   // h/hB ratios for a B map on another grid
 };
 
-// at most 80 VGPRs (6 waves per SIMD instead of 5): the electrons' global
-// gathers and atomics late in a sort cycle wait less (measured 1.09 -> 1.06 ms
-// per 1024^2 electron push, ions 0.93 -> 0.92 ms; 8 waves would spill)
-template <int BT>
-__global__ __launch_bounds__(BT, 6) void k_mover_mixed(MoverCommon a, MixedParams m, SoaMx in,
+// Bound by memory: 105 M particles at 48 B on 1024 x 1024 cells take 0.99 ms
+// (5.1 TB/s) with at most 80 VGPRs (6 waves per SIMD), 1.01 ms with 5 waves; 1.09
+// while tile and global gathers were merged into flat loads.
+template <int BT, int OCC>
+__global__ __launch_bounds__(BT, OCC) void k_mover_mixed(MoverCommon a, MixedParams m, SoaMx in,
                                                         SoaMxW out, int8_t* flag_dead,
                                                         const float* __restrict__ E,
                                                         const float* __restrict__ B) {
@@ -726,7 +807,8 @@ __global__ __launch_bounds__(BT, 6) void k_mover_mixed(MoverCommon a, MixedParam
     const int q = ty * kTileCols + tx;
     float2 e00, e10, e11, e01;
     if (in_tile) {
-      e00 = sE[q]; e10 = sE[q + 1]; e11 = sE[q + kTileCols + 1]; e01 = sE[q + kTileCols];
+      e00 = lds_get(sE + q); e10 = lds_get(sE + q + 1);
+      e11 = lds_get(sE + q + kTileCols + 1); e01 = lds_get(sE + q + kTileCols);
     } else {
       const int64_t n00 = node_index(ix, iy, n1), n01 = node_index(ix, iy + 1, n1);
       e00 = *(const float2*)(E + 2 * n00); e10 = *(const float2*)(E + 2 * (n00 + 1));
@@ -741,7 +823,8 @@ __global__ __launch_bounds__(BT, 6) void k_mover_mixed(MoverCommon a, MixedParam
         Bx = (float)a.Bc0; By = (float)a.Bc1; Bz = (float)a.Bc2;
         boris = true;
       } else if (tileB && in_tile) {
-        const float4 B00 = sB[q], B10 = sB[q + 1], B11 = sB[q + kTileCols + 1], B01 = sB[q + kTileCols];
+        const float4 B00 = lds_get(sB + q), B10 = lds_get(sB + q + 1);
+        const float4 B11 = lds_get(sB + q + kTileCols + 1), B01 = lds_get(sB + q + kTileCols);
         if (B00.w > 1.0e-5f) {
           Bx = fmaf(w3, B01.x, fmaf(w2, B11.x, fmaf(w1, B10.x, w0 * B00.x)));
           By = fmaf(w3, B01.y, fmaf(w2, B11.y, fmaf(w1, B10.y, w0 * B00.y)));
@@ -805,7 +888,9 @@ __global__ __launch_bounds__(BT, 6) void k_mover_mixed(MoverCommon a, MixedParam
     // part_expmover.f90:254-258, from the tile's wall flags when it holds the cell
     const int wx = cx - fx0, wy = cy - fy0;
     const bool w_tile = (unsigned)wx < (unsigned)kTileCols && (unsigned)wy < (unsigned)kTileRows;
-    const int8_t wall = w_tile ? sW[wy * kTileCols + wx] : a.cellwall[node_index(cx, cy, n1)];
+    int8_t wall;
+    if (w_tile) wall = *(lds_p<int8_t>)(sW + wy * kTileCols + wx);
+    else wall = a.cellwall[node_index(cx, cy, n1)];
     const bool lost = live && wall != 0;
     lostm |= lost ? 1u << k : 0u;
     IXU[k] = ix; IYU[k] = iy;
@@ -947,6 +1032,12 @@ __global__ __launch_bounds__(256) void k_np_from_acc(const unsigned long long* _
   }
 }
 
+ExactDiv exact_div(double h) {
+  ExactDiv d{h, 1.0 / h, 0.0};
+  d.rl = std::fma(-d.r, h, 1.0) / h;
+  return d;
+}
+
 MoverCommon common_args(lepic_ctx* ctx, int p) {
   Species& s = ctx->sp[p];
   MoverCommon a{};
@@ -954,6 +1045,7 @@ MoverCommon common_args(lepic_ctx* ctx, int p) {
   a.cellwall = ctx->d_cellwall;
   a.n1 = ctx->g.n1; a.n2 = ctx->g.n2;
   a.h1 = ctx->g.h1; a.h2 = ctx->g.h2; a.dt = ctx->g.dt;
+  a.d1 = exact_div(ctx->g.h1); a.d2 = exact_div(ctx->g.h2);
   a.k1 = ctx->g.dt * s.charge / (2.0 * s.mass);  // part_expmover.f90:61
   a.Nm = s.Nm; a.mass = s.mass; a.NmQ = s.Nm * s.charge;
   a.tagneg = (ctx->g.tag_neg == p + 1);
@@ -1010,9 +1102,17 @@ int mover_launch(lepic_ctx* ctx, int p, int deposit) {
     m.hB2r = ctx->flag_gridB ? (float)(ctx->g.h2 / ctx->hB2) : 1.0f;
     SoaMx in{s.cell[b], s.f[b][0], s.f[b][1], s.f[b][2], s.f[b][3], s.f[b][4], s.f[b][5]};
     SoaMxW out{s.cell[o], s.f[o][0], s.f[o][1], s.f[o][2], s.f[o][3], s.f[o][4], s.f[o][5]};
-    hipLaunchKernelGGL(k_mover_mixed<kMoverThreadsMixed>, dim3((unsigned)nb), dim3(kMoverThreadsMixed), 0,
-                       ctx->stream, a, m, in, out,
-                       s.flag_dead, (const float*)ctx->Ef, (const float*)(ctx->Bf ? ctx->Bf : (float*)ctx->Ef));
+    // A launch that gives every CU at most two blocks gains nothing from six
+    // waves per SIMD and takes the form with registers to spare, which overlaps
+    // more of a thread's loads (400 k particles: 24.0 us, 24.8 in the other).
+    const float* B = (const float*)(ctx->Bf ? ctx->Bf : (float*)ctx->Ef);
+    const dim3 g((unsigned)nb), bt(kMoverThreadsMixed);
+    if (nb <= 512)
+      hipLaunchKernelGGL((k_mover_mixed<kMoverThreadsMixed, 2>), g, bt, 0, ctx->stream, a, m, in, out, s.flag_dead,
+                         (const float*)ctx->Ef, B);
+    else
+      hipLaunchKernelGGL((k_mover_mixed<kMoverThreadsMixed, 6>), g, bt, 0, ctx->stream, a, m, in, out, s.flag_dead,
+                         (const float*)ctx->Ef, B);
   } else {
     Soa64 in{s.d[b][0], s.d[b][1], s.d[b][2], s.d[b][3], s.d[b][4], s.d[b][5]};
     Soa64W out{s.d[o][0], s.d[o][1], s.d[o][2], s.d[o][3], s.d[o][4], s.d[o][5]};
