@@ -444,11 +444,12 @@ __global__ __launch_bounds__(64 * NW) void k_tile32(TileArgs A) {
 // ---------------------------------------------------------------------------
 // a level of the single-workgroup kernel, arrays in LDS
 // ---------------------------------------------------------------------------
+template <typename T>
 struct StripLevel {
   int n1, n2;
   int Lx, SW, nst;             // lanes per strip row ((n1 + 1) / 2), strips per wave, strips
   int inv;                     // 65536 / Lx + 1: lane / Lx = lane inv >> 16 for lane < 64, Lx <= 64
-  StripCoef<float> k;
+  StripCoef<T> k;
 };
 
 // the lane's strip of a level: wave w holds strips w SW .. w SW + SW - 1,
@@ -459,7 +460,8 @@ struct StripPos {
   bool act;
 };
 
-__device__ __forceinline__ StripPos strip_pos(const StripLevel& L, int w) {
+template <typename T>
+__device__ __forceinline__ StripPos strip_pos(const StripLevel<T>& L, int w) {
   const int lane = threadIdx.x & 63;
   StripPos p;
   const int q = (lane * L.inv) >> 16;
@@ -471,12 +473,12 @@ __device__ __forceinline__ StripPos strip_pos(const StripLevel& L, int w) {
 }
 
 // All loads are issued before the first is used, from clamped positions.
-template <int R, bool ISO>
-__device__ __forceinline__ void strip_load(Strip<float, R, ISO>& s, const StripLevel& L, const StripPos& p, const float* u,
-                                           const float* b, const int8_t* bc) {
+template <typename T, int R, bool ISO>
+__device__ __forceinline__ void strip_load(Strip<T, R, ISO>& s, const StripLevel<T>& L, const StripPos& p, const T* u,
+                                           const T* b, const int8_t* bc) {
   const int W = L.n1 + 3;
   int8_t c[R][2];
-  float lu[R][2];
+  T lu[R][2];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int j = min(2 + p.strip * R + r, L.n2), i = min(p.i0, L.n1);
@@ -497,35 +499,56 @@ __device__ __forceinline__ void strip_load(Strip<float, R, ISO>& s, const StripL
 #pragma unroll
     for (int P = 0; P < 2; ++P) {
       s.m[r][P] = strip_mask(ok && c[r][P] <= 0);
-      s.u[r][P] = u ? strip_select(s.m[r][P], lu[r][P], 0.0f) : 0.0f;
+      s.u[r][P] = u ? strip_clear(s.m[r][P], lu[r][P]) : (T)0;
     }
   }
 }
 
 // The lane's edges: zero guards below the first and above the last strip, and
 // the starting state's black edges (north: their an u).
-template <int R, bool ISO>
-__device__ __forceinline__ void strip_edges(const Strip<float, R, ISO>& s, const StripLevel& L, const StripPos& p,
-                                            const Edges<float>& e) {
+template <typename T, int R, bool ISO>
+__device__ __forceinline__ void strip_edges(const Strip<T, R, ISO>& s, const StripLevel<T>& L, const StripPos& p,
+                                            const Edges<T>& e) {
   if (!p.act) return;
-  if (p.strip == 0) e.ed[e.E + p.lx] = e.ed[3 * e.E + p.lx] = 0.0f;
-  if (p.strip == L.nst - 1) e.ed[e.o + e.Lx] = e.ed[2 * e.E + e.o + e.Lx] = 0.0f;
-  strip_publish_black<float, R, ISO>(s, e);
+  if (p.strip == 0) e.ed[e.E + p.lx] = e.ed[3 * e.E + p.lx] = (T)0;
+  if (p.strip == L.nst - 1) e.ed[e.o + e.Lx] = e.ed[2 * e.E + e.o + e.Lx] = (T)0;
+  strip_publish_black<T, R, ISO>(s, e);
+}
+
+// where the lane reads and writes its edges
+template <typename T>
+__device__ __forceinline__ Edges<T> strip_edge_pos(const StripLevel<T>& L, const StripPos& p, T* ed) {
+  return Edges<T>{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
+}
+
+// the coarse correction u2 around the strip, prolonged onto it
+template <typename T, int R, bool ISO>
+__device__ __forceinline__ void strip_prolong_from(Strip<T, R, ISO>& s, const StripLevel<T>& L, const StripPos& p,
+                                                   const T* u2) {
+  const int m1 = L.n1 / 2, m2 = L.n2 / 2;
+  P2<T> c[R / 2 + 1];
+#pragma unroll
+  for (int t = 0; t <= R / 2; ++t) {
+    const int cj = min((p.act ? p.strip : 0) * (R / 2) + 1 + t, m2 + 1);
+    const int q = cj * (m1 + 3) + min(p.i0 / 2, m1);
+    c[t] = P2<T>{u2[q], u2[q + 1]};
+  }
+  strip_prolong<T, R, ISO>(s, c);
 }
 
 // Down visit: nsw sweeps from zero, the state to u, the restricted residual
 // to the coarse right-hand side b2.
 template <int R, bool ISO, bool WAVE>
-__device__ __forceinline__ void strip_down(const StripLevel& L, const StripCoef<float>& kl, int nsw, float* ed, float* u,
+__device__ __forceinline__ void strip_down(const StripLevel<float>& L, const StripCoef<float>& kl, int nsw, float* ed, float* u,
                                            const float* b, const int8_t* bc, float* b2) {
   const StripCoef<float> k = strip_hold(kl);
   const StripPos p = strip_pos(L, WAVE ? 0 : (int)(threadIdx.x >> 6));
-  Edges<float> e{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
+  const Edges<float> e = strip_edge_pos(L, p, ed);
   Strip<float, R, ISO> s;
-  strip_load<R, ISO>(s, L, p, nullptr, b, bc);
+  strip_load<float, R, ISO>(s, L, p, nullptr, b, bc);
 #pragma unroll
   for (int r = 0; r < R; ++r) s.p[r][0] = s.p[r][1] = s.q[r][0] = s.q[r][1] = 0.0f;
-  strip_edges<R, ISO>(s, L, p, e);
+  strip_edges<float, R, ISO>(s, L, p, e);
   strip_sync<WAVE>();
   strip_sweeps<R, ISO, WAVE>(s, k, nsw, e);
   const int W = L.n1 + 3, m1 = L.n1 / 2, j0 = 2 + p.strip * R;
@@ -550,28 +573,21 @@ __device__ __forceinline__ void strip_down(const StripLevel& L, const StripCoef<
 // Up visit: the coarse correction u2 prolonged onto u, nsw sweeps, the state
 // to u, to the global array gu, or added to phi.
 template <int R, bool ISO, bool WAVE>
-__device__ __forceinline__ void strip_up(const StripLevel& L, const StripCoef<float>& kl, int nsw, float* ed, float* u,
+__device__ __forceinline__ void strip_up(const StripLevel<float>& L, const StripCoef<float>& kl, int nsw, float* ed, float* u,
                                          const float* b, const int8_t* bc, const float* u2, float* gu, double* phi) {
   const StripCoef<float> k = strip_hold(kl);
   const StripPos p = strip_pos(L, WAVE ? 0 : (int)(threadIdx.x >> 6));
-  Edges<float> e{ed, (L.nst + 2) * L.Lx, L.Lx, p.act ? (p.strip + 1) * L.Lx + p.lx : L.Lx, p.act};
+  const Edges<float> e = strip_edge_pos(L, p, ed);
   Strip<float, R, ISO> s;
-  strip_load<R, ISO>(s, L, p, u, b, bc);
-  const int W = L.n1 + 3, m1 = L.n1 / 2, m2 = L.n2 / 2, j0 = 2 + p.strip * R;
-  F2 c[R / 2 + 1];
-#pragma unroll
-  for (int t = 0; t <= R / 2; ++t) {
-    const int cj = min((p.act ? p.strip : 0) * (R / 2) + 1 + t, m2 + 1);
-    const int q = cj * (m1 + 3) + min(p.i0 / 2, m1);
-    c[t] = F2{u2[q], u2[q + 1]};
-  }
-  strip_prolong<float, R, ISO>(s, c);
+  strip_load<float, R, ISO>(s, L, p, u, b, bc);
+  const int W = L.n1 + 3, j0 = 2 + p.strip * R;
+  strip_prolong_from<float, R, ISO>(s, L, p, u2);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     s.products(k, r, 0);
     s.products(k, r, 1);
   }
-  strip_edges<R, ISO>(s, L, p, e);
+  strip_edges<float, R, ISO>(s, L, p, e);
   strip_sync<WAVE>();
   strip_sweeps<R, ISO, WAVE>(s, k, nsw, e);
   if (p.act && p.i0 <= L.n1) {
@@ -583,6 +599,135 @@ __device__ __forceinline__ void strip_up(const StripLevel& L, const StripCoef<fl
         if (s.m[r][0]) phi[q] = phi[q] + (double)s.u[r][0];
         if (s.m[r][1]) phi[q + 1] = phi[q + 1] + (double)s.u[r][1];
       } else if (gu) {
+        gu[q] = s.u[r][0];
+        gu[q + 1] = s.u[r][1];
+      } else {
+        u[q] = s.u[r][0];
+        u[q + 1] = s.u[r][1];
+      }
+    }
+  }
+  strip_sync<WAVE>();
+}
+
+// ---- FP64 visits ----
+
+// sum over the participants, the same value in every participant; ws holds
+// two banks of 16 wave sums used alternately (par), so a bank is rewritten
+// only after the barriers of a whole sweep
+template <bool WAVE>
+__device__ __forceinline__ double strip_sum(double v, double* ws, int par) {
+  v = lepic::wave_sum(v);
+  if (WAVE) return v;
+  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  double* bank = ws + 16 * par;
+  if ((threadIdx.x & 63) == 0) bank[w] = v;
+  __syncthreads();
+  double t = 0.0;
+  for (int q = 0; q < nw; ++q) t += bank[q];
+  return t;
+}
+
+// What a visit needs of the exit test (sors.f90:371-377), and its outcome.
+struct VisitTest {
+  int dig, nr;
+  double eps;
+  double* ws;                  // strip_sum's banks
+  int ks;
+  double res;
+};
+
+// Sweeps until the exit test ends the visit; the black edges of the starting
+// state are in LDS.  The red nodes' residual after sweep k comes with the red
+// pass of sweep k + 1, whose result is dropped when the test ends the visit;
+// all edges are then in LDS again.  Ends with a synchronisation.
+template <int R, bool ISO, bool WAVE>
+__device__ __forceinline__ void strip_sweeps64(Strip<double, R, ISO>& s, const StripCoef<double>& k, VisitTest& v,
+                                               const Edges<double>& e) {
+  double red[R], prev = 0.0;
+  strip_pass64<R, ISO, true, false, true>(s, k, e);
+  for (v.ks = 1;; ++v.ks) {
+    strip_sync<WAVE>();
+    const double rb = strip_pass64<R, ISO, false, true, true>(s, k, e);
+    strip_sync<WAVE>();
+#pragma unroll
+    for (int r = 0; r < R; ++r) red[r] = s.u[r][1 - (r & 1)];
+    const double rr = strip_pass64<R, ISO, true, true, true>(s, k, e);
+    v.res = strip_sum<WAVE>(rr + rb, v.ws, v.ks & 1);
+    const bool stop = v.dig == 0 ? v.res <= v.eps : prev > 0.0 && v.res / prev <= 0.6;
+    if (stop || v.ks >= v.nr) break;
+    prev = v.res;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    s.u[r][1 - (r & 1)] = red[r];
+    s.products(k, r, 1 - (r & 1));
+  }
+  if (e.write) {
+    e.ed[e.o] = s.north(0, 1);
+    e.ed[e.E + e.o] = s.north(R - 1, 0);
+  }
+  strip_sync<WAVE>();
+}
+
+// strip_down under the exit test
+template <int R, bool ISO, bool WAVE>
+__device__ __forceinline__ void strip_down64(const StripLevel<double>& L, VisitTest& v, double* ed, double* u,
+                                             const double* b, const int8_t* bc, double* b2) {
+  const StripCoef<double> k = strip_hold(L.k);
+  const StripPos p = strip_pos(L, WAVE ? 0 : (int)(threadIdx.x >> 6));
+  const Edges<double> e = strip_edge_pos(L, p, ed);
+  Strip<double, R, ISO> s;
+  strip_load<double, R, ISO>(s, L, p, nullptr, b, bc);
+#pragma unroll
+  for (int r = 0; r < R; ++r) s.p[r][0] = s.p[r][1] = s.q[r][0] = s.q[r][1] = 0.0;
+  strip_edges<double, R, ISO>(s, L, p, e);
+  strip_sync<WAVE>();
+  strip_sweeps64<R, ISO, WAVE>(s, k, v, e);
+  const int W = L.n1 + 3, m1 = L.n1 / 2, j0 = 2 + p.strip * R;
+  if (p.act && p.i0 <= L.n1) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (j0 + r <= L.n2) {
+        u[(j0 + r) * W + p.i0] = s.u[r][0];
+        u[(j0 + r) * W + p.i0 + 1] = s.u[r][1];
+      }
+  }
+  double out[R / 2];
+  strip_restrict<double, R, ISO, WAVE>(s, k, e, out);
+  if (p.act && p.i0 + 1 <= L.n1) {
+#pragma unroll
+    for (int t = 0; t < R / 2; ++t)
+      if (j0 + 2 * t + 1 <= L.n2) b2[(j0 / 2 + t) * (m1 + 1) + p.i0 / 2] = out[t];
+  }
+  strip_sync<WAVE>();
+}
+
+// strip_up under the exit test; the state goes to u, or to gu where not null
+template <int R, bool ISO, bool WAVE>
+__device__ __forceinline__ void strip_up64(const StripLevel<double>& L, VisitTest& v, double* ed, double* u,
+                                           const double* b, const int8_t* bc, const double* u2, double* gu) {
+  const StripCoef<double> k = strip_hold(L.k);
+  const StripPos p = strip_pos(L, WAVE ? 0 : (int)(threadIdx.x >> 6));
+  const Edges<double> e = strip_edge_pos(L, p, ed);
+  Strip<double, R, ISO> s;
+  strip_load<double, R, ISO>(s, L, p, u, b, bc);
+  strip_prolong_from<double, R, ISO>(s, L, p, u2);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    s.products(k, r, 0);
+    s.products(k, r, 1);
+  }
+  strip_edges<double, R, ISO>(s, L, p, e);
+  strip_sync<WAVE>();
+  strip_sweeps64<R, ISO, WAVE>(s, k, v, e);
+  const int W = L.n1 + 3, j0 = 2 + p.strip * R;
+  if (p.act && p.i0 <= L.n1) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (j0 + r > L.n2) continue;
+      const int q = (j0 + r) * W + p.i0;
+      if (gu) {
         gu[q] = s.u[r][0];
         gu[q + 1] = s.u[r][1];
       } else {

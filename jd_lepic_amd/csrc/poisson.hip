@@ -22,8 +22,8 @@
 //  * Coarse levels (at most mg_tail_nodes nodes) run in one workgroup that
 //    performs the whole lower part of the V-cycle (down sweeps, restrictions,
 //    the coarsest solve, prolongations and up sweeps), with the levels that
-//    fit in its LDS (up to 158 KB) held there: k_tail (FP64; the mixed form
-//    where a level is too wide for strips) and k_tail32 (mixed).
+//    fit in its LDS (up to 158 KB) held there: k_tail_strips, or k_tail where a
+//    level is too wide for strips or is the finest one in FP64.
 //  * Mixed mode runs each visit of a multi-block level in one launch of
 //    k_tile32 (mg_strip.h): the sweeps of a fixed count on register strips,
 //    with the prolongation on load, the restriction after the last sweep, and
@@ -383,9 +383,7 @@ __global__ __launch_bounds__(64 * kVisitMaxWaves) void k_visit64(VisitArgs A) {
 }
 
 // restriction, mg.f90:335-444, from a multi-block level: resolves the fine
-// level's down visit and writes the coarse right-hand side; `zero`, when not
-// null, is the coarse correction, cleared for the single-workgroup kernel (a
-// multi-block level's down visit knows that it starts from zero).
+// level's down visit and writes the coarse right-hand side
 struct RestrictArgs {
   VisitRef vf;
   const double* frot[kRot];
@@ -394,7 +392,6 @@ struct RestrictArgs {
   int n1, n2;
   StripCoef<double> k;
   double* r2h;
-  double* zero;
 };
 
 // A block's region is 128 x 32 nodes with 2 around the tile; bound by latency
@@ -407,13 +404,9 @@ __global__ __launch_bounds__(64 * kRestrictWaves) void k_restrict64(RestrictArgs
   __shared__ double ed[4 * E];
   __shared__ double s_res[kS + 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int n1 = A.n1, n2 = A.n2, m1 = n1 / 2, m2 = n2 / 2;
-  const int nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
+  const int n1 = A.n1, n2 = A.n2, m1 = n1 / 2;
+  const int bid = blockIdx.y * gridDim.x + blockIdx.x;
   const int i0 = (int)blockIdx.x * 124 + 2 * lane, j0 = (int)blockIdx.y * (NW * kVR - 4) + w * kVR;
-  if (A.zero) {
-    const int64_t nc = (int64_t)(m1 + 3) * (m2 + 3);
-    for (int64_t q = (int64_t)bid * blockDim.x + threadIdx.x; q < nc; q += (int64_t)nb * blockDim.x) A.zero[q] = 0.0;
-  }
   const int buf = resolve_visit(A.vf, bid == 0, s_res).buf;
   Strip<double, kVR, ISO> s;
   strip_region_load<kVR, ISO>(s, A.frot[buf], A.frot[0], A.fb, A.fbc, n1, n2, i0, j0);
@@ -663,35 +656,6 @@ __device__ void t_smooth(PU u, PB b, PC bc, int n1, int n2, T aw, T an, T ac, T 
 // pass's update; the update is stored only if the exit test (sors.f90:371-377)
 // lets sweep k+1 run.  Expressions and exit tests are those of t_smooth.
 // WAVE: wave 0 alone (P = 64, no block barriers); else the whole block.
-template <bool WAVE>
-__device__ __forceinline__ void tail_sync() {
-  if (WAVE) {
-    // a level may live in global memory: wait for the wave's stores and
-    // order the later loads after them, as a block barrier would
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  } else {
-    __syncthreads();
-  }
-}
-
-// sum over the participants, the same value in every participant; ws holds
-// two banks of 16 wave sums used alternately (par), so a bank is rewritten
-// only after the barriers of a whole sweep
-template <bool WAVE>
-__device__ __forceinline__ double tail_sum(double v, double* ws, int par) {
-  v = wave_sum(v);
-  if (WAVE) return v;
-  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  double* bank = ws + 16 * par;
-  if ((threadIdx.x & 63) == 0) bank[w] = v;
-  __syncthreads();
-  double t = 0.0;
-  for (int q = 0; q < nw; ++q) t += bank[q];
-  return t;
-}
-
 template <typename T, int R, bool WAVE, typename PU, typename PB, typename PC>
 __device__ __forceinline__ void t_smooth_fused(PU u, PB b, PC bc, int n1, int n2, T aw, T an, T ac, T omega, double eps,
                                int dig, int nr, double* ws, int* ksor_out, double* res_out, int nfix) {
@@ -774,9 +738,9 @@ __device__ __forceinline__ void t_smooth_fused(PU u, PB b, PC bc, int n1, int n2
     for (int k = 1; k <= nfix; ++k) {
       red_pass(false);
       store_red();
-      tail_sync<WAVE>();
+      strip_sync<WAVE>();
       black_pass();
-      tail_sync<WAVE>();
+      strip_sync<WAVE>();
     }
     *ksor_out = nfix;
     *res_out = 0.0;
@@ -785,27 +749,27 @@ __device__ __forceinline__ void t_smooth_fused(PU u, PB b, PC bc, int n1, int n2
   // sweep 1
   red_pass(false);
   store_red();
-  tail_sync<WAVE>();
+  strip_sync<WAVE>();
   double rb = black_pass();
-  tail_sync<WAVE>();
+  strip_sync<WAVE>();
   int k = 1;
   double res_s = 0.0, res = 0.0;
   for (;;) {
     const double rs = red_pass(true);
-    res = tail_sum<WAVE>(rs + rb, ws, k & 1);
+    res = strip_sum<WAVE>(rs + rb, ws, k & 1);
     bool stop;
     if (dig == 0) stop = res <= eps;
     else stop = res_s > 0.0 && (res / res_s) <= 0.6;
     if (stop || k >= nr) break;
     res_s = res;
     store_red();
-    tail_sync<WAVE>();
+    strip_sync<WAVE>();
     rb = black_pass();
-    tail_sync<WAVE>();
+    strip_sync<WAVE>();
     ++k;
   }
   // the last red pass only read; the next phase may overwrite nothing it read
-  tail_sync<WAVE>();
+  strip_sync<WAVE>();
   *ksor_out = k;
   *res_out = res;
 }
@@ -1011,7 +975,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs<T> A) {
         smooth_level<T, true>(F, sU[l], sB[l], sBC[l], A.omega, A.eps, l - ng, kNr, ws, &ks, &res, A.fix_dn);
         if (tid == 0) { A.visit[l] = ks; A.vres[l] = res; }
         tail_restrict<T>(F, A.lv[l + 1], sU[l], sB[l], sBC[l], sU[l + 1], sB[l + 1], sBC[l + 1], tid, 64);
-        tail_sync<true>();
+        strip_sync<true>();
       }
       smooth_level<T, true>(A.lv[ng], sU[ng], sB[ng], sBC[ng], A.omega, A.eps, 0, A.k == 1 ? 1000000 : kNr, ws,
                             &ks, &res);
@@ -1019,7 +983,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs<T> A) {
       for (int l = ng - 1; l >= Lw; --l) {
         const TLevel<T>& F = A.lv[l];
         tail_prolong<T>(F, A.lv[l + 1], sU[l], sBC[l], (const T*)sU[l + 1], tid, 64);
-        tail_sync<true>();
+        strip_sync<true>();
         smooth_level<T, true>(F, sU[l], sB[l], sBC[l], A.omega, A.eps, ng - l, kNr, ws, &ks, &res, A.fix_up);
         if (tid == 0) { A.visit[2 * ng - l] = ks; A.vres[2 * ng - l] = res; }
       }
@@ -1041,98 +1005,116 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs<T> A) {
   if (L.lds) copy_l2g(L.gu, smem + L.ou, (L.n1 + 3) * (L.n2 + 3) * (int)sizeof(T));
 }
 
-// The same work for the mixed form, on register strips (mg_strip.h; 28 us a
-// launch at 65^2 nodes and below against 60 us for k_tail, of 65e3 cycles:
-// load 4e3, down visits 13e3 (65^2), 9e3 (33^2), 6.2-6.9e3 each below, up
-// visits 2.5-5.2e3; a pass costs about 225 cycles in one wave, most of them
-// the LDS exchange): every
-// level above the coarsest runs its fixed sweeps from registers, its arrays in
-// LDS between the visits.  Levels whose strips fit one wave run in wave 0
-// without block barriers.  The coarsest level keeps the exit test of
-// sors.f90:371-377 on the arrays in LDS.
-struct Tail32Level {
-  StripLevel s;
+// The same work on register strips (mg_strip.h): every level above the
+// coarsest runs its sweeps from registers, its arrays in LDS between the
+// visits.  Levels whose strips fit one wave run in wave 0 without block
+// barriers.  The coarsest level keeps the exit test of sors.f90:371-377 on the
+// arrays in LDS, in FP64 every level does (strip_sweeps64).  Bound by the
+// latency of the passes one after the other.  FP32 at 65^2 nodes and below: 28
+// us a launch against 60 for k_tail, of 65e3 cycles: load 4e3, down visits 13e3
+// (65^2), 9e3 (33^2), 6.2-6.9e3 each below, up visits 2.5-5.2e3; a pass costs
+// about 225 cycles in one wave, most of them the LDS exchange.  FP64 at 65 x 33
+// nodes and below: 44 us against 87 for k_tail.
+template <typename T>
+struct TailStripLevel {
+  StripLevel<T> s;
   int two;                     // strips of 2 rows (else 4); always in wave 0
   uint32_t ou, ob, obc;        // LDS offsets of the correction, right-hand side and bc arrays
 };
 
-struct Tail32Args {
+template <typename T>
+struct TailStripArgs {
   int Ls, ng, k;
   int Lw;                      // levels Ls .. Lw-1 by the whole block, Lw .. ng-1 by wave 0
   int cw;                      // the coarsest level by wave 0
-  int fix_dn, fix_up;
+  int fix_dn, fix_up;          // FP32: the sweeps of a visit
   double eps;
   const int8_t* bc_img;
   int bc_bytes;
   uint32_t u_begin, u_end, oed;
-  const float* gb;             // level Ls: right-hand side, and where its correction goes
-  float* gu;
-  double* phi;                 // not null when Ls is the finest level
-  float omega, caw, can, cac;  // coarsest level
+  const T* gb;                 // level Ls: right-hand side, and where its correction goes
+  T* gu;
+  double* phi;                 // FP32, not null when Ls is the finest level
+  T omega, caw, can, cac;      // coarsest level
   int* visit;
   double* vres;
-  Tail32Level lv[kMaxLevels + 1];
+  TailStripLevel<T> lv[kMaxLevels + 1];
 };
 
-template <bool ISO>
-__global__ __launch_bounds__(kTailThreads) void k_tail32(Tail32Args A) {
+template <typename T, bool ISO>
+__global__ __launch_bounds__(kTailThreads) void k_tail_strips(TailStripArgs<T> A) {
   extern __shared__ __align__(16) char smem[];
   __shared__ double ws[32];
   const int Ls = A.Ls, ng = A.ng, tid = threadIdx.x;
-  auto U = [&](int l) { return (float*)(smem + A.lv[l].ou); };
-  auto B = [&](int l) { return (float*)(smem + A.lv[l].ob); };
+  auto U = [&](int l) { return (T*)(smem + A.lv[l].ou); };
+  auto B = [&](int l) { return (T*)(smem + A.lv[l].ob); };
   auto M = [&](int l) { return (const int8_t*)(smem + A.lv[l].obc); };
-  float* ed = (float*)(smem + A.oed);
+  T* ed = (T*)(smem + A.oed);
   {
-    const StripLevel& L = A.lv[Ls].s;
-    copy3_g2l(smem, A.bc_img, A.bc_bytes, smem + A.lv[Ls].ob, A.gb, (L.n1 + 1) * (L.n2 + 1) * 4, smem, A.bc_img, 0);
+    const StripLevel<T>& L = A.lv[Ls].s;
+    copy3_g2l(smem, A.bc_img, A.bc_bytes, smem + A.lv[Ls].ob, A.gb, (L.n1 + 1) * (L.n2 + 1) * (int)sizeof(T), smem,
+              A.bc_img, 0);
   }
   for (uint32_t q = A.u_begin + 16u * tid; q < A.u_end; q += 16u * blockDim.x)
     *(float4*)(smem + q) = make_float4(0.f, 0.f, 0.f, 0.f);
   __syncthreads();
   int ks = 0;
   double res = 0.0;
-  TLevel<float> C;
+  TLevel<T> C;
   C.n1 = A.lv[ng].s.n1; C.n2 = A.lv[ng].s.n2;
   C.aw = A.caw; C.an = A.can; C.ac = A.cac;
   C.gu = nullptr; C.gb = nullptr; C.gbc = nullptr;
   C.lds = 1;
   C.ou = C.ob = C.obc = 0;
   const int nr = A.k == 1 ? 1000000 : kNr;
+  auto down = [&](int l, auto rows, auto wave) {
+    constexpr int R = decltype(rows)::value;
+    constexpr bool W = decltype(wave)::value;
+    const StripLevel<T>& L = A.lv[l].s;
+    if constexpr (sizeof(T) == 4) {
+      strip_down<R, ISO, W>(L, L.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
+      if (tid == 0) A.visit[l] = A.fix_dn;
+    } else {
+      VisitTest v{l - ng, kNr, A.eps, ws, 0, 0.0};
+      strip_down64<R, ISO, W>(L, v, ed, U(l), B(l), M(l), B(l + 1));
+      if (tid == 0) { A.visit[l] = v.ks; A.vres[l] = v.res; }
+    }
+  };
+  auto up = [&](int l, auto rows, auto wave) {
+    constexpr int R = decltype(rows)::value;
+    constexpr bool W = decltype(wave)::value;
+    const StripLevel<T>& L = A.lv[l].s;
+    T* gu = l == Ls ? A.gu : nullptr;
+    if constexpr (sizeof(T) == 4) {
+      strip_up<R, ISO, W>(L, L.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), gu, l == Ls ? A.phi : nullptr);
+      if (tid == 0) A.visit[2 * ng - l] = A.fix_up;
+    } else {
+      VisitTest v{ng - l, kNr, A.eps, ws, 0, 0.0};
+      strip_up64<R, ISO, W>(L, v, ed, U(l), B(l), M(l), U(l + 1), gu);
+      if (tid == 0) { A.visit[2 * ng - l] = v.ks; A.vres[2 * ng - l] = v.res; }
+    }
+  };
+  using Two = std::integral_constant<int, 2>;
+  using Four = std::integral_constant<int, 4>;
   for (int l = Ls; l < A.Lw; ++l) {
-    const Tail32Level& L = A.lv[l];
-    if (L.two) strip_down<2, ISO, false>(L.s, L.s.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
-    else strip_down<4, ISO, false>(L.s, L.s.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
-    if (tid == 0) A.visit[l] = A.fix_dn;
+    if (A.lv[l].two) down(l, Two{}, std::false_type{});
+    else down(l, Four{}, std::false_type{});
   }
   if (A.cw) {
     if (tid < 64) {
-      for (int l = A.Lw; l < ng; ++l) {
-        const Tail32Level& L = A.lv[l];
-        strip_down<2, ISO, true>(L.s, L.s.k, A.fix_dn, ed, U(l), B(l), M(l), B(l + 1));
-        if (tid == 0) A.visit[l] = A.fix_dn;
-      }
-      smooth_level<float, true>(C, U(ng), B(ng), M(ng), A.omega, A.eps, 0, nr, ws, &ks, &res);
+      for (int l = A.Lw; l < ng; ++l) down(l, Two{}, std::true_type{});
+      smooth_level<T, true>(C, U(ng), B(ng), M(ng), A.omega, A.eps, 0, nr, ws, &ks, &res);
       if (tid == 0) { A.visit[ng] = ks; A.vres[ng] = res; }
-      for (int l = ng - 1; l >= A.Lw; --l) {
-        const Tail32Level& L = A.lv[l];
-        strip_up<2, ISO, true>(L.s, L.s.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), l == Ls ? A.gu : nullptr,
-                               l == Ls ? A.phi : nullptr);
-        if (tid == 0) A.visit[2 * ng - l] = A.fix_up;
-      }
+      for (int l = ng - 1; l >= A.Lw; --l) up(l, Two{}, std::true_type{});
     }
   } else {                     // Lw == ng
-    smooth_level<float>(C, U(ng), B(ng), M(ng), A.omega, A.eps, 0, nr, ws, &ks, &res);
+    smooth_level<T>(C, U(ng), B(ng), M(ng), A.omega, A.eps, 0, nr, ws, &ks, &res);
     if (tid == 0) { A.visit[ng] = ks; A.vres[ng] = res; }
   }
   __syncthreads();
   for (int l = A.Lw - 1; l >= Ls; --l) {
-    const Tail32Level& L = A.lv[l];
-    float* gu = l == Ls ? A.gu : nullptr;
-    double* phi = l == Ls ? A.phi : nullptr;
-    if (L.two) strip_up<2, ISO, false>(L.s, L.s.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), gu, phi);
-    else strip_up<4, ISO, false>(L.s, L.s.k, A.fix_up, ed, U(l), B(l), M(l), U(l + 1), gu, phi);
-    if (tid == 0) A.visit[2 * ng - l] = A.fix_up;
+    if (A.lv[l].two) up(l, Two{}, std::false_type{});
+    else up(l, Four{}, std::false_type{});
   }
 }
 
@@ -1354,7 +1336,6 @@ int launch_restrict(lepic_ctx* ctx, int l, int epoch, double eps) {
   A.n1 = F.n1; A.n2 = F.n2;
   A.k = strip_coef64(F);
   A.r2h = C.b;
-  A.zero = C.mb ? nullptr : C.u;
   constexpr int tx = 124, ty = kRestrictWaves * kVR - 4;
   const dim3 g((unsigned)((F.n1 - 1 + tx - 1) / tx), (unsigned)((F.n2 - 1 + ty - 1) / ty));
   if (F.aw == F.an) hipLaunchKernelGGL(k_restrict64<true>, g, dim3(64 * kRestrictWaves), 0, ctx->stream, A);
@@ -1385,10 +1366,13 @@ int tail_bc_image(lepic_ctx* ctx, int Lr, bool f32) {
   return 0;
 }
 
-// k_tail32's layout, or false where a level above the coarsest does not fit
-// its strips (wider than 128 columns or more than 16 waves) or the LDS.
-bool tail32_plan(lepic_ctx* ctx, Tail32Args& A, size_t& lds, int& threads) {
+// k_tail_strips' layout, or false where a level above the coarsest does not fit
+// its strips (wider than 128 columns or more than 16 waves) or the LDS, or
+// holds wall values (FP64, the finest level).
+template <typename T>
+bool tail_strips_plan(lepic_ctx* ctx, TailStripArgs<T>& A, size_t& lds, int& threads) {
   if (ctx->Lc == ctx->ng) return false;   // the coarsest level alone
+  if (sizeof(T) == 8 && ctx->Lc == 1) return false;
   const int ng = ctx->ng, Ls = ctx->Lc;
   auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
   A.Ls = Ls; A.ng = ng; A.Lw = ng;
@@ -1396,8 +1380,8 @@ bool tail32_plan(lepic_ctx* ctx, Tail32Args& A, size_t& lds, int& threads) {
   size_t ed = 0;
   for (int l = Ls; l < ng; ++l) {
     const Level& L = ctx->lv[l];
-    Tail32Level& T = A.lv[l];
-    StripLevel& S = T.s;
+    TailStripLevel<T>& V = A.lv[l];
+    StripLevel<T>& S = V.s;
     S.n1 = L.n1; S.n2 = L.n2;
     S.Lx = (L.n1 + 1) / 2;
     if (S.Lx > 64) return false;
@@ -1406,16 +1390,17 @@ bool tail32_plan(lepic_ctx* ctx, Tail32Args& A, size_t& lds, int& threads) {
     // strips of two rows where they fit four waves, one per SIMD; strips of
     // four rows where a level has work for every SIMD anyway (65^2: 13e3
     // cycles a down visit in 8 waves of 4 rows, 18e3 in 4 waves of 8)
-    T.two = ((L.n2 - 1 + 1) / 2 + S.SW - 1) / S.SW <= 4;
-    const int R = T.two ? 2 : 4;
+    V.two = ((L.n2 - 1 + 1) / 2 + S.SW - 1) / S.SW <= 4;
+    const int R = V.two ? 2 : 4;
     S.nst = (L.n2 - 1 + R - 1) / R;
     const int w = (S.nst + S.SW - 1) / S.SW;
     if (w > 16) return false;
-    if (w == 1 && T.two) A.Lw = std::min(A.Lw, l);
+    if (w == 1 && V.two) A.Lw = std::min(A.Lw, l);
     else if (A.Lw < l) return false;
     waves = std::max(waves, w);
-    S.k = strip_coef(L, 1.4f);
-    ed = std::max(ed, (size_t)4 * (S.nst + 2) * S.Lx * 4);
+    if constexpr (sizeof(T) == 4) S.k = strip_coef(L, 1.4f);
+    else S.k = strip_coef64(L);
+    ed = std::max(ed, (size_t)4 * (S.nst + 2) * S.Lx * sizeof(T));
   }
   const Level& C = ctx->lv[ng];
   A.lv[ng].s.n1 = C.n1; A.lv[ng].s.n2 = C.n2;
@@ -1430,12 +1415,12 @@ bool tail32_plan(lepic_ctx* ctx, Tail32Args& A, size_t& lds, int& threads) {
   A.u_begin = (uint32_t)off;
   for (int l = ng; l >= Ls; --l) {
     A.lv[l].ou = (uint32_t)off;
-    off = al(off + (size_t)(ctx->lv[l].n1 + 3) * (ctx->lv[l].n2 + 3) * 4);
+    off = al(off + (size_t)(ctx->lv[l].n1 + 3) * (ctx->lv[l].n2 + 3) * sizeof(T));
   }
   A.u_end = (uint32_t)off;
   for (int l = ng; l >= Ls; --l) {
     A.lv[l].ob = (uint32_t)off;
-    off = al(off + (size_t)(ctx->lv[l].n1 + 1) * (ctx->lv[l].n2 + 1) * 4);
+    off = al(off + (size_t)(ctx->lv[l].n1 + 1) * (ctx->lv[l].n2 + 1) * sizeof(T));
   }
   A.oed = (uint32_t)off;
   lds = off + ed;
@@ -1446,42 +1431,48 @@ bool tail32_plan(lepic_ctx* ctx, Tail32Args& A, size_t& lds, int& threads) {
 template <typename T>
 int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps);
 
-int launch_tail32(lepic_ctx* ctx, int k, double eps) {
-  Tail32Args A{};
+// levels Ls .. ng of a V-cycle on strips where the plan allows, else in the
+// generic kernel, which starts from the state in global memory: zero on
+// coarser levels
+template <typename T>
+int launch_lower(lepic_ctx* ctx, int k, double eps) {
+  constexpr bool f32 = sizeof(T) == 4;
+  TailStripArgs<T> A{};
   size_t lds = 0;
   int threads = 0;
-  const Level& L = ctx->lv[ctx->Lc];
-  if (!tail32_plan(ctx, A, lds, threads)) {
-    // the generic kernel starts from the state in global memory: zero
+  Level& L = ctx->lv[ctx->Lc];
+  if (!tail_strips_plan(ctx, A, lds, threads)) {
     const int64_t n = (int64_t)(L.n1 + 3) * (L.n2 + 3);
-    if (int rc = zero_async(ctx, L.uf, n * 4)) return rc;
-    if (int rc = launch_tail<float>(ctx, true, k, eps)) return rc;
-    if (ctx->Lc == 1) {
+    if (f32 || ctx->Lc > 1)
+      if (int rc = zero_async(ctx, u_of<T>(L, f32), n * sizeof(T))) return rc;
+    if (int rc = launch_tail<T>(ctx, f32, k, eps)) return rc;
+    if (f32 && ctx->Lc == 1) {
       hipLaunchKernelGGL(k_add_corr, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, ctx->phi,
                          (const float*)L.uf, (const int8_t*)ctx->bc, n);
       LEPIC_HIP(hipGetLastError());
     }
     return 0;
   }
-  if (int rc = tail_bc_image(ctx, ctx->Lc, true)) return rc;
+  if (int rc = tail_bc_image(ctx, ctx->Lc, f32)) return rc;
   A.k = k; A.eps = eps;
   A.fix_dn = kFixDn; A.fix_up = kFixUp;
   A.bc_img = ctx->d_tail_bc;
-  A.gb = L.bf;
-  A.gu = L.uf;
+  A.gb = b_of<T>(L, f32);
+  A.gu = u_of<T>(L, f32);
   A.phi = ctx->Lc == 1 ? ctx->phi : nullptr;
   const Level& C = ctx->lv[ctx->ng];
-  A.omega = 1.4f; A.caw = (float)C.aw; A.can = (float)C.an; A.cac = (float)C.ac;
+  A.omega = (T)1.4; A.caw = (T)C.aw; A.can = (T)C.an; A.cac = (T)C.ac;
   A.visit = d_visit_of(ctx);
   A.vres = d_vres_of(ctx);
-  static bool attr_set = false;
+  static bool attr_set = false;   // per instantiation
   if (!attr_set) {
-    LEPIC_HIP(hipFuncSetAttribute((const void*)k_tail32<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
-    LEPIC_HIP(hipFuncSetAttribute((const void*)k_tail32<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
+    LEPIC_HIP(hipFuncSetAttribute((const void*)k_tail_strips<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
+    LEPIC_HIP(hipFuncSetAttribute((const void*)k_tail_strips<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTailLds));
     attr_set = true;
   }
-  if (strip_iso(L)) hipLaunchKernelGGL(k_tail32<true>, dim3(1), dim3(threads), lds, ctx->stream, A);
-  else hipLaunchKernelGGL(k_tail32<false>, dim3(1), dim3(threads), lds, ctx->stream, A);
+  if ((T)L.aw == (T)L.an)
+    hipLaunchKernelGGL((k_tail_strips<T, true>), dim3(1), dim3(threads), lds, ctx->stream, A);
+  else hipLaunchKernelGGL((k_tail_strips<T, false>), dim3(1), dim3(threads), lds, ctx->stream, A);
   LEPIC_HIP(hipGetLastError());
   return 0;
 }
@@ -1569,7 +1560,7 @@ int vcycle64(lepic_ctx* ctx, int k, double eps) {
     if (int rc = launch_visit(ctx, l, e_dn, false, eps)) return rc;
     if (int rc = launch_restrict(ctx, l, e_dn, eps)) return rc;
   }
-  if (int rc = launch_tail<double>(ctx, false, k, eps)) return rc;
+  if (int rc = launch_lower<double>(ctx, k, eps)) return rc;
   for (int l = Ls - 1; l >= 1; --l)  // up leg
     if (int rc = launch_visit(ctx, l, e_up, true, eps)) return rc;
   return ctx->lv[1].mb ? launch_finish64(ctx, cycle_visit_ref(ctx, 1, e_up, true, eps)) : launch_report(ctx, 0);
@@ -1580,7 +1571,7 @@ int vcycle64(lepic_ctx* ctx, int k, double eps) {
 int vcycle32(lepic_ctx* ctx, int k, double eps) {
   for (int l = 1; l < ctx->Lc; ++l)
     if (int rc = tile_down(ctx, l)) return rc;
-  if (int rc = launch_tail32(ctx, k, eps)) return rc;
+  if (int rc = launch_lower<float>(ctx, k, eps)) return rc;
   for (int l = ctx->Lc - 1; l >= 1; --l)
     if (int rc = tile_up(ctx, l)) return rc;
   return 0;

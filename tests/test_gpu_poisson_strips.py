@@ -1,9 +1,9 @@
 """The mixed form's multigrid on register strips: a level's visit gives the
 same bits in the tiled kernel (k_tile32), in the single-workgroup kernel
-(k_tail32) and in the generic single-workgroup kernel, so phi must not depend
+(k_tail_strips) and in the generic single-workgroup kernel, so phi must not depend
 on mg_tail_nodes as long as the finest level stays tiled.  Sides whose strips
 fill their lanes unevenly, cells that are not square, a grid electrode, and a
-level too wide for the strips of k_tail32 (512 x 32)."""
+level too wide for the strips of k_tail_strips (512 x 32)."""
 import numpy as np
 import pytest
 

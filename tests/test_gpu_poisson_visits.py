@@ -1,7 +1,9 @@
 """FP64 solves whose multi-block levels exercise every shape of the visit
 kernel: launches of 8, 12 and 16 waves, more blocks than CUs, tiles cut by the
 grid on both sides, odd sides (ng = 1), cells that are not square, outer walls
-that differ from node to node, and a second solve from other wall values."""
+that differ from node to node, and a second solve from other wall values; and
+levels below them on strips (lanes filled unevenly, one strip per wave) or, too
+wide or too many for LDS, in the generic single-workgroup kernel."""
 import numpy as np
 import pytest
 
@@ -16,7 +18,8 @@ pytestmark = pytest.mark.gpu
 # 256 of 12: 1280 x 768 nodes launch 8, 12 and 16 waves on its levels
 @pytest.mark.parametrize("n1,n2,ng,aspect,tail,eps", [
     (101, 67, 1, 1.0, 100, 1e-4), (66, 131, 1, 1.3, 100, 1e-4), (96, 160, 4, 0.7, 100, 1e-10),
-    (320, 64, 4, 1.0, 100, 1e-10), (1280, 768, 8, 1.0, 0, 1e-7), (1280, 768, 8, 1.2, 2000, 1e-7)])
+    (320, 64, 4, 1.0, 100, 1e-10), (256, 128, 7, 1.0, 0, 1e-10), (160, 160, 5, 0.8, 0, 1e-10),
+    (224, 32, 4, 1.0, 0, 1e-10), (512, 32, 5, 1.0, 0, 1e-10), (192, 192, 6, 1.0, 10000, 1e-10), (1280, 768, 8, 1.0, 0, 1e-7), (1280, 768, 8, 1.2, 2000, 1e-7)])
 def test_fp64_visits_match_oracle(n1, n2, ng, aspect, tail, eps):
     dom = S.box_domain(n1, n2, Bmode=None)
     h = (dom.h1, dom.h2 * aspect)
