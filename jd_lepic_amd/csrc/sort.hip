@@ -9,15 +9,16 @@
 //  1. k_seg_sort: one block per segment sorts the segment's keys stably in
 //     LDS (LSD passes of 8-bit digits of the key minus the segment's
 //     smallest key, as many as the segment's key span needs) and records,
-//     for every slot, its run (a maximal group of equal keys in the sorted
-//     segment) and its rank inside the run, and for every run its key and
+//     for every slot, its place in the sorted segment and its run (a maximal
+//     group of equal keys there), and for every run its key, first place and
 //     particle count.
 //  2. The runs of all segments, in segment order, are sorted stably by key
 //     (global LSD radix passes of up to 11 bits over the runs only), and an
 //     exclusive scan of their counts in sorted order gives every run its
 //     first output position.
-//  3. k_seg_scatter: one block per segment writes every particle to its
-//     run's position plus its rank, into the other particle buffer.
+//  3. k_seg_scatter: one block per segment brings its particles into sorted
+//     order in LDS and writes them, run by run, to the runs' positions in the
+//     other particle buffer.
 // A particle's output position is then the number of particles in lower
 // cells, plus those of its cell in earlier segments, plus those of its cell
 // earlier in its own segment: exactly the stable sort's.  The payload moves
@@ -31,6 +32,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "lepic_internal.h"
 
@@ -44,7 +46,8 @@ constexpr int kMaxRadix = 2048;   // buckets of the widest global digit (11 bits
 constexpr int kMaxDigitBits = 11;
 constexpr int kSegThreads = 256;  // one block per segment: 4 waves x 4 rounds of 64 slots
 constexpr int kSegRounds = kChunk / kSegThreads;
-constexpr int kRankBits = 10;     // rank inside a run and run index inside a segment: < kChunk
+constexpr int kRankBits = 10;     // place and run index inside a segment: < kChunk
+constexpr int kCntBits = 11;      // particles of a run: <= kChunk
 static_assert(kChunk == (1 << kRankBits), "meta packing assumes 1024-slot segments");
 
 __device__ __forceinline__ uint64_t lanemask_lt() { return (1ull << (threadIdx.x & 63)) - 1ull; }
@@ -83,9 +86,9 @@ struct SegSortArgs {
   const double* y;
   double h1, h2;
   int n1, n2;
-  uint32_t* meta;             // [slot] (run << kRankBits) | rank in run
+  uint32_t* meta;             // [slot] (run << kRankBits) | place in the sorted segment
   uint32_t* rkey;             // [segment * kChunk + run] cell key of the run
-  uint32_t* rcnt;             // [segment * kChunk + run] particles of the run
+  uint32_t* rcnt;             // [segment * kChunk + run] (first place << kCntBits) | particles of the run
   uint32_t* nrun;             // [segment] runs of the segment
 };
 
@@ -194,9 +197,9 @@ __global__ __launch_bounds__(kSegThreads, 8) void k_seg_sort(SegSortArgs A) {
   if (npass <= 1) {  // block-uniform
     // The compact key is a single 8-bit digit: its counts give every slot's
     // place directly.  The slot's run is the number of distinct keys below
-    // its own and its rank the number of equal keys before it (the wave's
-    // earlier rounds, earlier waves, then earlier lanes): the stable sort's
-    // runs without moving the keys.
+    // its own, its place the number of smaller keys and of equal keys before
+    // it (the wave's earlier rounds, earlier waves, then earlier lanes): the
+    // stable sort's runs without moving the keys.
     for (int e = t; e < 4 * 256; e += kSegThreads) (&s_wc[0][0])[e] = 0u;
     __syncthreads();
     uint32_t d[kSegRounds], pos[kSegRounds];
@@ -212,25 +215,23 @@ __global__ __launch_bounds__(kSegThreads, 8) void k_seg_sort(SegSortArgs A) {
     // key t: its count and its run index
     const uint32_t c0 = s_wc[0][t], c1 = s_wc[1][t], c2 = s_wc[2][t], c3 = s_wc[3][t];
     const uint32_t ck = c0 + c1 + c2 + c3;
-    uint32_t nrun;
-    const uint32_t run = block_excl_scan(ck > 0u ? 1u : 0u, s_tot, &nrun);
-    // the earlier waves' counts of key t, then the run index, in LDS
-    s_wc[1][t] = c0;
-    s_wc[2][t] = c0 + c1;
-    s_wc[3][t] = c0 + c1 + c2;
-    s_wc[0][t] = run;
+    uint32_t tot;
+    const uint32_t pre = block_excl_scan((ck > 0u ? 1u << 16 : 0u) | ck, s_tot, &tot);   // runs and slots before key t
+    const uint32_t run = pre >> 16, start = pre & 0xFFFFu, nrun = tot >> 16;
+    // each wave's first place for key t, with the run index
+    s_wc[0][t] = (run << kRankBits) + start;
+    s_wc[1][t] = (run << kRankBits) + start + c0;
+    s_wc[2][t] = (run << kRankBits) + start + c0 + c1;
+    s_wc[3][t] = (run << kRankBits) + start + c0 + c1 + c2;
     if (ck > 0u) {
       A.rkey[base + run] = (t % dxs + xmin) + (uint32_t)A.n1 * (t / dxs + ymin);
-      A.rcnt[base + run] = ck;
+      A.rcnt[base + run] = (start << kCntBits) | ck;
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kSegRounds; ++r) {
       const int q = w * 256 + r * 64 + lane;
-      if (q < cnt) {
-        const uint32_t rank = (w > 0 ? s_wc[w][d[r]] : 0u) + pos[r];
-        A.meta[base + q] = (s_wc[0][d[r]] << kRankBits) | rank;
-      }
+      if (q < cnt) A.meta[base + q] = s_wc[w][d[r]] + pos[r];
     }
     if (t == 0) A.nrun[sg] = nrun;
     return;
@@ -306,13 +307,13 @@ __global__ __launch_bounds__(kSegThreads, 8) void k_seg_sort(SegSortArgs A) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int q = 4 * t + j;
-    if (q < cnt) A.meta[base + s_i[cur][q]] = (rid[j] << kRankBits) | (uint32_t)(q - s_head[rid[j]]);
+    if (q < cnt) A.meta[base + s_i[cur][q]] = (rid[j] << kRankBits) | (uint32_t)q;
   }
   for (uint32_t r = t; r < nrun; r += kSegThreads) {
     const int h = s_head[r];
     const uint32_t ck = s_k[cur][h];
     A.rkey[base + r] = (ck % dxs + xmin) + (uint32_t)A.n1 * (ck / dxs + ymin);
-    A.rcnt[base + r] = (uint32_t)(s_head[r + 1] - h);
+    A.rcnt[base + r] = ((uint32_t)h << kCntBits) | (uint32_t)(s_head[r + 1] - h);
   }
   if (t == 0) A.nrun[sg] = nrun;
 }
@@ -416,17 +417,18 @@ __global__ __launch_bounds__(256) void k_scatter(const uint32_t* __restrict__ ki
 }
 
 // counts of the runs in sorted order (for the offset scan) and, after the
-// scan, each run's first output position by its dense index
+// scan, what leads from a place in a run's segment to its output position, by
+// the run's dense index (modulo 2^32)
 __global__ void k_runs_sorted_counts(const uint32_t* __restrict__ perm, const uint32_t* __restrict__ cnt,
                                      uint32_t* __restrict__ out, int64_t M) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < M) out[j] = cnt[perm[j]];
+  if (j < M) out[j] = cnt[perm[j]] & ((1u << kCntBits) - 1u);
 }
 
 __global__ void k_runs_offsets(const uint32_t* __restrict__ perm, const uint32_t* __restrict__ off,
-                               uint32_t* __restrict__ roff, int64_t M) {
+                               const uint32_t* __restrict__ cnt, uint32_t* __restrict__ roff, int64_t M) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < M && perm[j] < M) roff[perm[j]] = off[j];
+  if (j < M && perm[j] < M) roff[perm[j]] = off[j] - (cnt[perm[j]] >> kCntBits);
 }
 
 // Plist from the sorted run keys K[0..M) and their first positions off:
@@ -451,82 +453,89 @@ struct SegScatterArgs {
   const int32_t* seg;
   const uint32_t* meta;
   const uint32_t* rbase;      // first dense run of each segment
-  const uint32_t* roff;       // first output position of each dense run
+  const uint32_t* roff;       // output position less place, of each dense run
   const double* a[6];         // FP64 payload in
   double* b[6];               // FP64 payload out
   const int32_t* ci;          // mixed payload in: cell + 6 FP32 (z may be null)
   const float* f[6];
   int32_t* co;
   float* g[6];
+  int64_t nseg;
+  int64_t nchunk;             // the segments in nchunk chunks of at most wmax
+  int64_t wmax;
   int64_t cap;                // slots of the output buffer
   int32_t* err;               // set when a destination falls outside it
 };
 
+// Chunks of the segments that k_seg_scatter's blocks take in turn: an eighth of
+// a row of cells each, so that each of the eight XCDs (blocks go round them)
+// works down a stripe of columns.  A cell's particles come from the rows
+// around it, and the pieces that they write of a line meet in the XCD's L2
+// only if it still holds the line: with whole rows per XCD, or rows dealt out
+// block by block, it does not (105 M electrons: 2.35 ms either way, 1.26 in
+// stripes).  Below kStripeMin segments per chunk the stripes say little and
+// half of the blocks would be empty: a chunk is a segment.
+constexpr int kXcds = 8, kStripeMin = 4;
+
+// Bound by memory.  In slot order almost every lane wrote a line of its own;
+// sorted in LDS first, neighbouring lanes write the same run.  A thread has
+// kSegRounds slots (t + r kSegThreads, so every access of a round is
+// coalesced) whose loads are all issued before any store.  All arrays pass
+// through LDS at once, which also keeps few enough blocks on a CU (4 mixed, 3
+// FP64) that the lines in the making fit the L2 (see kXcds; with 6 to 8 blocks
+// 1.45 to 1.65 ms).  105 M electrons on 1024 x 1024 cells 2.35 to 1.26 ms, ions
+// 1.07 to 1.00 (5.0 TB/s); 26 M in FP64 on 512 x 512 0.83 to 0.62.
 template <bool kMixed>
 __global__ __launch_bounds__(kSegThreads) void k_seg_scatter(SegScatterArgs A) {
-  // kSegRounds slots per thread (slot t + r*kSegThreads, so every access of a
-  // round is coalesced); the payload and run loads of all rounds are issued
-  // before any store
-  constexpr int R = kSegRounds;
-  const int64_t sg = blockIdx.x;
+  using T = std::conditional_t<kMixed, uint32_t, double>;
+  constexpr int R = kSegRounds, kN = kMixed ? 7 : 6;
+  __shared__ T s_p[kN][kChunk];
+  __shared__ uint32_t s_o[kChunk];
+  const int64_t c = (blockIdx.x / kXcds) / A.wmax * kXcds + blockIdx.x % kXcds;
+  const int64_t sg = c * A.nseg / A.nchunk + (blockIdx.x / kXcds) % A.wmax;
+  if (c >= A.nchunk || sg >= (c + 1) * A.nseg / A.nchunk) return;
   const int cnt = A.seg[sg];
   const int64_t base = sg * (int64_t)kChunk;
   const uint32_t rb = A.rbase[sg];
   const int t = threadIdx.x;
-  bool v[R];
+  auto src = [&](int k) { return kMixed ? (const T*)(k == 0 ? (const void*)A.ci : (const void*)A.f[k - 1]) : (const T*)A.a[k]; };
+  auto dst = [&](int k) { return kMixed ? (T*)(k == 0 ? (void*)A.co : (void*)A.g[k - 1]) : (T*)A.b[k]; };
   uint32_t m[R];
+  T v[kN][R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int j = t + r * kSegThreads;
-    v[r] = j < cnt;
-    m[r] = v[r] ? A.meta[base + j] : 0u;
+    m[r] = j < cnt ? A.meta[base + j] : 0u;
+#pragma unroll
+    for (int k = 0; k < kN; ++k) {
+      v[k][r] = (T)0;
+      if (j < cnt && dst(k)) v[k][r] = src(k)[base + j];          // mixed: z may not be kept
+    }
   }
-  if (kMixed) {
-    int32_t c[R];
-    float f[6][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int64_t i = base + t + r * kSegThreads;
-      c[r] = v[r] ? A.ci[i] : 0;
-#pragma unroll
-      for (int k = 0; k < 6; ++k) f[k][r] = (v[r] && (k != 2 || A.g[2])) ? A.f[k][i] : 0.f;
+  for (int r = 0; r < R; ++r)
+    if (t + r * kSegThreads < cnt) {
+      const uint32_t q = m[r] & (kChunk - 1);
+      s_o[q] = A.roff[rb + (m[r] >> kRankBits)] + q;
     }
-    int64_t o[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) o[r] = v[r] ? (int64_t)A.roff[rb + (m[r] >> kRankBits)] + (m[r] & (kChunk - 1)) : 0;
+  for (int k = 0; k < kN; ++k)
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (!v[r]) continue;
-      if (o[r] >= A.cap) {        // cannot happen for consistent runs; never write past the buffer
-        *A.err = 1;
-        continue;
-      }
-      A.co[o[r]] = c[r];
+    for (int r = 0; r < R; ++r)
+      if (t + r * kSegThreads < cnt) s_p[k][m[r] & (kChunk - 1)] = v[k][r];
+  __syncthreads();
 #pragma unroll
-      for (int k = 0; k < 6; ++k)
-        if (k != 2 || A.g[2]) A.g[k][o[r]] = f[k][r];
+  for (int r = 0; r < R; ++r) {
+    const int j = t + r * kSegThreads;
+    if (j >= cnt) continue;
+    const int64_t o = s_o[j];
+    if (o >= A.cap) {             // cannot happen for consistent runs; never write past the buffer
+      *A.err = 1;
+      continue;
     }
-  } else {
-    double d[6][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int64_t i = base + t + r * kSegThreads;
-#pragma unroll
-      for (int k = 0; k < 6; ++k) d[k][r] = v[r] ? A.a[k][i] : 0.0;
-    }
-    int64_t o[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) o[r] = v[r] ? (int64_t)A.roff[rb + (m[r] >> kRankBits)] + (m[r] & (kChunk - 1)) : 0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (!v[r]) continue;
-      if (o[r] >= A.cap) {
-        *A.err = 1;
-        continue;
-      }
-#pragma unroll
-      for (int k = 0; k < 6; ++k) A.b[k][o[r]] = d[k][r];
-    }
+    for (int k = 0; k < kN; ++k)
+      if (T* d = dst(k)) d[o] = s_p[k][j];
   }
 }
 
@@ -674,7 +683,8 @@ int sort_core(lepic_ctx* ctx, int p, int32_t* Plist_host, const SortWork& W, int
     hipLaunchKernelGGL(k_runs_sorted_counts, gm, dim3(256), 0, ctx->stream, perm, (const uint32_t*)W.rcntd, off, M);
     LEPIC_HIP(hipGetLastError());
     if (int rc = scan_exclusive_u32(ctx, off, M, W.scan_ws)) return rc;
-    hipLaunchKernelGGL(k_runs_offsets, gm, dim3(256), 0, ctx->stream, perm, (const uint32_t*)off, W.rkey, M);
+    hipLaunchKernelGGL(k_runs_offsets, gm, dim3(256), 0, ctx->stream, perm, (const uint32_t*)off,
+                       (const uint32_t*)W.rcntd, W.rkey, M);
     LEPIC_HIP(hipGetLastError());
     // 3. the payload, once
     SegScatterArgs S{};
@@ -686,8 +696,13 @@ int sort_core(lepic_ctx* ctx, int p, int32_t* Plist_host, const SortWork& W, int
     S.ci = s.cell[b]; S.co = s.cell[o];
     S.cap = (s.nseg_cap - 1) * kChunk;   // alloc_species: nseg_cap = slots / kChunk + 1
     S.err = ctx->d_error + 12;
-    if (mixed) hipLaunchKernelGGL(k_seg_scatter<true>, dim3((unsigned)nseg), dim3(kSegThreads), 0, ctx->stream, S);
-    else hipLaunchKernelGGL(k_seg_scatter<false>, dim3((unsigned)nseg), dim3(kSegThreads), 0, ctx->stream, S);
+    const int64_t stripes = (int64_t)kXcds * n2;
+    S.nseg = nseg;
+    S.nchunk = nseg >= kStripeMin * stripes ? stripes : nseg;
+    S.wmax = (nseg + S.nchunk - 1) / S.nchunk;
+    const dim3 gs((unsigned)((S.nchunk + kXcds - 1) / kXcds * kXcds * S.wmax));
+    if (mixed) hipLaunchKernelGGL(k_seg_scatter<true>, gs, dim3(kSegThreads), 0, ctx->stream, S);
+    else hipLaunchKernelGGL(k_seg_scatter<false>, gs, dim3(kSegThreads), 0, ctx->stream, S);
     LEPIC_HIP(hipGetLastError());
   }
   s.cur = o;
