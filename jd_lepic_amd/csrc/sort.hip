@@ -40,8 +40,13 @@ using namespace lepic;
 
 namespace {
 
-constexpr int kSortItems = 64;
+// Keys per thread of the run sort's blocks: the most that still give every CU
+// a block, but no fewer keys per block than it has counters (the fewest only
+// for 256 buckets).  A pass over the runs of 400 k particles: 73 us at 64 keys
+// (three blocks), 10 at 4; of 105 M ions 100 us at 64, 46 at 16.
+constexpr int kSortItems = 64, kSortItemsMid = 16, kSortItemsMin = 4;
 constexpr int kTile = 256 * kSortItems;
+constexpr int kSortBlocks = 256;
 constexpr int kMaxRadix = 2048;   // buckets of the widest global digit (11 bits)
 constexpr int kMaxDigitBits = 11;
 constexpr int kSegThreads = 256;  // one block per segment: 4 waves x 4 rounds of 64 slots
@@ -334,46 +339,45 @@ __global__ __launch_bounds__(64) void k_runs_pack(const uint32_t* __restrict__ r
 // ---------------------------------------------------------------------------
 // 2. global stable radix sort of the runs by key
 // ---------------------------------------------------------------------------
-// Digit counts of a wave's kSortItems x 64 keys from base, added to cnt.  The
+// Digit counts of a wave's IT x 64 keys from base, added to cnt.  The
 // keys are loaded kLoadBatch per lane at a time, so a wave waits for one
 // memory latency per batch rather than one per 64 keys.
-constexpr int kLoadBatch = 16;
-static_assert(kSortItems % kLoadBatch == 0, "whole load batches per wave");
+template <int IT> constexpr int kLoadBatch = IT < 16 ? IT : 16;
 
-template <int R>
+template <int R, int IT>
 __device__ __forceinline__ void count_digits(const uint32_t* __restrict__ key, int64_t base, int64_t n, int shift,
                                              uint32_t* cnt) {
   const int lane = threadIdx.x & 63;
-  for (int j0 = 0; j0 < kSortItems; j0 += kLoadBatch) {
-    uint32_t d[kLoadBatch];
+  for (int j0 = 0; j0 < IT; j0 += kLoadBatch<IT>) {
+    uint32_t d[kLoadBatch<IT>];
 #pragma unroll
-    for (int u = 0; u < kLoadBatch; ++u) {
+    for (int u = 0; u < kLoadBatch<IT>; ++u) {
       const int64_t i = base + (int64_t)(j0 + u) * 64 + lane;
       d[u] = i < n ? (key[i] >> shift) & (uint32_t)(R - 1) : 0u;
     }
 #pragma unroll
-    for (int u = 0; u < kLoadBatch; ++u)
+    for (int u = 0; u < kLoadBatch<IT>; ++u)
       wave_match<Log2<R>::v>(base + (int64_t)(j0 + u) * 64 + lane < n, d[u], cnt);
   }
 }
 
-// Each wave owns a contiguous quarter of the tile (kTile/4 keys, read 64 at a
+// Each wave owns a contiguous quarter of the block's keys (read 64 at a
 // time), so stability across waves is a per-digit prefix over the four
 // waves and no barrier is needed inside the loops.
-template <int R>   // buckets per pass
+template <int R, int IT>   // buckets per pass, keys per thread
 __global__ __launch_bounds__(256) void k_hist(const uint32_t* __restrict__ key, int64_t n, int shift,
                                               uint32_t* __restrict__ hist, int nb) {
   __shared__ uint32_t wc[4][R];
   const int t = threadIdx.x, w = t >> 6;
   for (int q = t; q < R; q += 256) wc[0][q] = wc[1][q] = wc[2][q] = wc[3][q] = 0;
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)w * (kTile / 4);
-  count_digits<R>(key, base, n, shift, wc[w]);
+  const int64_t base = ((int64_t)blockIdx.x * 4 + w) * (IT * 64);
+  count_digits<R, IT>(key, base, n, shift, wc[w]);
   __syncthreads();
   for (int q = t; q < R; q += 256) hist[(int64_t)q * nb + blockIdx.x] = wc[0][q] + wc[1][q] + wc[2][q] + wc[3][q];
 }
 
-template <int R>
+template <int R, int IT>
 __global__ __launch_bounds__(256) void k_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                  uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                  const uint32_t* __restrict__ hist, int64_t n, int shift, int nb) {
@@ -381,8 +385,8 @@ __global__ __launch_bounds__(256) void k_scatter(const uint32_t* __restrict__ ki
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   for (int q = t; q < R; q += 256) wc[0][q] = wc[1][q] = wc[2][q] = wc[3][q] = 0;
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kTile + (int64_t)w * (kTile / 4);
-  count_digits<R>(kin, base, n, shift, wc[w]);
+  const int64_t base = ((int64_t)blockIdx.x * 4 + w) * (IT * 64);
+  count_digits<R, IT>(kin, base, n, shift, wc[w]);
   __syncthreads();
   for (int q = t; q < R; q += 256) {
     const uint32_t g = hist[(int64_t)q * nb + blockIdx.x];
@@ -393,17 +397,17 @@ __global__ __launch_bounds__(256) void k_scatter(const uint32_t* __restrict__ ki
     wc[3][q] = g + c0 + c1 + c2;
   }
   __syncthreads();
-  for (int j0 = 0; j0 < kSortItems; j0 += kLoadBatch) {
-    uint32_t kk[kLoadBatch], vv[kLoadBatch];
+  for (int j0 = 0; j0 < IT; j0 += kLoadBatch<IT>) {
+    uint32_t kk[kLoadBatch<IT>], vv[kLoadBatch<IT>];
 #pragma unroll
-    for (int u = 0; u < kLoadBatch; ++u) {
+    for (int u = 0; u < kLoadBatch<IT>; ++u) {
       const int64_t i = base + (int64_t)(j0 + u) * 64 + lane;
       const bool valid = i < n;
       kk[u] = valid ? kin[i] : 0u;
       vv[u] = valid ? (vin ? vin[i] : (uint32_t)i) : 0u;
     }
 #pragma unroll
-    for (int u = 0; u < kLoadBatch; ++u) {
+    for (int u = 0; u < kLoadBatch<IT>; ++u) {
       const bool valid = base + (int64_t)(j0 + u) * 64 + lane < n;
       const uint32_t d = (kk[u] >> shift) & (uint32_t)(R - 1);
       const uint32_t b = valid ? wc[w][d] : 0u;          // read before this round's counts are added
@@ -560,6 +564,7 @@ struct SortWork {
   uint32_t* rcntd;
   uint32_t* nrun;
   uint32_t* hist;
+  int64_t hist_cap;
   uint32_t* plist;
   uint32_t* scan_ws;
 };
@@ -612,17 +617,30 @@ static __device__ __align__(256) uint32_t scratch[kStaticWords];
 
 namespace lepic {
 
-template <int R>
-int radix_pass(lepic_ctx* ctx, const SortWork& W, int cur, int pass, int shift, int64_t n, int64_t nb) {
-  hipLaunchKernelGGL(k_hist<R>, dim3((unsigned)nb), dim3(256), 0, ctx->stream, W.key[cur], n, shift, W.hist,
+template <int R, int IT>
+int radix_pass_of(lepic_ctx* ctx, const SortWork& W, int cur, int pass, int shift, int64_t n) {
+  const int64_t nb = (n + 256 * IT - 1) / (256 * IT);
+  hipLaunchKernelGGL((k_hist<R, IT>), dim3((unsigned)nb), dim3(256), 0, ctx->stream, W.key[cur], n, shift, W.hist,
                      (int)nb);
   LEPIC_HIP(hipGetLastError());
   if (int rc = scan_exclusive_u32(ctx, W.hist, (int64_t)R * nb, W.scan_ws)) return rc;
-  hipLaunchKernelGGL(k_scatter<R>, dim3((unsigned)nb), dim3(256), 0, ctx->stream, W.key[cur],
+  hipLaunchKernelGGL((k_scatter<R, IT>), dim3((unsigned)nb), dim3(256), 0, ctx->stream, W.key[cur],
                      pass == 0 ? (const uint32_t*)nullptr : W.val[cur], W.key[1 - cur], W.val[1 - cur], W.hist, n,
                      shift, (int)nb);
   LEPIC_HIP(hipGetLastError());
   return 0;
+}
+
+template <int R>
+int radix_pass(lepic_ctx* ctx, const SortWork& W, int cur, int pass, int shift, int64_t n) {
+  // the histogram holds one word per bucket and block
+  auto fits = [&](int it) { return (n + 256 * it - 1) / (256 * it) * R <= W.hist_cap; };
+  if (n > (int64_t)kSortBlocks * 256 * kSortItems || !fits(kSortItemsMid))
+    return radix_pass_of<R, kSortItems>(ctx, W, cur, pass, shift, n);
+  if constexpr (R <= 256)
+    if (n <= (int64_t)kSortBlocks * 256 * kSortItemsMid && fits(kSortItemsMin))
+      return radix_pass_of<R, kSortItemsMin>(ctx, W, cur, pass, shift, n);
+  return radix_pass_of<R, kSortItemsMid>(ctx, W, cur, pass, shift, n);
 }
 
 // The sort of species p with its device buffers in W (sized for nseg
@@ -661,7 +679,6 @@ int sort_core(lepic_ctx* ctx, int p, int32_t* Plist_host, const SortWork& W, int
   // 2. the runs sorted by key (stable), in the fewest digits of at most 11 bits
   int cur = 0;
   if (M > 0) {
-    const int64_t nb = (M + kTile - 1) / kTile;
     int bits = 1;
     while ((1ll << bits) < ncell) ++bits;
     const int npass = (bits + kMaxDigitBits - 1) / kMaxDigitBits;
@@ -669,10 +686,10 @@ int sort_core(lepic_ctx* ctx, int p, int32_t* Plist_host, const SortWork& W, int
     for (int pass = 0; pass < npass; ++pass) {
       const int shift = pass * lo, width = std::min(lo, bits - shift);
       int rc;
-      if (width <= 8) rc = radix_pass<256>(ctx, W, cur, pass, shift, M, nb);
-      else if (width <= 9) rc = radix_pass<512>(ctx, W, cur, pass, shift, M, nb);
-      else if (width <= 10) rc = radix_pass<1024>(ctx, W, cur, pass, shift, M, nb);
-      else rc = radix_pass<2048>(ctx, W, cur, pass, shift, M, nb);
+      if (width <= 8) rc = radix_pass<256>(ctx, W, cur, pass, shift, M);
+      else if (width <= 9) rc = radix_pass<512>(ctx, W, cur, pass, shift, M);
+      else if (width <= 10) rc = radix_pass<1024>(ctx, W, cur, pass, shift, M);
+      else rc = radix_pass<2048>(ctx, W, cur, pass, shift, M);
       if (rc) return rc;
       cur = 1 - cur;
     }
@@ -738,7 +755,7 @@ int sort_launch(lepic_ctx* ctx, int p, int32_t* Plist_host) {
   SortWork W{};
   for (int k = 0; k < 2; ++k) { W.key[k] = ctx->s_key[k]; W.val[k] = ctx->s_val[k]; }
   W.meta = ctx->s_meta; W.rkey = ctx->s_rkey; W.rcnt = ctx->s_rcnt; W.rcntd = ctx->s_rcntd;
-  W.nrun = ctx->s_nrun; W.hist = ctx->s_hist; W.plist = (uint32_t*)ctx->d_plist; W.scan_ws = nullptr;
+  W.nrun = ctx->s_nrun; W.hist = ctx->s_hist; W.hist_cap = ctx->s_hist_cap; W.plist = (uint32_t*)ctx->d_plist; W.scan_ws = nullptr;
   return sort_core(ctx, p, Plist_host, W, nseg, pl_max);
 }
 
@@ -788,6 +805,7 @@ int sort_noalloc_launch(lepic_ctx* ctx, int p, int32_t* Plist_host) {
   W.rcntd = w; w += kStaticSlots;
   W.nrun = w; w += kStaticSeg + 2;
   W.hist = w; w += kStaticHist;
+  W.hist_cap = kStaticHist;
   W.plist = w; w += kStaticPlist;
   W.scan_ws = w;
   return sort_core(ctx, p, Plist_host, W, nseg, pl_max);
