@@ -59,3 +59,28 @@ def test_mixed_push_is_the_same_in_both_launch_forms(z):
             out.append(ctx.download(1))
     assert len(out[0]) > 0.9 * n
     assert np.array_equal(out[0], out[1][:len(out[0])])
+
+
+@pytest.mark.parametrize("precision", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("n1,n2,per_cell,push", [(96, 20, 30, True), (96, 20, 30, False), (300, 9, 7, True), (300, 9, 7, False)])
+def test_density_of_segments_over_the_end_of_a_row(n1, n2, per_cell, push, precision):
+    """Particles in cell order whose segments run over the end of a row of
+    cells, and (7 per cell) over 146 columns, more than either window holds."""
+    dom = S.box_domain(n1, n2, Bmode=None)
+    count = per_cell * n1 * n2
+    parts = S.particles(dom, count, 1.0, seed=n1, edge_frac=0.0)
+    parts = parts[np.lexsort(((parts[:, 0] / dom.h1).astype(int), (parts[:, 1] / dom.h2).astype(int)))]
+    with L.Context(n1, n2, dom.h1, dom.h2, dom.dt, [L.Species(-L.QE, L.ME, 55.0, count)], zmax=dom.zmax,
+                   ngrid=dom.ngrid, precision=precision) as ctx:
+        ctx.set_boundary(dom.bcnd, np.zeros((n2 + 3, n1 + 3)))
+        ctx.upload(1, parts)
+        if push:
+            ctx.part_mover(1, deposit=True)
+        else:
+            ctx.charge_deposition(1)
+        now, rho = ctx.download(1), ctx.get_grid(L.GRID_NP, 1)
+    ref = O.charge_deposition(dom, 55.0, now)
+    # mixed: every weight is rounded to 2^-20 (half: 4.8e-7) from FP32 factors
+    # (2^-23), and four times a cell's particles touch a node; FP64: 2^-42
+    tol = 4 * (2.0 ** -21 + 2.0 ** -22) if precision == L.MIXED else 1e-12
+    assert np.abs(rho - ref).max() <= tol * np.abs(ref).max()
