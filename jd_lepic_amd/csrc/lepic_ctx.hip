@@ -301,8 +301,10 @@ int alloc_species(lepic_ctx* ctx, int p) {
   s.packed = true;
   LEPIC_HIP(hipMalloc(&s.np, ctx->nodes * 8));
   LEPIC_HIP(hipMemsetAsync(s.np, 0, ctx->nodes * 8, ctx->stream));
-  LEPIC_HIP(hipMalloc(&s.acc, ctx->nodes * 8));
-  LEPIC_HIP(hipMemsetAsync(s.acc, 0, ctx->nodes * 8, ctx->stream));
+  for (int b = 0; b < 2; ++b) {
+    LEPIC_HIP(hipMalloc(&s.acc[b], ctx->nodes * 8));
+    LEPIC_HIP(hipMemsetAsync(s.acc[b], 0, ctx->nodes * 8, ctx->stream));
+  }
   LEPIC_HIP(hipMalloc(&s.np_red, ctx->nodes * 8));
   LEPIC_HIP(hipMemsetAsync(s.np_red, 0, ctx->nodes * 8, ctx->stream));
   LEPIC_HIP(hipMalloc(&s.sink, ctx->nodes * 8));
@@ -409,7 +411,7 @@ int lepic_destroy(lepic_ctx* ctx) {
   for (int p = 0; p < ctx->nsp; ++p) {
     Species& s = ctx->sp[p];
     for (int b = 0; b < 2; ++b) (void)hipFree(s.mem[b]);
-    (void)hipFree(s.flag_dead); (void)hipFree(s.np); (void)hipFree(s.acc); (void)hipFree(s.np_red); (void)hipFree(s.sink); (void)hipFree(s.src);
+    (void)hipFree(s.flag_dead); (void)hipFree(s.np); (void)hipFree(s.acc[0]); (void)hipFree(s.acc[1]); (void)hipFree(s.np_red); (void)hipFree(s.sink); (void)hipFree(s.src);
     (void)hipFree(s.seg[0]); (void)hipFree(s.seg[1]);
   }
   void* ptrs[] = {ctx->bc, ctx->phi, ctx->phi_given, ctx->rhs, ctx->E, ctx->Ef, ctx->Bi, ctx->Bf,

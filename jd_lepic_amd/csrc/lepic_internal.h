@@ -107,7 +107,10 @@ struct Species {
   // since the last push (a push consumes and clears every set flag)
   bool dead_maybe = true;
   double* np = nullptr;              // deposited density (nodes)
-  int64_t* acc = nullptr;            // fixed-point deposition accumulator (nodes), scaled into np
+  // fixed-point deposition accumulators (nodes): acc[acc_cur] holds the last
+  // deposition, scaled into np, the other one is zero for the next
+  int64_t* acc[2] = {nullptr, nullptr};
+  int acc_cur = 0;
   double* np_red = nullptr;
   double* sink = nullptr;            // ss2D(2): sink counts (nodes)
   double* src = nullptr;             // ss2D(1): source counts (nodes)
