@@ -138,15 +138,32 @@ int load_uniform_launch(lepic_ctx* ctx, int p, int ppc, double vt, double xl, do
   return set_packed_counts(ctx, p);
 }
 
-// SUM(p_mac(ptype, np_loss, 0:ngrid)) per species: particles lost at walls
-int lost_counts(lepic_ctx* ctx, double* out) {
-  for (int q = 0; q < ctx->nsp; ++q) {
-    double p_mac[2 * 65];
-    if (int rc = lepic_get_mover_tally(ctx, q + 1, nullptr, p_mac, nullptr)) return rc;
-    double s = 0.0;
-    for (int g = 0; g <= ctx->g.ngrid; ++g) s += p_mac[g];
-    out[q] = s;
-  }
+// SUM(p_mac(ptype, np_loss, 0:ngrid)) per species, particles lost at walls, to
+// word `slot` x kMaxSpecies of the scalar scratch.  Reading the tallies back
+// whole, once per species before and after the pushes, took 360 us of a 5.2 ms
+// step of the ion source.
+static_assert(kTallyCopies == 64, "a lane per copy");
+__global__ __launch_bounds__(64) void k_lost_counts(const Tally* __restrict__ tally, int ngrid, double* __restrict__ out) {
+  const Tally& t = tally[(size_t)blockIdx.x * kTallyCopies + threadIdx.x];
+  double s = 0.0;
+  for (int g = 0; g <= ngrid; ++g) s += t.p_mac[0][g];
+  s = wave_sum(s);                 // whole numbers: exact in any order
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
+int lost_counts_launch(lepic_ctx* ctx, int slot) {
+  static_assert(2 * kMaxSpecies <= 32, "the scalar scratch's first half");
+  hipLaunchKernelGGL(k_lost_counts, dim3((unsigned)ctx->nsp), dim3(64), 0, ctx->stream, (const Tally*)ctx->d_tally,
+                     ctx->g.ngrid, ctx->d_scalar + slot * kMaxSpecies);
+  LEPIC_HIP(hipGetLastError());
+  return 0;
+}
+
+// what the pushes between slots 0 and 1 lost, added to out
+int lost_counts_add(lepic_ctx* ctx, double* out) {
+  LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, ctx->d_scalar, 2 * kMaxSpecies * 8, hipMemcpyDeviceToHost, ctx->stream));
+  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
+  for (int q = 0; q < ctx->nsp; ++q) out[q] += ctx->h_pinned[kMaxSpecies + q] - ctx->h_pinned[q];
   return 0;
 }
 
@@ -177,14 +194,10 @@ extern "C" int lepic_step(lepic_ctx* ctx, int32_t it, lepic_step_args* a) {
   // opt_inj = +-2 re-injects the wall losses of every push since the last
   // injection: sav_np before and after each push (main.f90:1044-1056)
   const bool count_losses = a->inj && (a->inj->opt_inj == 2 || a->inj->opt_inj == -2);
-  double lost0[kMaxSpecies] = {};
-  if (!rc && count_losses) rc = lost_counts(ctx, lost0);
+  if (!rc && count_losses) rc = lost_counts_launch(ctx, 0);
   for (int p = 1; p <= ctx->nsp && !rc; ++p) rc = lepic_part_mover(ctx, p, 1);  // :1041-1086
-  if (!rc && count_losses) {
-    double lost1[kMaxSpecies] = {};
-    rc = lost_counts(ctx, lost1);
-    for (int q = 0; q < ctx->nsp; ++q) ctx->inj_lost[q] += lost1[q] - lost0[q];
-  }
+  if (!rc && count_losses) rc = lost_counts_launch(ctx, 1);
+  if (!rc && count_losses) rc = lost_counts_add(ctx, ctx->inj_lost);
   a->injected = 0;
   if (!rc && inject) {  // :1063-1071
     int64_t N_inj[kMaxSpecies] = {};
