@@ -46,7 +46,6 @@ struct SpeciesMcc {
   double nu_max;
   double nu_omp;                 // nu_max_OMP (collisions.f90:172)
   int64_t Nc;
-  double rg_inv[5];              // 1/np_tot_rg(ptype, rg)
 };
 
 struct PartPtrs {
@@ -331,7 +330,8 @@ struct ProdArgs {
   int8_t* st_type;               // [Nc*kMaxCreate] byproduct species (1-based) or 0
   int64_t* st_ip;                // [Nc] incident particle of the candidate
   double* st_v;                  // [Nc*kMaxCreate*3]
-  uint32_t* ncreate;             // [kMaxSpecies][Nc]
+  uint32_t* ncreate;             // [nsp][Nc], and a last zero: their exclusive scan has the total there
+  const double* rg_inv;          // [n_rg] 1/np_tot_rg(ptype, rg)
   int64_t Nc;
   double* cnt_col;
   double* ploss3;
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256) void k_mcc_prod(ProdArgs A) {
       const int* ci = T.col_info[c_ind - 1];
       const int n_re = ci[0], n_by = ci[1], rt = ci[2 + n_re + n_by];
       atomicAdd(&s_ev[icol_hit], 1ull);
-      if (rg_hit >= 0) atomicAdd(&s_cnt[2][icol_hit][rg_hit], S.rg_inv[rg_hit]);
+      if (rg_hit >= 0) atomicAdd(&s_cnt[2][icol_hit][rg_hit], A.rg_inv[rg_hit]);
       int slot = 0;
       A.st_ip[c] = ip;
       if (rt != 4) {
@@ -559,13 +559,14 @@ __global__ __launch_bounds__(256) void k_mcc_prod(ProdArgs A) {
 
 // append staged particles at N_b + exclusive(ncreate_b)[c], in candidate
 // order, at the position of the candidate's incident particle
-// (collisions.f90:804-816)
+// (collisions.f90:804-816); block row b is species b, offs the exclusive scan
+// of all species' create counts one after the other
 template <bool kMixed>
-__global__ void k_mcc_append(ProdArgs A, const uint32_t* __restrict__ offs, int b) {
+__global__ void k_mcc_append(ProdArgs A, const uint32_t* __restrict__ offs) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= A.Nc) return;
-  const int bt = b + 1, q = A.q;
-  const int64_t base = A.counts[b] + offs[c];
+  const int b = blockIdx.y, bt = b + 1, q = A.q;
+  const int64_t base = A.counts[b] + (offs[b * A.Nc + c] - offs[b * A.Nc]);
   int k = 0;
   for (int s = 0; s < kMaxCreate; ++s) {
     const int64_t so = c * kMaxCreate + s;
@@ -593,10 +594,11 @@ __global__ void k_mcc_append(ProdArgs A, const uint32_t* __restrict__ offs, int 
   }
 }
 
-__global__ void k_add_count(int64_t* counts, int b, const uint32_t* offs, const uint32_t* cnt,
-                            int64_t Nc, unsigned long long* created) {
-  if (threadIdx.x || blockIdx.x || Nc <= 0) return;
-  const uint64_t tot = (uint64_t)offs[Nc - 1] + cnt[Nc - 1];
+__global__ __launch_bounds__(64) void k_add_counts(int64_t* counts, const uint32_t* __restrict__ offs, int nsp,
+                                                   int64_t Nc, unsigned long long* created) {
+  const int b = threadIdx.x;
+  if (b >= nsp) return;
+  const uint32_t tot = offs[(b + 1) * Nc] - offs[b * Nc];
   counts[b] += (int64_t)tot;
   created[b] += tot;
 }
@@ -696,14 +698,14 @@ int mcc_run(lepic_ctx* ctx, int it, int mode, uint64_t seed, int32_t* iseed, lep
   MccTab* dtab = (MccTab*)ctx->d_mcc_tab;
   if (int rc = upload_tab(ctx, &dtab)) return rc;
   ctx->d_mcc_tab = dtab;
-  int32_t* d_status = ctx->d_error + 4;
-  unsigned long long* d_events = (unsigned long long*)ctx->d_mcc_i64;        // [32]
-  unsigned long long* d_created = (unsigned long long*)ctx->d_mcc_i64 + 40;  // [8]
-  unsigned long long* d_missed = (unsigned long long*)ctx->d_mcc_i64 + 48;
+  // the call's counters, cleared together and read back together: events [32],
+  // (another kernel's 8 words), created [8], missed, status
+  constexpr int kCreated = 40, kMissed = 48, kStatus = 49, kCounters = 50;
+  unsigned long long* d_cnt = (unsigned long long*)ctx->d_mcc_i64;
+  unsigned long long *d_events = d_cnt, *d_created = d_cnt + kCreated, *d_missed = d_cnt + kMissed;
+  int32_t* d_status = (int32_t*)(d_cnt + kStatus);
   if (R.ncol > 32) return ctx->fail(LEPIC_ERR_UNSUPPORTED, "more than 32 reactions");
-  if (int rc = zero_async(ctx, ctx->d_mcc_i64, 32 * 8)) return rc;
-  if (int rc = zero_async(ctx, d_created, 16 * 8)) return rc;
-  if (int rc = zero_async(ctx, d_status, 4)) return rc;
+  if (int rc = zero_async(ctx, d_cnt, kCounters * 8)) return rc;
   double* d_ploss3 = ctx->d_mcc_f64;  // [ptype], accumulated until lepic_reset_tallies
   // candidates are drawn by particle index: dense arrays
   for (int q = 0; q < ctx->nsp; ++q)
@@ -776,17 +778,17 @@ int mcc_run(lepic_ctx* ctx, int it, int mode, uint64_t seed, int32_t* iseed, lep
         hipLaunchKernelGGL(k_region_final, dim3(1), dim3(64), 0, ctx->stream, (const double*)part, kRegionBlocks,
                            kk, d_rg + rg);
       }
-      LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_rg, 5 * 8, hipMemcpyDeviceToHost, ctx->stream));
       // scratch: claim bitmap, staging
-      const int64_t words = (N[q] + 31) / 32;
+      const int64_t words = (N[q] + 63) / 64 * 2;
       if (words > ctx->claim_cap) {
         if (ctx->d_claim) LEPIC_HIP(hipFree(ctx->d_claim));
         LEPIC_HIP(hipMalloc(&ctx->d_claim, words * 4));
         ctx->claim_cap = words;
       }
-      // staging: velocities, incident index, per-species create counts, the
-      // scanned copy of one species' counts, byproduct types
-      const size_t stage_bytes = (size_t)Nc * (kMaxCreate * (1 + 24) + 8 + 4 * kMaxSpecies + 4) + 1024;
+      // staging: velocities, incident index, per-species create counts (and
+      // the zero behind them), byproduct types; the last two are cleared
+      const size_t clear_bytes = ((size_t)Nc * (4 * ctx->nsp + kMaxCreate) + 4 + 7) / 8 * 8;
+      const size_t stage_bytes = (size_t)Nc * (kMaxCreate * 24 + 8) + clear_bytes;
       if ((int64_t)stage_bytes > ctx->stage_cap) {
         if (ctx->d_mcc_stage) LEPIC_HIP(hipFree(ctx->d_mcc_stage));
         LEPIC_HIP(hipMalloc(&ctx->d_mcc_stage, stage_bytes));
@@ -795,14 +797,10 @@ int mcc_run(lepic_ctx* ctx, int it, int mode, uint64_t seed, int32_t* iseed, lep
       char* st = (char*)ctx->d_mcc_stage;
       double* st_v = (double*)st;                                   st += (size_t)Nc * kMaxCreate * 24;
       int64_t* st_ip = (int64_t*)st;                                st += (size_t)Nc * 8;
-      uint32_t* ncreate = (uint32_t*)st;                            st += (size_t)Nc * 4 * kMaxSpecies;
-      uint32_t* offs = (uint32_t*)st;                               st += (size_t)Nc * 4;
+      uint32_t* ncreate = (uint32_t*)st;                            st += ((size_t)Nc * ctx->nsp + 1) * 4;
       int8_t* st_type = (int8_t*)st;
       if (int rc = zero_async(ctx, ctx->d_claim, words * 4)) return rc;
-      if (int rc = zero_async(ctx, ncreate, (size_t)Nc * 4 * kMaxSpecies)) return rc;
-      if (int rc = zero_async(ctx, st_type, (size_t)Nc * kMaxCreate)) return rc;
-      LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-      for (int rg = 0; rg < R.n_rg; ++rg) std::memcpy(&Sq.rg_inv[rg], ctx->h_pinned + rg, 8);
+      if (int rc = zero_async(ctx, ncreate, clear_bytes)) return rc;
       ProdArgs A{};
       A.tab = dtab; A.sig_Er = R.d_sig_Er; A.sig = R.d_sig; A.P = P; A.counts = ctx->d_counts;
       A.N0 = N[q];
@@ -810,7 +808,7 @@ int mcc_run(lepic_ctx* ctx, int it, int mode, uint64_t seed, int32_t* iseed, lep
       A.h1 = ctx->g.h1; A.h2 = ctx->g.h2; A.qe = ctx->g.qe; A.pi = pi; A.S = Sq;
       A.k0 = k0; A.k1 = k1; A.it = (uint32_t)it;
       A.claim = ctx->d_claim; A.st_type = st_type; A.st_ip = st_ip; A.st_v = st_v;
-      A.ncreate = ncreate; A.Nc = Nc;
+      A.ncreate = ncreate; A.Nc = Nc; A.rg_inv = d_rg;
       A.cnt_col = R.d_cnt_col; A.ploss3 = d_ploss3; A.events = d_events; A.missed = d_missed;
       A.status = d_status;
       const dim3 g((unsigned)((Nc + 255) / 256));
@@ -822,37 +820,29 @@ int mcc_run(lepic_ctx* ctx, int it, int mode, uint64_t seed, int32_t* iseed, lep
       else if (lds) hipLaunchKernelGGL((k_mcc_prod<false, true>), g, dim3(256), tab_bytes, ctx->stream, A);
       else hipLaunchKernelGGL((k_mcc_prod<false, false>), g, dim3(256), 0, ctx->stream, A);
       LEPIC_HIP(hipGetLastError());
-      for (int b = 0; b < ctx->nsp; ++b) {
-        uint32_t* cnt = ncreate + (size_t)b * Nc;
-        // keep the raw counts for the total: scan a copy
-        LEPIC_HIP(hipMemcpyAsync(offs, cnt, (size_t)Nc * 4, hipMemcpyDeviceToDevice, ctx->stream));
-        if (int rc = scan_exclusive_u32(ctx, offs, Nc)) return rc;
-        if (A.mixed) hipLaunchKernelGGL(k_mcc_append<true>, g, dim3(256), 0, ctx->stream, A, (const uint32_t*)offs, b);
-        else hipLaunchKernelGGL(k_mcc_append<false>, g, dim3(256), 0, ctx->stream, A, (const uint32_t*)offs, b);
-        hipLaunchKernelGGL(k_add_count, dim3(1), dim3(64), 0, ctx->stream, ctx->d_counts, b,
-                           (const uint32_t*)offs, (const uint32_t*)cnt, Nc, d_created);
-        LEPIC_HIP(hipGetLastError());
-      }
+      // the created particles of every species in one scan and one launch
+      if (int rc = scan_exclusive_u32(ctx, ncreate, (int64_t)ctx->nsp * Nc + 1)) return rc;
+      const dim3 ga(g.x, (unsigned)ctx->nsp);
+      if (A.mixed) hipLaunchKernelGGL(k_mcc_append<true>, ga, dim3(256), 0, ctx->stream, A, (const uint32_t*)ncreate);
+      else hipLaunchKernelGGL(k_mcc_append<false>, ga, dim3(256), 0, ctx->stream, A, (const uint32_t*)ncreate);
+      hipLaunchKernelGGL(k_add_counts, dim3(1), dim3(64), 0, ctx->stream, ctx->d_counts, (const uint32_t*)ncreate,
+                         ctx->nsp, Nc, d_created);
+      LEPIC_HIP(hipGetLastError());
     }
-    int32_t st = 0;
-    LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_status, 4, hipMemcpyDeviceToHost, ctx->stream));
-    LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-    std::memcpy(&st, ctx->h_pinned, 4);
+  }
+  // counters and, in production mode, the status back to the host
+  LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_cnt, kCounters * 8, hipMemcpyDeviceToHost, ctx->stream));
+  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
+  unsigned long long cnt[kCounters];
+  std::memcpy(cnt, ctx->h_pinned, sizeof(cnt));
+  const unsigned long long *ev = cnt, *cr = cnt + kCreated, ms = cnt[kMissed];
+  if (mode != LEPIC_MCC_CHECK) {
+    const int32_t st = (int32_t)(uint32_t)cnt[kStatus];
     if (st & 8) return ctx->fail(LEPIC_ERR_CAPACITY, "particle capacity exceeded by collisions");
     if (st & 4) return ctx->fail(LEPIC_ERR_MCC, "negative collision energy");
     if (st & 2) return ctx->fail(LEPIC_ERR_MCC, "relative energy above the cross-section table");
     if (st & 16) return ctx->fail(LEPIC_ERR_UNSUPPORTED, "more than 4 target species for one incident species");
   }
-  // counts and tallies back to the host
-  unsigned long long ev[32], cr[8], ms = 0;
-  LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_events, 32 * 8, hipMemcpyDeviceToHost, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-  std::memcpy(ev, ctx->h_pinned, 32 * 8);
-  LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned, d_created, 8 * 8, hipMemcpyDeviceToHost, ctx->stream));
-  LEPIC_HIP(hipMemcpyAsync(ctx->h_pinned + 8, d_missed, 8, hipMemcpyDeviceToHost, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-  std::memcpy(cr, ctx->h_pinned, 8 * 8);
-  std::memcpy(&ms, ctx->h_pinned + 8, 8);
   for (int q = 0; q < ctx->nsp; ++q) {
     ctx->sp[q].ub = N[q] + (int64_t)cr[q];
     if (int rc = set_packed_counts(ctx, q)) return rc;  // appended particles extend the last segments
