@@ -423,6 +423,7 @@ __global__ __launch_bounds__(256) void k_mcc_prod(ProdArgs A) {
     // one Maxwellian target per distinct target species (collisions.f90:425-437)
     int tts[4] = {0, 0, 0, 0};
     double tv[4][3], tmu[4], tvr[4], tE[4], tcm[4][3];
+    int tlo[4];                  // a target's place in the energy grid serves all its reactions
     int nts = 0;
     double nu[kMaxPcol], sum_nu = 0.0;
     for (int icol = 0; icol < S.p_ncol; ++icol) {
@@ -446,15 +447,17 @@ __global__ __launch_bounds__(256) void k_mcc_prod(ProdArgs A) {
         tcm[k][0] = (mp * vx1 + mt * a) / (mp + mt);
         tcm[k][1] = (mp * vy1 + mt * b) / (mp + mt);
         tcm[k][2] = (mp * vz1 + mt * z0) / (mp + mt);
+        int lo = 0, hi = npt - 1;  // Er[lo] < E <= Er[hi]
+        while (hi - lo > 1) {
+          int mid = (lo + hi) >> 1;
+          if (Er[mid] < tE[k]) lo = mid; else hi = mid;
+        }
+        tlo[k] = lo;
       }
       nu[icol] = 0.0;
       const double E = tE[k];
       if (E > Er[0] && E <= Er[npt - 1]) {
-        int lo = 0, hi = npt - 1;  // Er[lo] < E <= Er[hi]
-        while (hi - lo > 1) {
-          int mid = (lo + hi) >> 1;
-          if (Er[mid] < E) lo = mid; else hi = mid;
-        }
+        const int lo = tlo[k], hi = lo + 1;
         const double* row = kLds ? s_tab + (int64_t)(1 + icol) * npt : A.sig + (int64_t)(S.reac[icol] - 1) * npt;
         double sL = row[lo], sR = row[hi];
         double EkL = Er[lo], EkR = Er[hi];
