@@ -1258,27 +1258,34 @@ bool strip_iso(const Level& L) { return (float)L.aw == (float)L.an; }
 
 // One launch of nsw sweeps.  Bound by VALU issue (eleven instructions of about
 // 4.7 cycles per node and pass) behind the launch's load latency of about
-// 3 us.  Regions of 128 x 64 nodes as 16 waves x 4 rows, four waves per SIMD to
-// cover the LDS exchange (8 waves x 8 rows: 9.9, 11.9, 11.7, 11.3 us for the
-// four down visits of 1025^2 .. 129^2 against 9.2, 12.3, 10.6, 10.0); for
-// halos of at most 4 nodes 128 x 32, whose passes take half as long.  The
-// sweeps on a region in LDS that this replaces took 23.5 us for the 1025^2
-// down visit (4 sweeps) and 29.6, 20.4, 21.2 us for the 10 sweeps of the
-// others in two launches each.
+// 3 us.  Regions of 128 columns by 4 rows for each of 16 waves, four waves per
+// SIMD to cover the LDS exchange (8 waves x 8 rows: 9.9, 11.9, 11.7, 11.3 us
+// for the four down visits of 1025^2 .. 129^2 against 9.2, 12.3, 10.6, 10.0);
+// fewer waves, whose passes take less long, where the launch then still has at
+// most one block per CU (129^2: 4 sweeps 7.0 us with 16 waves, 5.1 with 8; 3 sweeps
+// 7.3, 5.4).  The sweeps on a region in LDS that this replaces took 23.5 us for
+// the 1025^2 down visit (4 sweeps) and 29.6, 20.4, 21.2 us for the 10 sweeps of
+// the others in two launches each.
+template <int NW>
+void launch_tile_of(lepic_ctx* ctx, const Level& L, const TileArgs& A, dim3 g) {
+  if (strip_iso(L)) hipLaunchKernelGGL((k_tile32<4, NW, true>), g, dim3(64 * NW), 0, ctx->stream, A);
+  else hipLaunchKernelGGL((k_tile32<4, NW, false>), g, dim3(64 * NW), 0, ctx->stream, A);
+}
+
 int launch_tile32(lepic_ctx* ctx, const Level& L, TileArgs A) {
   A.halo = 2 * A.nsw + (A.r2h ? 2 : 0);
-  const int rows = A.halo <= 4 ? 32 : 64;
-  const int tx = 128 - 2 * A.halo, ty = rows - 2 * A.halo;
-  const dim3 g((unsigned)((L.n1 - 1 + tx - 1) / tx), (unsigned)((L.n2 - 1 + ty - 1) / ty));
-  if (strip_iso(L)) {
-    if (rows == 32) hipLaunchKernelGGL((k_tile32<4, 8, true>), g, dim3(512), 0, ctx->stream, A);
-    else hipLaunchKernelGGL((k_tile32<4, 16, true>), g, dim3(1024), 0, ctx->stream, A);
-  } else {
-    if (rows == 32) hipLaunchKernelGGL((k_tile32<4, 8, false>), g, dim3(512), 0, ctx->stream, A);
-    else hipLaunchKernelGGL((k_tile32<4, 16, false>), g, dim3(1024), 0, ctx->stream, A);
+  const int tx = 128 - 2 * A.halo;
+  for (int nw = 8;; nw += 4) {
+    const int ty = 4 * nw - 2 * A.halo;
+    if (ty < 8) continue;
+    const dim3 g((unsigned)((L.n1 - 1 + tx - 1) / tx), (unsigned)((L.n2 - 1 + ty - 1) / ty));
+    if (nw < 16 && (int64_t)g.x * g.y > kVisitBlocks) continue;
+    if (nw == 8) launch_tile_of<8>(ctx, L, A, g);
+    else if (nw == 12) launch_tile_of<12>(ctx, L, A, g);
+    else launch_tile_of<16>(ctx, L, A, g);
+    LEPIC_HIP(hipGetLastError());
+    return 0;
   }
-  LEPIC_HIP(hipGetLastError());
-  return 0;
 }
 
 TileArgs tile_args(lepic_ctx* ctx, int l) {
