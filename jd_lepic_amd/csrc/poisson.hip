@@ -56,9 +56,10 @@ constexpr size_t kTailLds = 160 * 1024 - 2048;  // dynamic LDS of k_tail (static
 constexpr int kTailThreads = 1024;
 constexpr int kS = kSweepsPerLaunch;          // most sweeps of one launch (kRot - 1 state buffers ahead)
 constexpr int kDefaultTailNodes = 5000;
-constexpr int kResidBlocks = 512;             // blocks of the FP64 finest-level residual
+constexpr int kResidBlocks = 2048;            // most blocks of the FP64 finest-level residual
 // byte offset of the residual partials behind the scalars and the visit log
 constexpr size_t kPartialsOff = (64 * 8 + kVisitLog * sizeof(int) + 7) / 8 * 8;
+constexpr size_t kScalarBytes = kPartialsOff + kResidBlocks * 8;
 constexpr int kNr = 10;                       // sweep limit of sors.f90:63-64
 // Mixed form: the FP32 correction V-cycle is a preconditioner inside FP64
 // refinement to the unchanged tolerance, so its schedule is chosen, not
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(64 * kVisitMaxWaves) void k_visit64(VisitArgs A) {
   const int TX = 128 - 2 * A.halo_x, TY = nw * kVR - 2 * A.halo_y;
   const int i0 = 2 + (int)blockIdx.x * TX - A.halo_x + 2 * lane;
   const int j0 = 2 + (int)blockIdx.y * TY - A.halo_y + w * kVR;
-  const int nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
+  const int bid = blockIdx.y * gridDim.x + blockIdx.x;
   LevelCtrl* c = A.ctrl;
   const int c0 = c->cur[(A.epoch - 1) & 1];
   Strip<double, kVR, ISO> s;
@@ -497,28 +498,50 @@ __global__ __launch_bounds__(256) void k_add_corr(double* __restrict__ phi, cons
 
 // FP64 L1 residual of phi on the finest level (the reference's definition,
 // sors.f90:348-349 order); in mixed mode it also becomes the FP32 right-hand
-// side of the next correction equation.  One partial sum per block; blocks
-// walk rows j = blockIdx.x + 1 + m*gridDim.x.
-__global__ __launch_bounds__(256) void k_resid64(const double* __restrict__ u, const double* __restrict__ b,
-                                                 const int8_t* __restrict__ bc, int n1, int n2, double aw,
-                                                 double an, double ac, float* __restrict__ bf,
-                                                 double* __restrict__ partials) {
-  __shared__ double ws[4];
-  const int64_t W = n1 + 3;
-  double r = 0.0;
-  for (int j = blockIdx.x + 1; j <= n2 + 1; j += gridDim.x) {
-    for (int i = threadIdx.x + 1; i <= n1 + 1; i += blockDim.x) {
-      const int64_t c = (int64_t)j * W + i;
-      const int64_t q = (int64_t)(j - 1) * (n1 + 1) + (i - 1);
-      double rij = 0.0;
-      if (bc[c] == -1)
-        rij = b[q] - (aw * u[c - 1] + an * u[c + W] + an * u[c - W] + aw * u[c + 1] + ac * u[c]);
-      if (bf) bf[q] = (float)rij;
-      r += fabs(rij);
+// side of the next correction equation (zero on walls; the outer ones are
+// never written and stay so).  A thread takes two columns of kResidRows rows,
+// all loads before the first use: 1025^2 nodes (22 MB) 6.2 us, 10.4 with a row
+// per block and a node per thread at a time.  k_report sums the blocks'
+// partial sums: letting the block that ends last do it takes as long at 129^2
+// (each block then makes its writes visible to the others) and 16 us longer at
+// 1025^2.
+constexpr int kResidRows = 4, kResidThreads = 256;
+__global__ __launch_bounds__(kResidThreads) void k_resid64(const double* __restrict__ u, const double* __restrict__ b,
+                                                           const int8_t* __restrict__ bc, int n1, int n2, double aw,
+                                                           double an, double ac, float* __restrict__ bf,
+                                                           double* __restrict__ partials) {
+  constexpr int R = kResidRows, NT = kResidThreads;
+  __shared__ double ws[NT / 64];
+  const int W = n1 + 3, np = n1 / 2;                       // column pairs (2, 3), (4, 5) ...
+  const int64_t n = (int64_t)np * ((n2 - 1 + R - 1) / R);
+  double sum = 0.0;
+  for (int64_t q = (int64_t)blockIdx.x * NT + threadIdx.x; q < n; q += (int64_t)gridDim.x * NT) {
+    const int i0 = 2 + 2 * (int)(q % np), j0 = 2 + R * (int)(q / np);
+    D2 um[R + 2], bb[R];
+    double uw[R], ue[R];
+    B2 m[R];
+#pragma unroll
+    for (int r = 0; r < R + 2; ++r) um[r] = *(const D2*)(u + (int64_t)min(j0 + r - 1, n2 + 1) * W + i0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t c = (int64_t)min(j0 + r, n2 + 1) * W + i0;
+      uw[r] = u[c - 1];
+      ue[r] = u[c + 2];
+      m[r] = *(const B2*)(bc + c);
+      bb[r] = *(const D2*)(b + (int64_t)(min(j0 + r, n2 + 1) - 1) * (n1 + 1) + i0 - 1);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (j0 + r > n2) break;
+      double r0 = 0.0, r1 = 0.0;
+      if (m[r].x == -1) r0 = bb[r].x - (aw * uw[r] + an * um[r + 2].x + an * um[r].x + aw * um[r + 1].y + ac * um[r + 1].x);
+      if (m[r].y == -1) r1 = bb[r].y - (aw * um[r + 1].x + an * um[r + 2].y + an * um[r].y + aw * ue[r] + ac * um[r + 1].y);
+      if (bf) *(F2*)(bf + (int64_t)(j0 + r - 1) * (n1 + 1) + i0 - 1) = F2{(float)r0, (float)r1};
+      sum += fabs(r0) + fabs(r1);
     }
   }
-  r = wave_sum(r);
-  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = r;
+  sum = wave_sum(sum);
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = sum;
   __syncthreads();
   if (threadIdx.x == 0) partials[blockIdx.x] = ((ws[0] + ws[1]) + ws[2]) + ws[3];
 }
@@ -1589,16 +1612,16 @@ double alpha_of(lepic_ctx* ctx) {
   return std::fabs((double)((ctx->g.n1 + 1) * (ctx->g.n2 + 1)) * ctx->lv[1].ac) * 1.0;
 }
 
-int resid_blocks(lepic_ctx* ctx) { return std::min(ctx->g.n2 + 1, kResidBlocks); }
-
 // FP64 residual of phi, reported; fills the FP32 right-hand side when fill_f32
 int launch_resid64(lepic_ctx* ctx, bool fill_f32, const double* u = nullptr) {
   Level& L = ctx->lv[1];
-  hipLaunchKernelGGL(k_resid64, dim3(resid_blocks(ctx)), dim3(256), 0, ctx->stream, u ? u : (const double*)ctx->phi,
+  const int64_t n = (int64_t)(L.n1 / 2) * ((L.n2 - 1 + kResidRows - 1) / kResidRows);
+  const int nb = (int)std::min<int64_t>(std::max<int64_t>((n + kResidThreads - 1) / kResidThreads, 1), kResidBlocks);
+  hipLaunchKernelGGL(k_resid64, dim3(nb), dim3(kResidThreads), 0, ctx->stream, u ? u : (const double*)ctx->phi,
                      (const double*)ctx->rhs, (const int8_t*)ctx->bc, L.n1, L.n2, L.aw, L.an, L.ac,
                      fill_f32 ? L.bf : nullptr, ctx->d_partials);
   LEPIC_HIP(hipGetLastError());
-  return launch_report(ctx, resid_blocks(ctx));
+  return launch_report(ctx, nb);
 }
 
 // Waits for the report launched last.  The stream is asked now and then, so
@@ -1693,8 +1716,8 @@ int poisson_setup(lepic_ctx* ctx) {
   ctx->mg_epoch = 0;
   // one allocation: 64 doubles of scalars (the visit residuals from 32), the
   // visit log, then the FP64 residual's block partials
-  LEPIC_HIP(hipMalloc(&ctx->d_scalar, kPartialsOff + kResidBlocks * 8));
-  LEPIC_HIP(hipMemsetAsync(ctx->d_scalar, 0, kPartialsOff + kResidBlocks * 8, ctx->stream));
+  LEPIC_HIP(hipMalloc(&ctx->d_scalar, kScalarBytes));
+  LEPIC_HIP(hipMemsetAsync(ctx->d_scalar, 0, kScalarBytes, ctx->stream));
   ctx->d_partials = (double*)((char*)ctx->d_scalar + kPartialsOff);
   if (!ctx->h_report) {
     LEPIC_HIP(hipHostMalloc((void**)&ctx->h_report, sizeof(SolveReport), hipHostMallocMapped | hipHostMallocCoherent));

@@ -49,3 +49,30 @@ def test_fp64_visits_match_oracle(n1, n2, ng, aspect, tail, eps):
             assert info["vcycles"] == ref["vcycles"], turn
             assert np.array_equal(info["sweeps"], ref["sweeps"][:len(info["sweeps"])]), turn
             assert np.array_equal(got[1:-1, 1:-1], ref_phi[1:-1, 1:-1]), turn
+
+
+@pytest.mark.parametrize("precision,n1,n2,ng", [
+    (L.FP64, 5, 3, 1), (L.FP64, 7, 12, 1), (L.FP64, 130, 66, 2), (L.FP64, 2050, 6, 2), (L.MIXED, 12, 8, 3),
+    (L.MIXED, 48, 264, 4), (L.MIXED, 1600, 1400, 4)])
+def test_starting_residual(precision, n1, n2, ng):
+    """The finest level's residual where its threads' two columns and four
+    rows meet the walls, in one block and in more blocks than it has."""
+    dom = S.box_domain(n1, n2, Bmode=None)
+    bc = dom.bcnd.copy()
+    if n1 > 40:
+        bc[4:6, 9:30] = 2
+    rng = np.random.default_rng(n1)
+    phi = rng.uniform(-5.0, 5.0, bc.shape)
+    b = rng.normal(0, 1e-3, (n2 + 1, n1 + 1))
+    with L.Context(n1, n2, dom.h1, dom.h2 * 1.25, dom.dt, [L.Species(-L.QE, L.ME, 1.0, 16)], ng=ng, ngrid=2,
+                   precision=precision) as ctx:
+        ctx.set_boundary(bc, phi)
+        ctx.set_grid(L.GRID_RHS, b)
+        info = ctx.iterative_solver(eps=1e30, start=L.START_PREV)
+    aw, an = O.EPS0 / dom.h1 ** 2, O.EPS0 / (dom.h2 * 1.25) ** 2
+    u = phi[1:-1, 1:-1]
+    r = b - (aw * (phi[1:-1, :-2] + phi[1:-1, 2:]) + an * (phi[2:, 1:-1] + phi[:-2, 1:-1]) - 2.0 * (aw + an) * u)
+    ref = np.abs(r[bc[1:-1, 1:-1] == -1]).sum() / O.mg_alpha(n1, n2, (dom.h1, dom.h2 * 1.25))
+    # sums of up to 2.2e6 positive terms in two orders, and terms that cancel
+    # to 1e-2 of their parts
+    assert abs(info["res0"] - ref) <= 1e-11 * ref
