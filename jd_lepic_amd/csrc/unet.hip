@@ -690,6 +690,21 @@ __global__ void k_fill_input(const float* __restrict__ xin, const float* __restr
   }
 }
 
+// a host batch, two interleaved FP32 channels per pixel, into the input tensor
+// and channel 0 in FP32
+__global__ void k_load_input(const float2* __restrict__ xin, bf16_t* __restrict__ X, float* __restrict__ Xf, int B,
+                             int H, int W) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= (int64_t)B * H * W) return;
+  const int x = (int)(q % W), y = (int)((q / W) % H), b = (int)(q / ((int64_t)W * H));
+  const float2 v = xin[q];
+  ushort2 o;
+  o.x = f2bf(v.x);
+  o.y = f2bf(v.y);
+  *(ushort2*)(X + px(b, y, x, H, W) * 16) = o;
+  Xf[q] = v.x;
+}
+
 // one pass of the 3x3 binomial filter [1 2 1]x[1 2 1]/16 over the image,
 // zero outside the mask (walls keep no correction)
 __global__ void k_smooth(const float* __restrict__ in, const float* __restrict__ mk, int W, int H,
@@ -770,6 +785,7 @@ struct Net {
   float* dY = nullptr;
   float* Xf = nullptr;               // FP32 normalized input channel 0
   float* Rr = nullptr;               // Poisson residual of the prediction
+  float* Xin = nullptr;              // a host batch as it comes: (B, H, W, 2)
   double* d_loss = nullptr;
   // samples on the node grid image (Hs x Ws)
   int Hs = 0, Ws = 0;
@@ -826,7 +842,7 @@ int alloc_tensors(lepic_ctx* ctx, Net& N, int B, int H, int W) {
   size_t total = 0;
   for (const Spec& s : specs) total += (elems(s.lvl, s.C) * 2 + 255) & ~(size_t)255;
   const size_t hw = (size_t)B * H * W;
-  const size_t fbytes = 6 * ((hw * 4 + 63) & ~(size_t)63);
+  const size_t fbytes = 8 * ((hw * 4 + 63) & ~(size_t)63);
   LEPIC_HIP(hipMalloc(&N.arena, total + fbytes + 256));
   LEPIC_HIP(hipMemsetAsync(N.arena, 0, total + fbytes + 256, ctx->stream));
   char* p = (char*)N.arena;
@@ -837,7 +853,7 @@ int alloc_tensors(lepic_ctx* ctx, Net& N, int B, int H, int W) {
   }
   const size_t fstride = (hw * 4 + 63) & ~(size_t)63;
   N.Y = (float*)p; N.Tt = (float*)(p + fstride); N.Mk = (float*)(p + 2 * fstride); N.dY = (float*)(p + 3 * fstride);
-  N.Xf = (float*)(p + 4 * fstride); N.Rr = (float*)(p + 5 * fstride);
+  N.Xf = (float*)(p + 4 * fstride); N.Rr = (float*)(p + 5 * fstride); N.Xin = (float*)(p + 6 * fstride);
   N.B = B; N.H = H; N.W = W;
   return 0;
 }
@@ -1055,31 +1071,19 @@ size_t logical_size(const Net& N) {
 
 Net* need_net(lepic_ctx* ctx) { return ctx ? ctx->net : nullptr; }
 
-// copy host (B,H,W,2) input and optional target/mask into the batch tensors
+// copy host (B,H,W,2) input and optional target/mask into the batch tensors;
+// the caller waits for the stream before it returns
 int load_batch(lepic_ctx* ctx, Net& N, const float* x, const float* t, const float* mk, int B, int H, int W) {
   if (int rc = alloc_tensors(ctx, N, B, H, W)) return rc;
   N.B = B;
-  const size_t hw = (size_t)H * W;
-  std::vector<float> a(hw), c(hw);
-  float* dx = nullptr;
-  LEPIC_HIP(hipMalloc(&dx, 2 * hw * 4));
-  for (int b = 0; b < B; ++b) {
-    for (size_t q = 0; q < hw; ++q) { a[q] = x[((size_t)b * hw + q) * 2]; c[q] = x[((size_t)b * hw + q) * 2 + 1]; }
-    LEPIC_HIP(hipMemcpyAsync(dx, a.data(), hw * 4, hipMemcpyHostToDevice, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-    LEPIC_HIP(hipMemcpyAsync(dx + hw, c.data(), hw * 4, hipMemcpyHostToDevice, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-    hipLaunchKernelGGL(k_fill_input, dim3(nblk(hw)), dim3(256), 0, ctx->stream, (const float*)dx,
-                       (const float*)(dx + hw), 1.0f, N.X.p, b, H, W, (const float*)nullptr, 0.f, (float*)nullptr,
-                       (float*)nullptr, N.Xf);
-    LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-  }
-  LEPIC_HIP(hipFree(dx));
+  const size_t n = (size_t)B * H * W;
+  LEPIC_HIP(hipMemcpyAsync(N.Xin, x, n * 8, hipMemcpyHostToDevice, ctx->stream));
+  hipLaunchKernelGGL(k_load_input, dim3(nblk((int64_t)n)), dim3(256), 0, ctx->stream, (const float2*)N.Xin, N.X.p, N.Xf,
+                     B, H, W);
+  LEPIC_HIP(hipGetLastError());
   if (t) {
-    LEPIC_HIP(hipMemcpyAsync(N.Tt, t, (size_t)B * hw * 4, hipMemcpyHostToDevice, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-    LEPIC_HIP(hipMemcpyAsync(N.Mk, mk, (size_t)B * hw * 4, hipMemcpyHostToDevice, ctx->stream));
-  LEPIC_HIP(hipStreamSynchronize(ctx->stream));
+    LEPIC_HIP(hipMemcpyAsync(N.Tt, t, n * 4, hipMemcpyHostToDevice, ctx->stream));
+    LEPIC_HIP(hipMemcpyAsync(N.Mk, mk, n * 4, hipMemcpyHostToDevice, ctx->stream));
   }
   return 0;
 }
@@ -1463,17 +1467,25 @@ int lepic_net_loss_grad(lepic_ctx* ctx, const float* x, const float* t, const fl
   if (B < 1 || H < 8 || W < 8 || H % 8 || W % 8) return ctx->fail(LEPIC_ERR_ARG, "B >= 1, H and W multiples of 8");
   if ((size_t)n != logical_size(*N)) return ctx->fail(LEPIC_ERR_ARG, "parameter count mismatch");
   if (int rc = load_batch(ctx, *N, x, t, mk, B, H, W)) return rc;
-  double nm = 0.0;
-  for (int64_t q = 0; q < (int64_t)B * H * W; ++q) nm += mk[q];
-  if (!(nm > 0.0)) return ctx->fail(LEPIC_ERR_ARG, "empty mask");
   if (int rc = forward(ctx, *N)) return rc;
+  double nm = 0.0;                   // while the forward pass runs
+  for (int64_t q = 0; q < (int64_t)B * H * W; ++q) nm += mk[q];
+  if (!(nm > 0.0)) {
+    LEPIC_HIP(hipStreamSynchronize(ctx->stream));
+    return ctx->fail(LEPIC_ERR_ARG, "empty mask");
+  }
   if (int rc = loss_launch(ctx, *N, nm, lam, cw, cn)) return rc;
   if (int rc = backward(ctx, *N)) return rc;
   *loss = read_d(ctx, N->d_loss) / nm;
-  std::vector<float> gpu(N->nparam);
-  LEPIC_HIP(hipMemcpyAsync(gpu.data(), N->g, N->nparam * 4, hipMemcpyDeviceToHost, ctx->stream));
+  // only the first layer is laid out differently (its input channels padded)
+  const Layer& L0 = N->L[0];
+  const size_t pad = (size_t)L0.cout * 9 * L0.cin, log = (size_t)L0.cout * 9 * L0.cin_logical;
+  std::vector<float> first(pad);
+  LEPIC_HIP(hipMemcpyAsync(first.data(), N->g, pad * 4, hipMemcpyDeviceToHost, ctx->stream));
+  LEPIC_HIP(hipMemcpyAsync(grad + log, N->g + pad, (N->nparam - pad) * 4, hipMemcpyDeviceToHost, ctx->stream));
   LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-  gpu_to_logical(*N, gpu.data(), grad);
+  for (size_t r = 0; r < (size_t)L0.cout * 9; ++r)
+    for (int c = 0; c < L0.cin_logical; ++c) grad[r * L0.cin_logical + c] = first[r * L0.cin + c];
   return 0;
 }
 
