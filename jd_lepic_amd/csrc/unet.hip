@@ -29,6 +29,7 @@
 #include <cmath>
 #include <cstring>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "lepic_internal.h"
@@ -70,7 +71,11 @@ struct ConvArgs {
 };
 
 // A block computes 64 pixels of ROWS rows (a wave per 16 pixels, all rows)
-// times all cout output channels.  Input channels are taken in chunks of
+// times all cout output channels.  The bands of ROWS rows of all images lie one
+// after the other, one border pixel between them, and a block takes 64 of
+// that line: with tiles of their own the rows of 2^k / 8 + 1 and the like wasted
+// up to half of the blocks (27 convolutions of a 520 x 520 batch of 4: 845 us,
+// 770 so).  Input channels are taken in chunks of
 // CC: the chunk of the ROWS + 2 input rows around the output rows (66
 // pixels, border included) and of the weights (cout x 9 taps) are staged in
 // LDS, each thread issuing its 16-byte loads in batches of kStageBatch
@@ -79,10 +84,11 @@ struct ConvArgs {
 // A operand and the pixels its B operand, so a lane ends with 4 consecutive
 // output channels of one pixel and writes them as one 8-byte vector.  CC
 // and ROWS shrink as cout grows so the LDS stays near 64 KB and the
-// accumulators in registers; rows are padded by 4 channels against bank
+// accumulators in registers, and is 16 where that is all there is (CIN; more
+// blocks per CU); rows are padded by 4 channels against bank
 // conflicts (8-byte aligned rows: the 16-byte loads are stored as halves).
-template <int NT> struct ConvShape {
-  static constexpr int CC = NT <= 4 ? 32 : 16;
+template <int NT, int CIN> struct ConvShape {
+  static constexpr int CC = NT <= 4 && CIN != 16 ? 32 : 16;
   static constexpr int ROWS = NT <= 4 ? 4 : 2;
   static constexpr int PAD = NT <= 8 ? 4 : 0;              // 192 output channels: no room for the padding
 };
@@ -118,14 +124,24 @@ __device__ __forceinline__ void stage_lds(int n, Src src, Dst dst) {
   }
 }
 
-template <int NT>
+template <int NT, int CIN>
 __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A) {
-  constexpr int CC = ConvShape<NT>::CC, ROWS = ConvShape<NT>::ROWS, CP = CC + ConvShape<NT>::PAD;
-  constexpr int COUT = 16 * NT, kPx = 66, kRin = ROWS + 2;  // pixels x0-1 .. x0+64, rows y0-1 .. y0+ROWS
+  using Shape = ConvShape<NT, CIN>;
+  constexpr int CC = Shape::CC, ROWS = Shape::ROWS, CP = CC + Shape::PAD;
+  constexpr int COUT = 16 * NT, kPx = 66, kRin = ROWS + 2;  // 64 pixels and one beside, rows y0-1 .. y0+ROWS
   __shared__ __align__(16) bf16_t s_in[kRin * kPx * CP];
   __shared__ __align__(16) bf16_t s_w[COUT * 9 * CP];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int x0 = blockIdx.x * 64, y0 = blockIdx.y * ROWS, b = blockIdx.z;
+  // staged pixel q: place of its row y0-1 in the tensor, and the rows from
+  // there to the bottom border (0: no pixel of the image)
+  __shared__ int s_pix[kPx], s_nr[kPx];
+  if (t < kPx) {
+    const int nb = (A.H + ROWS - 1) / ROWS, v = (int)blockIdx.x * 64 - 1 + t, band = v / (A.W + 1), x = v - band * (A.W + 1);
+    const bool in = v >= 0 && x < A.W && band < nb * A.B;
+    const int y0 = in ? band % nb * ROWS : 0;
+    s_pix[t] = in ? (int)px(band / nb, y0 - 1, x, A.H, A.W) : 0;
+    s_nr[t] = in ? A.H + 2 - y0 : 0;
+  }
   const int m = lane & 15, g = lane >> 4;
   f32x4 acc[ROWS][NT];
 #pragma unroll
@@ -137,14 +153,13 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A) {
     const int lv = cc == 32 ? 2 : 1;                       // log2 of the 16-byte vectors per pixel or weight row
     const int nv = 1 << lv;
     __syncthreads();                                       // the previous chunk's reads are done
-    // input rows y0-1 .. y0+ROWS, pixels x0-1 .. x0+64 (the tensors' zero
-    // border covers -1; beyond the bottom or right border: zero)
+    // input rows y0-1 .. y0+ROWS (the tensors' zero border covers -1; beyond
+    // the bottom border, and beside the image: zero)
     stage_lds(kRin * kPx * nv,
               [&](int q) -> const bf16_t* {
                 const int v = q & (nv - 1), pq = q >> lv, xx = pq % kPx, r = pq / kPx;
-                const int gx = x0 - 1 + xx, gy = y0 - 1 + r;
-                return gx <= A.W && gy <= A.H ? A.in + px(b, gy, gx, A.H, A.W) * A.in_C + A.in_off + c + 8 * v
-                                              : nullptr;
+                return r < s_nr[xx] ? A.in + (size_t)(s_pix[xx] + r * (A.W + 2)) * A.in_C + A.in_off + c + 8 * v
+                                    : nullptr;
               },
               [&](int q) { return s_in + (q >> lv) * CP + 8 * (q & (nv - 1)); });
     stage_lds(COUT * 9 * nv,
@@ -168,14 +183,12 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A) {
       }
     }
   }
-  // lane (m, g) holds output channels 16 j + 4 g .. + 3 of pixel x0 + 16 wv + m
-  const int xp = x0 + 16 * wv + m;
-  if (xp >= A.W) return;
+  // lane (m, g) holds output channels 16 j + 4 g .. + 3 of pixel 16 wv + m
+  const int pix = s_pix[16 * wv + m + 1], nr = s_nr[16 * wv + m + 1];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    const int y = y0 + r;
-    if (y >= A.H) break;
-    const size_t p = px(b, y, xp, A.H, A.W);
+    if (r + 2 >= nr) break;
+    const size_t p = (size_t)(pix + (r + 1) * (A.W + 2));
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int co = 16 * j + 4 * g;
@@ -868,15 +881,23 @@ int conv(lepic_ctx* ctx, Net& N, const T4& in, int in_off, int cin, const bf16_t
   A.out = out.p; A.out_C = out.C; A.out_off = out_off; A.cout = cout;
   A.mask = mask ? mask->p : nullptr; A.mask_C = mask ? mask->C : 0; A.mask_off = mask_off;
   A.relu = relu; A.B = B; A.H = H; A.W = W;
-  auto grid = [&](int rows) { return dim3((unsigned)((W + 63) / 64), (unsigned)((H + rows - 1) / rows), (unsigned)B); };
+  auto go = [&](auto nt, auto ci) {
+    constexpr int NT = decltype(nt)::value, CIN = decltype(ci)::value, R = ConvShape<NT, CIN>::ROWS;
+    const int64_t n = (int64_t)B * ((H + R - 1) / R) * (W + 1);
+    hipLaunchKernelGGL((k_conv3x3<NT, CIN>), dim3((unsigned)((n + 63) / 64)), dim3(256), 0, ctx->stream, A);
+  };
+  auto any = [&](auto nt) {
+    if (cin == 16) go(nt, std::integral_constant<int, 16>{});
+    else go(nt, std::integral_constant<int, 0>{});
+  };
   switch (cout / 16) {
-    case 1: hipLaunchKernelGGL(k_conv3x3<1>, grid(ConvShape<1>::ROWS), dim3(256), 0, ctx->stream, A); break;
-    case 2: hipLaunchKernelGGL(k_conv3x3<2>, grid(ConvShape<2>::ROWS), dim3(256), 0, ctx->stream, A); break;
-    case 3: hipLaunchKernelGGL(k_conv3x3<3>, grid(ConvShape<3>::ROWS), dim3(256), 0, ctx->stream, A); break;
-    case 4: hipLaunchKernelGGL(k_conv3x3<4>, grid(ConvShape<4>::ROWS), dim3(256), 0, ctx->stream, A); break;
-    case 6: hipLaunchKernelGGL(k_conv3x3<6>, grid(ConvShape<6>::ROWS), dim3(256), 0, ctx->stream, A); break;
-    case 8: hipLaunchKernelGGL(k_conv3x3<8>, grid(ConvShape<8>::ROWS), dim3(256), 0, ctx->stream, A); break;
-    case 12: hipLaunchKernelGGL(k_conv3x3<12>, grid(ConvShape<12>::ROWS), dim3(256), 0, ctx->stream, A); break;
+    case 1: any(std::integral_constant<int, 1>{}); break;
+    case 2: any(std::integral_constant<int, 2>{}); break;
+    case 3: any(std::integral_constant<int, 3>{}); break;
+    case 4: any(std::integral_constant<int, 4>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}, std::integral_constant<int, 0>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}, std::integral_constant<int, 0>{}); break;
+    case 12: go(std::integral_constant<int, 12>{}, std::integral_constant<int, 0>{}); break;
     default: return ctx->fail(LEPIC_ERR_ARG, "unsupported channel count");
   }
   LEPIC_HIP(hipGetLastError());
