@@ -191,9 +191,9 @@ struct lepic_ctx {
   double* d_partials = nullptr;      // FP64 residual partial sums of the finest level
   double* d_scalar = nullptr;        // small scratch (res0 etc.)
   double* h_pinned = nullptr;        // pinned host scratch (kPinnedDoubles)
-  lepic::SolveReport* h_report = nullptr;   // coherent host memory that a V-cycle's last kernel writes
+  lepic::SolveReport* h_report = nullptr;   // [2] coherent host memory that the solver's kernels report to
   lepic::SolveReport* d_report = nullptr;   // its device address
-  uint64_t report_seq = 0;
+  uint64_t report_seq[2] = {0, 0};
   double* d_resid64 = nullptr;       // FP64 residual grid for mixed refinement
   float* d_corr = nullptr;
 

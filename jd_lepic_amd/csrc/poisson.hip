@@ -1565,8 +1565,10 @@ int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps) {
 
 // One FP64 V-cycle (mg.f90:85-225): levels 1..Ls-1 multi-block, Ls..ng in
 // k_tail; then the end-of-cycle kernel.
-ReportArgs report_args(lepic_ctx* ctx) {
-  return ReportArgs{ctx->d_report, ++ctx->report_seq, d_visit_of(ctx), d_vres_of(ctx)};
+// slot 0: what the host waits for next; slot 1: the starting residual, which it
+// reads when it has something to wait for
+ReportArgs report_args(lepic_ctx* ctx, int slot = 0) {
+  return ReportArgs{ctx->d_report + slot, ++ctx->report_seq[slot], d_visit_of(ctx), d_vres_of(ctx)};
 }
 
 int launch_finish64(lepic_ctx* ctx, const VisitRef& v) {
@@ -1575,9 +1577,9 @@ int launch_finish64(lepic_ctx* ctx, const VisitRef& v) {
   return 0;
 }
 
-int launch_report(lepic_ctx* ctx, int nb) {
+int launch_report(lepic_ctx* ctx, int nb, int slot = 0) {
   hipLaunchKernelGGL(k_report, dim3(1), dim3(kReportThreads), 0, ctx->stream, (const double*)ctx->d_partials, nb,
-                     report_args(ctx));
+                     report_args(ctx, slot));
   LEPIC_HIP(hipGetLastError());
   return 0;
 }
@@ -1613,7 +1615,7 @@ double alpha_of(lepic_ctx* ctx) {
 }
 
 // FP64 residual of phi, reported; fills the FP32 right-hand side when fill_f32
-int launch_resid64(lepic_ctx* ctx, bool fill_f32, const double* u = nullptr) {
+int launch_resid64(lepic_ctx* ctx, bool fill_f32, const double* u = nullptr, int slot = 0) {
   Level& L = ctx->lv[1];
   const int64_t n = (int64_t)(L.n1 / 2) * ((L.n2 - 1 + kResidRows - 1) / kResidRows);
   const int nb = (int)std::min<int64_t>(std::max<int64_t>((n + kResidThreads - 1) / kResidThreads, 1), kResidBlocks);
@@ -1621,14 +1623,14 @@ int launch_resid64(lepic_ctx* ctx, bool fill_f32, const double* u = nullptr) {
                      (const double*)ctx->rhs, (const int8_t*)ctx->bc, L.n1, L.n2, L.aw, L.an, L.ac,
                      fill_f32 ? L.bf : nullptr, ctx->d_partials);
   LEPIC_HIP(hipGetLastError());
-  return launch_report(ctx, nb);
+  return launch_report(ctx, nb, slot);
 }
 
-// Waits for the report launched last.  The stream is asked now and then, so
-// that an error on it ends the wait.
-int read_report(lepic_ctx* ctx, int* visit, double* vres) {
-  const SolveReport* h = ctx->h_report;
-  auto arrived = [&]() { return __atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) == ctx->report_seq; };
+// Waits for the slot's report launched last.  The stream is asked now and
+// then, so that an error on it ends the wait.
+int read_report(lepic_ctx* ctx, int* visit, double* vres, int slot = 0) {
+  const SolveReport* h = ctx->h_report + slot;
+  auto arrived = [&]() { return __atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) == ctx->report_seq[slot]; };
   for (uint32_t spin = 1; !arrived(); ++spin) {
     if (spin % 65536 != 0) continue;
     const hipError_t q = hipStreamQuery(ctx->stream);
@@ -1720,8 +1722,8 @@ int poisson_setup(lepic_ctx* ctx) {
   LEPIC_HIP(hipMemsetAsync(ctx->d_scalar, 0, kScalarBytes, ctx->stream));
   ctx->d_partials = (double*)((char*)ctx->d_scalar + kPartialsOff);
   if (!ctx->h_report) {
-    LEPIC_HIP(hipHostMalloc((void**)&ctx->h_report, sizeof(SolveReport), hipHostMallocMapped | hipHostMallocCoherent));
-    std::memset((void*)ctx->h_report, 0, sizeof(SolveReport));
+    LEPIC_HIP(hipHostMalloc((void**)&ctx->h_report, 2 * sizeof(SolveReport), hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset((void*)ctx->h_report, 0, 2 * sizeof(SolveReport));
     LEPIC_HIP(hipHostGetDevicePointer((void**)&ctx->d_report, ctx->h_report, 0));
   }
   return 0;
@@ -1787,9 +1789,8 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
   LEPIC_HIP(hipGetLastError());
   // residual of the starting guess; in mixed mode it also fills the FP32
   // right-hand side of the first correction equation
-  if (int rc = launch_resid64(ctx, mixed)) return rc;
-  if (int rc = read_report(ctx, visit, vres)) return rc;
-  info->res0 = ctx->h_report->resid / alpha;
+  // (the first V-cycle runs whatever it is, so nothing waits for it here)
+  if (int rc = launch_resid64(ctx, mixed, nullptr, 1)) return rc;
   int k = 1;
   info->status = 0;
   // FP64 with a multi-block finest level: the buffer that holds its state
@@ -1834,6 +1835,12 @@ int poisson_solve(lepic_ctx* ctx, double eps, int ncycl, int start, lepic_solve_
       if (int rc = launch_resid64(ctx, true)) return rc;
       if (int rc = read_report(ctx, visit, vres)) return rc;
       vres[2 * ng - 1] = ctx->h_report->resid;
+    }
+    if (k == 1) {
+      int v0[kVisitLog];
+      double r0[kVisitLog];
+      if (int rc = read_report(ctx, v0, r0, 1)) return rc;
+      info->res0 = ctx->h_report[1].resid / alpha;
     }
     const int nvis = 2 * ng - 1;
     if (ctx->lv[1].mb && !mixed) state = (state + visit[1] + (ng > 1 ? visit[nvis] : 0)) % kRot;
