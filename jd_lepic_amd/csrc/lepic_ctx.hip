@@ -749,7 +749,7 @@ int lepic_set_grid(lepic_ctx* ctx, int32_t which, int32_t ptype, const double* i
 int lepic_part_mover(lepic_ctx* ctx, int32_t ptype, int32_t deposit) {
   if (!ctx || !valid_ptype(ctx, ptype)) return LEPIC_ERR_ARG;
   if (!ctx->boundary_set) return ctx->fail(LEPIC_ERR_STATE, "lepic_set_boundary not called");
-  return mover_launch(ctx, ptype - 1, deposit);
+  return movers_launch(ctx, ptype - 1, ptype, deposit);
 }
 
 int lepic_charge_deposition(lepic_ctx* ctx, int32_t ptype) {

@@ -278,7 +278,7 @@ int zero_async(lepic_ctx* ctx, void* p, size_t bytes);
 int deposit_range_launch(lepic_ctx* ctx, int p, int64_t seg0, int64_t nseg);   // push.hip
 
 // ---- phase entry points implemented per translation unit ----
-int mover_launch(lepic_ctx* ctx, int ptype, int deposit);
+int movers_launch(lepic_ctx* ctx, int p0, int p1, int deposit);   // species p0..p1-1, from 0
 int deposit_launch(lepic_ctx* ctx, int ptype);
 int rhs_launch(lepic_ctx* ctx);
 int efield_launch(lepic_ctx* ctx);

@@ -195,7 +195,7 @@ extern "C" int lepic_step(lepic_ctx* ctx, int32_t it, lepic_step_args* a) {
   // injection: sav_np before and after each push (main.f90:1044-1056)
   const bool count_losses = a->inj && (a->inj->opt_inj == 2 || a->inj->opt_inj == -2);
   if (!rc && count_losses) rc = lost_counts_launch(ctx, 0);
-  for (int p = 1; p <= ctx->nsp && !rc; ++p) rc = lepic_part_mover(ctx, p, 1);  // :1041-1086
+  if (!rc) rc = movers_launch(ctx, 0, ctx->nsp, 1);  // :1041-1086
   if (!rc && count_losses) rc = lost_counts_launch(ctx, 1);
   if (!rc && count_losses) rc = lost_counts_add(ctx, ctx->inj_lost);
   a->injected = 0;
