@@ -334,10 +334,9 @@ int alloc_species(lepic_ctx* ctx, int p) {
   s.packed = true;
   LEPIC_HIP(hipMalloc(&s.np, ctx->nodes * 8));
   LEPIC_HIP(hipMemsetAsync(s.np, 0, ctx->nodes * 8, ctx->stream));
-  for (int b = 0; b < 2; ++b) {
-    LEPIC_HIP(hipMalloc(&s.acc[b], ctx->nodes * 8));
-    LEPIC_HIP(hipMemsetAsync(s.acc[b], 0, ctx->nodes * 8, ctx->stream));
-  }
+  LEPIC_HIP(hipMalloc(&s.acc[0], 2 * ctx->nodes * 8));   // one allocation for both
+  LEPIC_HIP(hipMemsetAsync(s.acc[0], 0, 2 * ctx->nodes * 8, ctx->stream));
+  s.acc[1] = s.acc[0] + ctx->nodes;
   LEPIC_HIP(hipMalloc(&s.np_red, ctx->nodes * 8));
   LEPIC_HIP(hipMemsetAsync(s.np_red, 0, ctx->nodes * 8, ctx->stream));
   LEPIC_HIP(hipMalloc(&s.sink, ctx->nodes * 8));
@@ -417,8 +416,8 @@ int lepic_create(const lepic_grid_desc* g, const lepic_species_desc* sp, lepic_c
   H(hipMemset(ctx->d_tally, 0, kMaxSpecies * kTallyCopies * sizeof(Tally)), "tally");
   H(hipMalloc(&ctx->d_ticket, 8), "ticket");
   H(hipMemset(ctx->d_ticket, 0, 8), "ticket");
-  H(hipMalloc(&ctx->d_scan, kScanDirect * 4), "scan");
-  H(hipMalloc(&ctx->d_error, 64), "error");
+  H(hipMalloc(&ctx->d_error, 64 + kScanDirect * 4), "error");
+  ctx->d_scan = (uint32_t*)(ctx->d_error + 16);
   H(hipMemset(ctx->d_error, 0, 64), "error");
   H(hipMalloc(&ctx->d_mcc_i64, 64 * 8), "mcc");
   H(hipMemset(ctx->d_mcc_i64, 0, 64 * 8), "mcc");
@@ -445,12 +444,12 @@ int lepic_destroy(lepic_ctx* ctx) {
   for (int p = 0; p < ctx->nsp; ++p) {
     Species& s = ctx->sp[p];
     for (int b = 0; b < 2; ++b) (void)hipFree(s.mem[b]);
-    (void)hipFree(s.flag_dead); (void)hipFree(s.np); (void)hipFree(s.acc[0]); (void)hipFree(s.acc[1]); (void)hipFree(s.np_red); (void)hipFree(s.sink); (void)hipFree(s.src);
+    (void)hipFree(s.flag_dead); (void)hipFree(s.np); (void)hipFree(s.acc[0]); (void)hipFree(s.np_red); (void)hipFree(s.sink); (void)hipFree(s.src);
     (void)hipFree(s.seg[0]); (void)hipFree(s.seg[1]);
   }
   void* ptrs[] = {ctx->bc, ctx->phi, ctx->phi_given, ctx->rhs, ctx->E, ctx->Ef, ctx->Bi, ctx->Bf,
                   ctx->d_ctrl, ctx->d_scalar, ctx->d_resid64, ctx->d_corr,
-                  ctx->d_counts, ctx->d_tally, ctx->d_segoff, ctx->d_ticket, ctx->d_scan, ctx->d_error,
+                  ctx->d_counts, ctx->d_tally, ctx->d_segoff, ctx->d_ticket, ctx->d_error,
                   ctx->s_key[0], ctx->s_key[1], ctx->s_val[0], ctx->s_val[1], ctx->s_hist,
                   ctx->d_plist, ctx->d_scan_tmp, ctx->s_meta, ctx->s_rkey, ctx->s_rcnt, ctx->s_rcntd,
                   ctx->s_nrun, ctx->rx.d_sig_Er, ctx->rx.d_sig,
