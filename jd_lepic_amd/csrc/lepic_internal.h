@@ -108,9 +108,11 @@ struct Species {
   bool dead_maybe = true;
   double* np = nullptr;              // deposited density (nodes)
   // fixed-point deposition accumulators (nodes): acc[acc_cur] holds the last
-  // deposition, scaled into np, the other one is zero for the next
+  // deposition, scaled into np, the other one is zero for the next unless a
+  // call ended in an error between the two (acc_clean false)
   int64_t* acc[2] = {nullptr, nullptr};
   int acc_cur = 0;
+  bool acc_clean = true;
   double* np_red = nullptr;
   double* sink = nullptr;            // ss2D(2): sink counts (nodes)
   double* src = nullptr;             // ss2D(1): source counts (nodes)

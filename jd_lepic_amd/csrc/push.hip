@@ -1101,6 +1101,16 @@ int np_from_acc(lepic_ctx* ctx, int p0, int p1) {
   const dim3 grid((unsigned)std::min<int64_t>((ctx->nodes + 255) / 256, 2048), (unsigned)(p1 - p0));
   hipLaunchKernelGGL(k_np_from_acc, grid, dim3(256), 0, ctx->stream, all, (const int8_t*)ctx->bc, ctx->nodes);
   LEPIC_HIP(hipGetLastError());
+  for (int p = p0; p < p1; ++p) ctx->sp[p].acc_clean = true;
+  return 0;
+}
+
+// the species' next accumulator, zero, becomes the current one
+int next_acc(lepic_ctx* ctx, Species& s) {
+  if (!s.acc_clean)
+    if (int rc = zero_async(ctx, s.acc[1 - s.acc_cur], ctx->nodes * 8)) return rc;
+  s.acc_cur = 1 - s.acc_cur;
+  s.acc_clean = false;           // until np_from_acc has cleared the other one
   return 0;
 }
 
@@ -1110,7 +1120,8 @@ namespace lepic {
 
 static int mover_launch(lepic_ctx* ctx, int p, int deposit) {
   Species& s = ctx->sp[p];
-  if (deposit) s.acc_cur = 1 - s.acc_cur;
+  if (deposit)
+    if (int rc = next_acc(ctx, s)) return rc;
   MoverCommon a = common_args(ctx, p);
   a.deposit = deposit ? 1 : 0;
   a.check_dead = s.dead_maybe ? 1 : 0;
@@ -1161,6 +1172,7 @@ static int mover_launch(lepic_ctx* ctx, int p, int deposit) {
 }
 
 int movers_launch(lepic_ctx* ctx, int p0, int p1, int deposit) {
+  LEPIC_HIP(hipGetLastError());  // an error left by an earlier call is reported before any particle moves
   for (int p = p0; p < p1; ++p)
     if (int rc = mover_launch(ctx, p, deposit)) return rc;
   return deposit ? np_from_acc(ctx, p0, p1) : 0;
@@ -1168,7 +1180,8 @@ int movers_launch(lepic_ctx* ctx, int p0, int p1, int deposit) {
 
 int deposit_launch(lepic_ctx* ctx, int p) {
   Species& s = ctx->sp[p];
-  s.acc_cur = 1 - s.acc_cur;
+  LEPIC_HIP(hipGetLastError());
+  if (int rc = next_acc(ctx, s)) return rc;
   MoverCommon a = common_args(ctx, p);
   a.deposit = 1;
   const int64_t nb = std::max<int64_t>(nseg_of(s), 1);
