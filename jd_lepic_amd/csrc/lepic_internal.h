@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -312,6 +313,30 @@ __device__ __forceinline__ int64_t node_index(int ix, int iy, int n1) {
 }
 
 __device__ __forceinline__ void atomic_add_f64(double* p, double v) { unsafeAtomicAdd(p, v); }
+
+// ---- exact division by a constant ----
+// a divisor, its reciprocal rounded and what the rounding left
+struct ExactDiv { double h, r, rl; };
+
+inline ExactDiv exact_div(double h) {
+  ExactDiv d{h, 1.0 / h, 0.0};
+  d.rl = std::fma(-d.r, h, 1.0) / h;
+  return d;
+}
+
+// x / h for finite x, correctly rounded: the quotient from the reciprocal in
+// two parts is within one unit in the last place, so the remainder is exact and
+// one correction rounds it right (Markstein's theorem, IBM J. Res. Dev. 34,
+// 1990).
+__device__ __forceinline__ double div_finite(double x, const ExactDiv& d) {
+  const double q = __builtin_fma(x, d.r, x * d.rl);
+  return __builtin_fma(__builtin_fma(-d.h, q, x), d.r, q);
+}
+
+// the same with infinities, NaN and zeros as the division gives them
+__device__ __forceinline__ double div_exact(double x, const ExactDiv& d) {
+  return __builtin_amdgcn_div_fixup(div_finite(x, d), d.h, x);
+}
 
 // ---- wave reductions in a fixed order through DPP lane moves ----
 // (VALU data-parallel primitives: row_shr:1,2,4,8 build a scan inside each

@@ -9,9 +9,11 @@
 // particles in one coarse cell are summed in registers over a thread's
 // slots, then over adjacent lanes (segmented DPP sums), go to an LDS window
 // of coarse nodes around the segment's first particle and from there to the
-// FP64 moment grid, one atomic per node and quantity of a segment; only the
-// summation order differs from the reference's serial loop.  calc_avg and
-// the phi/E averages are elementwise over nodes.
+// FP64 moment grid, one atomic per node and quantity of a segment.  A
+// particle's cell and weights are the reference's bit for bit; the order of
+// the sums differs from its serial loop, and k1 kq multiplies a run's sum
+// instead of every term.  calc_avg and the phi/E averages are elementwise over
+// nodes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,15 +34,16 @@ struct MomArgs {
   const float *fx, *fy, *fvx, *fvy, *fvz;
   const int8_t* bc;              // fine bcnd: kq = 2 where bc != -1
   int n1, size_na, na1, na2;
-  double h1, h2, ra1, ra2, xmax, ymax, half_dt, k1;   // ra = 1/(size_na h)
+  double h1, h2, xmax, ymax, half_dt, k1;
+  ExactDiv d1, d2;               // the coarse cell's sides, size_na h
   double* pm;                    // (na2+1)(na1+1) x 4: |v|^2, vx, vy, vz
 };
 
 // LDS window of coarse nodes, kMomX0 columns left and kMomY0 rows below the
 // segment's first particle: a sorted segment spans up to 1024 / (particles
 // per cell) columns of one row and drifts a few cells between sorts; runs in
-// cells outside go to the moment grid directly.  16 KB of LDS: ten blocks per
-// CU.
+// cells outside go to the moment grid directly.  16 KB of LDS would let nine
+// blocks on a CU; the registers (94) let five.
 constexpr int kMomCols = 64, kMomRows = 8, kMomX0 = 8, kMomY0 = 3;
 constexpr int kMomWin = kMomCols * kMomRows;
 
@@ -82,10 +85,13 @@ __device__ __forceinline__ void mom_stage(double acc[16], bool take) {
   }
 }
 
-// Bound by FP64 issue: about 75 operations a particle and 290 a wave of 256
+// Bound by FP64 issue: about 90 operations a particle and 290 a wave of 256
 // particles for the lane sums, against 24 B (mixed) or 40 B (FP64) read.
-// 26.2e6 particles at 100 per cell, mixed, size_na 2: 0.206 ms, 3.05 TB/s of
+// 26.2e6 particles at 100 per cell, mixed, size_na 2: 0.213 ms, 2.95 TB/s of
 // the 24 B a particle; 7.11 ms with 16 atomics on the moment grid per thread.
+// The divisions by the cell's sides round as the reference's (a product with
+// the rounded reciprocal, 0.205 ms, puts a particle on a coarse column in the
+// cell below it now and then, and its place is 1.3 times less exact).
 template <bool MIXED>
 __global__ __launch_bounds__(kBlock) void k_part_moments(MomArgs a) {
   __shared__ double win[kMomWin][4];
@@ -122,8 +128,8 @@ __global__ __launch_bounds__(kBlock) void k_part_moments(MomArgs a) {
   }
   for (int e = t; e < 4 * kMomWin; e += kBlock) (&win[0][0])[e] = 0.0;
   if (t == 0) {
-    s_w[0] = max((int)(X[0] * a.ra1) + 1 - kMomX0, 1);
-    s_w[1] = max((int)(Y[0] * a.ra2) + 1 - kMomY0, 1);
+    s_w[0] = max((int)(X[0] * a.d1.r) + 1 - kMomX0, 1);
+    s_w[1] = max((int)(Y[0] * a.d2.r) + 1 - kMomY0, 1);
   }
   __syncthreads();
   const int wx0 = s_w[0], wy0 = s_w[1];
@@ -138,9 +144,8 @@ __global__ __launch_bounds__(kBlock) void k_part_moments(MomArgs a) {
     const double vx = V[k][0], vy = V[k][1], vz = V[k][2];
     const double xp = X[k] - vx * a.half_dt, yp = Y[k] - vy * a.half_dt;
     if (k >= nv || !(xp <= a.xmax && xp >= 0.0 && yp <= a.ymax && yp >= 0.0)) continue;
-    const double sx = xp * a.ra1, sy = yp * a.ra2;
-    const int ix = (int)sx + 1, iy = (int)sy + 1;
-    const double px = (double)ix - sx, py = (double)iy - sy;
+    const int ix = (int)div_finite(xp, a.d1) + 1, iy = (int)div_finite(yp, a.d2) + 1;
+    const double px = div_finite(ix * a.d1.h - xp, a.d1), py = div_finite(iy * a.d2.h - yp, a.d2);
     const int key = iy * S + ix;
     if (key != cur) {
       if (cur >= 0) mom_flush(a, win, wx0, wy0, cur % S, cur / S, acc);
@@ -336,7 +341,7 @@ int lepic_moments_accumulate(lepic_ctx* ctx, int32_t size_na) {
     a.n1 = ctx->g.n1; a.size_na = size_na; a.na1 = na1; a.na2 = na2;
     a.h1 = ctx->g.h1; a.h2 = ctx->g.h2;
     const double ha1 = size_na * ctx->g.h1, ha2 = size_na * ctx->g.h2;
-    a.ra1 = 1.0 / ha1; a.ra2 = 1.0 / ha2;
+    a.d1 = exact_div(ha1); a.d2 = exact_div(ha2);
     a.xmax = ctx->g.n1 * ctx->g.h1; a.ymax = ctx->g.n2 * ctx->g.h2;
     a.half_dt = ctx->g.dt / 2.0;
     a.k1 = s.Nm / (ha1 * ha2 * ctx->g.zmax);

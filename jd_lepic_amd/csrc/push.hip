@@ -86,9 +86,6 @@ constexpr float kFixMx = 1048576.0f;         // 2^20
 constexpr int kMoverThreadsMixed = kBlock;
 constexpr int kMoverThreads64 = kBlock;
 
-// a divisor, its reciprocal rounded and what the rounding left (div_exact)
-struct ExactDiv { double h, r, rl; };
-
 struct MoverCommon {
   const int8_t* bc;
   const int8_t* cellwall;       // 1 where all four corners of cell (ix,iy) are walls
@@ -506,16 +503,6 @@ __device__ __forceinline__ void deposit_global_runs(const MoverCommon& a, const 
 // ---------------------------------------------------------------------------
 // FP64 mover
 // ---------------------------------------------------------------------------
-// x / h for the cell sizes, correctly rounded: the quotient from the
-// reciprocal in two parts is within one unit in the last place, so the
-// remainder is exact and one correction rounds it right (Markstein's theorem,
-// IBM J. Res. Dev. 34, 1990); the fix-up gives infinities, NaN and zeros as
-// the division does.
-__device__ __forceinline__ double div_exact(double x, const ExactDiv& d) {
-  const double q = __builtin_fma(x, d.r, x * d.rl);
-  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.h, q, x), d.r, q), d.h, x);
-}
-
 // Bound by memory (96 B a particle) as far as the latencies overlap: a
 // thread's particles are all loaded at once, then the field tile (as the mixed
 // mover's; global memory for particles outside it), and everything up to the
@@ -1054,12 +1041,6 @@ __global__ __launch_bounds__(256) void k_np_from_acc(NpAll all, const int8_t* __
     A.np[i] = kq * ((double)(long long)A.acc[i] * A.scale);
     A.next[i] = 0ull;
   }
-}
-
-ExactDiv exact_div(double h) {
-  ExactDiv d{h, 1.0 / h, 0.0};
-  d.rl = std::fma(-d.r, h, 1.0) / h;
-  return d;
 }
 
 MoverCommon common_args(lepic_ctx* ctx, int p) {
