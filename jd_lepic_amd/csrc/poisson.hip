@@ -669,10 +669,19 @@ __device__ void t_smooth(PU u, PB b, PC bc, int n1, int n2, T aw, T an, T ac, T 
   *res_out = res;
 }
 
+// Interior node of participant m in a colour's pass (t_smooth_fused).
+__device__ __forceinline__ int colour_node(int m, bool red, int n1p) {
+  const int q = 2 * m + (red ? 1 : 0);
+  return (n1p & 1) ? q : q ^ ((q / n1p) & 1);
+}
+
 // Red-black sweeps of one tail level with the residual folded into the
-// sweeps.  Interior node q = (j-1)(n1+1) + (i-1) is red (i+j odd) exactly
-// when q is odd (n1+1 is odd), so a participant handles red nodes 2m+1 and
+// sweeps.  Where n1+1 is odd, interior node q = (j-1)(n1+1) + (i-1) is red
+// (i+j odd) exactly when q is odd, so a participant handles red nodes 2m+1 and
 // black nodes 2m for m = tid + P*r, r < R, with the indices computed once.
+// Where n1+1 is even (a coarsest level of an odd number of cells along x) the
+// nodes of a pair 2m, 2m+1 lie in one row and have the two colours, the other
+// way round in every second row (colour_node).
 // The residual after sweep k is the black nodes' residual, taken right after
 // their update (their red neighbours are final), plus the red nodes'
 // residual, taken in the red pass of sweep k+1 from the same loads as that
@@ -691,13 +700,13 @@ __device__ __forceinline__ void t_smooth_fused(PU u, PB b, PC bc, int n1, int n2
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int m = tid + P * r;
-    int q = 2 * m + 1;
+    int q = colour_node(m, true, n1p);
     bool ok = q < nint;
     q = ok ? q : 0;
     int x = (q / n1p + 1) * W + q % n1p + 1;
     int8_t mq = bc[x];
     xr[r] = x; qr[r] = q; ur[r] = ok && mq <= 0; rr[r] = ok && mq == -1;
-    q = 2 * m;
+    q = colour_node(m, false, n1p);
     ok = q < nint;
     q = ok ? q : 0;
     x = (q / n1p + 1) * W + q % n1p + 1;
