@@ -396,93 +396,102 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
 // ---------------------------------------------------------------------------
 // pooling, upsampling, skip gradients
 // ---------------------------------------------------------------------------
+// The four kernels below take 8 channels (16 B) of one pixel per thread, of each
+// of the batch's rows (b * H + y) gridDim.y apart: one row a block unless the
+// batch has more of them than a grid may have blocks along y.
+
 // out (Ho=H/2, Wo=W/2, C) = average of 2x2 input pixels (channels in_off..)
 __global__ void k_pool(const bf16_t* __restrict__ in, int in_C, int in_off, bf16_t* __restrict__ out, int C,
                        int B, int Ho, int Wo) {
-  // a thread averages 8 channels of one output pixel; block row blockIdx.y = b * Ho + y
   const int nv = C / 8;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= Wo * nv) return;
   const int x = q / nv, v = q - x * nv;
-  const int y = (int)blockIdx.y % Ho, b = (int)blockIdx.y / Ho;
   const int H = 2 * Ho, W = 2 * Wo;
-  bf16_t p00[8], p01[8], p10[8], p11[8], o[8];
-  *(int4*)p00 = *(const int4*)(in + px(b, 2 * y, 2 * x, H, W) * in_C + in_off + 8 * v);
-  *(int4*)p01 = *(const int4*)(in + px(b, 2 * y, 2 * x + 1, H, W) * in_C + in_off + 8 * v);
-  *(int4*)p10 = *(const int4*)(in + px(b, 2 * y + 1, 2 * x, H, W) * in_C + in_off + 8 * v);
-  *(int4*)p11 = *(const int4*)(in + px(b, 2 * y + 1, 2 * x + 1, H, W) * in_C + in_off + 8 * v);
+  for (int row = blockIdx.y; row < B * Ho; row += gridDim.y) {
+    const int y = row % Ho, b = row / Ho;
+    bf16_t p00[8], p01[8], p10[8], p11[8], o[8];
+    *(int4*)p00 = *(const int4*)(in + px(b, 2 * y, 2 * x, H, W) * in_C + in_off + 8 * v);
+    *(int4*)p01 = *(const int4*)(in + px(b, 2 * y, 2 * x + 1, H, W) * in_C + in_off + 8 * v);
+    *(int4*)p10 = *(const int4*)(in + px(b, 2 * y + 1, 2 * x, H, W) * in_C + in_off + 8 * v);
+    *(int4*)p11 = *(const int4*)(in + px(b, 2 * y + 1, 2 * x + 1, H, W) * in_C + in_off + 8 * v);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const float s = (bf2f(p00[k]) + bf2f(p01[k])) + (bf2f(p10[k]) + bf2f(p11[k]));
-    o[k] = f2bf(0.25f * s);
+    for (int k = 0; k < 8; ++k) {
+      const float s = (bf2f(p00[k]) + bf2f(p01[k])) + (bf2f(p10[k]) + bf2f(p11[k]));
+      o[k] = f2bf(0.25f * s);
+    }
+    *(int4*)(out + px(b, y, x, Ho, Wo) * C + 8 * v) = *(const int4*)o;
   }
-  *(int4*)(out + px(b, y, x, Ho, Wo) * C + 8 * v) = *(const int4*)o;
 }
 
 // nearest upsampling of in (H/2, W/2, C) into channels [0, C) of out (H, W,
-// out_C): a thread moves 8 channels (16 B) of one pixel; block row
-// blockIdx.y = b * H + y
+// out_C)
 __global__ void k_up(const bf16_t* __restrict__ in, int C, bf16_t* __restrict__ out, int out_C, int B, int H,
                      int W) {
   const int nv = C / 8;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= W * nv) return;
   const int x = q / nv, v = q - x * nv;
-  const int y = (int)blockIdx.y % H, b = (int)blockIdx.y / H;
-  *(int4*)(out + px(b, y, x, H, W) * out_C + 8 * v) = *(const int4*)(in + px(b, y / 2, x / 2, H / 2, W / 2) * C + 8 * v);
+  for (int row = blockIdx.y; row < B * H; row += gridDim.y) {
+    const int y = row % H, b = row / H;
+    *(int4*)(out + px(b, y, x, H, W) * out_C + 8 * v) = *(const int4*)(in + px(b, y / 2, x / 2, H / 2, W / 2) * C + 8 * v);
+  }
 }
 
 // gradient of the upsampling: sum of the 4 fine gradients (channels [0, C)
-// of g (H, W, g_C)), masked by the ReLU of the coarse activation act; a thread
-// takes 8 channels (16 B) of one coarse pixel, block row blockIdx.y = b * Ho +
-// y (one channel per thread took 42 us at 260 x 260 x 32 x 4, 30 so)
+// of g (H, W, g_C)), masked by the ReLU of the coarse activation act (one channel
+// per thread took 42 us at 260 x 260 x 32 x 4, 30 so)
 __global__ void k_up_bwd(const bf16_t* __restrict__ g, int g_C, const bf16_t* __restrict__ act,
                          bf16_t* __restrict__ out, int C, int B, int Ho, int Wo) {
   const int nv = C / 8;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= Wo * nv) return;
   const int x = q / nv, v = q - x * nv;
-  const int y = (int)blockIdx.y % Ho, b = (int)blockIdx.y / Ho;
   const int H = 2 * Ho, W = 2 * Wo;
-  const size_t p = px(b, y, x, Ho, Wo) * C + 8 * v;
-  bf16_t g00[8], g01[8], g10[8], g11[8], a[8], o[8];
-  *(int4*)g00 = *(const int4*)(g + px(b, 2 * y, 2 * x, H, W) * g_C + 8 * v);
-  *(int4*)g01 = *(const int4*)(g + px(b, 2 * y, 2 * x + 1, H, W) * g_C + 8 * v);
-  *(int4*)g10 = *(const int4*)(g + px(b, 2 * y + 1, 2 * x, H, W) * g_C + 8 * v);
-  *(int4*)g11 = *(const int4*)(g + px(b, 2 * y + 1, 2 * x + 1, H, W) * g_C + 8 * v);
-  *(int4*)a = *(const int4*)(act + p);
+  for (int row = blockIdx.y; row < B * Ho; row += gridDim.y) {
+    const int y = row % Ho, b = row / Ho;
+    const size_t p = px(b, y, x, Ho, Wo) * C + 8 * v;
+    bf16_t g00[8], g01[8], g10[8], g11[8], a[8], o[8];
+    *(int4*)g00 = *(const int4*)(g + px(b, 2 * y, 2 * x, H, W) * g_C + 8 * v);
+    *(int4*)g01 = *(const int4*)(g + px(b, 2 * y, 2 * x + 1, H, W) * g_C + 8 * v);
+    *(int4*)g10 = *(const int4*)(g + px(b, 2 * y + 1, 2 * x, H, W) * g_C + 8 * v);
+    *(int4*)g11 = *(const int4*)(g + px(b, 2 * y + 1, 2 * x + 1, H, W) * g_C + 8 * v);
+    *(int4*)a = *(const int4*)(act + p);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const float s = (bf2f(g00[k]) + bf2f(g01[k])) + (bf2f(g10[k]) + bf2f(g11[k]));
-    o[k] = bf_pos(a[k]) ? f2bf(s) : (bf16_t)0;
+    for (int k = 0; k < 8; ++k) {
+      const float s = (bf2f(g00[k]) + bf2f(g01[k])) + (bf2f(g10[k]) + bf2f(g11[k]));
+      o[k] = bf_pos(a[k]) ? f2bf(s) : (bf16_t)0;
+    }
+    *(int4*)(out + p) = *(const int4*)o;
   }
-  *(int4*)(out + p) = *(const int4*)o;
 }
 
 // skip gradient: the concat buffer's slice of g plus pool_bwd(gp), masked by the
-// ReLU of the skip activation (same slice of the activations); threads as in
-// k_up_bwd.  Bound by the lines that the slices touch (520 x 520 x 16 x 4, 32 of
-// each 96 bytes: 81 us, 51 by vectors).  The result is packed: 47 us, and the
-// weight and input gradients that read it next take 32 and 26 us, 36 and 34
-// when it stayed in the concat buffer.
+// ReLU of the skip activation (same slice of the activations).  Bound by the
+// lines that the slices touch (520 x 520 x 16 x 4, 32 of each 96 bytes: 81 us, 51
+// by vectors).  The result is packed: 47 us, and the weight and input gradients
+// that read it next take 32 and 26 us, 36 and 34 when it stayed in the concat
+// buffer.
 __global__ void k_skip_grad(const bf16_t* __restrict__ g, const bf16_t* __restrict__ act, int cat_C, int off,
                             const bf16_t* __restrict__ gp, bf16_t* __restrict__ out, int C, int B, int H, int W) {
   const int nv = C / 8;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= W * nv) return;
   const int x = q / nv, v = q - x * nv;
-  const int y = (int)blockIdx.y % H, b = (int)blockIdx.y / H;
-  const size_t i = px(b, y, x, H, W), p = i * cat_C + off + 8 * v;
-  bf16_t gv[8], a[8], gc[8];
-  *(int4*)gv = *(const int4*)(g + p);
-  *(int4*)a = *(const int4*)(act + p);
-  *(int4*)gc = *(const int4*)(gp + px(b, y / 2, x / 2, H / 2, W / 2) * C + 8 * v);
+  for (int row = blockIdx.y; row < B * H; row += gridDim.y) {
+    const int y = row % H, b = row / H;
+    const size_t i = px(b, y, x, H, W), p = i * cat_C + off + 8 * v;
+    bf16_t gv[8], a[8], gc[8];
+    *(int4*)gv = *(const int4*)(g + p);
+    *(int4*)a = *(const int4*)(act + p);
+    *(int4*)gc = *(const int4*)(gp + px(b, y / 2, x / 2, H / 2, W / 2) * C + 8 * v);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const float s = bf2f(gv[k]) + 0.25f * bf2f(gc[k]);
-    gv[k] = bf_pos(a[k]) ? f2bf(s) : (bf16_t)0;
+    for (int k = 0; k < 8; ++k) {
+      const float s = bf2f(gv[k]) + 0.25f * bf2f(gc[k]);
+      gv[k] = bf_pos(a[k]) ? f2bf(s) : (bf16_t)0;
+    }
+    *(int4*)(out + i * C + 8 * v) = *(const int4*)gv;
   }
-  *(int4*)(out + i * C + 8 * v) = *(const int4*)gv;
 }
 
 // ---------------------------------------------------------------------------
@@ -876,6 +885,9 @@ int alloc_tensors(lepic_ctx* ctx, Net& N, int B, int H, int W) {
 
 unsigned nblk(int64_t n, int t = 256) { return (unsigned)((n + t - 1) / t); }
 
+// blocks over n items of a row and the rows of a batch, as many as a grid may have along y
+dim3 row_grid(int64_t n, int rows) { return dim3(nblk(n), (unsigned)std::min(rows, 65535)); }
+
 int conv(lepic_ctx* ctx, Net& N, const T4& in, int in_off, int cin, const bf16_t* w, const T4& out, int out_off,
          int cout, int relu, const T4* mask, int mask_off, int B, int H, int W) {
   ConvArgs A;
@@ -951,7 +963,7 @@ int wgrad_layer(lepic_ctx* ctx, Net& N, int l, const T4& x, int x_off, const T4&
 
 int pool(lepic_ctx* ctx, Net& N, const T4& in, int in_off, const T4& out, int C, int lvl_out) {
   const int Ho = N.H >> lvl_out, Wo = N.W >> lvl_out;
-  hipLaunchKernelGGL(k_pool, dim3(nblk((int64_t)Wo * (C / 8)), (unsigned)(N.B * Ho)), dim3(256), 0, ctx->stream, in.p,
+  hipLaunchKernelGGL(k_pool, row_grid((int64_t)Wo * (C / 8), N.B * Ho), dim3(256), 0, ctx->stream, in.p,
                      in.C, in_off, out.p, C, N.B, Ho, Wo);
   LEPIC_HIP(hipGetLastError());
   return 0;
@@ -959,7 +971,7 @@ int pool(lepic_ctx* ctx, Net& N, const T4& in, int in_off, const T4& out, int C,
 
 int upsample(lepic_ctx* ctx, Net& N, const T4& in, int C, const T4& out, int lvl_out) {
   const int H = N.H >> lvl_out, W = N.W >> lvl_out;
-  hipLaunchKernelGGL(k_up, dim3(nblk((int64_t)W * (C / 8)), (unsigned)(N.B * H)), dim3(256), 0, ctx->stream, in.p, C,
+  hipLaunchKernelGGL(k_up, row_grid((int64_t)W * (C / 8), N.B * H), dim3(256), 0, ctx->stream, in.p, C,
                      out.p, out.C, N.B, H, W);
   LEPIC_HIP(hipGetLastError());
   return 0;
@@ -1000,7 +1012,7 @@ int forward(lepic_ctx* ctx, Net& N) {
 
 int up_bwd(lepic_ctx* ctx, Net& N, const T4& g, const T4& act, const T4& out, int C, int lvl_out) {
   const int Ho = N.H >> lvl_out, Wo = N.W >> lvl_out;
-  hipLaunchKernelGGL(k_up_bwd, dim3(nblk((int64_t)Wo * (C / 8)), (unsigned)(N.B * Ho)), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(k_up_bwd, row_grid((int64_t)Wo * (C / 8), N.B * Ho), dim3(256), 0, ctx->stream,
                      g.p, g.C, act.p, out.p, C, N.B, Ho, Wo);
   LEPIC_HIP(hipGetLastError());
   return 0;
@@ -1009,7 +1021,7 @@ int up_bwd(lepic_ctx* ctx, Net& N, const T4& g, const T4& act, const T4& out, in
 int skip_grad(lepic_ctx* ctx, Net& N, const T4& gcat, const T4& acat, int off, const T4& gp, const T4& out, int lvl) {
   const int C = out.C;
   const int H = N.H >> lvl, W = N.W >> lvl;
-  hipLaunchKernelGGL(k_skip_grad, dim3(nblk((int64_t)W * (C / 8)), (unsigned)(N.B * H)), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(k_skip_grad, row_grid((int64_t)W * (C / 8), N.B * H), dim3(256), 0, ctx->stream,
                      gcat.p, acat.p, gcat.C, off, gp.p, out.p, C, N.B, H, W);
   LEPIC_HIP(hipGetLastError());
   return 0;
