@@ -1124,8 +1124,16 @@ __attribute__((noinline, aligned(64))) void he_normal(Net& N, float* flat) {
 
 Net* need_net(lepic_ctx* ctx) { return ctx ? ctx->net : nullptr; }
 
+// Waits for the stream when a call ends, whatever its outcome: copies from and to
+// the caller's arrays are under way until then (from pinned memory nothing else
+// waits for them).
+struct StreamEnd {
+  hipStream_t stream;
+  ~StreamEnd() { (void)hipStreamSynchronize(stream); }
+};
+
 // copy host (B,H,W,2) input and optional target/mask into the batch tensors;
-// the caller waits for the stream before it returns
+// the caller holds a StreamEnd
 int load_batch(lepic_ctx* ctx, Net& N, const float* x, const float* t, const float* mk, int B, int H, int W) {
   if (int rc = alloc_tensors(ctx, N, B, H, W)) return rc;
   N.B = B;
@@ -1496,6 +1504,7 @@ int lepic_net_forward(lepic_ctx* ctx, const float* x, int32_t B, int32_t H, int3
   Net* N = need_net(ctx);
   if (!N || !x || !y) return ctx ? ctx->fail(LEPIC_ERR_STATE, "no network") : LEPIC_ERR_ARG;
   if (B < 1 || H < 8 || W < 8 || H % 8 || W % 8) return ctx->fail(LEPIC_ERR_ARG, "B >= 1, H and W multiples of 8");
+  const StreamEnd end{ctx->stream};
   if (int rc = load_batch(ctx, *N, x, nullptr, nullptr, B, H, W)) return rc;
   if (int rc = forward(ctx, *N)) return rc;
   LEPIC_HIP(hipStreamSynchronize(ctx->stream));
@@ -1511,14 +1520,12 @@ int lepic_net_loss_grad(lepic_ctx* ctx, const float* x, const float* t, const fl
   if (!N || !x || !t || !mk || !loss || !grad) return ctx ? ctx->fail(LEPIC_ERR_STATE, "no network") : LEPIC_ERR_ARG;
   if (B < 1 || H < 8 || W < 8 || H % 8 || W % 8) return ctx->fail(LEPIC_ERR_ARG, "B >= 1, H and W multiples of 8");
   if ((size_t)n != logical_size(*N)) return ctx->fail(LEPIC_ERR_ARG, "parameter count mismatch");
+  const StreamEnd end{ctx->stream};
   if (int rc = load_batch(ctx, *N, x, t, mk, B, H, W)) return rc;
   if (int rc = forward(ctx, *N)) return rc;
   double nm = 0.0;                   // while the forward pass runs
   for (int64_t q = 0; q < (int64_t)B * H * W; ++q) nm += mk[q];
-  if (!(nm > 0.0)) {
-    LEPIC_HIP(hipStreamSynchronize(ctx->stream));
-    return ctx->fail(LEPIC_ERR_ARG, "empty mask");
-  }
+  if (!(nm > 0.0)) return ctx->fail(LEPIC_ERR_ARG, "empty mask");
   if (int rc = loss_launch(ctx, *N, nm, lam, cw, cn)) return rc;
   if (int rc = backward(ctx, *N)) return rc;
   *loss = read_d(ctx, N->d_loss) / nm;
