@@ -43,7 +43,11 @@ namespace {
 // Keys per thread of the run sort's blocks: the most that still give every CU
 // a block, but no fewer keys per block than it has counters (the fewest only
 // for 256 buckets).  A pass over the runs of 400 k particles: 73 us at 64 keys
-// (three blocks), 10 at 4; of 105 M ions 100 us at 64, 46 at 16.
+// (three blocks), 10 at 4; of 105 M ions 100 us at 64, 46 at 16.  The histogram
+// has a word for every eighth slot (the static scratch's as well), so 4 keys
+// with 256 buckets and 16 with 1024 need two slots for each run, 16 with 2048
+// four: with more runs, which particles in no order have, the form with more
+// keys takes the pass.
 constexpr int kSortItems = 64, kSortItemsMid = 16, kSortItemsMin = 4;
 constexpr int kTile = 256 * kSortItems;
 constexpr int kSortBlocks = 256;
@@ -507,9 +511,9 @@ constexpr int kXcds = 8, kStripeMin = 4;
 // sorted in LDS first, neighbouring lanes write the same run.  A thread has
 // kSegRounds slots (t + r kSegThreads, so every access of a round is
 // coalesced) whose loads are all issued before any store.  All arrays pass
-// through LDS at once, which also keeps few enough blocks on a CU (4 mixed, 3
-// FP64) that the lines in the making fit the L2 (see kXcds; with 6 to 8 blocks
-// 1.45 to 1.65 ms).  105 M electrons on 1024 x 1024 cells 2.35 to 1.26 ms, ions
+// through LDS at once, which also keeps few enough blocks on a CU (5 mixed, 3
+// FP64) that the lines in the making fit the L2 (see kXcds; an array at a time
+// with 8 blocks 1.65 ms, with 4 and 3 1.24 and 1.26, with 2 1.45).  105 M electrons on 1024 x 1024 cells 2.35 to 1.26 ms, ions
 // 1.07 to 1.00 (5.0 TB/s); 26 M in FP64 on 512 x 512 0.83 to 0.62.
 template <bool kMixed>
 __global__ __launch_bounds__(kSegThreads) void k_seg_scatter(SegScatterArgs A) {
@@ -574,9 +578,10 @@ int grow(lepic_ctx* ctx, T** p, int64_t n) {
 }
 
 // Device buffers of one sort: keys and values of the run sort (two of each),
-// the per-slot (run, rank), the per-segment runs (key, count) at a stride
-// of kChunk, the dense run counts, the run bases, the digit histograms, the
-// cell-end list and the scans' block partials (null: allocated by the scan).
+// the per-slot (run, place), the per-segment runs (key, first place and count)
+// at a stride of kChunk, the dense ones, the run bases, the digit histograms and
+// how many words they have, the cell-end list and the scans' block partials
+// (null: the context's words or an allocation of the scan's).
 struct SortWork {
   uint32_t* key[2];
   uint32_t* val[2];
