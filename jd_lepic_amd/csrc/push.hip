@@ -115,9 +115,9 @@ struct Soa64W { double *x, *y, *z, *vx, *vy, *vz; };
 struct SoaMx { const int32_t* cell; const float *fx, *fy, *z, *vx, *vy, *vz; };
 struct SoaMxW { int32_t* cell; float *fx, *fy, *z, *vx, *vy, *vz; };
 
-// An element of an LDS tile or, where the tile does not hold it, of global
-// memory: the explicit address space keeps the two loads apart, which the
-// compiler would otherwise merge into one flat access.
+// An element of an LDS tile: the explicit address space keeps its load apart
+// from the one of global memory in the other branch, with which the compiler
+// would otherwise merge it into one flat access.
 template <typename T> using lds_p = __attribute__((address_space(3))) const T*;
 template <typename T>
 __device__ __forceinline__ T lds_get(const T* p) {
@@ -716,8 +716,11 @@ struct MixedParams {
 
 // Bound by memory: 105 M particles at 48 B on 1024 x 1024 cells take 0.99 ms
 // (5.1 TB/s) with at most 80 VGPRs (6 waves per SIMD), 1.01 ms with 5 waves; 1.09
-// while tile and global gathers were merged into flat loads.
-template <int BT, int OCC, bool WRAP>
+// with tile and global gathers merged into flat loads (FLAT: plain pointers, which
+// the compiler merges), which pass the tile's data through the memory pipe but
+// leave a thread's four particles in one block of code, their loads overlapping,
+// where segments run beyond the tile.
+template <int BT, int OCC, bool WRAP, bool FLAT>
 __global__ __launch_bounds__(BT, OCC) void k_mover_mixed(MoverCommon a, MixedParams m, SoaMx in,
                                                         SoaMxW out, int8_t* flag_dead,
                                                         const float* __restrict__ E,
@@ -812,7 +815,9 @@ __global__ __launch_bounds__(BT, OCC) void k_mover_mixed(MoverCommon a, MixedPar
     const bool in_tile = (unsigned)tx < (unsigned)(kTileCols - 1) && (unsigned)ty < (unsigned)(kTileRows - 1);
     const int q = ty * kTileCols + tx;
     float2 e00, e10, e11, e01;
-    if (in_tile) {
+    if (FLAT && in_tile) {
+      e00 = sE[q]; e10 = sE[q + 1]; e11 = sE[q + kTileCols + 1]; e01 = sE[q + kTileCols];
+    } else if (in_tile) {
       e00 = lds_get(sE + q); e10 = lds_get(sE + q + 1);
       e11 = lds_get(sE + q + kTileCols + 1); e01 = lds_get(sE + q + kTileCols);
     } else {
@@ -829,8 +834,13 @@ __global__ __launch_bounds__(BT, OCC) void k_mover_mixed(MoverCommon a, MixedPar
         Bx = (float)a.Bc0; By = (float)a.Bc1; Bz = (float)a.Bc2;
         boris = true;
       } else if (tileB && in_tile) {
-        const float4 B00 = lds_get(sB + q), B10 = lds_get(sB + q + 1);
-        const float4 B11 = lds_get(sB + q + kTileCols + 1), B01 = lds_get(sB + q + kTileCols);
+        float4 B00, B10, B11, B01;
+        if (FLAT) {
+          B00 = sB[q]; B10 = sB[q + 1]; B11 = sB[q + kTileCols + 1]; B01 = sB[q + kTileCols];
+        } else {
+          B00 = lds_get(sB + q); B10 = lds_get(sB + q + 1);
+          B11 = lds_get(sB + q + kTileCols + 1); B01 = lds_get(sB + q + kTileCols);
+        }
         if (B00.w > 1.0e-5f) {
           Bx = fmaf(w3, B01.x, fmaf(w2, B11.x, fmaf(w1, B10.x, w0 * B00.x)));
           By = fmaf(w3, B01.y, fmaf(w2, B11.y, fmaf(w1, B10.y, w0 * B00.y)));
@@ -895,7 +905,7 @@ __global__ __launch_bounds__(BT, OCC) void k_mover_mixed(MoverCommon a, MixedPar
     const int wx = cx - fx0, wy = cy - fy0;
     const bool w_tile = (unsigned)wx < (unsigned)kTileCols && (unsigned)wy < (unsigned)kTileRows;
     int8_t wall;
-    if (w_tile) wall = *(lds_p<int8_t>)(sW + wy * kTileCols + wx);
+    if (w_tile) wall = FLAT ? sW[wy * kTileCols + wx] : *(lds_p<int8_t>)(sW + wy * kTileCols + wx);
     else wall = a.cellwall[node_index(cx, cy, n1)];
     const bool lost = live && wall != 0;
     lostm |= lost ? 1u << k : 0u;
@@ -1126,14 +1136,19 @@ static int mover_launch(lepic_ctx* ctx, int p, int deposit) {
     // and the second window, for which the other has no registers (105 M
     // particles: 1.00 ms with it, 0.96 without; there hardly a segment in a
     // hundred runs over the end of a row).
+    // The others read tile and memory through flat loads where a segment spans
+    // more cells than the tile has columns from its first one on (1024 x 1024
+    // cells, ions at 8 and 16 per cell and electrons at 24: 138, 234 and 324 us,
+    // 150, 258 and 343 through separate loads; electrons at 64 735 and 690, at 40
+    // they meet).
     const float* B = (const float*)(ctx->Bf ? ctx->Bf : (float*)ctx->Ef);
     const dim3 g((unsigned)nb), bt(kMoverThreadsMixed);
-    if (nb <= 512)
-      hipLaunchKernelGGL((k_mover_mixed<kMoverThreadsMixed, 2, true>), g, bt, 0, ctx->stream, a, m, in, out, s.flag_dead,
-                         (const float*)ctx->Ef, B);
-    else
-      hipLaunchKernelGGL((k_mover_mixed<kMoverThreadsMixed, 6, false>), g, bt, 0, ctx->stream, a, m, in, out, s.flag_dead,
-                         (const float*)ctx->Ef, B);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, g, bt, 0, ctx->stream, a, m, in, out, s.flag_dead, (const float*)ctx->Ef, B);
+    };
+    if (nb <= 512) go(k_mover_mixed<kMoverThreadsMixed, 2, true, false>);
+    else if ((int64_t)a.n1 * a.n2 > nb * (kTileCols - 1 - kTileX0)) go(k_mover_mixed<kMoverThreadsMixed, 6, false, true>);
+    else go(k_mover_mixed<kMoverThreadsMixed, 6, false, false>);
   } else {
     Soa64 in{s.d[b][0], s.d[b][1], s.d[b][2], s.d[b][3], s.d[b][4], s.d[b][5]};
     Soa64W out{s.d[o][0], s.d[o][1], s.d[o][2], s.d[o][3], s.d[o][4], s.d[o][5]};
