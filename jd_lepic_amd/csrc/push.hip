@@ -1152,9 +1152,16 @@ static int mover_launch(lepic_ctx* ctx, int p, int deposit) {
   } else {
     Soa64 in{s.d[b][0], s.d[b][1], s.d[b][2], s.d[b][3], s.d[b][4], s.d[b][5]};
     Soa64W out{s.d[o][0], s.d[o][1], s.d[o][2], s.d[o][3], s.d[o][4], s.d[o][5]};
-    hipLaunchKernelGGL(k_mover64<kMoverThreads64>, dim3((unsigned)nb), dim3(kMoverThreads64), 0, ctx->stream,
-                       a, in, out,
-                       s.flag_dead, (const double*)ctx->E, (const double*)ctx->Bi);
+    // At most four blocks per CU: latency counts, and two particles per thread
+    // have less of it one after the other (128 x 128 cells, ions at 8 per cell,
+    // 128 blocks: 16.4 us a push, 20.4 with four per thread; 512 x 512, 4 per cell,
+    // 1024 blocks: 79.3 and 82.1; at 2048 blocks they meet).
+    auto go = [&](auto kernel, int threads) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(threads), 0, ctx->stream, a, in, out, s.flag_dead,
+                         (const double*)ctx->E, (const double*)ctx->Bi);
+    };
+    if (nb <= 1024) go(k_mover64<2 * kMoverThreads64>, 2 * kMoverThreads64);
+    else go(k_mover64<kMoverThreads64>, kMoverThreads64);
   }
   LEPIC_HIP(hipGetLastError());
   if (ctx->timing) {

@@ -23,8 +23,9 @@ def push(dom, E, parts, precision, pushes):
 
 
 # segments of the whole species: mixed above 512 through flat loads (more than 25
-# cells a segment) and separate ones, its halves below
-@pytest.mark.parametrize("precision,n1,n2,segs", [(L.MIXED, 200, 100, 602), (L.MIXED, 110, 100, 602)])
+# cells a segment) and separate ones, its halves below; FP64 above and below 1024
+@pytest.mark.parametrize("precision,n1,n2,segs", [(L.MIXED, 200, 100, 602), (L.MIXED, 110, 100, 602),
+                                                  (L.FP64, 200, 100, 1100), (L.FP64, 64, 50, 1026)])
 @pytest.mark.parametrize("Bmode,order", [("map", "sorted"), ("coarse", "random"), ("const", "sorted")])
 def test_forms_agree(precision, n1, n2, segs, Bmode, order):
     dom = S.box_domain(n1, n2, Bmode=Bmode)
