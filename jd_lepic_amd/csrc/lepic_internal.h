@@ -203,7 +203,7 @@ struct lepic_ctx {
   // device scalars
   int64_t* d_counts = nullptr;       // [kMaxSpecies]
   lepic::Tally* d_tally = nullptr;   // [kMaxSpecies][kTallyCopies]
-  uint32_t* d_scan = nullptr;        // block sums of a scan over few blocks
+  uint32_t* d_scan = nullptr;        // block sums of a scan over few blocks, behind d_error's words
   uint32_t* d_segoff = nullptr;      // segment offsets for packing (max nseg_cap)
   int64_t segoff_cap = 0;
   unsigned long long* d_ticket = nullptr;   // monotonic block ticket of the movers

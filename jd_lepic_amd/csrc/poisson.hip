@@ -9,11 +9,12 @@
 //    and a halo of 2S+1 nodes on register strips (mg_strip.h) and performs S
 //    red-black sweeps on it, recomputing the halo redundantly instead of
 //    exchanging it.  After every sweep it writes the tile to that sweep's
-//    state buffer (kRot rotating buffers per level) and its share of the L1
-//    residual.  The exit test of sors.f90:371-377 for those sweeps is taken
-//    at the start of the next launch (or by the kernel that consumes the
-//    level), by every block from the same partial sums in the same order, so
-//    all blocks agree and no atomics or host round trips are needed.  A visit
+//    state buffer (kRot = 9 rotating buffers per level, for a continuation's
+//    up to 8 sweeps) and its share of the L1 residual.  The exit test of
+//    sors.f90:371-377 for those sweeps is taken at the start of the next
+//    launch (or by the kernel that consumes the level), by every block from
+//    the same partial sums in the same order, so all blocks agree and no
+//    atomics or host round trips are needed.  A visit
 //    takes two launches, of which the second mostly finds it finished.  An up
 //    visit prolongs the coarse correction while it loads; the restriction
 //    needs the visit's outcome and is a kernel of its own (k_restrict64).
@@ -498,8 +499,7 @@ __global__ __launch_bounds__(256) void k_add_corr(double* __restrict__ phi, cons
 
 // FP64 L1 residual of phi on the finest level (the reference's definition,
 // sors.f90:348-349 order); in mixed mode it also becomes the FP32 right-hand
-// side of the next correction equation (zero on walls; the outer ones are
-// never written and stay so).  A thread takes two columns of kResidRows rows,
+// side of the next correction equation (zero on walls).  A thread takes two columns of kResidRows rows,
 // all loads before the first use: 1025^2 nodes (22 MB) 6.2 us, 10.4 with a row
 // per block and a node per thread at a time.  k_report sums the blocks'
 // partial sums: letting the block that ends last do it takes as long at 129^2
@@ -1572,8 +1572,6 @@ int launch_tail(lepic_ctx* ctx, bool f32, int k, double eps) {
   return 0;
 }
 
-// One FP64 V-cycle (mg.f90:85-225): levels 1..Ls-1 multi-block, Ls..ng in
-// k_tail; then the end-of-cycle kernel.
 // slot 0: what the host waits for next; slot 1: the starting residual, which it
 // reads when it has something to wait for
 ReportArgs report_args(lepic_ctx* ctx, int slot = 0) {
@@ -1593,6 +1591,8 @@ int launch_report(lepic_ctx* ctx, int nb, int slot = 0) {
   return 0;
 }
 
+// One FP64 V-cycle (mg.f90:85-225): levels 1..Ls-1 multi-block, Ls..ng in one
+// workgroup; then the end-of-cycle kernel.
 int vcycle64(lepic_ctx* ctx, int k, double eps) {
   const int Ls = ctx->Lc;
   const int e_dn = ctx->mg_epoch + 1, e_up = ctx->mg_epoch + 2;
@@ -1691,7 +1691,7 @@ int poisson_setup(lepic_ctx* ctx) {
     }
   }
   // levels with more nodes than the tail threshold run multi-block; the
-  // coarsest level always runs in k_tail (unless ng = 1)
+  // coarsest level always runs in the single workgroup (unless ng = 1)
   const int64_t tail_nodes = ctx->g.mg_tail_nodes > 0 ? ctx->g.mg_tail_nodes : kDefaultTailNodes;
   ctx->Lc = ng;
   for (int l = 1; l <= ng; ++l) {

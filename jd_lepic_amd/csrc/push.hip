@@ -4,7 +4,7 @@
 // One block handles one segment of kChunk = 1024 slots.  Mixed precision:
 // 256 threads, thread t owning the four consecutive slots 4t .. 4t+3 (16-byte
 // vector loads and stores); FP64: 256 threads, thread t owning slots t, t +
-// 256, ...  Survivors are compacted in particle order (part_expmover.f90:
+// 256, ..., or 512 in launches of few blocks.  Survivors are compacted in particle order (part_expmover.f90:
 // 495-503) by a block ballot scan into the same segment of the other particle
 // buffer; the segments' contents in segment order are the species'
 // particles, so no prefix across blocks is needed and blocks never wait for
@@ -507,8 +507,8 @@ __device__ __forceinline__ void deposit_global_runs(const MoverCommon& a, const 
 // thread's particles are all loaded at once, then the field tile (as the mixed
 // mover's; global memory for particles outside it), and everything up to the
 // deposition into the window runs from registers and LDS before the one
-// barrier that the compaction needs.  Four particles per thread at four waves
-// per SIMD: 26.2 M particles on 512 x 512 cells 748 us with E, B and the walls
+// barrier that the compaction needs.  Four particles per thread (two in small
+// launches) at four waves per SIMD: 26.2 M particles on 512 x 512 cells 748 us with E, B and the walls
 // gathered from memory particle by particle, 518 so (4.9 TB/s; two particles
 // per thread 570, one 570).
 template <int BT>

@@ -83,7 +83,7 @@ struct ConvArgs {
 // weight fragment serving the wave's ROWS rows.  The weights are the MFMA's
 // A operand and the pixels its B operand, so a lane ends with 4 consecutive
 // output channels of one pixel and writes them as one 8-byte vector.  CC
-// and ROWS shrink as cout grows so the LDS stays near 64 KB and the
+// and ROWS shrink as cout grows so the LDS stays at 22 to 70 KB and the
 // accumulators in registers, and is 16 where that is all there is (CIN; more
 // blocks per CU); rows are padded by 4 channels against bank
 // conflicts (8-byte aligned rows: the 16-byte loads are stored as halves).
