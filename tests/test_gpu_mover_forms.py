@@ -41,3 +41,20 @@ def test_forms_agree(precision, n1, n2, segs, Bmode, order):
     assert np.array_equal(lost_w, lost_a + lost_b)
     # whole numbers of 2^-42 or 2^-20 of a particle, scaled and rounded once each
     assert np.abs(np_w - (np_a + np_b)).max() <= 3 * 2.0 ** -53 * np_w.max()
+
+
+@pytest.mark.parametrize("precision", [L.FP64, L.MIXED])
+def test_deposition_forms_agree(precision):
+    """513 segments deposit through one window each, their halves through two."""
+    dom = S.box_domain(40, 30, Bmode=None)
+    parts = S.particles(dom, 513 * 1024 - 5, 1.0, seed=1, edge_frac=0.0)
+    parts = parts[np.lexsort((np.floor(parts[:, 0] / dom.h1), np.floor(parts[:, 1] / dom.h2)))]
+    out = []
+    for sel in (slice(None), slice(0, 256 * 1024), slice(256 * 1024, None)):
+        with L.Context(40, 30, dom.h1, dom.h2, dom.dt, [L.Species(-L.QE, L.ME, 1.0, len(parts))], zmax=dom.zmax,
+                       ngrid=dom.ngrid, precision=precision) as ctx:
+            ctx.set_boundary(dom.bcnd, np.zeros((33, 43)))
+            ctx.upload(1, parts[sel])
+            ctx.charge_deposition(1)
+            out.append(ctx.get_grid(L.GRID_NP, 1))
+    assert np.abs(out[0] - (out[1] + out[2])).max() <= 3 * 2.0 ** -53 * out[0].max()
