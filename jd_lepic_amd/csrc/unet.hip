@@ -252,7 +252,10 @@ __device__ __forceinline__ uint2 lds_tr4(const bf16_t* p) {
 // Bound by the latency of a step (one row's loads in flight, two barriers)
 // and by the atomics at its end.  The 14 layers of a 520 x 520 batch of 4:
 // 2300 us with operands gathered pixel by pixel from memory, 830 us staged
-// but with 1024 blocks and a row of x loaded for each dy, 505 us so.
+// but with 1024 blocks and a row of x loaded for each dy, 505 us so.  Small images
+// wait for the first rows' loads and the sums at the end: one wait for two rows,
+// and waves without pixels left out of the sums, take a training step on 40 x 40
+// images from 567 to 530 us (527 gathered), on 72 x 72 from 587 to 557.
 template <int AT, int BT>
 __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
   constexpr int CO = 16 * AT, CI = 16 * BT, PD = CO + kWgPad, PX = CI + kWgPad;
@@ -271,6 +274,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
   const int img = (int)blockIdx.x / (A.nstrip * A.nchunk);
   const int y0 = chunk * A.rows, y1 = min(y0 + A.rows, A.H);
   const int wlim = min(A.sw, A.W - strip * A.sw);        // columns of this strip
+  const int nwv = (wlim + 31) / 32;                      // waves with pixels
   f32x4 acc[9][AT][BT];
 #pragma unroll
   for (int q = 0; q < 9; ++q)
@@ -301,36 +305,36 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
   };
   // pixel of the strip's first column in row y of the image (-1: the border)
   auto pixel = [&](int y) { return px(img, y, strip * A.sw, A.H, A.W); };
-  v4i vd[AT], vx[kRx];
-  auto fetch_x = [&](int y) {
+  v4i vd[AT], vx[kRx], vp[kRx];
+  auto fetch_x = [&](int y, v4i (&v)[kRx]) {
     const auto rx = desc(A.x + (pixel(y) - 1) * A.x_C + A.x_off + ci0, x_end);
 #pragma unroll
     for (int r = 0; r < kRx; ++r)
-      if (t + 256 * r < kXr) vx[r] = __builtin_amdgcn_raw_buffer_load_b128(rx, vo_x[r], 0, 0);
+      if (t + 256 * r < kXr) v[r] = __builtin_amdgcn_raw_buffer_load_b128(rx, vo_x[r], 0, 0);
   };
   auto fetch_dz = [&](int y) {
     const auto rd = desc(A.dz + pixel(y) * A.dz_C + A.dz_off + co0, dz_end);
 #pragma unroll
     for (int r = 0; r < AT; ++r) vd[r] = __builtin_amdgcn_raw_buffer_load_b128(rd, vo_dz[r], 0, 0);
   };
-  auto store_x = [&](int y) {                            // y >= -1
+  auto store_x = [&](int y, const v4i (&v)[kRx]) {       // y >= -1
     bf16_t* d = s_x + ((y + 1) % 3) * kWgRow * PX;
 #pragma unroll
     for (int r = 0; r < kRx; ++r) {
       const int q = t + 256 * r;
-      if (q < kXr) *(v4i*)(d + q / (CI / 8) * PX + 8 * (q % (CI / 8))) = vx[r];
+      if (q < kXr) *(v4i*)(d + q / (CI / 8) * PX + 8 * (q % (CI / 8))) = v[r];
     }
   };
   const int px0 = 32 * wv + 8 * (lane >> 4) + ((lane & 15) >> 2), c0 = 4 * (lane & 3);
-  fetch_x(y0 - 1);
-  store_x(y0 - 1);
-  fetch_x(y0);
-  store_x(y0);
-  fetch_x(y0 + 1);
+  fetch_x(y0 - 1, vx);
+  fetch_x(y0, vp);
+  store_x(y0 - 1, vx);
+  fetch_x(y0 + 1, vx);
   fetch_dz(y0);
+  store_x(y0, vp);
   for (int y = y0; y < y1; ++y) {
     __syncthreads();                                     // the previous row's reads are done
-    store_x(y + 1);
+    store_x(y + 1, vx);
 #pragma unroll
     for (int r = 0; r < AT; ++r) {
       const int q = t + 256 * r;
@@ -338,7 +342,7 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
     }
     __syncthreads();
     if (y + 1 < y1) {
-      fetch_x(y + 2);
+      fetch_x(y + 2, vx);
       fetch_dz(y + 1);
     }
     union Op { uint32_t u[4]; bfv8 f; } a[AT];
@@ -369,7 +373,9 @@ __global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs A) {
   }
   // the waves' sums in wave order, then the block's to the gradient
   float* red = (float*)smem;
+#pragma unroll
   for (int w = 0; w < 4; ++w) {
+    if (w >= nwv) break;                                 // block-uniform
     __syncthreads();
     if (wv != w) continue;
 #pragma unroll
@@ -1125,8 +1131,8 @@ __attribute__((noinline, aligned(64))) void he_normal(Net& N, float* flat) {
 Net* need_net(lepic_ctx* ctx) { return ctx ? ctx->net : nullptr; }
 
 // Waits for the stream when a call ends, whatever its outcome: copies from and to
-// the caller's arrays are under way until then (from pinned memory nothing else
-// waits for them).
+// the caller's arrays are under way until then (also from pageable memory, where
+// a copy of 8.5 MB returns after 118 us and ends after 244).
 struct StreamEnd {
   hipStream_t stream;
   ~StreamEnd() { (void)hipStreamSynchronize(stream); }
